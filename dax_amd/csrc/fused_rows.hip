@@ -69,6 +69,11 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
                       pack_bf16_rne(f[6], f[7]));
 }
 
+// v, or zero where `keep` does not hold, as selects (an assignment under a condition makes v a merge of two paths)
+__device__ __forceinline__ void keep_if(bool keep, uint4& v) {
+    v.x = keep ? v.x : 0u, v.y = keep ? v.y : 0u, v.z = keep ? v.z : 0u, v.w = keep ? v.w : 0u;
+}
+
 // The row stays packed (bf16 pairs) between the passes over it.  Without this the compiler keeps the unpacked
 // fp32 copies of one pass alive for the next one, three times the registers, and the kernel loses half of its
 // wavefronts per SIMD.
@@ -95,7 +100,7 @@ __device__ __forceinline__ float gelu_tanh_f32(float x) {
 // PRE_GELU: y = bf16( gelu_tanh(x) ).
 // Requires k % 8 == 0, 16-byte aligned rows of x (and y), 8-byte aligned rows of q, kfill/8 <= NCH*64.
 // The quantise-only LayerNorm form for rows of up to 12 x 64 chunks holds two rows (the current and the requested
-// next one); rows of whole 512-element columns take ln_rows_exact below instead.
+// next one); what the blocks run, quantise-only rows in groups of four rows and more, takes ln_rows below instead.
 template <int NCH, int FMT, int PRE, bool WRITE_Y>
 __global__ __launch_bounds__(256, (PRE == PRE_LN && NCH <= 12 && !WRITE_Y) ? 2 : 1) void fused_rows_wave(
     const uint16_t* __restrict__ x, int64_t m, int k, int64_t ld_x, const float* __restrict__ mul,
@@ -278,68 +283,121 @@ __global__ __launch_bounds__(256, (PRE == PRE_LN && NCH <= 12 && !WRITE_Y) ? 2 :
     }
 }
 
-// The LayerNorm form for rows of exactly NCOL x 512 elements (every lane owns NCOL whole chunks), quantised bytes only,
-// groups of a multiple of four rows (the four rows of a workgroup pass share the staged vectors): the shapes the DiT
-// blocks have.  Against fused_rows_wave it has no lane predicates and no path that reads the vectors from memory, the row
-// number is a scalar (row base in SGPRs, one lane offset for all chunks), and the current and the requested row swap
-// roles from one pass to the next instead of being copied.  Same arithmetic, same bits.
+// The LayerNorm form, quantised bytes only, for rows of up to NCOL x 512 elements: what the DiT blocks run.  Against
+// fused_rows_wave it has no path that reads the vectors from memory (a row quad lies in one group: quads are counted per
+// group, the last quad of a group may hold fewer than four rows), the row number is a scalar (row base in SGPRs, one lane
+// offset for all chunks), the current and the requested row swap roles from one pass to the next instead of being copied,
+// and only the last chunks of a row can lie beyond its end.  Those are read from the row's last chunk instead (no load
+// sits under a condition) and set to zero after the load.  Same arithmetic, same bits.
+// Bound by HBM and VALU together (3 bytes and about ten VALU instructions per element).  Measured at 9450 x 5120 (one
+// group of 9450 rows, e4m3): 41.5 us in fused_rows_wave, where lane predicates and the path for rows of another group make
+// the compiler wait for the requested row in front of every chunk; 31.9 us here (behind a GEMM, vectors and rows far away:
+// 58.7 -> 38.7 us); 75600 x 5120 213 us = 5.4 TB/s.
+template <int NCOL>
+constexpr int kTailChunks = NCOL > 10 ? 2 : 1;  // chunks per lane that may lie beyond the row (NCOL > 10 exists in steps of two)
+
+// One of the two vectors of a group into LDS, in the lanes' read order: 16-byte pieces, all of a thread's loads in flight
+// before the first is stored.  (A loop over single elements waits for memory once per element and thread: the launch at
+// 9450 x 5120 behind a GEMM, vectors and rows far away, took 48.3 us with it.)
+template <int NCOL>
+__device__ __forceinline__ void stage_vector(float* dst, const float* src, float fill, int k) {
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int N = (NCOL + 1) / 2;
+    f4 r[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int p = i * 256 + threadIdx.x;  // piece: elements 4 p .. 4 p + 3
+        r[i] = f4{fill, fill, fill, fill};
+        if (src && 4 * p < k) r[i] = *reinterpret_cast<const f4*>(src + 4 * p);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int p = i * 256 + threadIdx.x, c = p >> 1;
+        if (4 * p < k) *reinterpret_cast<float4*>(dst + ((((c >> 6) * 2 + (p & 1)) * 64 + (c & 63)) << 2)) = make_float4(r[i].x, r[i].y, r[i].z, r[i].w);
+    }
+}
+
 template <int NCOL, int FMT>
-__global__ __launch_bounds__(256, NCOL <= 10 ? 3 : 2) void ln_rows_exact(const uint16_t* __restrict__ x, int64_t m, int64_t ld_x,
-                                                                          const float* __restrict__ mul, const float* __restrict__ add,
-                                                                          int64_t rows_per_group, float eps, uint8_t* __restrict__ q,
-                                                                          int64_t ld_q, float* __restrict__ scale, float qmax) {
-    constexpr int K = NCOL * 512;
+__global__ __launch_bounds__(256, NCOL <= 3 ? 7 : NCOL <= 4 ? 6 : NCOL <= 5 ? 5 : NCOL <= 10 ? 4 : NCOL <= 12 ? 3 : 2) void ln_rows(const uint16_t* __restrict__ x, int64_t m, int k, int64_t ld_x,
+                                                                   const float* __restrict__ mul, const float* __restrict__ add,
+                                                                   int64_t rows_per_group, int64_t quads_per_group, int64_t quads,
+                                                                   float eps, uint8_t* __restrict__ q, int64_t ld_q, int kfill,
+                                                                   float* __restrict__ scale, float qmax) {
+    constexpr int KP = NCOL * 512, FULL = NCOL - kTailChunks<NCOL>;
     extern __shared__ __attribute__((aligned(16))) float s_vec[];  // mul, then add, in the lanes' read order (as above)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t stride = (int64_t)gridDim.x * 4;
+    const int nch = k >> 3, npad = kfill >> 3;
     int64_t staged = -1;
+    // row of this wavefront in quad `qd` and the quad's group; row -1: the group has no such row, or there is no such quad
+    struct Pos {
+        int64_t row, g;
+    };
+    auto pos_of = [&](int64_t qd) __attribute__((always_inline)) {
+        Pos p{-1, 0};
+        if (qd >= quads) return p;
+        int64_t in = qd;
+        if (quads_per_group < quads) {  // more than one group
+            p.g = qd / quads_per_group;
+            in = qd - p.g * quads_per_group;
+        }
+        in = in * 4 + wave;
+        const int64_t row = p.g * rows_per_group + in;
+        if (in < rows_per_group && row < m) p.row = row;
+        return p;
+    };
     auto load_row = [&](int64_t r, uint4 (&dst)[NCOL]) __attribute__((always_inline)) {
-        const uint4* xr = reinterpret_cast<const uint4*>(x + r * ld_x) + lane;
+        const char* xr = reinterpret_cast<const char*>(x + (r >= 0 ? r : 0) * ld_x);  // (a scalar base and 32-bit lane offsets)
 #pragma unroll
-        for (int i = 0; i < NCOL; ++i) dst[i] = load_stream_16(xr + i * 64);
+        for (int i = 0; i < NCOL; ++i) {
+            const int c = i * 64 + lane;
+            if (i < FULL) dst[i] = load_stream_16(reinterpret_cast<const uint4*>(xr + i * 1024 + (uint32_t)(lane * 16)));
+            else dst[i] = load_stream_16(reinterpret_cast<const uint4*>(xr + (uint32_t)(c < nch ? c : nch - 1) * 16u));
+        }
     };
     // one pass: stage the vectors of the quad's group if they changed, request the row of the next pass, work on `cur`
-    auto pass = [&](int64_t row0, uint4 (&cur)[NCOL], uint4 (&nxt)[NCOL]) __attribute__((always_inline)) {
-        const int64_t g0 = row0 / rows_per_group;
+    Pos at = pos_of(blockIdx.x);
+    auto pass = [&](int64_t qd, uint4 (&cur)[NCOL], uint4 (&nxt)[NCOL]) __attribute__((always_inline)) {
+        const int64_t row = at.row, g0 = at.g;
         if (g0 != staged) {
             __syncthreads();  // everyone is done with the previous group's vectors
-            for (int e = threadIdx.x; e < K; e += 256) {
-                const int c = e >> 3;
-                const int pos = (((((c >> 6) << 1) + ((e >> 2) & 1)) * 64 + (c & 63)) << 2) | (e & 3);
-                s_vec[pos] = mul ? mul[g0 * K + e] : 1.0f;
-                s_vec[K + pos] = add ? add[g0 * K + e] : 0.0f;
-            }
+            stage_vector<NCOL>(s_vec, mul ? mul + g0 * k : nullptr, 1.0f, k);
+            stage_vector<NCOL>(s_vec + KP, add ? add + g0 * k : nullptr, 0.0f, k);
             staged = g0;
             __syncthreads();
         }
-        const int64_t row = row0 + wave;
-        // always requested, beyond the last row that row again: a load under a condition makes the registers of `nxt` a
+        // always requested, without a quad behind this one row 0: a load under a condition makes the registers of `nxt` a
         // merge of two values, which the compiler resolves with copies right behind the loads, i.e. by waiting for them
-        load_row(row + stride < m ? row + stride : m - 1, nxt);
-        if (row >= m) return;
+        at = pos_of(qd + gridDim.x);
+        load_row(at.row, nxt);
+        if (row < 0) return;
 
+#pragma unroll
+        for (int i = FULL; i < NCOL; ++i)
+            keep_if(i * 64 + lane < nch, cur[i]);
         float sum = 0.0f, sq = 0.0f;  // see fused_rows_wave for the statistics
 #pragma unroll
         for (int i = 0; i < NCOL; ++i) dot_sums(cur[i], sum, sq);
         dot_sums_done(sum, sq);
-        float mean = wave_sum_f32(sum) / (float)K;
-        float var = wave_sum_f32(sq) / (float)K - mean * mean;
+        float mean = wave_sum_f32(sum) / (float)k;
+        float var = wave_sum_f32(sq) / (float)k - mean * mean;
         if (!(mean * mean <= 7.0f * var)) {
             float sd = 0.0f, ssq = 0.0f;
 #pragma unroll
             for (int i = 0; i < NCOL; ++i) {
-                float f[8];
-                unpack8(cur[i], f);
+                if (i < FULL || i * 64 + lane < nch) {
+                    float f[8];
+                    unpack8(cur[i], f);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float d = f[e] - mean;
-                    sd += d;
-                    ssq += d * d;
+                    for (int e = 0; e < 8; ++e) {
+                        const float d = f[e] - mean;
+                        sd += d;
+                        ssq += d * d;
+                    }
                 }
             }
-            const float dm = wave_sum_f32(sd) / (float)K;
-            var = wave_sum_f32(ssq) / (float)K - dm * dm;
+            const float dm = wave_sum_f32(sd) / (float)k;
+            var = wave_sum_f32(ssq) / (float)k - dm * dm;
             mean += dm;
         }
         forget_values(cur);
@@ -352,13 +410,14 @@ __global__ __launch_bounds__(256, NCOL <= 10 ? 3 : 2) void ln_rows_exact(const u
             const float* sv = s_vec + (i * 128 + lane) * 4;
             const float4 a0 = *reinterpret_cast<const float4*>(sv);
             const float4 a1 = *reinterpret_cast<const float4*>(sv + 256);
-            const float4 b0 = *reinterpret_cast<const float4*>(sv + K);
-            const float4 b1 = *reinterpret_cast<const float4*>(sv + K + 256);
+            const float4 b0 = *reinterpret_cast<const float4*>(sv + KP);
+            const float4 b1 = *reinterpret_cast<const float4*>(sv + KP + 256);
             const float a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
             const float b[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
 #pragma unroll
             for (int e = 0; e < 8; ++e) f[e] = __builtin_fmaf(__fmul_rn(f[e], rstd), a[e], b[e]);
             cur[i] = pack8(f);
+            if (i >= FULL) keep_if(i * 64 + lane < nch, cur[i]);
         }
         uint32_t mx = 0;
 #pragma unroll
@@ -370,17 +429,21 @@ __global__ __launch_bounds__(256, NCOL <= 10 ? 3 : 2) void ln_rows_exact(const u
         const float inv = 1.0f / s;
         uint2* qr = reinterpret_cast<uint2*>(q + row * ld_q) + lane;
 #pragma unroll
-        for (int i = 0; i < NCOL; ++i) store_stream_8(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv));
+        for (int i = 0; i < NCOL; ++i) {
+            if (i < FULL) store_stream_8(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv));
+            else if (i * 64 + lane < npad)  // (zeros in the padding columns [k, kfill), whatever the scale is)
+                store_stream_8(qr + i * 64, i * 64 + lane < nch ? quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv) : make_uint2(0, 0));
+        }
     };
     uint4 ra[NCOL], rb[NCOL];
-    int64_t row0 = (int64_t)blockIdx.x * 4;
-    load_row(row0 + wave < m ? row0 + wave : m - 1, ra);
-    while (row0 < m) {
-        pass(row0, ra, rb);
-        row0 += stride;
-        if (row0 >= m) break;
-        pass(row0, rb, ra);
-        row0 += stride;
+    int64_t qd = blockIdx.x;
+    load_row(at.row, ra);
+    while (qd < quads) {
+        pass(qd, ra, rb);
+        qd += gridDim.x;
+        if (qd >= quads) break;
+        pass(qd, rb, ra);
+        qd += gridDim.x;
     }
 }
 
@@ -421,20 +484,21 @@ __global__ __launch_bounds__(256) void gelu_rows_exact(const uint16_t* __restric
 }
 
 template <int NCOL, int FMT>
-static int launch_ln_exact(const char* what, const uint16_t* x, int64_t m, int64_t ld_x, const float* mul, const float* add,
-                           int64_t rows_per_group, float eps, uint8_t* q, int64_t ld_q, float* scale, float qmax, int cus,
-                           hipStream_t st) {
+static int launch_ln_rows(const char* what, const uint16_t* x, int64_t m, int64_t k, int64_t ld_x, const float* mul, const float* add,
+                          int64_t rows_per_group, float eps, uint8_t* q, int64_t ld_q, int64_t kfill, float* scale, float qmax, int cus,
+                          hipStream_t st) {
     constexpr size_t lds = (size_t)NCOL * 512 * 8;
     static int per_cu = 0;  // asked once per instantiation; a race between two threads stores the same value twice
     if (per_cu <= 0) {
         int v = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, ln_rows_exact<NCOL, FMT>, 256, lds) != hipSuccess || v <= 0)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, ln_rows<NCOL, FMT>, 256, lds) != hipSuccess || v <= 0)
             return fail(DAXQ_ERR_LAUNCH, "%s: occupancy query failed", what);
         per_cu = v;
     }
-    const int64_t quads = (m + 3) / 4, want = (int64_t)cus * per_cu;
-    hipLaunchKernelGGL((ln_rows_exact<NCOL, FMT>), dim3((unsigned)(quads < want ? quads : want)), dim3(256), lds, st, x, m, ld_x, mul,
-                       add, rows_per_group, eps, q, ld_q, scale, qmax);
+    const int64_t rpg = rows_per_group < m ? rows_per_group : m, qpg = (rpg + 3) / 4, quads = (m / rpg) * qpg + (m % rpg + 3) / 4;
+    const int64_t want = (int64_t)cus * per_cu;
+    hipLaunchKernelGGL((ln_rows<NCOL, FMT>), dim3((unsigned)(quads < want ? quads : want)), dim3(256), lds, st, x, m, (int)k, ld_x, mul,
+                       add, rpg, qpg, quads, eps, q, ld_q, (int)kfill, scale, qmax);
     return check_launch(what);
 }
 
@@ -464,21 +528,26 @@ static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         return fail(DAXQ_ERR_LAUNCH, "%s: cannot read the CU count", what);
     if constexpr (PRE == PRE_LN) {
-        // whole 512-element columns, groups of whole row quads, bytes only: the kernel without predicates
-        if (!yp && k % 512 == 0 && kfill == k && rows_per_group % 4 == 0) {
-            switch (k / 512) {
-#define DAXQ_LN_EXACT(N) \
-    case N: return launch_ln_exact<N, FMT>(what, xp, m, ld_x, mul, add, rows_per_group, eps, qp, ld_q, scale, qmax, cus, st);
-                DAXQ_LN_EXACT(3)
-                DAXQ_LN_EXACT(4)
-                DAXQ_LN_EXACT(6)
-                DAXQ_LN_EXACT(8)
-                DAXQ_LN_EXACT(10)
-                DAXQ_LN_EXACT(12)
-                DAXQ_LN_EXACT(16)
-#undef DAXQ_LN_EXACT
-                default: break;
-            }
+        // bytes only, and groups that hold a few row quads each (or one group): quads are counted per group, so groups of
+        // one to three rows would leave most wavefronts of every quad idle
+        if (!yp && (rows_per_group >= 4 || rows_per_group >= m)) {
+            const int cols = (int)((k + 511) / 512);
+#define DAXQ_LN_ROWS(N) \
+    if (cols <= N) return launch_ln_rows<N, FMT>(what, xp, m, k, ld_x, mul, add, rows_per_group, eps, qp, ld_q, kfill, scale, qmax, cus, st);
+            DAXQ_LN_ROWS(1)
+            DAXQ_LN_ROWS(2)
+            DAXQ_LN_ROWS(3)
+            DAXQ_LN_ROWS(4)
+            DAXQ_LN_ROWS(5)
+            DAXQ_LN_ROWS(6)
+            DAXQ_LN_ROWS(7)
+            DAXQ_LN_ROWS(8)
+            DAXQ_LN_ROWS(9)
+            DAXQ_LN_ROWS(10)
+            DAXQ_LN_ROWS(12)
+            DAXQ_LN_ROWS(14)
+            DAXQ_LN_ROWS(16)
+#undef DAXQ_LN_ROWS
         }
     }
     if constexpr (PRE == PRE_GELU) {

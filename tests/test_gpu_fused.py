@@ -93,6 +93,28 @@ def test_layernorm_multiply_add(ops, fmt, m, k, rpg, vecs):
     assert torch.equal(q2, q) and torch.equal(s2, s)
 
 
+@pytest.mark.parametrize("m,k,rpg", [(9, 8, 9), (23, 504, 5), (9, 520, 4), (6001, 1000, 2999), (30, 1544, 7), (30, 2056, 30), (13, 2560, 6), (30, 3080, 15), (30, 3592, 30),
+                                     (30, 4088, 11), (30, 4608, 9), (4500, 5112, 1501), (21, 5632, 5), (22, 6120, 8), (21, 6656, 21), (22, 7200, 5),
+                                     (21, 7680, 21), (22, 8184, 6)])
+def test_layernorm_rows_of_any_length_and_group(ops, m, k, rpg):
+    """Quantise-only rows of every number of 512-element columns, whole and partial (the last chunks of a lane lie beyond
+    the row), in groups that do not divide into row quads, resident workgroups that make several passes among them: bytes,
+    padding and scales equal those of the kernel that writes y as well.  One row has an offset that sends it through the second statistics
+    pass, one holds a NaN."""
+    g = torch.Generator().manual_seed(m + k)
+    x = (torch.randn(m, k, generator=g) * 2).bfloat16()
+    x[m // 2] += 100
+    x[m - 1, k // 2] = float("nan")
+    groups = -(-m // rpg)
+    mul, add = 1 + 0.2 * torch.randn(groups, k, generator=g), 0.1 * torch.randn(groups, k, generator=g)
+    for fmt in ("i8", "e4m3"):
+        fn = getattr(ops, "layernorm_act_quant_" + fmt)
+        q, s, _ = fn(dev(x), dev(mul), dev(add), rpg, 1e-6, True)
+        q2, s2, _ = fn(dev(x), dev(mul), dev(add), rpg, 1e-6, False)
+        assert torch.isnan(s[m - 1]) and torch.equal(s2[:m - 1], s[:m - 1]) and torch.isnan(s2[m - 1])
+        assert torch.equal(q2[:m - 1], q[:m - 1]) and int(q2[:, k:].to(torch.int32).abs().sum()) == 0
+
+
 @pytest.mark.parametrize("fmt", ["i8", "e4m3"])
 def test_layernorm_rows_with_an_offset(ops, fmt):
     """The variance comes from sum(x^2) / K - mean^2 while the mean is small against the spread and from the second
