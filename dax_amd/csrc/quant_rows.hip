@@ -10,88 +10,248 @@
 //   e4m3:  e4m3fn_rne(clamp(f32(x) / s, -448, 448))         true division
 //   e5m2:  e5m2_rne(clamp(f32(x) / s, -57344, 57344))       true division (activations only)
 //
-// HBM-bound: 2 B read + 1 B written per element.  The fast kernel gives one
-// 64-lane wavefront a whole row, keeps the row in VGPRs between the abs-max pass
-// and the quantise pass (so HBM is read once), reduces the abs-max with packed
-// u16 max + wavefront shuffles, and writes 8 quantised bytes per lane per store.
+// HBM-bound: 2 B read + 1 B written per element.  The row stays in VGPRs between the abs-max pass and the quantise pass,
+// so memory is read once.
+#include <type_traits>
+
 #include "quant_rows.h"
 
 namespace daxq {
 
-// Fast path: one wavefront per row, the row lives in registers.
-// Requires k % 8 == 0, ld_x % 8 == 0, ld_q % 8 == 0, 16-byte aligned x, 8-byte aligned q,
-// and kfill / 8 <= NCH * 64.
-// SCALE_IN: the per-row scale is an input (leaf quantiser) instead of being derived from the row.
-// XT: element type of x, DAXQ_BF16 or DAXQ_F16 (8 elements per 16-byte chunk either way).
-template <int NCH, int FMT, bool ROUND_BF16, bool SCALE_IN, int XT = DAXQ_BF16>
-__global__ __launch_bounds__(256) void quant_rows_wave(const uint16_t* __restrict__ x, int64_t m, int k,
-                                                       int64_t ld_x, uint8_t* __restrict__ q, int64_t ld_q, int kfill,
-                                                       float* __restrict__ scale, float qmax, float eps, int round_x) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= m) return;
-    const uint4* xr = reinterpret_cast<const uint4*>(x + row * ld_x);
-    const int nch = k >> 3;
-    const int npad = kfill >> 3;  // columns [k, kfill) are written as zeros
+// A row is cut into chunks of 8 elements.  Any alignment is taken: the loads and stores are the same 16- and 8-byte
+// instructions whatever the address (gfx950 runs them on any byte address of global memory).
+template <int XT>
+struct Chunk {
+    daxq_v4u w[XT == DAXQ_F32 ? 2 : 1];
+};
 
-    uint4 v[NCH];
-    uint32_t mx = 0;
+template <int XT>
+__device__ __forceinline__ void load_chunk(Chunk<XT>& v, const char* p) {
+    typedef daxq_v4u loose __attribute__((aligned(2)));
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-        const int c = i * 64 + lane;
-        if (c < nch) {
-            v[i] = load_stream_16(xr + c);
+    for (int h = 0; h < (XT == DAXQ_F32 ? 2 : 1); ++h) v.w[h] = __builtin_nontemporal_load(reinterpret_cast<const loose*>(p) + h);
+}
+
+__device__ __forceinline__ void store_chunk(uint8_t* p, uint2 v) {
+    typedef daxq_v2u loose __attribute__((aligned(1)));
+    const daxq_v2u t = {v.x, v.y};
+    __builtin_nontemporal_store(t, reinterpret_cast<loose*>(p));
+}
+
+// running abs-max of chunks: packed 16-bit magnitudes or 32-bit ones
+template <int XT>
+__device__ __forceinline__ uint32_t chunk_amax(uint32_t mx, const Chunk<XT>& v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (XT != DAXQ_F32) {
+            mx = pk_max_u16(mx, v.w[0][i] & 0x7fff7fffu);
         } else {
-            v[i] = make_uint4(0, 0, 0, 0);
+            const uint32_t a = v.w[0][i] & 0x7fffffffu, b = v.w[1][i] & 0x7fffffffu;
+            mx = a > mx ? a : mx;
+            mx = b > mx ? b : mx;
         }
     }
-    float s;
-    if constexpr (SCALE_IN) {
-        s = scale[row];
-    } else {
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            mx = pk_max_u16(mx, v[i].x & 0x7fff7fffu);
-            mx = pk_max_u16(mx, v[i].y & 0x7fff7fffu);
-            mx = pk_max_u16(mx, v[i].z & 0x7fff7fffu);
-            mx = pk_max_u16(mx, v[i].w & 0x7fff7fffu);
-        }
-        uint32_t amax = (mx & 0xffffu) > (mx >> 16) ? (mx & 0xffffu) : (mx >> 16);
-        amax = wave_max_u32(amax);
-        s = scale_from_amax_bits_rt<XT>(amax, qmax, eps, round_x);
-        if (lane == 0) scale[row] = s;
-    }
-    const float inv = 1.0f / s;  // IEEE division, not v_rcp_f32
+    return mx;
+}
+template <int XT>
+__device__ __forceinline__ uint32_t amax_of_lane(uint32_t mx) {
+    if constexpr (XT == DAXQ_F32) return mx;
+    return (mx & 0xffffu) > (mx >> 16) ? (mx & 0xffffu) : (mx >> 16);
+}
 
-    uint2* qr = reinterpret_cast<uint2*>(q + row * ld_q);
-    // Two forms of the store loop.  The fast one, for a bf16 row quantised with its own scale at no more than the
-    // format's maximum: no clamp (dead code there, quant_rows.h), and for FP8 the reciprocal sequence, which is verified
-    // exhaustively for bf16 elements under bf16-rounded scales.  The general one -- fp16 rows, a scale from the caller,
-    // a quant_max beyond the format's maximum, an FP8 row whose scale stays in fp32 -- divides and clamps.  The choice
-    // is uniform over the launch.
-    constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
-    constexpr bool kFastForm = !SCALE_IN && XT == DAXQ_BF16;
-    if (kFastForm && qmax <= kFmtMax && (FMT == 0 || round_x)) {
+template <int XT>
+__device__ __forceinline__ void chunk_values(const Chunk<XT>& v, float (&f)[8]) {
 #pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            const int c = i * 64 + lane;
-            if (c < nch) store_stream_8(qr + c, quant_chunk<FMT, false, XT, false>(v[i], s, inv));
-            else if (c < npad) store_stream_8(qr + c, make_uint2(0, 0));
-        }
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-        const int c = i * 64 + lane;
-        if (c < nch) {
-            store_stream_8(qr + c, quant_chunk<FMT, (FMT != 0), XT>(v[i], s, inv));
-        } else if (c < npad) {
-            store_stream_8(qr + c, make_uint2(0, 0));
-        }
+    for (int i = 0; i < 8; ++i) {
+        if constexpr (XT == DAXQ_F32) f[i] = __uint_as_float(v.w[i >> 2][i & 3]);
+        else if constexpr (XT == DAXQ_BF16) f[i] = __uint_as_float(i & 1 ? v.w[0][i >> 1] & 0xffff0000u : v.w[0][i >> 1] << 16);
+        else f[i] = x_bits_to_f32<XT>(i & 1 ? v.w[0][i >> 1] >> 16 : v.w[0][i >> 1] & 0xffffu);
     }
 }
 
-// General path: any k / alignment / row length / element type; one 256-thread block per row, two passes.
+// How the elements of a row become bytes, one choice per row:
+//   kOwn       a bf16 row under its own scale at no more than the format's maximum: no clamp (dead code there,
+//              quant_rows.h), for FP8 the reciprocal sequence verified exhaustively for bf16 elements under bf16 scales
+//   kDivide    x / s by IEEE division (int8: x * inv), clamped
+//   kNear      FP8 under any other scale: x * inv, whose error is at most 1.5 steps of fp32, rounds to the byte of x / s
+//              unless it lies that close to a value where the byte changes.  Those values, in the normal and the subnormal
+//              range of either format, have at most five significant bits, i.e. zeros in the low 19 bits of the fp32
+//              pattern, so a product within three steps of such a pattern sends its chunk through the division (five
+//              elements in 10^6 under an arbitrary scale; zeros and infinities too).  Measured with a scale from the
+//              caller, 4096 x 5120 e5m2: 18.9 us dividing every element (26 VALU issue slots), 11.4 us here.
+//   kExact     FP8 under a power of two: x * inv is the quotient
+//   kShort     bf16 elements under a bf16 scale from the caller (a per-tensor scale): their quotients hit such values all
+//              the time; the sequence of kOwn, clamped, and the division for chunks that hold an infinity or a NaN
+enum { kOwn = 0, kDivide = 1, kNear = 2, kExact = 3, kShort = 4 };
+
+template <int FMT, int XT>
+__device__ __forceinline__ int form_of_scale(float s) {
+    if constexpr (FMT == 0) return kDivide;
+    const uint32_t b = __float_as_uint(s);
+    if (!(s >= 0x1p-100f && s <= 0x1p100f)) return kDivide;  // (NaN too)
+    if ((b & 0x7fffffu) == 0) return kExact;
+    return XT == DAXQ_BF16 && (b & 0xffffu) == 0 ? kShort : kNear;
+}
+
+template <int FMT, int FORM, int XT>
+__device__ __forceinline__ uint2 quant8(const float (&f)[8], float s, float inv) {
+    uint32_t o[2];
+    if constexpr (FMT == 0) {
+        constexpr bool CLAMP = FORM != kOwn;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {  // byte 0 of each of the four words: three v_perm_b32
+            const uint32_t p01 = __builtin_amdgcn_perm(q_i8_bits<CLAMP>(f[4 * h + 1], inv), q_i8_bits<CLAMP>(f[4 * h], inv), 0x0c0c0400u);
+            const uint32_t p23 = __builtin_amdgcn_perm(q_i8_bits<CLAMP>(f[4 * h + 3], inv), q_i8_bits<CLAMP>(f[4 * h + 2], inv), 0x0c0c0400u);
+            o[h] = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+        }
+    } else {
+        constexpr float kMax = FMT == 2 ? 57344.0f : 448.0f;
+        float v[8];
+        if constexpr (FORM == kNear || FORM == kExact || FORM == kShort) {
+            uint32_t near = 0xffffffffu;
+            bool nan = false;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float q0 = FORM == kShort ? q_f8_pre<FMT, false, false>(f[i], s, inv) : f[i] * inv;
+                if constexpr (FORM == kNear) {
+                    const uint32_t d = (__float_as_uint(q0) << 13) + (3u << 13);
+                    near = d < near ? d : near;
+                }
+                if (XT != DAXQ_BF16 || FORM != kNear) nan |= q0 != q0;  // (a bf16 NaN has zeros in its low bits)
+                v[i] = __builtin_amdgcn_fmed3f(q0, -kMax, kMax);
+            }
+            if (__ballot((FORM == kNear && near <= (6u << 13)) || nan)) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = q_f8_pre<FMT, true>(f[i], s, inv);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = q_f8_pre<FMT, FORM != kOwn, FORM != kOwn>(f[i], s, inv);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int p = cvt_pk_f8<FMT>(v[4 * h], v[4 * h + 1], 0, false);
+            o[h] = (uint32_t)cvt_pk_f8<FMT>(v[4 * h + 2], v[4 * h + 3], p, true);
+        }
+    }
+    return make_uint2(o[0], o[1]);
+}
+
+struct QuantArgs {
+    const char* x;
+    int64_t m, ld_x;  // ld_x in elements
+    int k, kfill;     // columns [k, kfill) of q are written as zeros
+    uint8_t* q;
+    int64_t ld_q;
+    float* scale;           // [m], written (dynamic scale) or read (the caller's)
+    float qmax, eps;        // dynamic scale: divisor and floor,
+    int round_x;            // and whether both are rounded to the element type
+};
+
+// W wavefronts share a row (4 / W rows per workgroup), lane l of wavefront w holding chunks (i W + w) 64 + l.  One
+// wavefront per row for short rows, four for long ones: the chunks of a row then arrive in a quarter of the instructions,
+// which is what a launch of few rows waits for (512 x 5120: 4.1 -> 3.0 us, 17 x 5120 3.5 -> 2.4 us; a wavefront alone on
+// its SIMD issues one instruction in eight cycles), and a launch of many keeps more, smaller pieces of work in flight
+// (9450 x 5120: 25.9 -> 23.9 us = 6.1 TB/s, 75600 x 5120 186.2 -> 180.3 us = 6.4 TB/s, x 13824 543.8 -> 529.3 us); at
+// K = 1536 the barrier costs more than it returns (6.06 against 4.78 TB/s).  fp32 rows, and rows of any length or
+// address, against one workgroup per row that read them twice, element by element: 4096 x 5120 fp32 43.9 -> 19.7 us,
+// 2900 x 1001 bf16 6.1 -> 3.7 us.
+// SCALE_IN: the per-row scale is an input (leaf quantiser) instead of being derived from the row.
+template <int NCH, int W, int FMT, bool SCALE_IN, int XT>
+__global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
+    constexpr int XB = XT == DAXQ_F32 ? 4 : 2;
+    __shared__ uint32_t s_max[4];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row0 = (int64_t)blockIdx.x * (4 / W) + wave / W;
+    if (W == 1 && row0 >= a.m) return;
+    const int64_t row = row0 < a.m ? row0 : a.m - 1;  // (rows beyond the last: the wavefront still reaches the barrier)
+    const int part = wave % W, nch = a.k >> 3, npad = a.kfill >> 3;
+    const char* xr = a.x + row * a.ld_x * XB;
+    // what whole chunks do not cover -- the columns behind the last of them, and a width or fill that is no multiple of
+    // 8 -- is one element per lane of the row's first wavefront
+    const bool ragged = ((a.k | a.kfill) & 7) != 0;
+
+    Chunk<XT> v[NCH];
+    if (nch > 0) {
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            const int c = (i * W + part) * 64 + lane;
+            // (beyond the row: its last chunk once more, which leaves the maximum as it is and is not stored)
+            load_chunk<XT>(v[i], xr + (uint32_t)(c < nch ? c : nch - 1) * (8u * XB));
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) v[i] = Chunk<XT>{};
+    }
+    uint32_t tail = 0;
+    if (ragged && part == 0 && lane < (a.k & 7)) {
+        if constexpr (XT == DAXQ_F32) tail = reinterpret_cast<const uint32_t*>(xr)[nch * 8 + lane];
+        else tail = reinterpret_cast<const uint16_t*>(xr)[nch * 8 + lane];
+    }
+    float s;
+    if constexpr (SCALE_IN) {
+        s = a.scale[row];
+    } else {
+        uint32_t mx = 0;
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) mx = chunk_amax<XT>(mx, v[i]);
+        mx = amax_of_lane<XT>(mx);
+        const uint32_t t = tail & (XT == DAXQ_F32 ? 0x7fffffffu : 0x7fffu);
+        uint32_t amax = wave_max_u32(t > mx ? t : mx);
+        if constexpr (W > 1) {
+            if (lane == 0) s_max[wave] = amax;
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                const uint32_t o = s_max[wave / W * W + i];
+                amax = o > amax ? o : amax;
+            }
+        }
+        s = scale_from_amax_bits_rt<XT>(amax, a.qmax, a.eps, a.round_x);
+        if (part == 0 && lane == 0) a.scale[row] = s;
+    }
+    if (W > 1 && row0 >= a.m) return;
+    const float inv = 1.0f / s;  // IEEE division, not v_rcp_f32
+
+    uint8_t* qr = a.q + row * a.ld_q;
+    auto store = [&](auto FORM) __attribute__((always_inline)) {
+        constexpr int F = decltype(FORM)::value;
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            const int c = (i * W + part) * 64 + lane;
+            float f[8];
+            chunk_values<XT>(v[i], f);
+            const uint2 o = quant8<FMT, F, XT>(f, s, inv);
+            if (c < nch) store_chunk(qr + (uint32_t)c * 8u, o);
+            else if (!ragged && c < npad) store_chunk(qr + (uint32_t)c * 8u, make_uint2(0, 0));
+        }
+    };
+    constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
+    constexpr bool kOwnForm = !SCALE_IN && XT == DAXQ_BF16;
+    if (kOwnForm && a.qmax <= kFmtMax && (FMT == 0 || a.round_x)) {
+        store(std::integral_constant<int, kOwn>{});
+    } else if constexpr (FMT == 0) {
+        store(std::integral_constant<int, kDivide>{});
+    } else {
+        // (fp16 rows under their own fp16 scale: both have few significant bits, the products hit the values that need the
+        // division all the time)
+        const int form = XT == DAXQ_F16 && !SCALE_IN && a.round_x ? kDivide : form_of_scale<FMT, XT>(s);
+        if (form == kNear) store(std::integral_constant<int, kNear>{});
+        else if (XT == DAXQ_BF16 && form == kShort) store(std::integral_constant<int, XT == DAXQ_BF16 ? kShort : kDivide>{});
+        else if (form == kExact) store(std::integral_constant<int, kExact>{});
+        else store(std::integral_constant<int, kDivide>{});
+    }
+    if (ragged && part == 0) {
+        const float f = x_bits_to_f32<XT>(tail);
+        uint8_t o;
+        if constexpr (FMT == 0) o = (uint8_t)q_i8_bits(f, inv);
+        else o = (uint8_t)cvt_pk_f8<FMT>(q_f8_pre<FMT, true>(f, s, inv), 0.0f, 0, false);
+        for (int c = nch * 8 + lane; c < a.kfill; c += 64) qr[c] = c < a.k ? o : 0;
+    }
+}
+
+// Rows too long for the registers of four wavefronts: one 256-thread workgroup per row, two passes over memory.
 template <int XT>
 struct XWord {
     typedef uint16_t type;
@@ -101,7 +261,7 @@ struct XWord<DAXQ_F32> {
     typedef uint32_t type;
 };
 
-template <int FMT, bool ROUND_BF16, bool SCALE_IN, int XT = DAXQ_BF16>
+template <int FMT, bool SCALE_IN, int XT = DAXQ_BF16>
 __global__ __launch_bounds__(256) void quant_rows_block(const void* __restrict__ xv, int64_t m, int64_t k,
                                                         int64_t ld_x, uint8_t* __restrict__ q, int64_t ld_q, int64_t kfill,
                                                         float* __restrict__ scale, float qmax, float eps, int round_x) {
@@ -148,7 +308,7 @@ __global__ __launch_bounds__(256) void quant_rows_block(const void* __restrict__
     }
 }
 
-template <int FMT, bool ROUND_BF16, bool SCALE_IN, int XT>
+template <int FMT, bool SCALE_IN, int XT>
 static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q, float* scale,
                                float qmax, hipStream_t st, float eps, int round_x) {
     constexpr int XB = XT == DAXQ_F32 ? 4 : 2;
@@ -159,56 +319,58 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
     const int64_t kfill = fill_width(k, ld_q);
     if (((uintptr_t)x & (XB - 1)) != 0 || ((uintptr_t)scale & 3) != 0) return fail(DAXQ_ERR_ALIGN, "quant_rows: x must be element aligned and scale 4-byte aligned");
     uint8_t* qp = static_cast<uint8_t*>(q);
-    if constexpr (XT != DAXQ_F32) {
-        const uint16_t* xp = static_cast<const uint16_t*>(x);
-        const bool vec_ok = (k % 8 == 0) && (ld_x % 8 == 0) && (ld_q % 8 == 0) && (((uintptr_t)x & 15) == 0) &&
-                            (((uintptr_t)q & 7) == 0) && (kfill / 8 <= 36 * 64) && (m <= (int64_t)4 * 0x7fffffff);
-        if (vec_ok) {
-            const int nchunks = (int)((kfill / 8 + 63) / 64);
-            const dim3 grid((unsigned)((m + 3) / 4)), block(256);
-#define DAXQ_Q_CASE(N)                                                                                      \
-    if (nchunks <= N) {                                                                                     \
-        hipLaunchKernelGGL((quant_rows_wave<N, FMT, ROUND_BF16, SCALE_IN, XT>), grid, block, 0, st, xp, m, (int)k, ld_x, qp, \
-                           ld_q, (int)kfill, scale, qmax, eps, round_x);                                              \
-        return check_launch("quant_rows_wave");                                                             \
+    if (kfill <= 36 * 512 && m <= 0x7fffffff) {
+        QuantArgs a{static_cast<const char*>(x), m, ld_x, (int)k, (int)kfill, qp, ld_q, scale, qmax, eps, round_x};
+        const int cols = (int)((kfill + 511) / 512);
+#define DAXQ_Q_CASE(N, W)                                                                                                  \
+    if (cols <= N * W) {                                                                                                   \
+        hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT>), dim3((unsigned)((m + 4 / W - 1) / (4 / W))), dim3(256), 0, st, a); \
+        return check_launch("quant_rows");                                                                                 \
     }
-            DAXQ_Q_CASE(2)
-            DAXQ_Q_CASE(4)
-            DAXQ_Q_CASE(8)
-            DAXQ_Q_CASE(12)
-            DAXQ_Q_CASE(20)
-            DAXQ_Q_CASE(28)
-            DAXQ_Q_CASE(36)
-#undef DAXQ_Q_CASE
+        DAXQ_Q_CASE(1, 1)
+        DAXQ_Q_CASE(2, 1)
+        if constexpr (XT != DAXQ_F32) {
+            DAXQ_Q_CASE(3, 1)
+            DAXQ_Q_CASE(4, 1)
+            DAXQ_Q_CASE(3, 2)
         }
+        DAXQ_Q_CASE(2, 4)
+        DAXQ_Q_CASE(3, 4)
+        if constexpr (XT == DAXQ_BF16) {
+            DAXQ_Q_CASE(4, 4)
+        }
+        DAXQ_Q_CASE(5, 4)
+        DAXQ_Q_CASE(7, 4)
+        DAXQ_Q_CASE(9, 4)
+#undef DAXQ_Q_CASE
     }
-    if (m > 0x7fffffff) return fail(DAXQ_ERR_ARG, "quant_rows: too many rows for the general kernel");
-    hipLaunchKernelGGL((quant_rows_block<FMT, ROUND_BF16, SCALE_IN, XT>), dim3((unsigned)m), dim3(256), 0, st, x, m, k, ld_x, qp,
+    if (m > 0x7fffffff) return fail(DAXQ_ERR_ARG, "quant_rows: too many rows");
+    hipLaunchKernelGGL((quant_rows_block<FMT, SCALE_IN, XT>), dim3((unsigned)m), dim3(256), 0, st, x, m, k, ld_x, qp,
                        ld_q, kfill, scale, qmax, eps, round_x);
     return check_launch("quant_rows_block");
 }
 
 // eps, round_x: floor and rounding of a dynamic scale (scale_from_amax_bits_rt); unused when the scale is an input
-template <int FMT, bool ROUND_BF16, bool SCALE_IN>
+template <int FMT, bool SCALE_IN>
 static int launch_quant_rows(const void* x, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q, float* scale,
                              float qmax, hipStream_t st, int x_dtype = DAXQ_BF16, float eps = kEps, int round_x = 1) {
     if (!SCALE_IN && (!(qmax > 0.0f) || !(eps >= 0.0f))) return fail(DAXQ_ERR_ARG, "quant_rows: quant_max must be positive and eps not negative");
     switch (x_dtype) {
-        case DAXQ_BF16: return launch_quant_rows_t<FMT, ROUND_BF16, SCALE_IN, DAXQ_BF16>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x);
-        case DAXQ_F16: return launch_quant_rows_t<FMT, ROUND_BF16, SCALE_IN, DAXQ_F16>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x);
-        case DAXQ_F32: return launch_quant_rows_t<FMT, ROUND_BF16, SCALE_IN, DAXQ_F32>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x);
+        case DAXQ_BF16: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_BF16>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x);
+        case DAXQ_F16: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_F16>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x);
+        case DAXQ_F32: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_F32>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x);
         default: return fail(DAXQ_ERR_ARG, "quant_rows: unknown element type %d", x_dtype);
     }
 }
 
 // qmax <= 0: the format's own maximum
-template <bool ROUND_BF16, bool SCALE_IN>
+template <bool SCALE_IN>
 static int launch_quant_rows_fmt(int q_fmt, const void* x, int x_dtype, int64_t m, int64_t k, int64_t ld_x, void* q,
                                  int64_t ld_q, float* scale, hipStream_t st, float qmax = 0.0f, float eps = kEps, int round_x = 1) {
     switch (q_fmt) {
-        case DAXQ_FMT_I8: return launch_quant_rows<0, ROUND_BF16, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 127.0f, st, x_dtype, eps, round_x);
-        case DAXQ_FMT_E4M3: return launch_quant_rows<1, ROUND_BF16, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 448.0f, st, x_dtype, eps, round_x);
-        case DAXQ_FMT_E5M2: return launch_quant_rows<2, ROUND_BF16, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 57344.0f, st, x_dtype, eps, round_x);
+        case DAXQ_FMT_I8: return launch_quant_rows<0, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 127.0f, st, x_dtype, eps, round_x);
+        case DAXQ_FMT_E4M3: return launch_quant_rows<1, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 448.0f, st, x_dtype, eps, round_x);
+        case DAXQ_FMT_E5M2: return launch_quant_rows<2, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 57344.0f, st, x_dtype, eps, round_x);
         default: return fail(DAXQ_ERR_ARG, "quant_rows: unknown quantised format %d", q_fmt);
     }
 }
@@ -260,34 +422,34 @@ extern "C" {
 
 int daxq_act_quant_i8(const void* x, int64_t m, int64_t k, int64_t ld_x, int8_t* q, int64_t ld_q, float* scale,
                       daxq_stream_t stream) {
-    return daxq::launch_quant_rows<0, true, false>(x, m, k, ld_x, q, ld_q, scale, 127.0f, (hipStream_t)stream);
+    return daxq::launch_quant_rows<0, false>(x, m, k, ld_x, q, ld_q, scale, 127.0f, (hipStream_t)stream);
 }
 
 int daxq_act_quant_e4m3(const void* x, int64_t m, int64_t k, int64_t ld_x, uint8_t* q, int64_t ld_q, float* scale,
                         daxq_stream_t stream) {
-    return daxq::launch_quant_rows<1, true, false>(x, m, k, ld_x, q, ld_q, scale, 448.0f, (hipStream_t)stream);
+    return daxq::launch_quant_rows<1, false>(x, m, k, ld_x, q, ld_q, scale, 448.0f, (hipStream_t)stream);
 }
 
 int daxq_act_quant_e5m2(const void* x, int64_t m, int64_t k, int64_t ld_x, uint8_t* q, int64_t ld_q, float* scale,
                         daxq_stream_t stream) {
-    return daxq::launch_quant_rows<2, true, false>(x, m, k, ld_x, q, ld_q, scale, 57344.0f, (hipStream_t)stream);
+    return daxq::launch_quant_rows<2, false>(x, m, k, ld_x, q, ld_q, scale, 57344.0f, (hipStream_t)stream);
 }
 
 int daxq_quantize_rows_i8(const void* x, int64_t m, int64_t k, int64_t ld_x, const float* scale, int8_t* q,
                           int64_t ld_q, daxq_stream_t stream) {
-    return daxq::launch_quant_rows<0, false, true>(x, m, k, ld_x, q, ld_q, const_cast<float*>(scale), 127.0f,
+    return daxq::launch_quant_rows<0, true>(x, m, k, ld_x, q, ld_q, const_cast<float*>(scale), 127.0f,
                                                        (hipStream_t)stream);
 }
 
 int daxq_quantize_rows_e4m3(const void* x, int64_t m, int64_t k, int64_t ld_x, const float* scale, uint8_t* q,
                             int64_t ld_q, daxq_stream_t stream) {
-    return daxq::launch_quant_rows<1, false, true>(x, m, k, ld_x, q, ld_q, const_cast<float*>(scale), 448.0f,
+    return daxq::launch_quant_rows<1, true>(x, m, k, ld_x, q, ld_q, const_cast<float*>(scale), 448.0f,
                                                       (hipStream_t)stream);
 }
 
 int daxq_quantize_rows_e5m2(const void* x, int64_t m, int64_t k, int64_t ld_x, const float* scale, uint8_t* q,
                             int64_t ld_q, daxq_stream_t stream) {
-    return daxq::launch_quant_rows<2, false, true>(x, m, k, ld_x, q, ld_q, const_cast<float*>(scale), 57344.0f,
+    return daxq::launch_quant_rows<2, true>(x, m, k, ld_x, q, ld_q, const_cast<float*>(scale), 57344.0f,
                                                       (hipStream_t)stream);
 }
 
@@ -314,7 +476,7 @@ int daxq_row_minmax(const void* x, int64_t m, int64_t k, int64_t ld_x, float* mi
 
 int daxq_act_quant_rows(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q,
                         float* scale, daxq_stream_t stream) {
-    return daxq::launch_quant_rows_fmt<true, false>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, scale, (hipStream_t)stream);
+    return daxq::launch_quant_rows_fmt<false>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, scale, (hipStream_t)stream);
 }
 
 int daxq_act_quant_rows_ex(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q,
@@ -322,13 +484,13 @@ int daxq_act_quant_rows_ex(const void* x, int x_dtype, int q_fmt, int64_t m, int
     if (scale_round != DAXQ_SCALE_ROUND_X && scale_round != DAXQ_SCALE_ROUND_NONE)
         return daxq::fail(DAXQ_ERR_ARG, "act_quant_rows_ex: unknown scale rounding %d", scale_round);
     if (!(quant_max > 0.0f)) return daxq::fail(DAXQ_ERR_ARG, "act_quant_rows_ex: quant_max must be positive");
-    return daxq::launch_quant_rows_fmt<true, false>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, scale, (hipStream_t)stream, quant_max,
+    return daxq::launch_quant_rows_fmt<false>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, scale, (hipStream_t)stream, quant_max,
                                                     eps, scale_round == DAXQ_SCALE_ROUND_X);
 }
 
 int daxq_quantize_rows(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, const float* scale,
                        void* q, int64_t ld_q, daxq_stream_t stream) {
-    return daxq::launch_quant_rows_fmt<false, true>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, const_cast<float*>(scale),
+    return daxq::launch_quant_rows_fmt<true>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, const_cast<float*>(scale),
                                                     (hipStream_t)stream);
 }
 

@@ -1,0 +1,86 @@
+"""The row quantiser at the sizes where it can go wrong: every split of a row over wavefronts, whole and partial chunks,
+rows that start on odd addresses, the three element types; and the FP8 bytes it takes without dividing."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import daxq_oracle as O
+from tests.util import FINITE_BF16, from_bits
+
+pytestmark = pytest.mark.gpu
+
+FP8 = {"e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}
+
+
+@pytest.fixture(scope="module")
+def ops():
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    import dax_amd.ops as ops
+
+    return ops
+
+
+def _bytes(t):
+    return t.cpu().contiguous().view(torch.uint8).numpy()
+
+
+# one row length on either side of every change of the kernel's split, then lengths that are no multiple of a chunk
+LENGTHS = [1, 7, 8, 9, 504, 512, 520, 1023, 1024, 1032, 1536, 1544, 2041, 2048, 2056, 3072, 3080, 4096, 4104, 6143, 6144,
+           6152, 8192, 8200, 10240, 10248, 14336, 14344, 18303, 18432, 18440]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k", LENGTHS)
+def test_rows_of_any_length(ops, dtype, k):
+    g = torch.Generator().manual_seed(k)
+    m = 6
+    wide = torch.randn(m, k + 3, generator=g) * torch.tensor([1e-4, 1.0, 30.0, 1.0, 0.0, 3.0])[:, None]
+    for x in (wide[:, :k].to(dtype).contiguous(), wide.to(dtype)[:, 3:]):   # the second: rows that start anywhere
+        xd = torch.empty(m, x.stride(0), dtype=dtype, device="cuda")[:, :k]
+        xd.copy_(x)
+        for fmt in ("i8", "e4m3"):
+            target = torch.int8 if fmt == "i8" else FP8[fmt]
+            qo, so = O.dynamic_quantize(x.contiguous(), (1, k), target, ops.QMAX[fmt], ops.EPS_F32, torch.float32)
+            q, s = getattr(ops, "act_quant_" + fmt)(xd)
+            assert torch.equal(s.cpu(), so.view(-1))
+            np.testing.assert_array_equal(_bytes(q[:, :k]), _bytes(qo))
+            assert not q[:, k:].any()
+            scale = so.view(-1) * 1.37                                      # the leaf quantiser, rows without padding
+            ql = getattr(ops, "quantize_rows_" + fmt)(xd, scale.to("cuda"))
+            ref = O.quantize_to_int8(x, scale[:, None]) if fmt == "i8" else O.quantize_to_fp8(x, scale[:, None], target)
+            np.testing.assert_array_equal(_bytes(ql), _bytes(ref))
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+def test_fp8_bytes_without_a_division(ops, fmt):
+    """FP8 under a scale of any 24 significant bits: x * (1 / s) decides the byte unless it lies within a few fp32 steps of a value
+    where the byte changes.  Every finite bf16 element (zeros, subnormals and values beyond the clamp among them) under
+    arbitrary scales, scales with few significant bits, powers of two, scales with all bits set and scales at and beyond the
+    ends of the range in which the product is used; infinities and NaN; then fp32 elements on and next to the values
+    where bytes change."""
+    g = torch.Generator().manual_seed(5)
+    scales = torch.cat([torch.rand(40, generator=g) * 10 ** (torch.rand(40, generator=g) * 12 - 6),
+                        torch.tensor([1.0, 0.5, 2.0 ** -23, 2.0 ** -99, 2.0 ** 99, 2.0 ** -120, 2.0 ** 120, 0.75, 1.25, 3.0, 0.0625 * 7,
+                                      float(np.float32(2) - np.float32(2) ** -23), float(np.float32(1) - np.float32(2) ** -24), 1e-38])])
+    x = torch.cat([from_bits(FINITE_BF16), torch.tensor([float("inf"), -float("inf"), float("nan")], dtype=torch.bfloat16),
+                   torch.zeros(5, dtype=torch.bfloat16)])
+    for xs in (x[:32768], x[32768:]):
+        for lo in range(0, xs.numel(), 8192):
+            row = xs[lo:lo + 8192]
+            rows = row.expand(scales.numel(), -1).contiguous()
+            q = getattr(ops, "quantize_rows_" + fmt)(rows.to("cuda"), scales.to("cuda"))
+            ref = O.quantize_to_fp8(rows, scales[:, None], FP8[fmt])
+            nan = torch.isnan(rows.float() / scales[:, None])
+            got = q.cpu()
+            assert torch.equal(got[~nan], ref.view(torch.uint8)[~nan])
+            assert bool(torch.isnan(got.view(FP8[fmt]).float()[nan]).all())
+    # fp32 elements: values t at and half-way between the format's, times s, and their fp32 neighbours
+    t = torch.arange(0, 127 if fmt == "e4m3" else 124, dtype=torch.uint8).view(FP8[fmt]).float()
+    t = torch.cat([t, (t[1:] + t[:-1]) / 2]).double()
+    for s in (0.1, 0.003, 1.0 / 3.0, 7.7, 1.0):
+        c = (t * s).float().view(torch.int32)[:, None] + torch.arange(-4, 5)
+        xf = c.clamp_min(0).to(torch.int32).view(torch.float32).reshape(1, -1)
+        xf = torch.cat([xf, -xf], 1)
+        sc = torch.tensor([s])
+        q = getattr(ops, "quantize_rows_" + fmt)(xf.to("cuda"), sc.to("cuda"))
+        assert torch.equal(q.cpu(), O.quantize_to_fp8(xf, sc[:, None], FP8[fmt]).view(torch.uint8))
