@@ -40,6 +40,8 @@ SIGNATURES = {
     "daxq_tensor_scale": [_P, _P, _I64, _F32, _F32, _INT, _P, _P, _I64, _P],
     "daxq_tensor_minmax_update": [_P, _P, _I64, _P, _P, _P],
     "daxq_broadcast_f32": [_P, _P, _I64, _P],
+    "daxq_act_quant_tensor": [_P, _INT, _INT, _I64, _I64, _I64, _P, _I64, _P, _P, _P, _F32, _F32, _INT, _P],
+    "daxq_quantize_tensor": [_P, _INT, _INT, _I64, _I64, _I64, _P, _P, _I64, _P, _P],
     "daxq_row_minmax": [_P, _I64, _I64, _I64, _P, _P, _P],
     "daxq_row_minmax_t": [_P, _INT, _I64, _I64, _I64, _P, _P, _P],
     "daxq_act_quant_rows": [_P, _INT, _INT, _I64, _I64, _I64, _P, _I64, _P, _P],

@@ -143,10 +143,15 @@ struct QuantArgs {
     int k, kfill;     // columns [k, kfill) of q are written as zeros
     uint8_t* q;
     int64_t ld_q;
-    float* scale;           // [m], written (dynamic scale) or read (the caller's)
-    float qmax, eps;        // dynamic scale: divisor and floor,
-    int round_x;            // and whether both are rounded to the element type
+    float* scale;             // [m]: the scale of every row, written; null = not wanted
+    const float* scale_in;    // SCALE_IN: the caller's scale, of row r at [r * scale_stride]
+    int scale_stride;         // 1, or 0: one scale for the tensor
+    const uint32_t* partials; // dynamic scale of the whole tensor: kPartials abs-max patterns, their maximum is the tensor's; null = per row
+    float* scale1;            // ... and where that one scale goes besides (or null)
+    float qmax, eps;          // dynamic scale: divisor and floor,
+    int round_x;              // and whether both are rounded to the element type
 };
+constexpr int kPartials = 256;  // workgroups of tensor_amax_kernel, one per CU
 
 // W wavefronts share a row (4 / W rows per workgroup), lane l of wavefront w holding chunks (i W + w) 64 + l.  One
 // wavefront per row for short rows, four for long ones: the chunks of a row then arrive in a quarter of the instructions,
@@ -191,15 +196,23 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
     }
     float s;
     if constexpr (SCALE_IN) {
-        s = a.scale[row];
+        s = a.scale_in[row * a.scale_stride];
+        if (a.scale && part == 0 && lane == 0) a.scale[row] = s;
     } else {
         uint32_t mx = 0;
+        if (a.partials) {  // every wavefront finds the tensor's maximum in 1 KB of L2 while its row arrives
+            const uint4 p = reinterpret_cast<const uint4*>(a.partials)[lane];
+            const uint32_t lo = p.x > p.y ? p.x : p.y, hi = p.z > p.w ? p.z : p.w;
+            mx = lo > hi ? lo : hi;
+        } else {
 #pragma unroll
-        for (int i = 0; i < NCH; ++i) mx = chunk_amax<XT>(mx, v[i]);
-        mx = amax_of_lane<XT>(mx);
-        const uint32_t t = tail & (XT == DAXQ_F32 ? 0x7fffffffu : 0x7fffu);
-        uint32_t amax = wave_max_u32(t > mx ? t : mx);
-        if constexpr (W > 1) {
+            for (int i = 0; i < NCH; ++i) mx = chunk_amax<XT>(mx, v[i]);
+            mx = amax_of_lane<XT>(mx);
+            const uint32_t t = tail & (XT == DAXQ_F32 ? 0x7fffffffu : 0x7fffu);
+            mx = t > mx ? t : mx;
+        }
+        uint32_t amax = wave_max_u32(mx);
+        if (W > 1 && !a.partials) {
             if (lane == 0) s_max[wave] = amax;
             __syncthreads();
 #pragma unroll
@@ -209,7 +222,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
             }
         }
         s = scale_from_amax_bits_rt<XT>(amax, a.qmax, a.eps, a.round_x);
-        if (part == 0 && lane == 0) a.scale[row] = s;
+        if (part == 0 && lane == 0) {
+            a.scale[row] = s;
+            if (a.scale1 && row == 0) a.scale1[0] = s;
+        }
     }
     if (W > 1 && row0 >= a.m) return;
     const float inv = 1.0f / s;  // IEEE division, not v_rcp_f32
@@ -308,9 +324,17 @@ __global__ __launch_bounds__(256) void quant_rows_block(const void* __restrict__
     }
 }
 
+// One scale for the whole tensor instead of one per row (QuantArgs)
+struct TensorScale {
+    bool one_scale = false;              // the caller's scale is one value; scale_rows: where it goes once per row (or null)
+    float* scale_rows = nullptr;
+    const uint32_t* partials = nullptr;  // the scale comes from the tensor's abs-max; scale1: where it goes besides (or null)
+    float* scale1 = nullptr;
+};
+
 template <int FMT, bool SCALE_IN, int XT>
 static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q, float* scale,
-                               float qmax, hipStream_t st, float eps, int round_x) {
+                               float qmax, hipStream_t st, float eps, int round_x, const TensorScale& t) {
     constexpr int XB = XT == DAXQ_F32 ? 4 : 2;
     if (m < 0 || k <= 0 || ld_x < k || ld_q < k) return fail(DAXQ_ERR_ARG, "quant_rows: bad shape m=%lld k=%lld ld_x=%lld ld_q=%lld",
                                                                (long long)m, (long long)k, (long long)ld_x, (long long)ld_q);
@@ -320,7 +344,8 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
     if (((uintptr_t)x & (XB - 1)) != 0 || ((uintptr_t)scale & 3) != 0) return fail(DAXQ_ERR_ALIGN, "quant_rows: x must be element aligned and scale 4-byte aligned");
     uint8_t* qp = static_cast<uint8_t*>(q);
     if (kfill <= 36 * 512 && m <= 0x7fffffff) {
-        QuantArgs a{static_cast<const char*>(x), m, ld_x, (int)k, (int)kfill, qp, ld_q, scale, qmax, eps, round_x};
+        QuantArgs a{static_cast<const char*>(x), m, ld_x, (int)k, (int)kfill, qp, ld_q, SCALE_IN ? t.scale_rows : scale, scale,
+                    t.one_scale ? 0 : 1, t.partials, t.scale1, qmax, eps, round_x};
         const int cols = (int)((kfill + 511) / 512);
 #define DAXQ_Q_CASE(N, W)                                                                                                  \
     if (cols <= N * W) {                                                                                                   \
@@ -344,6 +369,7 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
         DAXQ_Q_CASE(9, 4)
 #undef DAXQ_Q_CASE
     }
+    if (t.one_scale || t.partials) return fail(DAXQ_ERR_ARG, "quant_rows: one scale for the tensor is taken for rows of at most %d columns", 36 * 512);
     if (m > 0x7fffffff) return fail(DAXQ_ERR_ARG, "quant_rows: too many rows");
     hipLaunchKernelGGL((quant_rows_block<FMT, SCALE_IN, XT>), dim3((unsigned)m), dim3(256), 0, st, x, m, k, ld_x, qp,
                        ld_q, kfill, scale, qmax, eps, round_x);
@@ -353,12 +379,12 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
 // eps, round_x: floor and rounding of a dynamic scale (scale_from_amax_bits_rt); unused when the scale is an input
 template <int FMT, bool SCALE_IN>
 static int launch_quant_rows(const void* x, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q, float* scale,
-                             float qmax, hipStream_t st, int x_dtype = DAXQ_BF16, float eps = kEps, int round_x = 1) {
+                             float qmax, hipStream_t st, int x_dtype = DAXQ_BF16, float eps = kEps, int round_x = 1, const TensorScale& t = {}) {
     if (!SCALE_IN && (!(qmax > 0.0f) || !(eps >= 0.0f))) return fail(DAXQ_ERR_ARG, "quant_rows: quant_max must be positive and eps not negative");
     switch (x_dtype) {
-        case DAXQ_BF16: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_BF16>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x);
-        case DAXQ_F16: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_F16>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x);
-        case DAXQ_F32: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_F32>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x);
+        case DAXQ_BF16: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_BF16>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x, t);
+        case DAXQ_F16: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_F16>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x, t);
+        case DAXQ_F32: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_F32>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x, t);
         default: return fail(DAXQ_ERR_ARG, "quant_rows: unknown element type %d", x_dtype);
     }
 }
@@ -366,15 +392,58 @@ static int launch_quant_rows(const void* x, int64_t m, int64_t k, int64_t ld_x, 
 // qmax <= 0: the format's own maximum
 template <bool SCALE_IN>
 static int launch_quant_rows_fmt(int q_fmt, const void* x, int x_dtype, int64_t m, int64_t k, int64_t ld_x, void* q,
-                                 int64_t ld_q, float* scale, hipStream_t st, float qmax = 0.0f, float eps = kEps, int round_x = 1) {
+                                 int64_t ld_q, float* scale, hipStream_t st, float qmax = 0.0f, float eps = kEps, int round_x = 1, const TensorScale& t = {}) {
     switch (q_fmt) {
-        case DAXQ_FMT_I8: return launch_quant_rows<0, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 127.0f, st, x_dtype, eps, round_x);
-        case DAXQ_FMT_E4M3: return launch_quant_rows<1, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 448.0f, st, x_dtype, eps, round_x);
-        case DAXQ_FMT_E5M2: return launch_quant_rows<2, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 57344.0f, st, x_dtype, eps, round_x);
+        case DAXQ_FMT_I8: return launch_quant_rows<0, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 127.0f, st, x_dtype, eps, round_x, t);
+        case DAXQ_FMT_E4M3: return launch_quant_rows<1, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 448.0f, st, x_dtype, eps, round_x, t);
+        case DAXQ_FMT_E5M2: return launch_quant_rows<2, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 57344.0f, st, x_dtype, eps, round_x, t);
         default: return fail(DAXQ_ERR_ARG, "quant_rows: unknown quantised format %d", q_fmt);
     }
 }
 
+// Abs-max of a whole matrix as kPartials bit patterns (sign cleared; their maximum is the abs-max, NaN above infinity):
+// one workgroup of sixteen wavefronts per CU, four 16-byte loads per lane in flight.
+template <int XT>
+__global__ __launch_bounds__(1024) void tensor_amax_kernel(const char* __restrict__ x, int64_t m, int k, int64_t ld_x, uint32_t* __restrict__ partials) {
+    constexpr int XB = XT == DAXQ_F32 ? 4 : 2, U = XT == DAXQ_F32 ? 2 : 4;
+    constexpr uint32_t kAbs = XT == DAXQ_F32 ? 0x7fffffffu : 0x7fffu;
+    __shared__ uint32_t s_max[16];
+    int64_t len = k;
+    if (ld_x == k || m == 1) {  // one long row
+        len = (int64_t)k * m;
+        m = 1;
+    }
+    const int64_t nch = len >> 3;
+    uint32_t mx = 0, tl = 0;
+    // a long row is spread over the grid, rows of a strided matrix are dealt to the workgroups
+    const int64_t first = m == 1 ? (int64_t)blockIdx.x * 1024 : 0, step = m == 1 ? (int64_t)kPartials * 1024 : 1024;
+    for (int64_t r = m == 1 ? 0 : blockIdx.x; r < m; r += kPartials) {
+        const char* xr = x + r * ld_x * XB;
+        for (int64_t c = first + threadIdx.x; c < nch; c += U * step) {
+            Chunk<XT> v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t cu = c + u * step;
+                load_chunk<XT>(v[u], xr + (cu < nch ? cu : c) * (8 * XB));  // (beyond the end: the lane's first chunk again)
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) mx = chunk_amax<XT>(mx, v[u]);
+        }
+        const int64_t e = (nch << 3) + threadIdx.x;
+        if (e < len) {
+            const uint32_t t = (XT == DAXQ_F32 ? reinterpret_cast<const uint32_t*>(xr)[e] : reinterpret_cast<const uint16_t*>(xr)[e]) & kAbs;
+            tl = t > tl ? t : tl;
+        }
+    }
+    mx = amax_of_lane<XT>(mx);
+    mx = wave_max_u32(tl > mx ? tl : mx);
+    if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        mx = wave_max_u32(threadIdx.x < 16 ? s_max[threadIdx.x] : 0u);
+        if (threadIdx.x == 0) partials[blockIdx.x] = mx;
+    }
+}
 
 // Per-row min and max of a bf16 / fp16 / fp32 matrix in fp32 (weight observer statistics).
 template <int XT>
@@ -492,6 +561,43 @@ int daxq_quantize_rows(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t
                        void* q, int64_t ld_q, daxq_stream_t stream) {
     return daxq::launch_quant_rows_fmt<true>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, const_cast<float*>(scale),
                                                     (hipStream_t)stream);
+}
+
+int daxq_act_quant_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q,
+                          float* scale_rows, float* scale1, void* scratch, float quant_max, float eps, int scale_round, daxq_stream_t stream) {
+    using namespace daxq;
+    if (m < 0 || k <= 0 || ld_x < k || ld_q < k || m > 0x7fffffff || k > 36 * 512)
+        return fail(DAXQ_ERR_ARG, "act_quant_tensor: bad shape m=%lld k=%lld (at most %d columns)", (long long)m, (long long)k, 36 * 512);
+    if (scale_round != DAXQ_SCALE_ROUND_X && scale_round != DAXQ_SCALE_ROUND_NONE)
+        return fail(DAXQ_ERR_ARG, "act_quant_tensor: unknown scale rounding %d", scale_round);
+    if (m == 0) return DAXQ_OK;
+    if (!x || !q || !scale_rows || !scratch) return fail(DAXQ_ERR_ARG, "act_quant_tensor: null pointer");
+    if ((uintptr_t)scratch & 15) return fail(DAXQ_ERR_ALIGN, "act_quant_tensor: the scratch must be 16-byte aligned");
+    if ((uintptr_t)x & (x_dtype == DAXQ_F32 ? 3 : 1)) return fail(DAXQ_ERR_ALIGN, "act_quant_tensor: x must be element aligned");
+    hipStream_t st = (hipStream_t)stream;
+    uint32_t* part = static_cast<uint32_t*>(scratch);
+    const char* xp = static_cast<const char*>(x);
+    const dim3 grid(kPartials), block(1024);
+    switch (x_dtype) {
+        case DAXQ_BF16: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_BF16>, grid, block, 0, st, xp, m, (int)k, ld_x, part); break;
+        case DAXQ_F16: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_F16>, grid, block, 0, st, xp, m, (int)k, ld_x, part); break;
+        case DAXQ_F32: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_F32>, grid, block, 0, st, xp, m, (int)k, ld_x, part); break;
+        default: return fail(DAXQ_ERR_ARG, "act_quant_tensor: unknown element type %d", x_dtype);
+    }
+    if (int rc = check_launch("tensor_amax")) return rc;
+    TensorScale t;
+    t.partials = part;
+    t.scale1 = scale1;
+    return launch_quant_rows_fmt<false>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, scale_rows, st, quant_max, eps, scale_round == DAXQ_SCALE_ROUND_X, t);
+}
+
+int daxq_quantize_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, const float* scale1, void* q,
+                         int64_t ld_q, float* scale_rows, daxq_stream_t stream) {
+    daxq::TensorScale t;
+    t.one_scale = true;
+    t.scale_rows = scale_rows;
+    return daxq::launch_quant_rows_fmt<true>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, const_cast<float*>(scale1), (hipStream_t)stream, 0.0f,
+                                             daxq::kEps, 1, t);
 }
 
 int daxq_scale_from_minmax(const float* min_in, const float* max_in, int64_t n, float qmax, float* scale,

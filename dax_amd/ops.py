@@ -336,6 +336,70 @@ quantize_rows_e4m3.register_fake(
     lambda x, scale, padded=False: x.new_empty((x.shape[0], pad_k(x.shape[1]) if padded else x.shape[1]), dtype=torch.uint8))
 
 
+# ----------------------------------------------------------------------------- one scale for the whole tensor
+MAX_TENSOR_QUANT_K = 18432  # longest row daxq_act_quant_tensor / daxq_quantize_tensor take
+
+
+def _tensor_q(m: int, k: int, fmt: str, padded: bool, device) -> torch.Tensor:
+    dtype = torch.int8 if fmt == "i8" else torch.uint8
+    return _alloc_q(m, pad_k(k), dtype, device) if padded else torch.empty((m, k), dtype=dtype, device=device)
+
+
+def _tensor_q_fake(x, fmt: str, padded: bool) -> torch.Tensor:
+    dtype = torch.int8 if fmt == "i8" else torch.uint8
+    return _fake_q(x, x.shape[0], pad_k(x.shape[1]), dtype) if padded else x.new_empty(x.shape, dtype=dtype)
+
+
+@torch.library.custom_op("daxq::act_quant_tensor", mutates_args=(), device_types="cuda")
+def act_quant_tensor(x: torch.Tensor, fmt: str, quant_max: float, eps: float, round_scale: bool,
+                     padded: bool) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Dynamic per-tensor quantisation of a bf16 / fp16 / fp32 matrix of at most 18432 columns: (bytes [M, pad128(K)] zero
+    padded, or [M, K]; the scale once per row, fp32 [M]; the scale, fp32 [1]).  Arguments as for act_quant_rows."""
+    name = "act_quant_tensor"
+    kind = _rows_float(x, name)
+    if fmt not in FMT:
+        raise ValueError(f"daxq::{name}: unknown format {fmt}")
+    m, k = x.shape
+    with _on_device(x):
+        q = _tensor_q(m, k, fmt, padded, x.device)
+        s = torch.empty((m,), dtype=torch.float32, device=x.device)
+        s1 = torch.empty((1,), dtype=torch.float32, device=x.device)
+        if m:
+            scratch = torch.empty((256,), dtype=torch.int32, device=x.device)
+            _capi.check(_capi.lib().daxq_act_quant_tensor(
+                x.data_ptr(), kind, FMT[fmt], m, k, x.stride(0) if m > 1 else k, q.data_ptr(), q.stride(0) if m > 1 else q.shape[1],
+                s.data_ptr(), s1.data_ptr(), scratch.data_ptr(), quant_max, eps, 1 if round_scale else 0, _stream(x)), name)
+    return q, s, s1
+
+
+act_quant_tensor.register_fake(lambda x, fmt, quant_max, eps, round_scale, padded: (
+    _tensor_q_fake(x, fmt, padded), x.new_empty((x.shape[0],), dtype=torch.float32), x.new_empty((1,), dtype=torch.float32)))
+
+
+@torch.library.custom_op("daxq::quantize_tensor", mutates_args=(), device_types="cuda")
+def quantize_tensor(x: torch.Tensor, scale: torch.Tensor, fmt: str, padded: bool) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Leaf quantiser with one scale (fp32 [1]) for a matrix of at most 18432 columns: (bytes as in act_quant_tensor, the
+    scale once per row)."""
+    name = "quantize_tensor"
+    kind = _rows_float(x, name)
+    if fmt not in FMT:
+        raise ValueError(f"daxq::{name}: unknown format {fmt}")
+    if scale.dtype != torch.float32 or scale.numel() != 1 or scale.device != x.device:
+        raise ValueError(f"daxq::{name}: scale must hold one fp32 value on {x.device}")
+    m, k = x.shape
+    with _on_device(x):
+        q = _tensor_q(m, k, fmt, padded, x.device)
+        s = torch.empty((m,), dtype=torch.float32, device=x.device)
+        if m:
+            _capi.check(_capi.lib().daxq_quantize_tensor(
+                x.data_ptr(), kind, FMT[fmt], m, k, x.stride(0) if m > 1 else k, scale.data_ptr(), q.data_ptr(),
+                q.stride(0) if m > 1 else q.shape[1], s.data_ptr(), _stream(x)), name)
+    return q, s
+
+
+quantize_tensor.register_fake(lambda x, scale, fmt, padded: (_tensor_q_fake(x, fmt, padded), x.new_empty((x.shape[0],), dtype=torch.float32)))
+
+
 # ----------------------------------------------------------------------------- weight observer statistics
 @torch.library.custom_op("daxq::row_minmax", mutates_args=(), device_types="cuda")
 def row_minmax(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:

@@ -5,8 +5,9 @@ one on the DiT hot path, is a single fused HIP kernel (row abs-max with wavefron
 bf16-rounded scale floored at 2^-23, quantise from registers).  The scale recipe follows the
 reference's eager dtype chain for a bf16 input: the division by quant_max and the clamp
 happen in bf16, and only then is the scale widened to fp32 (:124-129).  The per-tensor scheme
-(one block = the whole tensor) runs the row statistics kernel, a single-workgroup reduction to
-the scalar scale by the same rule, and the leaf quantiser with that scale.
+(one block = the whole tensor) is the tensor's abs-max and, in the quantiser of the rows, the scale by
+the same rule; rows of more than 18432 elements take the row statistics kernel, a single-workgroup
+reduction to the scalar scale and the leaf quantiser with that scale.
 """
 from typing import List, Optional, Tuple, Union
 
@@ -128,6 +129,9 @@ def per_tensor_scale(x2: torch.Tensor, quant_max: float, eps: float = ops.EPS_F3
 def _per_tensor_quantize(x, fmt, quant_max, eps=ops.EPS_F32, round_x=True):
     k = x.shape[-1] if x.dim() else 1
     x2 = x.reshape(-1, k)
+    if 0 < k <= ops.MAX_TENSOR_QUANT_K:
+        q, _, s1 = ops.act_quant_tensor(x2, fmt, quant_max, eps, round_x, False)
+        return q, s1
     s1, rows = per_tensor_scale(x2, quant_max, eps, round_x)
     return getattr(ops, "quantize_rows_" + fmt)(x2, rows), s1
 

@@ -151,6 +151,9 @@ class Linear(DerivedOperands, nn.Module):
             flat = flat.contiguous()
         if self.input_qscheme == per_token_symmetric:
             xq, sx = getattr(ops, _ACT_QUANT[self.input_dtype])(flat, self.act_scale_fp32)
+        elif self.in_features <= ops.MAX_TENSOR_QUANT_K:
+            fmt = ops.FMT_OF_DTYPE[self.input_dtype]
+            xq, sx, _ = ops.act_quant_tensor(flat, fmt, ops.QMAX[fmt], ops.EPS_F32, not self.act_scale_fp32, True)
         else:
             from .functional import per_tensor_scale
 

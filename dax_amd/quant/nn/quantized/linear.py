@@ -69,10 +69,13 @@ class Linear(DerivedOperands, nn.Module):
         flat = input.view(-1, self.in_features)
         if flat.stride(-1) != 1:
             flat = flat.contiguous()
-        sx = ops.broadcast_f32(self.input_scale.reshape(1), flat.shape[0])
         bias = None if self.bias is None else self.bias.detach()  # inference-only kernels
         x_fmt, w_fmt = ops.FMT_OF_DTYPE[self.input_dtype], ops.FMT_OF_DTYPE[self.weight_dtype]
-        xq = getattr(ops, "quantize_rows_" + x_fmt)(flat, sx, True)
+        if self.in_features <= ops.MAX_TENSOR_QUANT_K:
+            xq, sx = ops.quantize_tensor(flat, self.input_scale, x_fmt, True)
+        else:
+            sx = ops.broadcast_f32(self.input_scale.reshape(1), flat.shape[0])
+            xq = getattr(ops, "quantize_rows_" + x_fmt)(flat, sx, True)
         # row-wise weight scales: the matmul writes bf16 and the result is cast afterwards (:96-104, :116-117)
         mm_dtype = torch.bfloat16 if self.row_wise_scale else self.out_dtype
         out = ops.linear_w8a8(xq, sx, self._gemm_weight(), self._weight_scale_vector(), bias, x_fmt, w_fmt, mm_dtype)

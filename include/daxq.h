@@ -218,6 +218,21 @@ int daxq_tensor_minmax_update(const float* row_min, const float* row_max, int64_
 int daxq_broadcast_f32(const float* src, float* dst, int64_t n, daxq_stream_t stream);
 
 /*
+ * The same two schemes without the statistics per row, for rows of at most 18432 columns (any alignment):
+ * daxq_act_quant_tensor: dynamic per-tensor quantisation in two passes over x -- the abs-max of the tensor into `scratch`
+ *   (1 KiB, 16-byte aligned, contents unspecified before and after), then scale and bytes.  Arguments and arithmetic as for
+ *   daxq_act_quant_rows_ex with the whole matrix as one row; scale_rows [m] receives the one scale once per row (the vector
+ *   the GEMM reads), scale1 [1] once more, or NULL.
+ * daxq_quantize_tensor: daxq_quantize_rows with the one scale scale1[0] for every row; scale_rows [m] receives it once per
+ *   row, or NULL.   dax/quant/nn/quantized/linear.py:91-118
+ */
+int daxq_act_quant_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q,
+                          float* scale_rows, float* scale1, void* scratch, float quant_max, float eps, int scale_round,
+                          daxq_stream_t stream);
+int daxq_quantize_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, const float* scale1,
+                         void* q, int64_t ld_q, float* scale_rows, daxq_stream_t stream);
+
+/*
  * Per-row min and max of a bf16 matrix, in fp32: the statistics of the per-channel weight observer.
  * Replaces PerChannelMinMaxObserver.forward   dax/quant/quantization/observer.py:284-312
  */

@@ -84,3 +84,34 @@ def test_fp8_bytes_without_a_division(ops, fmt):
         sc = torch.tensor([s])
         q = getattr(ops, "quantize_rows_" + fmt)(xf.to("cuda"), sc.to("cuda"))
         assert torch.equal(q.cpu(), O.quantize_to_fp8(xf, sc[:, None], FP8[fmt]).view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,k,pitch", [(1, 8, 8), (1, 5, 5), (3, 7, 9), (255, 33, 33), (300, 1000, 1000), (77, 1001, 1003), (70, 5120, 5128), (2500, 1536, 1536),
+                                       (260, 18432, 18432), (5000, 520, 520), (257, 4096, 4104)])
+def test_one_scale_for_the_tensor(ops, dtype, m, k, pitch):
+    """The abs-max of a tensor over the grid (flat, and rows apart from one another), its last element, first element and a
+    place in between as the largest; the scale by the rule of the tensor's type, and bytes, scales and padding against the
+    oracle's quantiser of the flattened tensor.  A NaN anywhere makes the scale NaN."""
+    g = torch.Generator().manual_seed(m + k)
+    base = torch.randn(m, pitch, generator=g).to(dtype)
+    for at in ((m - 1, k - 1), (0, 0), (m // 2, k // 3)):
+        x = base.clone()
+        x[at] = -9.5
+        xd = x.to("cuda")[:, :k]
+        xc = x[:, :k].contiguous()
+        for fmt in ("i8", "e5m2"):
+            target = torch.int8 if fmt == "i8" else FP8[fmt]
+            qo, so = O.dynamic_quantize(xc.view(1, -1), (1, m * k), target, ops.QMAX[fmt], ops.EPS_F32, torch.float32)
+            q, s, s1 = ops.act_quant_tensor(xd, fmt, ops.QMAX[fmt], ops.EPS_F32, True, True)
+            assert torch.equal(s1.cpu(), so.view(1)) and torch.equal(s.cpu(), so.view(1).expand(m))
+            np.testing.assert_array_equal(_bytes(q[:, :k]), _bytes(qo).reshape(m, k))
+            assert q.shape[1] == ops.pad_k(k) and not q[:, k:].any()
+            scale = so.view(1) * 0.61                                       # the same with a scale from the caller
+            q, s = ops.quantize_tensor(xd, scale.to("cuda"), fmt, False)
+            ref = O.quantize_to_int8(xc, scale) if fmt == "i8" else O.quantize_to_fp8(xc, scale, target)
+            np.testing.assert_array_equal(_bytes(q), _bytes(ref))
+            assert torch.equal(s.cpu(), scale.expand(m))
+    x[m // 2, k // 2] = float("nan")
+    _, s, s1 = ops.act_quant_tensor(x.to("cuda")[:, :k], "i8", 127.0, ops.EPS_F32, True, True)
+    assert bool(torch.isnan(s).all()) and bool(torch.isnan(s1).all())
