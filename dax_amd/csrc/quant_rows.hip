@@ -445,33 +445,87 @@ __global__ __launch_bounds__(1024) void tensor_amax_kernel(const char* __restric
     }
 }
 
-// Per-row min and max of a bf16 / fp16 / fp32 matrix in fp32 (weight observer statistics).
+// Per-row min and max of a bf16 / fp16 / fp32 matrix in fp32 (observer statistics), one workgroup per row, 16-byte loads.
+// The bit patterns are compared as two's-complement integers (magnitude bits of negative values flipped), two 16-bit
+// values per instruction; a NaN sorts beyond either infinity and makes both results NaN.  HBM-bound; measured against two-byte
+// loads and NaN-aware fp32 comparisons: 13824 x 5120 bf16 56.1 -> 22.9 us, 75600 x 5120 409 -> 118 us = 6.5 TB/s.
+typedef short daxq_s2 __attribute__((ext_vector_type(2)));
 template <int XT>
-__global__ __launch_bounds__(256) void row_minmax_kernel(const void* __restrict__ xv, int64_t k, int64_t ld_x,
-                                                         float* __restrict__ mn, float* __restrict__ mx) {
-    typedef typename XWord<XT>::type word_t;
-    __shared__ float rlo[4], rhi[4];
-    const int64_t row = blockIdx.x;
-    const word_t* xr = static_cast<const word_t*>(xv) + row * ld_x;
-    float lo = __builtin_inff(), hi = -__builtin_inff();
-    for (int64_t c = threadIdx.x; c < k; c += 256) {
-        float f = x_bits_to_f32<XT>(xr[c]);
-        lo = min_nan(lo, f);
-        hi = max_nan(hi, f);
+__device__ __forceinline__ int order_key(uint32_t w) {  // (a pair of values per word for the 16-bit types)
+    if constexpr (XT == DAXQ_F32) return (int)(w ^ (((int)w >> 31) & 0x7fffffff));
+    const daxq_s2 v = __builtin_bit_cast(daxq_s2, w);
+    return (int)(w ^ (__builtin_bit_cast(uint32_t, (daxq_s2)(v >> 15)) & 0x7fff7fffu));
+}
+template <int XT>
+__device__ __forceinline__ void keys_minmax(int& lo, int& hi, int key) {
+    if constexpr (XT == DAXQ_F32) {
+        lo = key < lo ? key : lo;
+        hi = key > hi ? key : hi;
+    } else {
+        const daxq_s2 k = __builtin_bit_cast(daxq_s2, key);
+        lo = __builtin_bit_cast(int, __builtin_elementwise_min(__builtin_bit_cast(daxq_s2, lo), k));
+        hi = __builtin_bit_cast(int, __builtin_elementwise_max(__builtin_bit_cast(daxq_s2, hi), k));
+    }
+}
+template <int XT>
+__device__ __forceinline__ float value_of_key(int key) {
+    if constexpr (XT == DAXQ_F32) return __uint_as_float((uint32_t)key ^ ((uint32_t)(key >> 31) & 0x7fffffffu));
+    const uint32_t w = (uint32_t)key & 0xffffu;
+    return x_bits_to_f32<XT>(w & 0x8000u ? w ^ 0x7fffu : w);
+}
+
+// U: loads per lane in flight, as many as the row has for 256 lanes, up to four
+template <int XT, int U>
+__global__ __launch_bounds__(256) void row_minmax_kernel(const char* __restrict__ x, int64_t k, int64_t ld_x, float* __restrict__ mn,
+                                                         float* __restrict__ mx) {
+    constexpr int XB = XT == DAXQ_F32 ? 4 : 2;
+    __shared__ int s_lo[4], s_hi[4];
+    const int64_t row = blockIdx.x, nch = k >> 3;
+    const char* xr = x + row * ld_x * XB;
+    int lo = XT == DAXQ_F32 ? 0x7fffffff : 0x7fff7fff, hi = XT == DAXQ_F32 ? (int)0x80000000 : (int)0x80008000;
+    for (int64_t c = threadIdx.x; c < nch; c += U * 256) {
+        Chunk<XT> v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) load_chunk<XT>(v[u], xr + (c + u * 256 < nch ? c + u * 256 : c) * (8 * XB));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < (XT == DAXQ_F32 ? 2 : 1); ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) keys_minmax<XT>(lo, hi, order_key<XT>(v[u].w[h][i]));
+    }
+    const int64_t e = (nch << 3) + threadIdx.x;
+    if (e < k) {
+        uint32_t w;
+        if constexpr (XT == DAXQ_F32) w = reinterpret_cast<const uint32_t*>(xr)[e];
+        else w = reinterpret_cast<const uint16_t*>(xr)[e] * 0x10001u;
+        keys_minmax<XT>(lo, hi, order_key<XT>(w));
+    }
+    if constexpr (XT != DAXQ_F32) {  // the pair's own minimum and maximum, sign-extended
+        const int l0 = (int)(short)lo, l1 = lo >> 16, h0 = (int)(short)hi, h1 = hi >> 16;
+        lo = l0 < l1 ? l0 : l1;
+        hi = h0 > h1 ? h0 : h1;
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
-        lo = min_nan(lo, __shfl_xor(lo, off, 64));
-        hi = max_nan(hi, __shfl_xor(hi, off, 64));
+        const int ol = __shfl_xor(lo, off, 64), oh = __shfl_xor(hi, off, 64);
+        lo = ol < lo ? ol : lo;
+        hi = oh > hi ? oh : hi;
     }
     if ((threadIdx.x & 63) == 0) {
-        rlo[threadIdx.x >> 6] = lo;
-        rhi[threadIdx.x >> 6] = hi;
+        s_lo[threadIdx.x >> 6] = lo;
+        s_hi[threadIdx.x >> 6] = hi;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        mn[row] = min_nan(min_nan(rlo[0], rlo[1]), min_nan(rlo[2], rlo[3]));
-        mx[row] = max_nan(max_nan(rhi[0], rhi[1]), max_nan(rhi[2], rhi[3]));
+#pragma unroll
+        for (int w = 1; w < 4; ++w) {
+            lo = s_lo[w] < lo ? s_lo[w] : lo;
+            hi = s_hi[w] > hi ? s_hi[w] : hi;
+        }
+        const float l = value_of_key<XT>(lo), h = value_of_key<XT>(hi);
+        mn[row] = h != h ? h : l;
+        mx[row] = l != l ? l : h;
     }
 }
 
@@ -529,10 +583,18 @@ int daxq_row_minmax_t(const void* x, int x_dtype, int64_t m, int64_t k, int64_t 
     if (m == 0) return DAXQ_OK;
     if (!x || !min_out || !max_out) return fail(DAXQ_ERR_ARG, "row_minmax: null pointer");
     const dim3 grid((unsigned)m), block(256);
+    hipStream_t st = (hipStream_t)stream;
+    const char* xp = static_cast<const char*>(x);
+    auto launch = [&](auto XT) {
+        constexpr int X = decltype(XT)::value;
+        if (k <= 2048) hipLaunchKernelGGL((row_minmax_kernel<X, 1>), grid, block, 0, st, xp, k, ld_x, min_out, max_out);
+        else if (k <= 4096 || X == DAXQ_F32) hipLaunchKernelGGL((row_minmax_kernel<X, 2>), grid, block, 0, st, xp, k, ld_x, min_out, max_out);
+        else hipLaunchKernelGGL((row_minmax_kernel<X, 4>), grid, block, 0, st, xp, k, ld_x, min_out, max_out);
+    };
     switch (x_dtype) {
-        case DAXQ_BF16: hipLaunchKernelGGL(row_minmax_kernel<DAXQ_BF16>, grid, block, 0, (hipStream_t)stream, x, k, ld_x, min_out, max_out); break;
-        case DAXQ_F16: hipLaunchKernelGGL(row_minmax_kernel<DAXQ_F16>, grid, block, 0, (hipStream_t)stream, x, k, ld_x, min_out, max_out); break;
-        case DAXQ_F32: hipLaunchKernelGGL(row_minmax_kernel<DAXQ_F32>, grid, block, 0, (hipStream_t)stream, x, k, ld_x, min_out, max_out); break;
+        case DAXQ_BF16: launch(std::integral_constant<int, DAXQ_BF16>{}); break;
+        case DAXQ_F16: launch(std::integral_constant<int, DAXQ_F16>{}); break;
+        case DAXQ_F32: launch(std::integral_constant<int, DAXQ_F32>{}); break;
         default: return fail(DAXQ_ERR_ARG, "row_minmax: unknown element type %d", x_dtype);
     }
     return check_launch("row_minmax");

@@ -438,6 +438,29 @@ def scale_from_minmax(min_val: torch.Tensor, max_val: torch.Tensor, qmax: float,
 scale_from_minmax.register_fake(lambda min_val, max_val, qmax, eps=EPS_F32: torch.empty_like(min_val))
 
 
+@torch.library.custom_op("daxq::weight_quant", mutates_args=(), device_types="cuda")
+def weight_quant(w: torch.Tensor, fmt: str, quant_max: float, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Symmetric per-row (per-output-channel) quantisation of a bf16 / fp16 / fp32 weight in one pass: (bytes [N, K] without
+    padding, fp32 scale [N]).  The same bits as row_minmax, scale_from_minmax and quantize_rows: the row's abs-max is the
+    larger of -min and max, and the scale is not rounded."""
+    name = "weight_quant"
+    kind = _rows_float(w, name)
+    if fmt not in FMT:
+        raise ValueError(f"daxq::{name}: unknown format {fmt}")
+    n, k = w.shape
+    with _on_device(w):
+        q = torch.empty((n, k), dtype=torch.int8 if fmt == "i8" else torch.uint8, device=w.device)
+        s = torch.empty((n,), dtype=torch.float32, device=w.device)
+        if n:
+            _capi.check(_capi.lib().daxq_act_quant_rows_ex(w.data_ptr(), kind, FMT[fmt], n, k, w.stride(0) if n > 1 else k, q.data_ptr(), k,
+                                                           s.data_ptr(), quant_max, eps, 0, _stream(w)), name)
+    return q, s
+
+
+weight_quant.register_fake(lambda w, fmt, quant_max, eps: (
+    w.new_empty(w.shape, dtype=torch.int8 if fmt == "i8" else torch.uint8), w.new_empty((w.shape[0],), dtype=torch.float32)))
+
+
 # ----------------------------------------------------------------------------- GEMM + epilogue
 # Workspaces of the split-K launches: one per (device, stream), zero-filled when it is made (the kernels leave the
 # counters at its head zero).  Launches on one stream are ordered, so they can share it; another stream gets its own.

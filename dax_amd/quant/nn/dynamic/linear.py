@@ -21,6 +21,7 @@ a plain library matmul on the cold path.
 from __future__ import annotations
 
 import logging
+from functools import partial
 
 import torch
 from torch import Tensor, nn
@@ -57,6 +58,12 @@ class QuantizedActivation:
 _ACT_QUANT = {torch.int8: "act_quant_i8", torch.float8_e4m3fn: "act_quant_e4m3", torch.float8_e5m2: "act_quant_e5m2"}
 _DYNAMIC_LINEAR = {torch.int8: "dynamic_linear_i8", torch.float8_e4m3fn: "dynamic_linear_e4m3",
                    torch.float8_e5m2: "dynamic_linear_e5m2_e4m3"}
+
+
+def _is_per_channel_observer(cls) -> bool:
+    from ...quantization.observer import PerChannelMinMaxObserver  # (that package imports this module)
+
+    return cls is PerChannelMinMaxObserver
 
 
 class Linear(DerivedOperands, nn.Module):
@@ -266,8 +273,10 @@ class Linear(DerivedOperands, nn.Module):
     # ------------------------------------------------------------------ conversion
     @classmethod
     @torch.no_grad()
-    def get_qlinear(cls, mod, activation_post_process, weight_post_process, reserve_float_weight):
-        """Builds the quantised module from a float ``nn.Linear`` (:240-309).
+    def get_qlinear(cls, mod, activation_post_process, weight_post_process, reserve_float_weight, fresh_observer=False):
+        """Builds the quantised module from a float ``nn.Linear`` (:240-309).  ``fresh_observer``: the weight observer is a
+        ``PerChannelMinMaxObserver`` that has seen nothing and is dropped afterwards, so its running statistics need not be
+        left in it.
 
         The weight statistics, the per-channel scale and the quantised weight are computed by
         HIP kernels; a module that still lives on the CPU is staged through the current
@@ -300,25 +309,21 @@ class Linear(DerivedOperands, nn.Module):
                                    f"(module is on {home}); there is no CPU implementation")
             w = w.to(torch.device("cuda", torch.cuda.current_device()))
 
-        weight_post_process.to(w.device)
-        weight_post_process(w)
-        if weight_post_process.dtype in FP8_ALLOWED_DTYPES:
-            from ..quantized.functional import quantize_to_fp8 as quantize_func
-        elif weight_post_process.dtype == torch.int8:
-            from ..quantized.functional import quantize_to_int8 as quantize_func
-        else:
+        if weight_post_process.dtype not in FP8_ALLOWED_DTYPES and weight_post_process.dtype != torch.int8:
             raise NotImplementedError(f"Unsupported dtype {weight_post_process.dtype}")
-
-        weight_scale = weight_post_process.calculate_qparams()
+        if fresh_observer and weight_post_process.ch_axis == 0:
+            # nobody looks at this observer again: its statistics, the scales and the bytes are one pass over the weight
+            if w.stride(1) != 1:
+                w = w.contiguous()
+            qweight, weight_scale = ops.weight_quant(w, ops.FMT_OF_DTYPE[weight_post_process.dtype],
+                                                     float(weight_post_process.quant_max), float(weight_post_process.eps))
+            if weight_post_process.dtype != torch.int8:
+                qweight = qweight.view(weight_post_process.dtype)
+        else:
+            qweight, weight_scale = cls._quantize_observed(w, weight_post_process)
         if weight_scale is not None:
-            if weight_scale.numel() > 1:
-                assert mod.weight.shape[0] == weight_scale.numel()
-                scale_arg = weight_scale.reshape(-1, 1)
-            else:
-                scale_arg = weight_scale.reshape(1)
-            qweight = quantize_func(w, scale=scale_arg, dtype=weight_post_process.dtype)
             qlinear.qweight = qweight.to(home)
-            qlinear.weight_scale.copy_(weight_scale.reshape(qlinear.weight_scale.shape))
+            qlinear.weight_scale = weight_scale.reshape(qlinear.weight_scale.shape).to(home)
         if qlinear.bias is not None:
             qlinear.bias.copy_(mod.bias)
 
@@ -327,6 +332,25 @@ class Linear(DerivedOperands, nn.Module):
             del mod.bias
         qlinear.refresh_derived()
         return qlinear
+
+    @staticmethod
+    def _quantize_observed(w, observer):
+        """(quantised weight, scale) by way of the observer: its running statistics, its scales, the leaf quantiser."""
+        observer.to(w.device)
+        observer(w)
+        if observer.dtype in FP8_ALLOWED_DTYPES:
+            from ..quantized.functional import quantize_to_fp8 as quantize_func
+        else:
+            from ..quantized.functional import quantize_to_int8 as quantize_func
+        weight_scale = observer.calculate_qparams()
+        if weight_scale is None:
+            return None, None
+        if weight_scale.numel() > 1:
+            assert w.shape[0] == weight_scale.numel()
+            scale_arg = weight_scale.reshape(-1, 1)
+        else:
+            scale_arg = weight_scale.reshape(1)
+        return quantize_func(w, scale=scale_arg, dtype=observer.dtype), weight_scale
 
     @classmethod
     def from_float(cls, mod, reserve_float_weight=False):
@@ -340,4 +364,7 @@ class Linear(DerivedOperands, nn.Module):
             assert hasattr(mod, "qconfig"), "Input float module must have qconfig defined."
             activation_post_process = mod.qconfig.activation()
             weight_post_process = mod.qconfig.weight()
+            # (the factory is the observer's class with arguments: a new object every time)
+            fresh = isinstance(mod.qconfig.weight, partial) and _is_per_channel_observer(mod.qconfig.weight.func)
+            return cls.get_qlinear(mod, activation_post_process, weight_post_process, reserve_float_weight, fresh)
         return cls.get_qlinear(mod, activation_post_process, weight_post_process, reserve_float_weight)

@@ -115,3 +115,28 @@ def test_one_scale_for_the_tensor(ops, dtype, m, k, pitch):
     x[m // 2, k // 2] = float("nan")
     _, s, s1 = ops.act_quant_tensor(x.to("cuda")[:, :k], "i8", 127.0, ops.EPS_F32, True, True)
     assert bool(torch.isnan(s).all()) and bool(torch.isnan(s1).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,k,pitch", [(1, 1, 1), (5, 7, 9), (3, 8, 8), (4, 2047, 2047), (3, 2048, 2051), (7, 8193, 8193), (2, 20001, 20001)])
+def test_row_statistics_and_weights_in_one_pass(ops, dtype, n, k, pitch):
+    """Row minima and maxima with 16-byte loads (chunks, leftover elements, rows that start anywhere; all-negative, zero and
+    NaN rows), and the one-pass weight quantiser against them: the same scales and bytes as statistics, scale and leaf
+    quantiser one after the other."""
+    g = torch.Generator().manual_seed(n * k)
+    w = torch.randn(n, pitch, generator=g)
+    w[0] = -w[0].abs() - 0.01
+    w[-1, k - 1] = 7.5
+    w = w.to(dtype).to("cuda")[:, :k]
+    lo, hi = ops.row_minmax(w)
+    assert torch.equal(lo, w.float().amin(1)) and torch.equal(hi, w.float().amax(1))
+    for fmt in ("i8", "e4m3"):
+        s = ops.scale_from_minmax(lo, hi, ops.QMAX[fmt])
+        q = getattr(ops, "quantize_rows_" + fmt)(w, s)
+        q1, s1 = ops.weight_quant(w, fmt, ops.QMAX[fmt], ops.EPS_F32)
+        assert torch.equal(s1, s) and torch.equal(q1, q)
+    for sign in (1.0, -1.0):
+        bad = w.clone()
+        bad[n // 2, k // 2] = sign * float("nan")
+        lo, hi = ops.row_minmax(bad)
+        assert torch.equal(torch.isnan(lo), torch.arange(n, device="cuda") == n // 2) and torch.equal(torch.isnan(hi), torch.isnan(lo))
