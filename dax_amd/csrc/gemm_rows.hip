@@ -1,0 +1,312 @@
+// W8A8 GEMM for a handful of rows (gfx950): every wavefront streams its own part of the weight, no barriers in the K loop.
+//
+// What bounds it: every byte of the weight is needed once and multiplied with a few rows, so the launch is a stream of the
+// weight from HBM (26 MB at N = K = 5120: 4.3 us at 6.2 TB/s) and what counts is how many bytes are in flight.  The tiled
+// kernels put such a launch on N / 128 workgroups (40 of them at N = 5120).
+//
+// Work decomposition
+//   workgroup  16 output columns x MB blocks of 16 rows, KS wavefronts that share K
+//   wavefront  K / KS bytes of the 16 weight rows and of the activation rows, in steps of 128 bytes, through a ring of R
+//              steps in an LDS region of its own
+// Loads go straight into LDS (global_load_lds_dwordx4, four lanes to 64 consecutive bytes of a row); fragments are read
+// back in the MFMA's layout with the chunk swizzle of the tiled kernels.  Loading the fragments directly into registers, lane
+// l from row l % 16, was built first: neighbouring lanes then sit in different rows, every lane is a cache line of its own,
+// and a CU takes 14 bytes per cycle instead of the 60 that four lanes to a row segment give.
+// A wavefront reads only what it loaded itself, so a wait on its own load counter is all the synchronisation there is.
+// INT8 runs KS = 4 or 1: sums of integers do not depend on how K is cut; partial sums meet in LDS.  FP8 runs KS = 1: an
+// output element is then the same sequence of MFMAs over the same K bytes in the same register positions as in
+// gemm_tile_fp8.hip, and an output row does not depend on how many rows the launch has.
+// Rows and columns beyond the matrix repeat its last row / column and are not stored.
+#include "gemm_tile.h"
+
+namespace daxq {
+
+// FP8 formats as in the tiled kernels: the weight is the MFMA "A" operand (cbsz), the activations the "B" operand (blgp)
+template <bool FP8, int F8>
+__device__ __forceinline__ typename Acc16<FP8>::type mfma_step(v8i w, v8i x, typename Acc16<FP8>::type c) {
+    if constexpr (FP8) {
+        return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, x, c, (F8 & kF8WE5) ? 1 : 0, (F8 & kF8XE5) ? 1 : 0, 0, 0, 0, 0);
+    } else {
+        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_shufflevector(w, w, 0, 1, 2, 3), __builtin_shufflevector(x, x, 0, 1, 2, 3), c, 0, 0, 0);
+        return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_shufflevector(w, w, 4, 5, 6, 7), __builtin_shufflevector(x, x, 4, 5, 6, 7), c, 0, 0, 0);
+    }
+}
+
+template <int T, typename F>
+__device__ __forceinline__ void for_down(F&& f) {
+    f(Int<T>{});
+    if constexpr (T > 0) for_down<T - 1>(f);
+}
+
+constexpr int rows_step_bytes(int mb) { return 2048 * (1 + mb); }  // LDS of a step: 16 weight rows, then MB x 16 activation rows
+
+template <bool FP8, int F8, int MB, int R, int KS, int OUTK>
+__global__ __launch_bounds__(64 * KS) void gemm_rows_kernel(const GemmArgs p) {
+    typedef typename Acc16<FP8>::type acc_t;
+    constexpr int STEP = rows_step_bytes(MB), L = 2 * (1 + MB);  // load instructions of a step
+    static_assert(R >= 2 && (R - 1) * L < 64, "the load counter holds 63");
+    static_assert(KS == 1 || KS * MB * 1024 <= KS * R * STEP, "the partial sums fit the ring");
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l15 = lane & 15, g4 = lane >> 4;
+    const int n0 = (int)blockIdx.x * 16, mbase = (int)blockIdx.y * (16 * MB);
+
+    const int steps = p.k >> 7;
+    const int first = steps * wave / KS, cnt = steps * (wave + 1) / KS - first;
+
+    // ---- memory side: a load instruction takes 16 rows x 64 bytes, lane l row l / 4 and the 16-byte chunk that the swizzle
+    //      stores at chunk l % 4 of the row
+    const int lrow = lane >> 2;
+    const uint32_t gsw = (uint32_t)(((lane & 3) ^ ((lrow >> 1) & 3)) << 4);
+    const uint8_t* wbase = p.b + (int64_t)n0 * p.ldb + (int64_t)first * 128;
+    const uint8_t* xbase = p.a + (int64_t)first * 128;
+    const uint32_t wcol = n0 + lrow < p.n ? lrow : p.n - 1 - n0;
+    uint32_t woff = wcol * (uint32_t)p.ldb + gsw, xoff[MB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i) xoff[i] = (uint32_t)(mbase + i * 16 + lrow < p.m ? mbase + i * 16 + lrow : p.m - 1) * (uint32_t)p.lda + gsw;
+    const uint32_t ring = (uint32_t)(uintptr_t)(DAXQ_LDS uint8_t*)smem + (uint32_t)wave * (R * STEP);
+    auto load = [&](int step, uint32_t slot) __attribute__((always_inline)) {
+        const uint8_t* w = wbase + (int64_t)step * 128;
+        const uint8_t* x = xbase + (int64_t)step * 128;
+        const uint32_t dst = ring + slot;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(w + h * 64 + woff), (DAXQ_LDS void*)(uintptr_t)(dst + h * 1024), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(x + h * 64 + xoff[i]),
+                                                 (DAXQ_LDS void*)(uintptr_t)(dst + 2048 * (1 + i) + h * 1024), 16, 0, 0);
+    };
+
+    // ---- LDS side: row l % 16, K chunk l / 16 of either half
+    const uint8_t* rd = smem + wave * (R * STEP) + l15 * 64 + ((g4 ^ ((l15 >> 1) & 3)) << 4);
+    acc_t acc[MB] = {};
+    auto fragment = [&](uint32_t at) __attribute__((always_inline)) {
+        const v4i lo = *reinterpret_cast<const v4i*>(rd + at), up = *reinterpret_cast<const v4i*>(rd + at + 1024);
+        return __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    auto next_slot = [](uint32_t slot) { return slot == (R - 1) * STEP ? 0 : slot + STEP; };
+    // U steps that have landed: their fragments into registers, the steps R later into their places, their MFMAs.  Two at a
+    // time with one row block: the wait for the LDS reads is then paid half as often (one row, N = 1536, K = 8960, FP8: 9.0 ->
+    // 7.8 us; with two row blocks and more the loads' own issue is what a step takes, and two steps at a time lose 3 %)
+    auto work = [&](auto STEPS, auto MORE, int step, uint32_t slot) __attribute__((always_inline)) {
+        constexpr int U = decltype(STEPS)::value;
+        v8i w[U], x[U][MB];
+        uint32_t at[U];
+        at[0] = slot;
+#pragma unroll
+        for (int u = 1; u < U; ++u) at[u] = next_slot(at[u - 1]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            w[u] = fragment(at[u]);
+#pragma unroll
+            for (int i = 0; i < MB; ++i) x[u][i] = fragment(at[u] + 2048 * (1 + i));
+        }
+        if constexpr (MORE.value) {
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(63) & lgkmcnt0_mask());  // the reads are over
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) load(step + u + R, at[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < MB; ++i) acc[i] = mfma_step<FP8, F8>(w[u], x[u][i], acc[i]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // (loads retire in order: a step has landed when no more than the loads issued behind it are in flight)
+    const int ahead = cnt < R ? cnt : R;
+#pragma unroll
+    for (int s = 0; s < R; ++s)
+        if (s < ahead) load(s, s * STEP);
+    __builtin_amdgcn_sched_barrier(0);
+    int step = 0;
+    uint32_t slot = 0;
+    for (; MB == 1 && step + R + 1 < cnt; step += 2) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((R - 2) * L));
+        __builtin_amdgcn_sched_barrier(0);
+        work(Int<2>{}, Yes{}, step, slot);
+        slot = next_slot(next_slot(slot));
+    }
+    for (; step + R < cnt; ++step) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((R - 1) * L));
+        __builtin_amdgcn_sched_barrier(0);
+        work(Int<1>{}, Yes{}, step, slot);
+        slot = next_slot(slot);
+    }
+    auto tail = [&](auto T) __attribute__((always_inline)) {  // T steps behind this one
+        constexpr int t = decltype(T)::value;
+        if (t >= ahead) return;
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(t * L));
+        __builtin_amdgcn_sched_barrier(0);
+        work(Int<1>{}, No{}, 0, slot);
+        slot = next_slot(slot);
+    };
+    for_down<R - 1>(tail);
+
+    // ---- epilogue (the arithmetic of tile_epilogue16): a lane owns output row l % 16 of a block and 4 consecutive columns
+    const int nc = n0 + 4 * g4;
+    float sw[4], bias[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int c = nc + e < p.n ? nc + e : p.n - 1;
+        sw[e] = p.sw[c];
+        if (!p.bias) bias[e] = -0.0f;  // x + (-0.0) == x bit for bit
+        else if constexpr (OUTK == DAXQ_F32) bias[e] = reinterpret_cast<const float*>(p.bias)[c];
+        else if constexpr (OUTK == DAXQ_F16) bias[e] = f16_bits_to_f32(p.bias[c]);
+        else bias[e] = bf16_bits_to_f32(p.bias[c]);
+    }
+    v4i* s_part = reinterpret_cast<v4i*>(smem);
+    if constexpr (KS > 1) {
+        __syncthreads();  // every wavefront is done with the ring
+#pragma unroll
+        for (int i = 0; i < MB; ++i) s_part[(wave * MB + i) * 64 + lane] = __builtin_bit_cast(v4i, acc[i]);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+        if (KS > 1 && i % KS != wave) continue;  // the wavefronts share the row blocks out
+        if constexpr (KS > 1) {
+            v4i sum = s_part[i * 64 + lane];
+#pragma unroll
+            for (int s = 1; s < KS; ++s) sum += s_part[(s * MB + i) * 64 + lane];
+            acc[i] = __builtin_bit_cast(acc_t, sum);
+        }
+        const int m = mbase + i * 16 + l15;
+        if (m >= p.m || nc >= p.n) continue;
+        const float sxv = p.sx[m];
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float y = (float)acc[i][e];  // (int8: v_cvt_f32_i32, round to nearest even)
+            y = y * sxv;
+            y = y * sw[e];
+            if constexpr (OUTK == DAXQ_F32 || FP8) {
+                o[e] = y + bias[e];
+                if constexpr (OUTK == DAXQ_F16) asm("" : "+v"(o[e]));  // the sum is rounded to fp32 before the cast to fp16
+            } else if constexpr (OUTK == DAXQ_F16) {
+                asm("" : "+v"(y));
+                float z = (float)(_Float16)y + bias[e];
+                asm("" : "+v"(z));
+                o[e] = z;
+            } else {
+                o[e] = bf16_bits_to_f32(pack_bf16_rne(y, 0.0f) & 0xffffu) + bias[e];
+            }
+        }
+        const int64_t at = (int64_t)m * p.ldo + nc;
+        if constexpr (OUTK == DAXQ_F32) {
+            float* dst = reinterpret_cast<float*>(p.out) + at;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (nc + e < p.n) dst[e] = o[e];
+        } else {
+            uint32_t lo, hi;
+            if constexpr (OUTK == DAXQ_F16) lo = pack_f16_rne(o[0], o[1]), hi = pack_f16_rne(o[2], o[3]);
+            else lo = pack_bf16_rne(o[0], o[1]), hi = pack_bf16_rne(o[2], o[3]);
+            typedef v2u loose __attribute__((aligned(2)));
+            uint16_t* dst = p.out + at;
+            if (nc + 4 <= p.n) {
+                *reinterpret_cast<loose*>(dst) = v2u{lo, hi};
+            } else {
+                const uint32_t w[4] = {lo & 0xffffu, lo >> 16, hi & 0xffffu, hi >> 16};
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (nc + e < p.n) dst[e] = (uint16_t)w[e];
+            }
+        }
+    }
+}
+
+// args null: only raises the kernel's LDS limit on the current device.
+template <bool FP8, int F8, int MB, int R, int KS, int OUTK>
+static int launch_rows_one(const GemmArgs* args, hipStream_t st) {
+    constexpr int lds = KS * R * rows_step_bytes(MB);
+    auto kern = gemm_rows_kernel<FP8, F8, MB, R, KS, OUTK>;
+    static std::atomic<uint64_t> lds_set{0};  // per instantiation
+    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_set)) return rc;
+    if (!args) return DAXQ_OK;
+    const dim3 grid((unsigned)((args->n + 15) / 16), (unsigned)((args->m + 16 * MB - 1) / (16 * MB)));
+    hipLaunchKernelGGL(kern, grid, dim3(64 * KS), lds, st, *args);
+    return check_launch("gemm_rows");
+}
+
+// Which form: the number of workgroups per row block (n / 16) and of rows decide how many bytes are in flight and how often
+// the activation is fetched.  Measured, us, weight in the caches / never touched before (INT8; FP8 the same where KS = 1):
+//                            MB,R,KS   1,10,1      1,5,1       2,5,1       1,5,4       2,3,4       4,2,4      128x128 tiles
+//   m = 16,  5120 x 5120           6.1 / 9.3   6.3 / 9.9   9.4 / 10.2  6.8 / 11.4  7.4 / 11.7  9.1 / 13.3   18.8 / 33.6
+//   m = 32,  5120 x 5120           7.4 / 11.9  7.1 / 11.6  9.7 / 11.1  8.2 / 11.9  8.9 / 14.5  10.0 / 15.6  18.7 / 33.5
+//   m = 64,  5120 x 5120          16.5 / 21.4 12.4 / 17.9 10.3 / 15.5 14.4 / 17.6 10.9 / 14.7  12.6 / 19.0  20.5 / 33.6
+//   m = 128, 5120 x 5120          24.7 / 29.4 24.0 / 29.5 18.0 / 25.2 23.8 / 27.0 20.2 / 23.3  16.5 / 19.8  18.6 / 33.3
+//   m = 32,  N = 15360            25.6 / 27.8 23.5 / 26.9 15.0 / 20.1 27.6 / 31.2 18.1 / 26.9  20.2 / 28.3  23.8 / 34.7
+//   m = 64,  N = 15360            47.6 / 50.1 44.6 / 48.5 31.2 / 37.7 51.1 / 54.5 33.1 / 39.5  24.5 / 35.8  24.0 / 35.0
+//   m = 16,  N = 1536, K = 8960    7.8 / 8.0   7.9 / 9.2  14.5 / 14.5  4.5 / 6.0   5.7 / 6.2    7.7 / 7.9   26.4 / 30.0
+//   m = 64,  N = 1536, K = 8960    8.2 / 8.5   8.3 / 9.4  14.8 / 14.7  7.4 / 8.2   5.8 / 7.5    7.8 / 10.3  26.3 / 29.5
+//   m = 128, N = 1536, K = 8960   10.5 / 11.7  9.9 / 11.2 14.9 / 15.1 12.6 / 12.9  9.6 / 10.9   8.0 / 10.2  26.3 / 29.4
+// Few workgroups (small n): cut K where the sums allow it, one row block per workgroup where they do not; many: two row
+// blocks, so that the activation is fetched half as often.  With more than 32 rows and N > 8192 the tiles, which fetch it
+// once per 128 columns, are as fast.
+template <bool FP8, int F8, int OUTK>
+static int launch_rows_out(const GemmArgs* a, hipStream_t st) {
+    if (!a) {
+        int rc = launch_rows_one<FP8, F8, 1, 10, 1, OUTK>(a, st);
+        if (!rc) rc = launch_rows_one<FP8, F8, 1, 5, 1, OUTK>(a, st);
+        if (!rc) rc = launch_rows_one<FP8, F8, 2, 5, 1, OUTK>(a, st);
+        if constexpr (!FP8) {
+            if (!rc) rc = launch_rows_one<FP8, F8, 1, 5, 4, OUTK>(a, st);
+            if (!rc) rc = launch_rows_one<FP8, F8, 2, 3, 4, OUTK>(a, st);
+            if (!rc) rc = launch_rows_one<FP8, F8, 4, 2, 4, OUTK>(a, st);
+        }
+        return rc;
+    }
+    if constexpr (!FP8) {
+        if (a->n < 4096 || a->m > 64) {
+            if (a->m <= 32) return launch_rows_one<FP8, F8, 1, 5, 4, OUTK>(a, st);
+            if (a->m <= 64) return launch_rows_one<FP8, F8, 2, 3, 4, OUTK>(a, st);
+            return launch_rows_one<FP8, F8, 4, 2, 4, OUTK>(a, st);
+        }
+    }
+    if (a->m <= 16) return launch_rows_one<FP8, F8, 1, 10, 1, OUTK>(a, st);
+    if (a->n <= 2048 || (a->m <= 32 && a->n <= 8192)) return launch_rows_one<FP8, F8, 1, 5, 1, OUTK>(a, st);
+    return launch_rows_one<FP8, F8, 2, 5, 1, OUTK>(a, st);
+}
+
+template <bool FP8, int F8>
+static int launch_rows_fmt(const GemmArgs* a, int out_kind, hipStream_t st) {
+    if (out_kind == DAXQ_F16) return launch_rows_out<FP8, F8, DAXQ_F16>(a, st);
+    if (out_kind == DAXQ_F32) return launch_rows_out<FP8, F8, DAXQ_F32>(a, st);
+    return launch_rows_out<FP8, F8, DAXQ_BF16>(a, st);
+}
+
+static int launch_rows_any(const GemmArgs* a, int out_kind, bool fp8, int f8, hipStream_t st) {
+    if (!fp8) return launch_rows_fmt<false, 0>(a, out_kind, st);
+    switch (f8) {
+        case 1: return launch_rows_fmt<true, 1>(a, out_kind, st);
+        case 2: return launch_rows_fmt<true, 2>(a, out_kind, st);
+        case 3: return launch_rows_fmt<true, 3>(a, out_kind, st);
+        default: return launch_rows_fmt<true, 0>(a, out_kind, st);
+    }
+}
+
+// every instantiation on the current device, so that a first launch may sit inside a stream capture
+int prepare_rows_kernels() {
+    int rc = 0;
+    for (int out_kind : {DAXQ_BF16, DAXQ_F16, DAXQ_F32}) {
+        if (!rc) rc = launch_rows_any(nullptr, out_kind, false, 0, nullptr);
+        for (int f8 = 0; f8 < 4 && !rc; ++f8) rc = launch_rows_any(nullptr, out_kind, true, f8, nullptr);
+    }
+    return rc;
+}
+
+bool rows_applies(int64_t m, int64_t n) { return m <= (n > 8192 ? 32 : 128); }
+
+// at most 128 rows (32-bit row offsets), no accumulator dump
+int launch_rows(const GemmArgs& a, bool fp8, int f8, hipStream_t st) {
+    if (a.m > 128 || a.acc || a.lda >= (1 << 26) || a.ldb >= (1 << 26))
+        return fail(DAXQ_ERR_ARG, "linear: the kernel for few rows takes at most 128, row strides below 2^26 and no accumulator dump");
+    return launch_rows_any(&a, a.out_kind, fp8, f8, st);
+}
+
+}  // namespace daxq

@@ -245,6 +245,8 @@ int launch_tile_i8(const GemmArgs& a, bool small, int tail, hipStream_t st);    
 int launch_tile_fp8(const GemmArgs& a, int f8, bool small, int tail, hipStream_t st);  // gemm_tile_fp8.hip
 int launch_halves_i8(const GemmArgs& a, hipStream_t st);                                // gemm_tile256.hip
 int launch_halves_fp8(const GemmArgs& a, int f8, hipStream_t st);                       // gemm_tile_fp8.hip
+int launch_rows(const GemmArgs& a, bool fp8, int f8, hipStream_t st);                    // gemm_rows.hip
+bool rows_applies(int64_t m, int64_t n);
 template <bool FP8>
 int launch_tile128_splitk(const GemmArgs& a, int f8, hipStream_t st);
 
@@ -261,6 +263,7 @@ static int launch_halves(const GemmArgs& a, int f8, hipStream_t st) {
 }
 
 int prepare_tile_fp8_kernels();
+int prepare_rows_kernels();
 int prepare_tile256_kernels();
 
 template <bool FP8, int BM, int BN, int BK, int WM, int WN, bool DIRECT, int F8 = 0>
@@ -301,7 +304,7 @@ static int launch_generic(const GemmArgs& a, int f8, hipStream_t st) {
 
 // Kernel choices of the `kernel` argument (daxq_linear_w8a8): low 16 bits pick the implementation, bits 16-23 the
 // depth of the tile-order groups (0 = 4 tile rows).
-enum { K_DEFAULT = 0, K_GENERIC256 = 2, K_GENERIC128 = 5, K_TILED_256 = 8, K_TILED_128 = 11, K_TILED_HALVES = 14 };
+enum { K_DEFAULT = 0, K_GENERIC256 = 2, K_GENERIC128 = 5, K_TILED_256 = 8, K_TILED_128 = 11, K_TILED_HALVES = 14, K_ROWS = 17 };
 
 // Tile order a launch of 256x256 tiles takes when the caller names none.  The banded order (tile_order.h: patches of
 // 8 x 4 tiles per XCD, the eight XCDs of a round on the same activation rows and on different weight bands) reads the
@@ -378,7 +381,7 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
             // fp16 / fp32 outputs together with the accumulator dump (tests): the generic kernel
             if (acc && out_kind != DAXQ_BF16)
                 return (m >= 256 && n >= 256) ? launch_generic<FP8, 256>(a, f8, st) : launch_generic<FP8, 128>(a, f8, st);
-            // library default: the tiled kernel on 256x256 tiles once there is one for every second CU, on 128x128
+            // library default: the kernel for few rows (rows_applies, gemm_rows.hip); the tiled kernel on 256x256 tiles once there is one for every second CU, on 128x128
             // tiles (4x as many workgroups, two per CU) below that, and the generic kernel for operands smaller than
             // one such tile.  Measured at N = K = 5120 (INT8, T-op/s, 128 / 256 tiles):
             // M = 512 -> 1127 / 551, M = 1024 (80 large tiles) -> 1275 / 1055, M = 2048 (160) -> 1542 / 1817;
@@ -390,6 +393,7 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
             // 2048 x 4096 x 4096 (128) 39.6 -> 30.7 / 38.7 -> 31.2, 1024 x 5120, K = 13824 95.9 -> 69.3 / 93.1 -> 66.8,
             // 4096 x 1536, K = 8960 62.3 -> 50.7 / 60.5 -> 50.3, K = 3072 +9 to +15 % / +16 %, K = 2048 0 to +10 % / +2 %;
             // at K = 1536 -2 / -5 %, and with 60 tiles (768 x 5120 x 5120) the quadrants' 23.8 us become 30.5.
+            if (rows_applies(m, n) && fits32 && !acc) return launch_rows(a, FP8, f8, st);
             const int64_t tiles256 = ((m + 255) / 256) * ((n + 255) / 256);
             const int cus = cu_count();
             if (tile256_applies(a) && k >= 2048 && cus >= 8 && 4 * tiles256 > cus && 2 * tiles256 <= cus) return launch_halves<FP8>(a, f8, st);
@@ -408,6 +412,7 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
         case K_TILED_HALVES:
             if (!tile256_applies(a)) return fail(DAXQ_ERR_ARG, "linear: the 256x128 kernel needs m, n >= 256");
             return launch_halves<FP8>(a, f8, st);
+        case K_ROWS: return launch_rows(a, FP8, f8, st);
         default: return fail(DAXQ_ERR_ARG, "linear: unknown kernel choice %d", which);
     }
 }
@@ -427,7 +432,7 @@ constexpr int64_t kMaxSplitTiles = kCounterBytes / 4;
 // 2 / 4 ranges): M = 256 (80 tiles) 34 / 28 / 40, M = 512 (160 tiles) 24 / 35 / 52, M = 1024 52 / 71 / -: the partial
 // results make a round trip through device-coherent memory (about 10 us for 20 MB), which only idle CUs pay for.
 static int splitk_choice(int64_t m, int64_t n, int64_t k) {
-    if (m < 128 || n < 128 || k % DAXQ_K_ALIGN) return 1;
+    if (m < 128 || n < 128 || k % DAXQ_K_ALIGN || rows_applies(m, n)) return 1;
     const int64_t tiles = splitk_tiles(m, n), units = k / DAXQ_K_ALIGN;
     int best = 1;
     for (int s = 2; s <= 8; ++s)
@@ -591,6 +596,7 @@ int daxq_init(void) {
     using namespace daxq;
     int rc = prepare_tile256_kernels();
     if (!rc) rc = prepare_tile_fp8_kernels();
+    if (!rc) rc = prepare_rows_kernels();
 #define DAXQ_PREP_ALL(FP8, BT, WN)                                        \
     if (!rc) rc = prepare_cfg<FP8, BT, BT, 128, 2, WN, true, 0>();
     DAXQ_PREP_ALL(false, 128, 2)
@@ -647,13 +653,14 @@ int daxq_dynamic_linear(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int ac
     // the quantiser zero-fills columns [k, kp) of the rows it writes
     const float qmax = x_fmt == DAXQ_FMT_I8 ? 127.0f : x_fmt == DAXQ_FMT_E4M3 ? 448.0f : 57344.0f;
     if (int rc = daxq_act_quant_rows_ex(x, x_dtype, x_fmt, m, k, ld_x, xq, ld_xq, sx, qmax, kEps, act_scale_round, stream)) return rc;
-    // Fewer rows than the smallest tile of the tiled kernels: run them on 128 rows of the caller's buffers when those
-    // reach that far (the rows beyond m hold whatever the buffers held; an output row depends on its own operand row only).
-    const int64_t mg = (m < 128 && rows_alloc >= 128 && n >= 128) ? 128 : m;
+    // Fewer rows than the smallest tile of the tiled kernels, and more columns than the kernel for few rows is taken for: run
+    // the tiled kernels on 128 rows of the caller's buffers when those reach that far (the rows beyond m hold whatever the buffers held; an output row depends on its own operand row only).
+    const bool rows = kernel == 0 && rows_applies(m, n);
+    const int64_t mg = (!rows && m < 128 && rows_alloc >= 128 && n >= 128) ? 128 : m;
     hipStream_t st = (hipStream_t)stream;
     // INT8 launches with few tiles cut K into ranges when the caller brings a workspace (integer partial sums: the
     // same bits as the plain launch); FP8 sums would change with the number of rows, so they stay whole.
-    if (!fp8 && workspace && out_dtype == DAXQ_BF16 && kernel == 0) {
+    if (!fp8 && workspace && out_dtype == DAXQ_BF16 && kernel == 0 && !rows) {
         const int splits = splitk_choice(mg, n, kp);
         if (splits > 1 && workspace_bytes >= kCounterBytes + splitk_tiles(mg, n) * splits * kPartialBytes)
             return launch_gemm_splitk<false>(xq, ld_xq, sx, wq, ld_wq, sw, bias, out, ld_out, mg, n, kp, splits, workspace,

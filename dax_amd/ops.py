@@ -114,6 +114,7 @@ def _rows_bf16(x: torch.Tensor, what: str) -> None:
 # written.
 Q_ROW_PAD = 128
 MIN_TILE_ROWS = 128  # rows of the smallest tile of the tiled GEMM kernels
+ROWS_KERNEL_MAX_N = 8192  # columns up to which 33 to 128 rows run in the kernel for few rows (fewer rows always do)
 
 
 def _row_pad(kp: int) -> int:
@@ -671,9 +672,10 @@ def _dynamic_linear(x, wq, sw, bias, fmt: str, scale_fp32: bool = False):
         raise ValueError(f"daxq::dynamic_linear_{fmt}: sw must be contiguous fp32 [N]")
     if bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != n or not bias.is_contiguous()):
         raise ValueError(f"daxq::dynamic_linear_{fmt}: bias must be contiguous bfloat16 [N]")
-    # Fewer rows than one 128-row tile: the buffers get 128 rows and the tiled kernel runs on all of them (twice as fast
-    # as the kernel that takes fewer rows); what the rows beyond M hold is never looked at, and their outputs are cut off.
-    rows = MIN_TILE_ROWS if 0 < m < MIN_TILE_ROWS <= n else m
+    # Fewer rows than one 128-row tile but more columns than the kernel for few rows is taken for: the buffers get 128
+    # rows and the tiled kernel runs on all of them; what the rows beyond M hold is never looked at, and their outputs are
+    # cut off.
+    rows = MIN_TILE_ROWS if 32 < m < MIN_TILE_ROWS and n > ROWS_KERNEL_MAX_N else m
     ld_q = kp + (Q_ROW_PAD if kp % 1024 == 0 else 0)
     with _on_device(x):
         # quantised rows, then the fp32 scales (the row stride is a multiple of 128, so they are aligned)

@@ -1,0 +1,81 @@
+"""The GEMM for a handful of rows: every row block count and ring depth, ragged in both dimensions, K from one step to more
+steps than the ring holds, every output type and operand format.  INT8 against the integer oracle's epilogue, bit for bit;
+FP8 the same bits as the tiled kernel (an output row does not depend on how many rows the launch has)."""
+import pytest
+import torch
+
+from oracle import daxq_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture()
+def select():
+    from dax_amd import _capi
+
+    yield _capi.debug_select_gemm
+    _capi.debug_select_gemm(0)
+
+
+# n on either side of the widths at which the form changes (2048, 4096, 8192) and ragged; k / 128 = 1 .. 44 steps
+SHAPES = [(5, 128), (16, 256), (17, 384), (130, 640), (264, 1408), (133, 1536), (2048, 1280), (2052, 1152), (4095, 512), (4097, 640),
+          (8192, 256), (8200, 384), (520, 5632)]
+ROWS = [1, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65, 100, 127, 128]
+
+
+@pytest.mark.parametrize("n,k", SHAPES)
+def test_rows_int8(select, n, k):
+    import dax_amd.ops as ops
+
+    g = torch.Generator().manual_seed(n + k)
+    xq = torch.randint(-128, 128, (128, k), generator=g, dtype=torch.int8)
+    wq = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8)
+    sx, sw = torch.rand(128, generator=g) * 0.01, torch.rand(n, generator=g) * 0.01
+    acc = O.int_mm(xq, wq)
+    select(17)
+    xd, wd = xq.to("cuda"), wq.to("cuda")
+    for i, m in enumerate(ROWS):
+        dtype = (torch.bfloat16, torch.float16, torch.float32)[i % 3]
+        bias = torch.randn(n, generator=g).to(dtype) if i % 2 else None
+        ref = O.epilogue_int8(acc[:m], sx[:m, None], sw, bias, out_dtype=dtype)
+        y = ops.linear_w8a8(xd[:m], sx[:m].to("cuda"), wd, sw.to("cuda"), None if bias is None else bias.to("cuda"), "i8", "i8", dtype)
+        assert y.dtype == dtype and torch.equal(y.cpu(), ref), (m, dtype)
+
+
+@pytest.mark.parametrize("x_fmt,w_fmt", [("e4m3", "e4m3"), ("e5m2", "e4m3"), ("e4m3", "e5m2"), ("e5m2", "e5m2")])
+@pytest.mark.parametrize("n,k", [s for s in SHAPES if s[0] >= 128])
+def test_rows_fp8_bits_of_the_tiled_kernel(select, n, k, x_fmt, w_fmt):
+    import dax_amd.ops as ops
+
+    g = torch.Generator().manual_seed(n * 3 + k)
+    f8 = {"e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}
+    xq = torch.randn(128, k, generator=g).to(f8[x_fmt]).view(torch.uint8).to("cuda")
+    wq = torch.randn(n, k, generator=g).to(f8[w_fmt]).view(torch.uint8).to("cuda")
+    sx, sw = torch.rand(128, generator=g).to("cuda"), torch.rand(n, generator=g).to("cuda")
+    for dtype in (torch.bfloat16, torch.float16, torch.float32):
+        bias = torch.randn(n, generator=g).to(dtype).to("cuda")
+        select(11)
+        ref = ops.linear_w8a8(xq, sx, wq, sw, bias, x_fmt, w_fmt, dtype)
+        select(17)
+        for m in ROWS:
+            assert torch.equal(ops.linear_w8a8(xq[:m], sx[:m], wq, sw, bias, x_fmt, w_fmt, dtype), ref[:m]), (m, dtype)
+
+
+def test_rows_outputs_as_a_slice_of_a_wider_buffer():
+    """Strided operands and output through the C ABI: nothing outside the M x N outputs is touched."""
+    import dax_amd.ops as ops
+    from dax_amd import _capi
+
+    g = torch.Generator().manual_seed(3)
+    m, n, k = 19, 83, 384
+    xq = torch.randint(-128, 128, (m, k + 128), generator=g, dtype=torch.int8).to("cuda")[:, :k]
+    wq = torch.randint(-128, 128, (n, k + 256), generator=g, dtype=torch.int8).to("cuda")[:, :k]
+    sx, sw = torch.rand(m, generator=g).to("cuda"), torch.rand(n, generator=g).to("cuda")
+    out = torch.full((m + 2, n + 10), 7.0, dtype=torch.bfloat16, device="cuda")
+    view = out[1:m + 1, 3:n + 3]
+    _capi.check(_capi.lib().daxq_linear_w8a8(0, 0, 0, xq.data_ptr(), xq.stride(0), sx.data_ptr(), wq.data_ptr(), wq.stride(0), sw.data_ptr(), None,
+                                             view.data_ptr(), out.stride(0), None, 0, m, n, k, 17, torch.cuda.current_stream().cuda_stream), "rows")
+    ref = O.epilogue_int8(O.int_mm(xq.cpu(), wq.cpu()), sx.cpu()[:, None], sw.cpu(), None)
+    assert torch.equal(view.cpu(), ref)
+    view.fill_(7.0)
+    assert bool((out == 7.0).all())
