@@ -8,6 +8,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -15,6 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libdaxq.so")
 ROOT = os.path.dirname(HERE)
+TORCH_LIB = os.path.join(LIBDIR, "_daxq_torch.so")
 MFMA_RATE = os.path.join(ROOT, "bench", "mfma_rate")
 SOURCES = ["capi.hip", "quant_rows.hip", "quant_blocks.hip", "fused_rows.hip", "per_tensor.hip", "gemm_w8a8.hip", "gemm_rows.hip", "gemm_tile256.hip", "gemm_tile_fp8.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -48,16 +50,50 @@ def _compile(src: str, verbose: bool) -> str:
     return obj
 
 
+def _compile_torch_entry(verbose: bool) -> str:
+    """torch_linear.cpp (host code against torch's headers), linked once libdaxq.so is there."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    obj = os.path.join(LIBDIR, "torch_linear.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{d}" for d in (*include_paths("cuda"), sysconfig.get_paths()["include"])),
+           "-c", os.path.join(CSRC, "torch_linear.cpp"), "-o", obj]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on torch_linear.cpp:\n{r.stderr}")
+    return obj
+
+
+def _link_torch_entry(obj: str, verbose: bool) -> None:
+    import torch
+
+    # libdaxq.so beside it is the library that ctypes loads, too; torch's libraries are loaded before this one
+    cmd = ["g++", "-shared", "-o", TORCH_LIB, obj, "-L" + LIBDIR, "-l:libdaxq.so", "-Wl,-rpath,$ORIGIN",
+           "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"link of _daxq_torch.so failed:\n{r.stderr}")
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(LIBDIR, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
+    with ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as ex:
+        entry = ex.submit(_compile_torch_entry, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), SOURCES))
+        entry = entry.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs]
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr}")
+    _link_torch_entry(entry, verbose)
     # stand-alone microbenchmark behind bench.py's sustained-MFMA-rate figure
     cmd = [HIPCC, *FLAGS, os.path.join(ROOT, "bench", "mfma_rate.hip"), "-o", MFMA_RATE]
     if verbose:

@@ -94,6 +94,23 @@ def lib() -> C.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The extension module that runs a whole linear from one Python call (csrc/torch_linear.cpp)."""
+    global _native
+    if _native is None:
+        lib()  # checks the ABI; raises if nothing is built
+        try:
+            from .lib import _daxq_torch
+        except ImportError as e:
+            raise RuntimeError(f"dax_amd/lib/_daxq_torch.so does not load ({e}); run "
+                               "`python -c 'import __graft_entry__ as g; g.build()'`") from e
+        _native = _daxq_torch
+    return _native
+
+
 def last_error() -> str:
     msg = lib().daxq_last_error()
     return msg.decode() if msg else ""

@@ -11,7 +11,7 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from ... import ops
+from ... import _capi, ops
 
 
 def _capturing(t: Tensor) -> bool:
@@ -24,6 +24,62 @@ def _refresh_after_load(module, incompatible_keys) -> None:
 
 class DerivedOperands:
     """Mixin for a module with ``qweight``, ``weight_scale`` and ``out_features``."""
+
+    # A module whose forward is quantiser + GEMM and whose state lives on the device keeps the arguments of that one call
+    # ready: every torch call in a forward costs the host a microsecond or two, and a small linear's time is the host's.
+    # The tensors alias the module's state (or are derived from it), so in-place updates of the aliased ones show through;
+    # the tuple also remembers which state tensors it was built from, where they lived and, where a derived copy stands
+    # for one, at which version, and a forward that finds anything else (a buffer or parameter replaced by assignment, by a
+    # hook of an off-loading framework, or through `.data`) rebuilds it.  Whatever sets the state afresh
+    # (conversion, load_state_dict, .to()) rebuilds it too.  Plain data only: a module must stay deep-copyable, and a
+    # copy finds the addresses changed and rebuilds.
+    _fast = None
+
+    def _fast_arguments(self):
+        """(x_fmt, w_fmt, element type of the output, scheme) of the one call, or None where the module needs more."""
+        raise NotImplementedError
+
+    def _fast_state(self):
+        raise NotImplementedError
+
+    def _build_fast(self) -> None:
+        object.__setattr__(self, "_fast", None)
+        args = self._fast_arguments()
+        qw, ws, bp, xs = self._fast_state()
+        if (args is None or qw.device.type != "cuda" or not qw.is_contiguous() or ops.is_tracing(qw)
+                or torch.cuda.is_current_stream_capturing()):
+            return
+        wq, sw = self._gemm_weight(), self._weight_scale_vector()
+        # (a tensor made in inference mode counts no versions: nothing can be derived from it that stays checkable)
+        derived = [t for t, of in ((qw, wq), (ws, sw)) if of.data_ptr() != t.data_ptr()]
+        if any(t.is_inference() for t in derived):
+            return
+        bias = None if bp is None else bp.detach()
+        in_scale = None if xs is None else xs.detach()
+        object.__setattr__(self, "_fast", (
+            (wq, sw, bias, in_scale, self.in_features, *args), qw.device.index, qw, ws, bp, xs, qw.data_ptr(), ws.data_ptr(),
+            0 if bp is None else bp.data_ptr(), 0 if xs is None else xs.data_ptr(),
+            tuple((t, t._version) for t in derived)))
+
+    def _fast_forward(self, input: Tensor, scale_fp32: bool):
+        """The output, or None where the general forward has to look at the call."""
+        f = self._fast
+        if f is None or input.__class__ is not Tensor or torch.compiler.is_compiling():
+            return None
+        qw, ws, bp, xs = self._fast_state()
+        if (qw is not f[2] or ws is not f[3] or bp is not f[4] or xs is not f[5] or qw.data_ptr() != f[6] or ws.data_ptr() != f[7]
+                or (bp is not None and bp.data_ptr() != f[8]) or (xs is not None and xs.data_ptr() != f[9])
+                or any(t._version != v for t, v in f[10])):
+            self.refresh_derived()
+            f = self._fast
+            if f is None:
+                return None
+        if f[1] not in _capi._checked_devices:
+            _capi.require_gfx950(f[1])
+        out = _capi.native().linear(input, *f[0], scale_fp32, _capi.kernel_arg())
+        if out is not None and out.__class__ is int:
+            _capi.check(out, "linear")
+        return out
 
     def _init_derived(self) -> None:
         self._packed = None  # (key, K-padded byte view of qweight)
@@ -43,6 +99,7 @@ class DerivedOperands:
         if self.qweight.device.type == "cuda":
             self._gemm_weight()
             self._weight_scale_vector()
+        self._build_fast()
 
     def _gemm_weight(self) -> Tensor:
         """qweight as the byte matrix [N, pad128(K)] the GEMM reads."""

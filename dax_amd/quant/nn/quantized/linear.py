@@ -63,7 +63,21 @@ class Linear(DerivedOperands, nn.Module):
         """De-quantised weight in out_dtype (:87-89)."""
         return self.qweight.to(self.out_dtype) * self.weight_scale.reshape(-1, 1).to(self.out_dtype)
 
+    def _fast_arguments(self):
+        mm_dtype = torch.bfloat16 if self.row_wise_scale else self.out_dtype
+        if mm_dtype != self.out_dtype or (self.bias is not None and self.bias.dtype != mm_dtype):
+            return None
+        return (ops.FMT[ops.FMT_OF_DTYPE[self.input_dtype]], ops.FMT[ops.FMT_OF_DTYPE[self.weight_dtype]],
+                ops.FLOAT_KIND[mm_dtype], 2)
+
+    def _fast_state(self):
+        p, b = self._parameters, self._buffers
+        return p["qweight"], b["weight_scale"], p["bias"], b["input_scale"]
+
     def forward(self, input: Tensor) -> Tensor:
+        out = self._fast_forward(input, False)
+        if out is not None:
+            return out
         self._check_device(input.device)
         prev_dims = input.shape[:-1]
         flat = input.view(-1, self.in_features)

@@ -1,0 +1,137 @@
+"""The forward of a quantised linear through the one native call (csrc/torch_linear.cpp): the bits of the general forward
+over every scheme, element type and layout it takes, and None wherever the dispatcher would do more than launch kernels."""
+import pytest
+import torch
+from torch import nn
+
+from dax_amd.quant.quantization import convert, prepare, quantize_dynamic
+from dax_amd.quant.quantization import qconfig as Q
+
+pytestmark = pytest.mark.gpu
+
+DYNAMIC = {
+    "token_i8": Q.get_dynamic_int8_per_token_act_per_channel_weight_qconfig,
+    "token_e4m3": lambda: Q.get_dynamic_fp8_per_token_act_per_channel_weight_qconfig(activation_dtype=torch.float8_e4m3fn),
+    "token_e5m2": lambda: Q.get_dynamic_fp8_per_token_act_per_channel_weight_qconfig(activation_dtype=torch.float8_e5m2),
+    "tensor_i8": Q.get_default_dynamic_int8_qconfig,
+    "tensor_e4m3": lambda: Q.get_default_dynamic_fp8_qconfig(activation_dtype=torch.float8_e4m3fn),
+    "tensor_e5m2": lambda: Q.get_default_dynamic_fp8_qconfig(activation_dtype=torch.float8_e5m2),
+}
+
+
+def _module(scheme, k, n, dtype, bias, x):
+    torch.manual_seed(k + n)
+    model = nn.Sequential(nn.Linear(k, n, bias=bias)).to("cuda", dtype)
+    if scheme.startswith("static"):
+        act = torch.float8_e4m3fn if scheme.endswith("e4m3") else torch.float8_e5m2
+        prepare(model, {"": Q.get_fp8_per_channel_weight_qconfig(activation_dtype=act)})
+        model(x)
+        convert(model)
+    else:
+        quantize_dynamic(model, {"": DYNAMIC[scheme]()})
+    return model[0]
+
+
+def _general(lin, x):
+    """The same forward by way of the custom ops."""
+    lin._fast_forward = lambda *a: None
+    try:
+        return lin(x)
+    finally:
+        del lin._fast_forward
+
+
+def _native(lin, x):
+    return lin._fast_forward(x, getattr(lin, "act_scale_fp32", False))
+
+
+@pytest.mark.parametrize("scheme", [*DYNAMIC, "static_e4m3", "static_e5m2"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,k,n,bias", [(1, 128, 16, True), (3, 1000, 40, False), (40, 1024, 264, True), (300, 333, 129, True)])
+@torch.no_grad()
+def test_bits_of_the_general_forward(scheme, dtype, m, k, n, bias):
+    x = torch.randn(m, k, device="cuda").to(dtype)
+    lin = _module(scheme, k, n, dtype, bias, x)
+    want = _general(lin, x)
+    row_wise_16 = dtype != torch.bfloat16 and (scheme.startswith("static") or scheme in ("token_e4m3", "token_e5m2"))
+    got = _native(lin, x)
+    assert (got is None) == row_wise_16  # a row-wise FP8 module that is not bf16 casts behind the matmul
+    assert torch.equal(lin(x), want)
+    wide = torch.randn(m, k + 24, device="cuda").to(dtype)
+    for y in (x.view(1, m, k), wide[:, 8:8 + k], x.t().contiguous().t(), x[:0]):  # any shape, row stride, strided columns, no rows
+        out = lin(y)
+        assert out.shape == (*y.shape[:-1], n) and out.dtype == dtype
+        assert torch.equal(out, _general(lin, y))
+
+
+@torch.no_grad()
+def test_calls_that_are_not_plain_take_the_op():
+    x = torch.randn(24, 256, device="cuda").bfloat16()
+    lin = _module("token_i8", 256, 64, torch.bfloat16, True, x)
+    want = lin(x)
+    assert _native(lin, x) is not None
+    assert _native(lin, x.cpu()) is None and _native(lin, x[:, :128]) is None and _native(lin, x.double()) is None
+    with pytest.raises(RuntimeError):
+        lin(x.cpu())
+    with torch.enable_grad():
+        assert _native(lin, x.clone().requires_grad_()) is None
+    with torch.autograd.forward_ad.dual_level():
+        assert _native(lin, torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))) is None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert _native(lin, x) is None and torch.equal(lin(x), want)
+    seen = []
+
+    class Mode(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert torch.equal(lin(x), want)
+    assert any("daxq.dynamic_linear_i8" in s for s in seen)
+    seen.clear()
+
+    class Functions(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Functions():
+        out = lin(x)
+    assert torch.equal(out, want) and any("dynamic_linear_i8" in s for s in seen)
+    with torch.inference_mode():
+        assert torch.equal(lin(x), want)
+
+
+@torch.no_grad()
+def test_derived_operands_follow_updates_in_place():
+    """K = 200: the GEMM reads a zero-padded copy of the weight, which an update of the weight in place makes stale."""
+    x = torch.randn(24, 200, device="cuda").bfloat16()
+    lin = _module("token_i8", 200, 64, torch.bfloat16, True, x)
+    assert _native(lin, x) is not None
+    lin.qweight.neg_()
+    lin.weight_scale.mul_(2)
+    want = _general(lin, x)
+    assert torch.equal(_native(lin, x), want)
+
+
+@torch.no_grad()
+def test_streams_and_capture():
+    x = torch.randn(24, 256, device="cuda").bfloat16()
+    lin = _module("tensor_e4m3", 256, 64, torch.bfloat16, True, x)
+    want = lin(x)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        on_side = lin(x)
+    side.synchronize()
+    assert torch.equal(on_side, want)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = lin(x)
+    for _ in range(3):
+        x.mul_(-1)
+        want = _general(lin, x)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
