@@ -1,4 +1,4 @@
-// W8A8 GEMM for a handful of rows (gfx950): every wavefront streams its own part of the weight, no barriers in the K loop.
+// W8A8 GEMM for a handful of rows, or few outputs at all (gfx950): every wavefront streams its own part of the weight, no barriers in the K loop.
 //
 // What bounds it: every byte of the weight is needed once and multiplied with a few rows, so the launch is a stream of the
 // weight from HBM (26 MB at N = K = 5120: 4.3 us at 6.2 TB/s) and what counts is how many bytes are in flight.  The tiled
@@ -60,11 +60,11 @@ __global__ __launch_bounds__(64 * KS) void gemm_rows_kernel(const GemmArgs p) {
     const int lrow = lane >> 2;
     const uint32_t gsw = (uint32_t)(((lane & 3) ^ ((lrow >> 1) & 3)) << 4);
     const uint8_t* wbase = p.b + (int64_t)n0 * p.ldb + (int64_t)first * 128;
-    const uint8_t* xbase = p.a + (int64_t)first * 128;
+    const uint8_t* xbase = p.a + (int64_t)mbase * p.lda + (int64_t)first * 128;  // (32-bit offsets reach 64 rows)
     const uint32_t wcol = n0 + lrow < p.n ? lrow : p.n - 1 - n0;
     uint32_t woff = wcol * (uint32_t)p.ldb + gsw, xoff[MB];
 #pragma unroll
-    for (int i = 0; i < MB; ++i) xoff[i] = (uint32_t)(mbase + i * 16 + lrow < p.m ? mbase + i * 16 + lrow : p.m - 1) * (uint32_t)p.lda + gsw;
+    for (int i = 0; i < MB; ++i) xoff[i] = (uint32_t)(mbase + i * 16 + lrow < p.m ? i * 16 + lrow : p.m - 1 - mbase) * (uint32_t)p.lda + gsw;
     const uint32_t ring = (uint32_t)(uintptr_t)(DAXQ_LDS uint8_t*)smem + (uint32_t)wave * (R * STEP);
     auto load = [&](int step, uint32_t slot) __attribute__((always_inline)) {
         const uint8_t* w = wbase + (int64_t)step * 128;
@@ -248,18 +248,36 @@ static int launch_rows_one(const GemmArgs* args, hipStream_t st) {
 // Few workgroups (small n): cut K where the sums allow it, one row block per workgroup where they do not; many: two row
 // blocks, so that the activation is fetched half as often.  With more than 32 rows and N > 8192 the tiles, which fetch it
 // once per 128 columns, are as fast.
+// More than 128 rows (rows_applies says which): `blocks` of 16 x 16 outputs count the work.  us, 1,5,1 / 2,5,1 / 4,3,1 and for
+// INT8 2,3,4, beside the tiles (or, n < 128, the generic kernel):
+//   INT8  390 x 176, K = 3456 (275 blocks)  4.7 / 7.2 / - / 4.0, 11.9     543 x 254, K = 2688 (544)    4.4 / 6.3 / - / 5.0, 10.4
+//         392 x 819, K = 1408 (1300)        5.1 / 5.1 / 6.6 / 5.6, 8.7    242 x 2100, K = 8448 (2112) 32.3 / 26.0 / 23.4 / 26.3, 28.6
+//   e4m3  443 x 275, K = 3200 (504)         4.6 / 5.9 / 7.8, 12.0         331 x 644, K = 5888 (861)   11.7 / 10.9 / 12.0, 19.5
+//         338 x 1233, K = 6016 (1716)      18.1 / 15.5 / 14.2, 21.7       2032 x 46, K = 256 (381)     2.8 / 3.1 / 3.6, 13.6
+static int64_t row_blocks(int64_t m, int64_t n) { return ((m + 15) / 16) * ((n + 15) / 16); }
+
 template <bool FP8, int F8, int OUTK>
 static int launch_rows_out(const GemmArgs* a, hipStream_t st) {
     if (!a) {
         int rc = launch_rows_one<FP8, F8, 1, 10, 1, OUTK>(a, st);
         if (!rc) rc = launch_rows_one<FP8, F8, 1, 5, 1, OUTK>(a, st);
         if (!rc) rc = launch_rows_one<FP8, F8, 2, 5, 1, OUTK>(a, st);
+        if (!rc) rc = launch_rows_one<FP8, F8, 4, 3, 1, OUTK>(a, st);
         if constexpr (!FP8) {
             if (!rc) rc = launch_rows_one<FP8, F8, 1, 5, 4, OUTK>(a, st);
             if (!rc) rc = launch_rows_one<FP8, F8, 2, 3, 4, OUTK>(a, st);
             if (!rc) rc = launch_rows_one<FP8, F8, 4, 2, 4, OUTK>(a, st);
         }
         return rc;
+    }
+    if (a->m > 128) {
+        const int64_t blocks = row_blocks(a->m, a->n);
+        if constexpr (!FP8) {
+            if (blocks <= 512) return launch_rows_one<FP8, F8, 2, 3, 4, OUTK>(a, st);
+        }
+        if (blocks <= (FP8 ? 640 : 1024)) return launch_rows_one<FP8, F8, 1, 5, 1, OUTK>(a, st);
+        if (blocks <= 1280 || a->k < 2048) return launch_rows_one<FP8, F8, 2, 5, 1, OUTK>(a, st);
+        return launch_rows_one<FP8, F8, 4, 3, 1, OUTK>(a, st);
     }
     if constexpr (!FP8) {
         if (a->n < 4096 || a->m > 64) {
@@ -300,12 +318,25 @@ int prepare_rows_kernels() {
     return rc;
 }
 
-bool rows_applies(int64_t m, int64_t n) { return m <= (n > 8192 ? 32 : 128); }
+// Launches this kernel is the library's choice for.  At most 128 rows: see above.  More rows, where 128x128 tiles are few or
+// do not exist: such a tile takes 0.16 to 0.2 us per 64 bytes of K on its CU (its LDS traffic, 48 KB) while the CUs without
+// a tile idle, here every 16 x 16 outputs or a few of them are a wavefront.  A tile in five CUs is where the two meet
+// (2048 blocks of 16 x 16; e4m3 217 x 2391, K = 1408, 2100 blocks: 7.2 against 8.8 us, 418 x 1558, K = 3840, 2646: 13.8 / 14.9,
+// 784 x 1360, K = 384, 4165: 5.2 / 5.7, 291 x 3671, K = 2176, 4370: 14.7 / 11.3); INT8 launches of long K have split-K
+// beside them (450 x 1137, K = 12800: 32 against 27 us).  Fewer than 128 columns leave only the generic kernel (9191 x 79, K = 512:
+// 15.4 -> 6.9 us, 2404 x 74, K = 3072: 25.6 -> 8.2), which is as fast from about 4000 blocks at K = 4096 on.
+bool rows_applies(int64_t m, int64_t n, int64_t k, bool fp8) {
+    if (m <= 128) return m <= (n > 8192 ? 32 : 128);
+    if (m > (1 << 20) || n > (1 << 20)) return false;
+    const int64_t blocks = row_blocks(m, n), work = blocks * (k / 128);
+    if (n < 128) return work <= 65536;
+    return blocks <= 2048 && (fp8 || work <= 131072);
+}
 
-// at most 128 rows (32-bit row offsets), no accumulator dump
+// 32-bit row offsets, no accumulator dump
 int launch_rows(const GemmArgs& a, bool fp8, int f8, hipStream_t st) {
-    if (a.m > 128 || a.acc || a.lda >= (1 << 26) || a.ldb >= (1 << 26))
-        return fail(DAXQ_ERR_ARG, "linear: the kernel for few rows takes at most 128, row strides below 2^26 and no accumulator dump");
+    if (a.acc || a.lda >= (1 << 26) || a.ldb >= (1 << 26))
+        return fail(DAXQ_ERR_ARG, "linear: the kernel for few rows takes row strides below 2^26 and no accumulator dump");
     return launch_rows_any(&a, a.out_kind, fp8, f8, st);
 }
 

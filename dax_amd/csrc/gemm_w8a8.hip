@@ -246,7 +246,7 @@ int launch_tile_fp8(const GemmArgs& a, int f8, bool small, int tail, hipStream_t
 int launch_halves_i8(const GemmArgs& a, hipStream_t st);                                // gemm_tile256.hip
 int launch_halves_fp8(const GemmArgs& a, int f8, hipStream_t st);                       // gemm_tile_fp8.hip
 int launch_rows(const GemmArgs& a, bool fp8, int f8, hipStream_t st);                    // gemm_rows.hip
-bool rows_applies(int64_t m, int64_t n);
+bool rows_applies(int64_t m, int64_t n, int64_t k, bool fp8);
 template <bool FP8>
 int launch_tile128_splitk(const GemmArgs& a, int f8, hipStream_t st);
 
@@ -393,7 +393,7 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
             // 2048 x 4096 x 4096 (128) 39.6 -> 30.7 / 38.7 -> 31.2, 1024 x 5120, K = 13824 95.9 -> 69.3 / 93.1 -> 66.8,
             // 4096 x 1536, K = 8960 62.3 -> 50.7 / 60.5 -> 50.3, K = 3072 +9 to +15 % / +16 %, K = 2048 0 to +10 % / +2 %;
             // at K = 1536 -2 / -5 %, and with 60 tiles (768 x 5120 x 5120) the quadrants' 23.8 us become 30.5.
-            if (rows_applies(m, n) && fits32 && !acc) return launch_rows(a, FP8, f8, st);
+            if (rows_applies(m, n, k, FP8) && fits32 && !acc) return launch_rows(a, FP8, f8, st);
             const int64_t tiles256 = ((m + 255) / 256) * ((n + 255) / 256);
             const int cus = cu_count();
             if (tile256_applies(a) && k >= 2048 && cus >= 8 && 4 * tiles256 > cus && 2 * tiles256 <= cus) return launch_halves<FP8>(a, f8, st);
@@ -412,7 +412,9 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
         case K_TILED_HALVES:
             if (!tile256_applies(a)) return fail(DAXQ_ERR_ARG, "linear: the 256x128 kernel needs m, n >= 256");
             return launch_halves<FP8>(a, f8, st);
-        case K_ROWS: return launch_rows(a, FP8, f8, st);
+        case K_ROWS:
+            if (m > 128) return fail(DAXQ_ERR_ARG, "linear: the kernel for few rows takes at most 128 by name");
+            return launch_rows(a, FP8, f8, st);
         default: return fail(DAXQ_ERR_ARG, "linear: unknown kernel choice %d", which);
     }
 }
@@ -432,7 +434,7 @@ constexpr int64_t kMaxSplitTiles = kCounterBytes / 4;
 // 2 / 4 ranges): M = 256 (80 tiles) 34 / 28 / 40, M = 512 (160 tiles) 24 / 35 / 52, M = 1024 52 / 71 / -: the partial
 // results make a round trip through device-coherent memory (about 10 us for 20 MB), which only idle CUs pay for.
 static int splitk_choice(int64_t m, int64_t n, int64_t k) {
-    if (m < 128 || n < 128 || k % DAXQ_K_ALIGN || rows_applies(m, n)) return 1;
+    if (m < 128 || n < 128 || k % DAXQ_K_ALIGN || rows_applies(m, n, k, false)) return 1;
     const int64_t tiles = splitk_tiles(m, n), units = k / DAXQ_K_ALIGN;
     int best = 1;
     for (int s = 2; s <= 8; ++s)
@@ -655,7 +657,7 @@ int daxq_dynamic_linear(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int ac
     if (int rc = daxq_act_quant_rows_ex(x, x_dtype, x_fmt, m, k, ld_x, xq, ld_xq, sx, qmax, kEps, act_scale_round, stream)) return rc;
     // Fewer rows than the smallest tile of the tiled kernels, and more columns than the kernel for few rows is taken for: run
     // the tiled kernels on 128 rows of the caller's buffers when those reach that far (the rows beyond m hold whatever the buffers held; an output row depends on its own operand row only).
-    const bool rows = kernel == 0 && rows_applies(m, n);
+    const bool rows = kernel == 0 && rows_applies(m, n, kp, fp8);
     const int64_t mg = (!rows && m < 128 && rows_alloc >= 128 && n >= 128) ? 128 : m;
     hipStream_t st = (hipStream_t)stream;
     // INT8 launches with few tiles cut K into ranges when the caller brings a workspace (integer partial sums: the

@@ -302,7 +302,7 @@ int daxq_linear_e5m2_e4m3(const uint8_t* xq, int64_t ld_xq, const float* sx,
  * bits 2 / 5 = the generic kernel on 256x256 / 128x128 tiles (an implementation of its own, any shape), 8 / 11 / 14 =
  * the tiled kernel on 256x256 / 128x128 / 256x128 tiles (int8: 16x16x64 MFMAs; fp8: 16x16x128 MFMAs; needs m, n >= the
  * tile edge, 256 for the 256x128 tiles);
- * 17 = the kernel for at most 128 rows (weights streamed through a ring per wavefront; no accumulator dump);
+ * 17 = the kernel for at most 128 rows, by itself also taken for few outputs (weights streamed through a ring per wavefront; no accumulator dump);
  * bits 16-23, when not zero, set the depth of the tile-order groups; bits 24-27 the tile order of the 256x256 kernels
  * (0 = by shape, 1 = groups of tile rows, 2 = banded patches of 8 x 4 tiles per XCD; every order computes every tile
  * once, the results are the same bits); bits 28-29 the treatment of the last, partial round of workgroups of a launch
@@ -313,7 +313,7 @@ int daxq_linear_e5m2_e4m3(const uint8_t* xq, int64_t ld_xq, const float* sx,
  * 1 = never; 2 = whenever they number at most a quarter / half of the CUs).
  * int8 results are the same bits for every choice.  fp8 results are the same bits for every choice of tile size, tile
  * order and cut of the tiled kernel (one sequence of MFMAs per output element), so an output row does not depend on
- * how many rows the launch has; the generic kernel (any fp8 launch of more than 128 rows with n < 128) adds in another
+ * how many rows the launch has; the generic kernel (the larger fp8 launches with n < 128) adds in another
  * order and agrees to fp32 rounding.  Every kernel writes bf16, fp16 and fp32; the accumulator dump of the tiled
  * kernels exists with bf16 outputs.  The choice is an argument of the call: the library keeps no process-wide
  * selection.

@@ -79,3 +79,31 @@ def test_rows_outputs_as_a_slice_of_a_wider_buffer():
     assert torch.equal(view.cpu(), ref)
     view.fill_(7.0)
     assert bool((out == 7.0).all())
+
+
+# more than 128 rows: outputs of 16 x 16 blocks on either side of every count at which the form or the kernel changes, ragged in
+# both dimensions, fewer than 128 columns, K below and above 2048
+MANY = [(129, 40, 256), (130, 800, 384), (512, 256, 2176), (513, 260, 256), (640, 250, 640), (641, 256, 2176), (1023, 255, 2048), (1040, 257, 128),
+        (200, 1570, 2176), (300, 1715, 256), (257, 1936, 1920), (16, 1, 128), (5000, 17, 256), (2047, 127, 1152), (6001, 100, 384)]
+
+
+@pytest.mark.parametrize("m,n,k", MANY)
+def test_few_outputs_of_many_rows(m, n, k):
+    import dax_amd.ops as ops
+
+    g = torch.Generator().manual_seed(m + n)
+    sx, sw = torch.rand(m, generator=g) * 0.01, torch.rand(n, generator=g) * 0.01
+    xq = torch.randint(-128, 128, (m, k), generator=g, dtype=torch.int8)
+    wq = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8)
+    acc = O.int_mm(xq, wq)
+    for dtype in (torch.bfloat16, torch.float16, torch.float32):
+        bias = torch.randn(n, generator=g).to(dtype)
+        y = ops.linear_w8a8(xq.to("cuda"), sx.to("cuda"), wq.to("cuda"), sw.to("cuda"), bias.to("cuda"), "i8", "i8", dtype)
+        assert torch.equal(y.cpu(), O.epilogue_int8(acc, sx[:, None], sw, bias, out_dtype=dtype)), dtype
+    # FP8: an output row's bits do not depend on how many rows the launch has (128 at a time is the same kernel's other form)
+    x8 = torch.randn(m, k, generator=g).to(torch.float8_e4m3fn).view(torch.uint8).to("cuda")
+    w8 = torch.randn(n, k, generator=g).to(torch.float8_e4m3fn).view(torch.uint8).to("cuda")
+    sxd, swd = sx.to("cuda"), sw.to("cuda")
+    y = ops.linear_w8a8(x8, sxd, w8, swd, None, "e4m3", "e4m3", torch.bfloat16)
+    parts = [ops.linear_w8a8(x8[i:i + 128], sxd[i:i + 128].contiguous(), w8, swd, None, "e4m3", "e4m3", torch.bfloat16) for i in range(0, m, 128)]
+    assert torch.equal(y, torch.cat(parts))
