@@ -387,17 +387,28 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
             // M = 512 -> 1127 / 551, M = 1024 (80 large tiles) -> 1275 / 1055, M = 2048 (160) -> 1542 / 1817;
             // 4096 x 1536 x 1536 (96) -> 1182 / 895, 8192 x 1536 x 1536 (192) -> 1517 / 1587.
             // Between a quarter and a half of the CUs' worth of large tiles, every tile runs as its two 256x128 halves with
-            // a CU each (K >= 2048).  Measured against what these launches took before (128x128 tiles up to 127 large
+            // a CU each (K >= 2048), unless the 128x128 tiles get a CU each as well.  Measured against what these launches took
+            // before (128x128 tiles up to 127 large
             // tiles, whole 256x256 tiles at 128), INT8 / e4m3, us: 1024 x 5120 x 5120 (80 tiles) 38.7 -> 31.0 / 37.7 -> 29.6,
             // 1536 x 5120 x 5120 (120) 41.1 -> 35.0 / 40.3 -> 35.3, 1100 x 4352 x 5120 (85) 42.4 -> 31.6 / 41.1 -> 31.1,
             // 2048 x 4096 x 4096 (128) 39.6 -> 30.7 / 38.7 -> 31.2, 1024 x 5120, K = 13824 95.9 -> 69.3 / 93.1 -> 66.8,
-            // 4096 x 1536, K = 8960 62.3 -> 50.7 / 60.5 -> 50.3, K = 3072 +9 to +15 % / +16 %, K = 2048 0 to +10 % / +2 %;
-            // at K = 1536 -2 / -5 %, and with 60 tiles (768 x 5120 x 5120) the quadrants' 23.8 us become 30.5.
+            // 4096 x 1536, K = 8960 62.3 -> 50.7 / 60.5 -> 50.3; with 60 tiles (768 x 5120 x 5120) the quadrants' 23.8 us
+            // become 30.5, and ragged ones (3312 x 1070, K = 7424: 65 large tiles or 234 small ones) lose as much: 28.2 / 39.6;
+            // 5588 x 584, K = 6272 (66 / 220) 23.8 / 35.3.  Below K = 2048 a repeated launch gains 5 to 10 % (4096 x 1536 x 1536
+            // 16.7 -> 15.4), but behind its quantiser and on other operands each time, as in a model, it loses 10 (23.2 -> 26.0
+            // for the pair).
+            // A launch whose 128x128 tiles all fit at two per CU takes them although its large tiles number 128 and more
+            // (ragged edges: 2358 x 3239 is 130 large tiles or 494 small ones).  256x256 -> 128x128 tiles, INT8 / e4m3: that shape
+            // at K = 256 16.9 -> 11.3 / 17.6 -> 11.4, K = 1536 26.4 -> 20.5 / 26.4 -> 19.4 (behind its quantiser 34.0 -> 27.1),
+            // K = 5120 55.3 -> 49.5 / 52.3 -> 46.0, K = 13824 116 -> 110 / 113 -> 104; 2176 x 3840 (135 / 510) K = 13824 111 -> 110 /
+            // 108 -> 105.  From 513 small tiles on a second round of them starts: 4600 x 1800 (144 / 540) K = 1024 17.2 -> 18.3 /
+            // 16.4 -> 16.4, K = 3072 32.1 -> 37.4.
             if (rows_applies(m, n, k, FP8) && fits32 && !acc) return launch_rows(a, FP8, f8, st);
             const int64_t tiles256 = ((m + 255) / 256) * ((n + 255) / 256);
             const int cus = cu_count();
-            if (tile256_applies(a) && k >= 2048 && cus >= 8 && 4 * tiles256 > cus && 2 * tiles256 <= cus) return launch_halves<FP8>(a, f8, st);
-            if (tile256_applies(a) && tiles256 >= 128) return launch_tiled<FP8>(a, f8, false, tail, st);
+            const int64_t tiles128 = ((m + 127) / 128) * ((n + 127) / 128);
+            if (tile256_applies(a) && k >= 2048 && cus >= 8 && 4 * tiles256 > cus && 2 * tiles256 <= cus && tiles128 > cus) return launch_halves<FP8>(a, f8, st);
+            if (tile256_applies(a) && tiles256 >= 128 && tiles128 > 2 * cus) return launch_tiled<FP8>(a, f8, false, tail, st);
             if (m >= 128 && n >= 128 && fits32) return launch_tiled<FP8>(a, f8, true, 1, st);
             return launch_generic<FP8, 128>(a, f8, st);
         }
