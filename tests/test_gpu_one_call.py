@@ -116,16 +116,11 @@ def test_derived_operands_follow_updates_in_place():
 
 
 @torch.no_grad()
-def test_streams_and_capture():
+def test_capture():
+    """On the capture's own stream, which is not the default one."""
     x = torch.randn(24, 256, device="cuda").bfloat16()
     lin = _module("tensor_e4m3", 256, 64, torch.bfloat16, True, x)
-    want = lin(x)
-    side = torch.cuda.Stream()
-    side.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(side):
-        on_side = lin(x)
-    side.synchronize()
-    assert torch.equal(on_side, want)
+    lin(x)
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
         out = lin(x)
