@@ -104,6 +104,17 @@ def test_calls_that_are_not_plain_take_the_op():
 
 
 @torch.no_grad()
+def test_a_lazily_negated_tensor_is_materialised():
+    """The bytes of a tensor with the negative bit are those of -x."""
+    x = torch.randn(24, 256, device="cuda").bfloat16()
+    for scheme in ("token_i8", "tensor_e4m3", "static_e5m2"):
+        lin = _module(scheme, 256, 64, torch.bfloat16, True, x)
+        neg = torch._neg_view(x)
+        assert neg.is_neg() and _native(lin, neg) is None
+        assert torch.equal(lin(neg), lin(-x))
+
+
+@torch.no_grad()
 def test_derived_operands_follow_updates_in_place():
     """K = 200: the GEMM reads a zero-padded copy of the weight, which an update of the weight in place makes stale."""
     x = torch.randn(24, 200, device="cuda").bfloat16()
