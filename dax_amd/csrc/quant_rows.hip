@@ -162,7 +162,11 @@ constexpr int kPartials = 256;  // workgroups of tensor_amax_kernel, one per CU
 // address, against one workgroup per row that read them twice, element by element: 4096 x 5120 fp32 43.9 -> 19.7 us,
 // 2900 x 1001 bf16 6.1 -> 3.7 us.
 // SCALE_IN: the per-row scale is an input (leaf quantiser) instead of being derived from the row.
-template <int NCH, int W, int FMT, bool SCALE_IN, int XT>
+// PLAIN: bf16 rows of whole chunks under their own scales, bytes as kOwn: what the DiT's linears launch.  The loads and the
+// stores then sit in one straight piece of code; with the other forms' branches between them a wavefront issues later, which
+// short rows feel most.  us, all forms in one / PLAIN, INT8 (e4m3): 32760 x 1536 26.0 / 24.3 (26.2 / 24.5), 4096 x 2048 6.2 / 6.0
+// (6.3 / 6.2), 9450 x 5120 24.2 / 23.4 (24.4 / 23.8), 516 x 5120 3.4 / 3.2 (3.6 / 3.4); none of eighteen slower.
+template <int NCH, int W, int FMT, bool SCALE_IN, int XT, bool PLAIN>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
     constexpr int XB = XT == DAXQ_F32 ? 4 : 2;
     __shared__ uint32_t s_max[4];
@@ -175,10 +179,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
     const char* xr = a.x + row * a.ld_x * XB;
     // what whole chunks do not cover -- the columns behind the last of them, and a width or fill that is no multiple of
     // 8 -- is one element per lane of the row's first wavefront
-    const bool ragged = ((a.k | a.kfill) & 7) != 0;
+    const bool ragged = !PLAIN && ((a.k | a.kfill) & 7) != 0;
 
     Chunk<XT> v[NCH];
-    if (nch > 0) {
+    if (PLAIN || nch > 0) {
 #pragma unroll
         for (int i = 0; i < NCH; ++i) {
             const int c = (i * W + part) * 64 + lane;
@@ -200,7 +204,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
         if (a.scale && part == 0 && lane == 0) a.scale[row] = s;
     } else {
         uint32_t mx = 0;
-        if (a.partials) {  // every wavefront finds the tensor's maximum in 1 KB of L2 while its row arrives
+        if (!PLAIN && a.partials) {  // every wavefront finds the tensor's maximum in 1 KB of L2 while its row arrives
             const uint4 p = reinterpret_cast<const uint4*>(a.partials)[lane];
             const uint32_t lo = p.x > p.y ? p.x : p.y, hi = p.z > p.w ? p.z : p.w;
             mx = lo > hi ? lo : hi;
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
             mx = t > mx ? t : mx;
         }
         uint32_t amax = wave_max_u32(mx);
-        if (W > 1 && !a.partials) {
+        if (W > 1 && (PLAIN || !a.partials)) {
             if (lane == 0) s_max[wave] = amax;
             __syncthreads();
 #pragma unroll
@@ -224,7 +228,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
         s = scale_from_amax_bits_rt<XT>(amax, a.qmax, a.eps, a.round_x);
         if (part == 0 && lane == 0) {
             a.scale[row] = s;
-            if (a.scale1 && row == 0) a.scale1[0] = s;
+            if (!PLAIN && a.scale1 && row == 0) a.scale1[0] = s;
         }
     }
     if (W > 1 && row0 >= a.m) return;
@@ -245,7 +249,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
     };
     constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
     constexpr bool kOwnForm = !SCALE_IN && XT == DAXQ_BF16;
-    if (kOwnForm && a.qmax <= kFmtMax && (FMT == 0 || a.round_x)) {
+    if (PLAIN || (kOwnForm && a.qmax <= kFmtMax && (FMT == 0 || a.round_x))) {
         store(std::integral_constant<int, kOwn>{});
     } else if constexpr (FMT == 0) {
         store(std::integral_constant<int, kDivide>{});
@@ -347,9 +351,14 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
         QuantArgs a{static_cast<const char*>(x), m, ld_x, (int)k, (int)kfill, qp, ld_q, SCALE_IN ? t.scale_rows : scale, scale,
                     t.one_scale ? 0 : 1, t.partials, t.scale1, qmax, eps, round_x};
         const int cols = (int)((kfill + 511) / 512);
+        constexpr bool kMayBePlain = !SCALE_IN && XT == DAXQ_BF16;
+        constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
+        const bool plain = kMayBePlain && ((k | kfill) & 7) == 0 && !t.partials && qmax <= kFmtMax && (FMT == 0 || round_x);
 #define DAXQ_Q_CASE(N, W)                                                                                                  \
     if (cols <= N * W) {                                                                                                   \
-        hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT>), dim3((unsigned)((m + 4 / W - 1) / (4 / W))), dim3(256), 0, st, a); \
+        const dim3 grid((unsigned)((m + 4 / W - 1) / (4 / W)));                                                            \
+        if (plain) hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain>), grid, dim3(256), 0, st, a); \
+        else hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false>), grid, dim3(256), 0, st, a);            \
         return check_launch("quant_rows");                                                                                 \
     }
         DAXQ_Q_CASE(1, 1)

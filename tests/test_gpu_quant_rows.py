@@ -140,3 +140,22 @@ def test_row_statistics_and_weights_in_one_pass(ops, dtype, n, k, pitch):
         bad[n // 2, k // 2] = sign * float("nan")
         lo, hi = ops.row_minmax(bad)
         assert torch.equal(torch.isnan(lo), torch.arange(n, device="cuda") == n // 2) and torch.equal(torch.isnan(hi), torch.isnan(lo))
+
+
+@pytest.mark.parametrize("fmt", ["i8", "e4m3", "e5m2"])
+@pytest.mark.parametrize("k", [8, 64, 504, 512, 520, 1024, 1536, 2048, 2056, 3072, 4104, 6144, 8192, 14336, 18424])
+@pytest.mark.parametrize("m", [1, 5])
+def test_rows_of_whole_chunks_and_rows_with_a_ragged_end_agree(ops, fmt, k, m):
+    """The kernel for rows of whole chunks against the one for any row: a zero column more changes neither scale nor bytes."""
+    g = torch.Generator().manual_seed(k + m)
+    x = (torch.randn(m, k, generator=g) * 3).bfloat16()
+    if m > 1:
+        x[1] = 0
+        x[2, k // 2] = float("inf")
+        x[3, k - 1] = float("nan")
+    wide = torch.cat([x, torch.zeros(m, 1, dtype=x.dtype)], dim=1)
+    quant = getattr(ops, "act_quant_" + fmt)
+    q, s = quant(x.cuda())
+    qw, sw = quant(wide.cuda())
+    assert torch.equal(s.view(torch.int32), sw.view(torch.int32))
+    assert torch.equal(q[:, :k].view(torch.uint8), qw[:, :k].view(torch.uint8)) and not q[:, k:].view(torch.uint8).any()
