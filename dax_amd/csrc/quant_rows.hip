@@ -76,9 +76,11 @@ __device__ __forceinline__ void chunk_values(const Chunk<XT>& v, float (&f)[8]) 
 //   kNear      FP8 under any other scale: x * inv, whose error is at most 1.5 steps of fp32, rounds to the byte of x / s
 //              unless it lies that close to a value where the byte changes.  Those values, in the normal and the subnormal
 //              range of either format, have at most five significant bits, i.e. zeros in the low 19 bits of the fp32
-//              pattern, so a product within three steps of such a pattern sends its chunk through the division (five
-//              elements in 10^6 under an arbitrary scale; zeros and infinities too).  Measured with a scale from the
-//              caller, 4096 x 5120 e5m2: 18.9 us dividing every element (26 VALU issue slots), 11.4 us here.
+//              pattern, so a product within three steps of such a pattern sends the wavefront's chunks through the
+//              division (seven patterns in 2^19, 13 elements in 10^6 under an arbitrary scale; zeros and infinities
+//              too).  A NaN does as well: a bf16 NaN has zeros in 16 low bits only, the rest of its payload lies in
+//              those 19, so it is looked for by itself.  Measured with a scale from the
+//              caller, 4096 x 5120 e5m2: 18.9 us dividing every element (26 VALU issue slots), 11.6 us here.
 //   kExact     FP8 under a power of two: x * inv is the quotient
 //   kShort     bf16 elements under a bf16 scale from the caller (a per-tensor scale): their quotients hit such values all
 //              the time; the sequence of kOwn, clamped, and the division for chunks that hold an infinity or a NaN
@@ -117,7 +119,7 @@ __device__ __forceinline__ uint2 quant8(const float (&f)[8], float s, float inv)
                     const uint32_t d = (__float_as_uint(q0) << 13) + (3u << 13);
                     near = d < near ? d : near;
                 }
-                if (XT != DAXQ_BF16 || FORM != kNear) nan |= q0 != q0;  // (a bf16 NaN has zeros in its low bits)
+                nan |= q0 != q0;
                 v[i] = __builtin_amdgcn_fmed3f(q0, -kMax, kMax);
             }
             if (__ballot((FORM == kNear && near <= (6u << 13)) || nan)) {

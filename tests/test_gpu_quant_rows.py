@@ -159,3 +159,23 @@ def test_rows_of_whole_chunks_and_rows_with_a_ragged_end_agree(ops, fmt, k, m):
     qw, sw = quant(wide.cuda())
     assert torch.equal(s.view(torch.int32), sw.view(torch.int32))
     assert torch.equal(q[:, :k].view(torch.uint8), qw[:, :k].view(torch.uint8)) and not q[:, k:].view(torch.uint8).any()
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+@pytest.mark.parametrize("scale", [0.1, 1.0 / 3.0, 0.75, 0.5, 2.0 ** 110])  # arbitrary, bf16, a power of two, one that divides
+def test_every_bf16_nan_stays_nan_under_a_scale_from_the_caller(ops, fmt, scale):
+    """Every NaN pattern of bf16, both signs, as the only special value of its row, among elements whose quotients lie far
+    from every value where a byte changes: the NaN element becomes the format's NaN byte, the others their own bytes."""
+    bits = np.concatenate([np.arange(0x7f81, 0x8000), np.arange(0xff81, 0x10000)]).astype(np.uint16)
+    m, k = bits.size, 520
+    x = torch.full((m, k), 1.296875, dtype=torch.bfloat16)
+    at = torch.arange(m) * 37 % k
+    x.view(torch.int16)[torch.arange(m), at] = torch.from_numpy(bits.view(np.int16))
+    sc = torch.tensor([scale])
+    row = O.quantize_to_fp8(torch.full((1, k), 1.296875, dtype=torch.bfloat16), sc[:, None], FP8[fmt]).view(torch.uint8)
+    for q in (getattr(ops, "quantize_rows_" + fmt)(x.to("cuda"), sc.expand(m).contiguous().to("cuda")),
+              ops.quantize_tensor(x.to("cuda"), sc.to("cuda"), fmt, False)[0]):
+        got = q.cpu()
+        nan = torch.isnan(got.view(FP8[fmt]).float())
+        assert torch.equal(nan, torch.arange(k)[None, :] == at[:, None])
+        assert torch.equal(got[~nan], row.expand(m, k)[~nan])
