@@ -250,8 +250,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
         }
     };
     constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
+    // (an infinity makes the tensor's scale infinite: the other elements are then x / inf = 0, which the reciprocal sequence
+    // gives as NaN, and the infinity itself is inf / inf)
     constexpr bool kOwnForm = !SCALE_IN && XT == DAXQ_BF16;
-    if (PLAIN || (kOwnForm && a.qmax <= kFmtMax && (FMT == 0 || a.round_x))) {
+    if (PLAIN || (kOwnForm && a.qmax <= kFmtMax && (FMT == 0 || a.round_x) && (!a.partials || s < __builtin_inff()))) {
         store(std::integral_constant<int, kOwn>{});
     } else if constexpr (FMT == 0) {
         store(std::integral_constant<int, kDivide>{});

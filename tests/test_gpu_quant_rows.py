@@ -179,3 +179,23 @@ def test_every_bf16_nan_stays_nan_under_a_scale_from_the_caller(ops, fmt, scale)
         nan = torch.isnan(got.view(FP8[fmt]).float())
         assert torch.equal(nan, torch.arange(k)[None, :] == at[:, None])
         assert torch.equal(got[~nan], row.expand(m, k)[~nan])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("fmt", ["i8", "e4m3", "e5m2"])
+@pytest.mark.parametrize("k", [8, 520, 1001, 5120])
+def test_an_infinity_in_a_tensor_under_one_scale(ops, dtype, fmt, k):
+    """The scale of the tensor is infinite: every finite element is x / inf, a zero with x's sign, and the infinity itself is
+    inf / inf: the bytes of the leaf quantiser under that scale."""
+    x = torch.randn(5, k, generator=torch.Generator().manual_seed(k)).to(dtype)
+    for bad in (float("inf"), -float("inf")):
+        x[2, k // 3] = bad
+        q, s, s1 = ops.act_quant_tensor(x.to("cuda"), fmt, ops.QMAX[fmt], ops.EPS_F32, True, False)
+        assert bool(torch.isinf(s1).all()) and torch.equal(s, s1.expand(5))
+        assert torch.equal(q, getattr(ops, "quantize_rows_" + fmt)(x.to("cuda"), s))
+        finite = torch.isfinite(x)
+        if fmt == "i8":
+            assert not q.cpu()[finite].any()
+        else:
+            assert torch.equal(q.cpu()[finite] & 0x7f, torch.zeros_like(q.cpu()[finite]))
+            assert bool(torch.isnan(q.cpu().view(FP8[fmt]).float()[~finite]).all())
