@@ -45,6 +45,7 @@ SIGNATURES = {
     "daxq_row_minmax": [_P, _I64, _I64, _I64, _P, _P, _P],
     "daxq_row_minmax_t": [_P, _INT, _I64, _I64, _I64, _P, _P, _P],
     "daxq_act_quant_rows": [_P, _INT, _INT, _I64, _I64, _I64, _P, _I64, _P, _P],
+    "daxq_weight_quant_rows": [_P, _INT, _INT, _I64, _I64, _I64, _P, _I64, _P, _F32, _F32, _P],
     "daxq_act_quant_rows_ex": [_P, _INT, _INT, _I64, _I64, _I64, _P, _I64, _P, _F32, _F32, _INT, _P],
     "daxq_quantize_rows": [_P, _INT, _INT, _I64, _I64, _I64, _P, _P, _I64, _P],
     "daxq_block_scale": [_P, _INT, _INT, C.POINTER(_I64), C.POINTER(C.c_int32), _F32, _F32, _INT, _P, _P],

@@ -152,6 +152,7 @@ struct QuantArgs {
     float* scale1;            // ... and where that one scale goes besides (or null)
     float qmax, eps;          // dynamic scale: divisor and floor,
     int round_x;              // and whether both are rounded to the element type
+    int leaf;                 // the scale is a tensor's or a weight's: the leaf quantiser's bytes also where it is not finite
 };
 constexpr int kPartials = 256;  // workgroups of tensor_amax_kernel, one per CU
 
@@ -250,10 +251,10 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
         }
     };
     constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
-    // (an infinity makes the tensor's scale infinite: the other elements are then x / inf = 0, which the reciprocal sequence
-    // gives as NaN, and the infinity itself is inf / inf)
+    // (leaf: under an infinite scale a finite element is x / inf = 0, which the reciprocal sequence gives as NaN, and an
+    // infinity is inf / inf, whose int8 byte depends on the clamp; so does that of a NaN)
     constexpr bool kOwnForm = !SCALE_IN && XT == DAXQ_BF16;
-    if (PLAIN || (kOwnForm && a.qmax <= kFmtMax && (FMT == 0 || a.round_x) && (!a.partials || s < __builtin_inff()))) {
+    if (PLAIN || (kOwnForm && a.qmax <= kFmtMax && (FMT == 0 || a.round_x) && (!a.leaf || s < __builtin_inff()))) {
         store(std::integral_constant<int, kOwn>{});
     } else if constexpr (FMT == 0) {
         store(std::integral_constant<int, kDivide>{});
@@ -332,17 +333,18 @@ __global__ __launch_bounds__(256) void quant_rows_block(const void* __restrict__
     }
 }
 
-// One scale for the whole tensor instead of one per row (QuantArgs)
-struct TensorScale {
+// Anything but a dynamic scale per token or the caller's per row (QuantArgs)
+struct ScaleKind {
     bool one_scale = false;              // the caller's scale is one value; scale_rows: where it goes once per row (or null)
     float* scale_rows = nullptr;
     const uint32_t* partials = nullptr;  // the scale comes from the tensor's abs-max; scale1: where it goes besides (or null)
     float* scale1 = nullptr;
+    bool weight = false;                 // rows of a weight: the leaf quantiser's bytes also under a scale that is not finite
 };
 
 template <int FMT, bool SCALE_IN, int XT>
 static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q, float* scale,
-                               float qmax, hipStream_t st, float eps, int round_x, const TensorScale& t) {
+                               float qmax, hipStream_t st, float eps, int round_x, const ScaleKind& t) {
     constexpr int XB = XT == DAXQ_F32 ? 4 : 2;
     if (m < 0 || k <= 0 || ld_x < k || ld_q < k) return fail(DAXQ_ERR_ARG, "quant_rows: bad shape m=%lld k=%lld ld_x=%lld ld_q=%lld",
                                                                (long long)m, (long long)k, (long long)ld_x, (long long)ld_q);
@@ -353,11 +355,11 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
     uint8_t* qp = static_cast<uint8_t*>(q);
     if (kfill <= 36 * 512 && m <= 0x7fffffff) {
         QuantArgs a{static_cast<const char*>(x), m, ld_x, (int)k, (int)kfill, qp, ld_q, SCALE_IN ? t.scale_rows : scale, scale,
-                    t.one_scale ? 0 : 1, t.partials, t.scale1, qmax, eps, round_x};
+                    t.one_scale ? 0 : 1, t.partials, t.scale1, qmax, eps, round_x, t.partials || t.weight};
         const int cols = (int)((kfill + 511) / 512);
         constexpr bool kMayBePlain = !SCALE_IN && XT == DAXQ_BF16;
         constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
-        const bool plain = kMayBePlain && ((k | kfill) & 7) == 0 && !t.partials && qmax <= kFmtMax && (FMT == 0 || round_x);
+        const bool plain = kMayBePlain && ((k | kfill) & 7) == 0 && !a.leaf && qmax <= kFmtMax && (FMT == 0 || round_x);
 #define DAXQ_Q_CASE(N, W)                                                                                                  \
     if (cols <= N * W) {                                                                                                   \
         const dim3 grid((unsigned)((m + 4 / W - 1) / (4 / W)));                                                            \
@@ -392,7 +394,7 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
 // eps, round_x: floor and rounding of a dynamic scale (scale_from_amax_bits_rt); unused when the scale is an input
 template <int FMT, bool SCALE_IN>
 static int launch_quant_rows(const void* x, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q, float* scale,
-                             float qmax, hipStream_t st, int x_dtype = DAXQ_BF16, float eps = kEps, int round_x = 1, const TensorScale& t = {}) {
+                             float qmax, hipStream_t st, int x_dtype = DAXQ_BF16, float eps = kEps, int round_x = 1, const ScaleKind& t = {}) {
     if (!SCALE_IN && (!(qmax > 0.0f) || !(eps >= 0.0f))) return fail(DAXQ_ERR_ARG, "quant_rows: quant_max must be positive and eps not negative");
     switch (x_dtype) {
         case DAXQ_BF16: return launch_quant_rows_t<FMT, SCALE_IN, DAXQ_BF16>(x, m, k, ld_x, q, ld_q, scale, qmax, st, eps, round_x, t);
@@ -405,7 +407,7 @@ static int launch_quant_rows(const void* x, int64_t m, int64_t k, int64_t ld_x, 
 // qmax <= 0: the format's own maximum
 template <bool SCALE_IN>
 static int launch_quant_rows_fmt(int q_fmt, const void* x, int x_dtype, int64_t m, int64_t k, int64_t ld_x, void* q,
-                                 int64_t ld_q, float* scale, hipStream_t st, float qmax = 0.0f, float eps = kEps, int round_x = 1, const TensorScale& t = {}) {
+                                 int64_t ld_q, float* scale, hipStream_t st, float qmax = 0.0f, float eps = kEps, int round_x = 1, const ScaleKind& t = {}) {
     switch (q_fmt) {
         case DAXQ_FMT_I8: return launch_quant_rows<0, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 127.0f, st, x_dtype, eps, round_x, t);
         case DAXQ_FMT_E4M3: return launch_quant_rows<1, SCALE_IN>(x, m, k, ld_x, q, ld_q, scale, qmax > 0.0f ? qmax : 448.0f, st, x_dtype, eps, round_x, t);
@@ -632,6 +634,14 @@ int daxq_act_quant_rows_ex(const void* x, int x_dtype, int q_fmt, int64_t m, int
                                                     eps, scale_round == DAXQ_SCALE_ROUND_X);
 }
 
+int daxq_weight_quant_rows(const void* w, int w_dtype, int q_fmt, int64_t n, int64_t k, int64_t ld_w, void* q, int64_t ld_q, float* scale,
+                           float quant_max, float eps, daxq_stream_t stream) {
+    if (!(quant_max > 0.0f)) return daxq::fail(DAXQ_ERR_ARG, "weight_quant_rows: quant_max must be positive");
+    daxq::ScaleKind t;
+    t.weight = true;
+    return daxq::launch_quant_rows_fmt<false>(q_fmt, w, w_dtype, n, k, ld_w, q, ld_q, scale, (hipStream_t)stream, quant_max, eps, 0, t);
+}
+
 int daxq_quantize_rows(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, const float* scale,
                        void* q, int64_t ld_q, daxq_stream_t stream) {
     return daxq::launch_quant_rows_fmt<true>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, const_cast<float*>(scale),
@@ -660,7 +670,7 @@ int daxq_act_quant_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int6
         default: return fail(DAXQ_ERR_ARG, "act_quant_tensor: unknown element type %d", x_dtype);
     }
     if (int rc = check_launch("tensor_amax")) return rc;
-    TensorScale t;
+    ScaleKind t;
     t.partials = part;
     t.scale1 = scale1;
     return launch_quant_rows_fmt<false>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, scale_rows, st, quant_max, eps, scale_round == DAXQ_SCALE_ROUND_X, t);
@@ -668,7 +678,7 @@ int daxq_act_quant_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int6
 
 int daxq_quantize_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, const float* scale1, void* q,
                          int64_t ld_q, float* scale_rows, daxq_stream_t stream) {
-    daxq::TensorScale t;
+    daxq::ScaleKind t;
     t.one_scale = true;
     t.scale_rows = scale_rows;
     return daxq::launch_quant_rows_fmt<true>(q_fmt, x, x_dtype, m, k, ld_x, q, ld_q, const_cast<float*>(scale1), (hipStream_t)stream, 0.0f,

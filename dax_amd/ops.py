@@ -453,8 +453,8 @@ def weight_quant(w: torch.Tensor, fmt: str, quant_max: float, eps: float) -> Tup
         q = torch.empty((n, k), dtype=torch.int8 if fmt == "i8" else torch.uint8, device=w.device)
         s = torch.empty((n,), dtype=torch.float32, device=w.device)
         if n:
-            _capi.check(_capi.lib().daxq_act_quant_rows_ex(w.data_ptr(), kind, FMT[fmt], n, k, w.stride(0) if n > 1 else k, q.data_ptr(), k,
-                                                           s.data_ptr(), quant_max, eps, 0, _stream(w)), name)
+            _capi.check(_capi.lib().daxq_weight_quant_rows(w.data_ptr(), kind, FMT[fmt], n, k, w.stride(0) if n > 1 else k, q.data_ptr(), k,
+                                                           s.data_ptr(), quant_max, eps, _stream(w)), name)
     return q, s
 
 

@@ -177,6 +177,11 @@ int daxq_act_quant_rows_ex(const void* x, int x_dtype, int q_fmt, int64_t m, int
                            daxq_stream_t stream);
 int daxq_quantize_rows(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, const float* scale,
                        void* q, int64_t ld_q, daxq_stream_t stream);
+/* Per-output-channel quantisation of a weight in one pass: daxq_act_quant_rows_ex with DAXQ_SCALE_ROUND_NONE, and the bytes
+ * of daxq_quantize_rows under the scale it writes for every row, rows that hold an infinity or a NaN among them.
+ *   dax/quant/quantization/observer.py:97-134, dax/quant/nn/quantized/functional.py:11-20 */
+int daxq_weight_quant_rows(const void* w, int w_dtype, int q_fmt, int64_t n, int64_t k, int64_t ld_w, void* q, int64_t ld_q,
+                           float* scale, float quant_max, float eps, daxq_stream_t stream);
 
 /*
  * Any other block shape of _dynamic_quantize_func (dax/quant/nn/dynamic/functional.py:54-148: per-channel

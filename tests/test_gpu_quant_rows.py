@@ -199,3 +199,23 @@ def test_an_infinity_in_a_tensor_under_one_scale(ops, dtype, fmt, k):
         else:
             assert torch.equal(q.cpu()[finite] & 0x7f, torch.zeros_like(q.cpu()[finite]))
             assert bool(torch.isnan(q.cpu().view(FP8[fmt]).float()[~finite]).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("fmt", ["i8", "e4m3", "e5m2"])
+@pytest.mark.parametrize("k", [8, 77, 1024, 18440])
+def test_weights_that_hold_infinities_and_nans(ops, dtype, fmt, k):
+    """The one-pass weight quantiser gives such rows the scale and the bytes of statistics, scale and leaf quantiser, too."""
+    w = torch.randn(6, k, generator=torch.Generator().manual_seed(k))
+    for row, bad in ((1, float("inf")), (2, -float("inf")), (4, float("nan"))):
+        w[row, k // 2] = bad
+    w = w.to(dtype).to("cuda")
+    s = ops.scale_from_minmax(*ops.row_minmax(w), ops.QMAX[fmt])
+    q = getattr(ops, "quantize_rows_" + fmt)(w, s)
+    q1, s1 = ops.weight_quant(w, fmt, ops.QMAX[fmt], ops.EPS_F32)
+    assert torch.equal(torch.isnan(s1), torch.isnan(s)) and torch.equal(torch.nan_to_num(s1, nan=1.0), torch.nan_to_num(s, nan=1.0))
+    if fmt == "i8":
+        assert torch.equal(q1, q)
+    else:  # (a NaN's sign is not compared)
+        a, b = q1.view(FP8[fmt]).float(), q.view(FP8[fmt]).float()
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(q1[~torch.isnan(a)], q[~torch.isnan(a)])
