@@ -275,7 +275,7 @@ class Linear(DerivedOperands, nn.Module):
 
         if weight_post_process.dtype not in FP8_ALLOWED_DTYPES and weight_post_process.dtype != torch.int8:
             raise NotImplementedError(f"Unsupported dtype {weight_post_process.dtype}")
-        if fresh_observer and weight_post_process.ch_axis == 0:
+        if fresh_observer and weight_post_process.ch_axis == 0 and w.numel():  # (an empty weight gives no statistics)
             # nobody looks at this observer again: its statistics, the scales and the bytes are one pass over the weight
             if w.stride(1) != 1:
                 w = w.contiguous()

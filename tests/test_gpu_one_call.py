@@ -141,3 +141,13 @@ def test_capture():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("k,n", [(0, 8), (16, 0)])
+@torch.no_grad()
+def test_conversion_of_an_empty_weight(k, n):
+    """A weight without elements gives its observer no statistics: the module is built and its scales stay ones."""
+    model = nn.Sequential(nn.Linear(k, n, bias=True).to("cuda", torch.bfloat16))
+    quantize_dynamic(model, {"": DYNAMIC["token_i8"]()})
+    assert model[0].qweight.shape == (n, k) and model[0].weight_scale.shape == (1, n)
+    assert bool((model[0].weight_scale == 1).all())
