@@ -342,6 +342,20 @@ struct ScaleKind {
     bool weight = false;                 // rows of a weight: the leaf quantiser's bytes also under a scale that is not finite
 };
 
+// at most `count` rows of `a` from row r on
+template <int XB>
+static QuantArgs rows_from(const QuantArgs& a, int64_t r, int64_t count) {
+    QuantArgs b = a;
+    if (b.m - r < count) count = b.m - r;
+    b.m = count;
+    b.x += r * a.ld_x * XB;
+    b.q += r * a.ld_q;
+    if (b.scale) b.scale += r;
+    b.scale_in += r * a.scale_stride;
+    if (r) b.scale1 = nullptr;
+    return b;
+}
+
 template <int FMT, bool SCALE_IN, int XT>
 static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q, float* scale,
                                float qmax, hipStream_t st, float eps, int round_x, const ScaleKind& t) {
@@ -353,18 +367,23 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
     const int64_t kfill = fill_width(k, ld_q);
     if (((uintptr_t)x & (XB - 1)) != 0 || ((uintptr_t)scale & 3) != 0) return fail(DAXQ_ERR_ALIGN, "quant_rows: x must be element aligned and scale 4-byte aligned");
     uint8_t* qp = static_cast<uint8_t*>(q);
-    if (kfill <= 36 * 512 && m <= 0x7fffffff) {
-        QuantArgs a{static_cast<const char*>(x), m, ld_x, (int)k, (int)kfill, qp, ld_q, SCALE_IN ? t.scale_rows : scale, scale,
+    if (kfill <= 36 * 512) {
+        const QuantArgs a{static_cast<const char*>(x), m, ld_x, (int)k, (int)kfill, qp, ld_q, SCALE_IN ? t.scale_rows : scale, scale,
                     t.one_scale ? 0 : 1, t.partials, t.scale1, qmax, eps, round_x, t.partials || t.weight};
         const int cols = (int)((kfill + 511) / 512);
         constexpr bool kMayBePlain = !SCALE_IN && XT == DAXQ_BF16;
         constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
         const bool plain = kMayBePlain && ((k | kfill) & 7) == 0 && !a.leaf && qmax <= kFmtMax && (FMT == 0 || round_x);
+        // A launch holds fewer than 2^32 work items, i.e. 2^24 workgroups: more rows are as many launches as they need
 #define DAXQ_Q_CASE(N, W)                                                                                                  \
     if (cols <= N * W) {                                                                                                   \
-        const dim3 grid((unsigned)((m + 4 / W - 1) / (4 / W)));                                                            \
-        if (plain) hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain>), grid, dim3(256), 0, st, a); \
-        else hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false>), grid, dim3(256), 0, st, a);            \
+        constexpr int64_t kRows = 4 / W, kSlab = kRows << 23;                                                              \
+        for (int64_t r = 0; r < m; r += kSlab) {                                                                           \
+            const QuantArgs b = rows_from<XB>(a, r, kSlab);                                                                \
+            const dim3 grid((unsigned)((b.m + kRows - 1) / kRows));                                                        \
+            if (plain) hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain>), grid, dim3(256), 0, st, b); \
+            else hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false>), grid, dim3(256), 0, st, b);        \
+        }                                                                                                                  \
         return check_launch("quant_rows");                                                                                 \
     }
         DAXQ_Q_CASE(1, 1)

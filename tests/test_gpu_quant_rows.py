@@ -219,3 +219,40 @@ def test_weights_that_hold_infinities_and_nans(ops, dtype, fmt, k):
     else:  # (a NaN's sign is not compared)
         a, b = q1.view(FP8[fmt]).float(), q.view(FP8[fmt]).float()
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(q1[~torch.isnan(a)], q[~torch.isnan(a)])
+
+
+def test_more_rows_than_one_launch_holds(ops):
+    """2^25 rows of one wavefront each per launch: scales, bytes and the single scale on either side of the cut."""
+    cut, k = 1 << 25, 8
+    m = cut + 5
+    x = torch.ones(m, k, dtype=torch.bfloat16, device="cuda")
+    at = torch.tensor([0, 1, cut - 1, cut, cut + 1, m - 1], device="cuda")
+    x[at] = (torch.arange(1, 7, device="cuda")[:, None] * torch.arange(1, k + 1, device="cuda")).bfloat16()
+    q, s = ops.act_quant_i8(x[:, :k])
+    qs, ss = ops.act_quant_i8(x[at])
+    assert torch.equal(q[at], qs) and torch.equal(s[at], ss)
+    assert bool((s[7:cut - 7] == s[7]).all())
+    del q
+    scale = torch.full((m,), 0.25, device="cuda")
+    scale[at] = torch.arange(1, 7, device="cuda") * 0.125
+    q = ops.quantize_rows_e4m3(x, scale)
+    assert torch.equal(q[at], ops.quantize_rows_e4m3(x[at], scale[at]))
+    q, s = ops.quantize_tensor(x, scale[:1], "i8", False)
+    assert torch.equal(q[at], ops.quantize_tensor(x[at], scale[:1], "i8", False)[0]) and bool((s == scale[0]).all())
+
+
+def test_more_long_rows_than_one_launch_holds(ops):
+    """Rows that take a workgroup each, more of them than the work items of one launch: 2^24 rows of more than 3072 columns."""
+    m, k = (1 << 24) + 5, 3080
+    if torch.cuda.mem_get_info()[0] < m * k * 3 + (8 << 30):
+        pytest.skip("needs 163 GB of free device memory")
+    x = torch.empty(m, k, dtype=torch.bfloat16, device="cuda").fill_(1.0)
+    scale = torch.full((m,), 0.25, device="cuda")
+    at = torch.tensor([0, (1 << 23) - 1, 1 << 23, (1 << 24) - 1, 1 << 24, m - 1], device="cuda")
+    x[at] = torch.randn(6, k, device="cuda").bfloat16()
+    scale[at] = torch.arange(1, 7, device="cuda") * 0.125
+    q = ops.quantize_rows_i8(x, scale)
+    assert torch.equal(q[at], ops.quantize_rows_i8(x[at], scale[at]))
+    assert bool((q[5:9] == 4).all()) and bool((q[(1 << 24) - 9:(1 << 24) - 5] == 4).all())
+    del x, q
+    torch.cuda.empty_cache()
