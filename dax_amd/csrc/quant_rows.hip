@@ -674,6 +674,7 @@ int daxq_act_quant_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int6
         return fail(DAXQ_ERR_ARG, "act_quant_tensor: bad shape m=%lld k=%lld (at most %d columns)", (long long)m, (long long)k, 36 * 512);
     if (scale_round != DAXQ_SCALE_ROUND_X && scale_round != DAXQ_SCALE_ROUND_NONE)
         return fail(DAXQ_ERR_ARG, "act_quant_tensor: unknown scale rounding %d", scale_round);
+    if (!(quant_max > 0.0f) || !(eps >= 0.0f)) return fail(DAXQ_ERR_ARG, "act_quant_tensor: quant_max must be positive and eps not negative");
     if (m == 0) return DAXQ_OK;
     if (!x || !q || !scale_rows || !scratch) return fail(DAXQ_ERR_ARG, "act_quant_tensor: null pointer");
     if ((uintptr_t)scratch & 15) return fail(DAXQ_ERR_ALIGN, "act_quant_tensor: the scratch must be 16-byte aligned");

@@ -113,6 +113,20 @@ def test_kernel_argument_fields():
     assert _capi.kernel_arg() == 0
 
 
+def test_quantisers_refuse_a_quant_max_that_is_not_positive():
+    """Before anything is launched, and also for no rows at all (a null matrix here)."""
+    from dax_amd import _capi
+
+    lib = _capi.lib()
+    for bad in (0.0, -1.0, float("nan")):
+        assert lib.daxq_act_quant_rows_ex(None, 0, 0, 0, 8, 8, None, 8, None, bad, 1e-7, 1, None) == -1
+        assert lib.daxq_weight_quant_rows(None, 0, 0, 0, 8, 8, None, 8, None, bad, 1e-7, None) == -1
+        assert lib.daxq_act_quant_tensor(None, 0, 0, 0, 8, 8, None, 8, None, None, None, bad, 1e-7, 1, None) == -1
+    for bad in (-1.0, float("nan")):
+        assert lib.daxq_act_quant_tensor(None, 0, 0, 0, 8, 8, None, 8, None, None, None, 127.0, bad, 1, None) == -1
+    assert lib.daxq_act_quant_tensor(None, 0, 0, 0, 8, 8, None, 8, None, None, None, 127.0, 0.0, 1, None) == 0
+
+
 def test_no_cpu_kernels_and_clear_errors():
     import dax_amd.ops as ops
 
