@@ -253,7 +253,7 @@ static int launch_rows_one(const GemmArgs* args, hipStream_t st) {
 //   INT8  390 x 176, K = 3456 (275 blocks)  4.7 / 7.2 / - / 4.0, 11.9     543 x 254, K = 2688 (544)    4.4 / 6.3 / - / 5.0, 10.4
 //         392 x 819, K = 1408 (1300)        5.1 / 5.1 / 6.6 / 5.6, 8.7    242 x 2100, K = 8448 (2112) 32.3 / 26.0 / 23.4 / 26.3, 28.6
 //   e4m3  443 x 275, K = 3200 (504)         4.6 / 5.9 / 7.8, 12.0         331 x 644, K = 5888 (861)   11.7 / 10.9 / 12.0, 19.5
-//         338 x 1233, K = 6016 (1716)      18.1 / 15.5 / 14.2, 21.7       2032 x 46, K = 256 (381)     2.8 / 3.1 / 3.6, 13.6
+//         338 x 1233, K = 6016 (1716)      18.1 / 15.5 / 14.2, 21.7
 static int64_t row_blocks(int64_t m, int64_t n) { return ((m + 15) / 16) * ((n + 15) / 16); }
 
 template <bool FP8, int F8, int OUTK>
@@ -323,9 +323,13 @@ int prepare_rows_kernels() {
 // a tile idle, here every 16 x 16 outputs or a few of them are a wavefront.  A tile in five CUs is where the two meet
 // (2048 blocks of 16 x 16; e4m3 217 x 2391, K = 1408, 2100 blocks: 7.2 against 8.8 us, 418 x 1558, K = 3840, 2646: 13.8 / 14.9,
 // 784 x 1360, K = 384, 4165: 5.2 / 5.7, 291 x 3671, K = 2176, 4370: 14.7 / 11.3); INT8 launches of long K have split-K
-// beside them (450 x 1137, K = 12800: 32 against 27 us).  Fewer than 128 columns leave only the generic kernel (9191 x 79, K = 512:
+// beside them (450 x 1137, K = 12800: 32 against 27 us).  Fewer than 128 columns leave only the generic kernel (INT8, 9191 x 79, K = 512:
 // 15.4 -> 6.9 us, 2404 x 74, K = 3072: 25.6 -> 8.2), which is as fast from about 4000 blocks at K = 4096 on.
+// FP8 with fewer than 128 columns keeps the generic kernel at any number of rows: it adds in another order, and beyond a few
+// thousand blocks this kernel is too slow to be the only one (e4m3 75600 x 64, K = 5120: 212 against 125 us), so a
+// line between the two would change a row's bits with the rows around it.
 bool rows_applies(int64_t m, int64_t n, int64_t k, bool fp8) {
+    if (fp8 && n < 128) return false;
     if (m <= 128) return m <= (n > 8192 ? 32 : 128);
     if (m > (1 << 20) || n > (1 << 20)) return false;
     const int64_t blocks = row_blocks(m, n), work = blocks * (k / 128);

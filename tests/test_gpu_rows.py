@@ -107,3 +107,17 @@ def test_few_outputs_of_many_rows(m, n, k):
     y = ops.linear_w8a8(x8, sxd, w8, swd, None, "e4m3", "e4m3", torch.bfloat16)
     parts = [ops.linear_w8a8(x8[i:i + 128], sxd[i:i + 128].contiguous(), w8, swd, None, "e4m3", "e4m3", torch.bfloat16) for i in range(0, m, 128)]
     assert torch.equal(y, torch.cat(parts))
+
+
+@pytest.mark.parametrize("n,k,m", [(64, 5120, 6600), (1, 384, 300), (127, 13824, 700), (40, 256, 50000)])
+def test_fp8_rows_of_a_narrow_layer_do_not_depend_on_the_others(n, k, m):
+    """Fewer than 128 output channels: the same bits for a row alone, among a few and in a launch of many."""
+    import dax_amd.ops as ops
+
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, k, generator=g).to(torch.float8_e4m3fn).view(torch.uint8).to("cuda")
+    w = torch.randn(n, k, generator=g).to(torch.float8_e4m3fn).view(torch.uint8).to("cuda")
+    sx, sw = torch.rand(m, generator=g).to("cuda"), torch.rand(n, generator=g).to("cuda")
+    y = ops.linear_w8a8(x, sx, w, sw, None, "e4m3", "e4m3", torch.float32)
+    for rows in (1, 16, 17, 128, 129, m // 2):
+        assert torch.equal(ops.linear_w8a8(x[:rows], sx[:rows], w, sw, None, "e4m3", "e4m3", torch.float32), y[:rows]), rows
