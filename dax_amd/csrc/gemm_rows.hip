@@ -178,6 +178,14 @@ __global__ __launch_bounds__(64 * KS) void gemm_rows_kernel(const GemmArgs p) {
         const int m = mbase + i * 16 + l15;
         if (m >= p.m || nc >= p.n) continue;
         const float sxv = p.sx[m];
+        if (p.acc) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (nc + e >= p.n) continue;
+                if constexpr (FP8) static_cast<float*>(p.acc)[(int64_t)m * p.ldacc + nc + e] = acc[i][e];
+                else static_cast<int32_t*>(p.acc)[(int64_t)m * p.ldacc + nc + e] = acc[i][e];
+            }
+        }
         float o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -337,10 +345,10 @@ bool rows_applies(int64_t m, int64_t n, int64_t k, bool fp8) {
     return blocks <= 2048 && (fp8 || work <= 131072);
 }
 
-// 32-bit row offsets, no accumulator dump
+// 32-bit row offsets
 int launch_rows(const GemmArgs& a, bool fp8, int f8, hipStream_t st) {
-    if (a.acc || a.lda >= (1 << 26) || a.ldb >= (1 << 26))
-        return fail(DAXQ_ERR_ARG, "linear: the kernel for few rows takes row strides below 2^26 and no accumulator dump");
+    if (a.lda >= (1 << 26) || a.ldb >= (1 << 26))
+        return fail(DAXQ_ERR_ARG, "linear: the kernel for few rows takes row strides below 2^26");
     return launch_rows_any(&a, a.out_kind, fp8, f8, st);
 }
 

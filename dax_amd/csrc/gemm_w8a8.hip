@@ -378,6 +378,8 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
         return fail(DAXQ_ERR_ARG, "linear: the tiled kernels dump their accumulators with bf16 outputs only");
     switch (which) {
         case K_DEFAULT: {
+            // (with the accumulator dump, too: the outputs beside it are the same bits as without)
+            if (rows_applies(m, n, k, FP8) && fits32) return launch_rows(a, FP8, f8, st);
             // fp16 / fp32 outputs together with the accumulator dump (tests): the generic kernel
             if (acc && out_kind != DAXQ_BF16)
                 return (m >= 256 && n >= 256) ? launch_generic<FP8, 256>(a, f8, st) : launch_generic<FP8, 128>(a, f8, st);
@@ -403,7 +405,6 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
             // K = 5120 55.3 -> 49.5 / 52.3 -> 46.0, K = 13824 116 -> 110 / 113 -> 104; 2176 x 3840 (135 / 510) K = 13824 111 -> 110 /
             // 108 -> 105.  From 513 small tiles on a second round of them starts: 4600 x 1800 (144 / 540) K = 1024 17.2 -> 18.3 /
             // 16.4 -> 16.4, K = 3072 32.1 -> 37.4.
-            if (rows_applies(m, n, k, FP8) && fits32 && !acc) return launch_rows(a, FP8, f8, st);
             const int64_t tiles256 = ((m + 255) / 256) * ((n + 255) / 256);
             const int cus = cu_count();
             const int64_t tiles128 = ((m + 127) / 128) * ((n + 127) / 128);
@@ -424,7 +425,7 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
             if (!tile256_applies(a)) return fail(DAXQ_ERR_ARG, "linear: the 256x128 kernel needs m, n >= 256");
             return launch_halves<FP8>(a, f8, st);
         case K_ROWS:
-            if (m > 128) return fail(DAXQ_ERR_ARG, "linear: the kernel for few rows takes at most 128 by name");
+            if (m > 128 || acc) return fail(DAXQ_ERR_ARG, "linear: the kernel for few rows takes at most 128, and no accumulator dump, by name");
             return launch_rows(a, FP8, f8, st);
         default: return fail(DAXQ_ERR_ARG, "linear: unknown kernel choice %d", which);
     }

@@ -307,7 +307,7 @@ int daxq_linear_e5m2_e4m3(const uint8_t* xq, int64_t ld_xq, const float* sx,
  * bits 2 / 5 = the generic kernel on 256x256 / 128x128 tiles (an implementation of its own, any shape), 8 / 11 / 14 =
  * the tiled kernel on 256x256 / 128x128 / 256x128 tiles (int8: 16x16x64 MFMAs; fp8: 16x16x128 MFMAs; needs m, n >= the
  * tile edge, 256 for the 256x128 tiles);
- * 17 = the kernel for at most 128 rows, by itself also taken for few outputs (weights streamed through a ring per wavefront; no accumulator dump);
+ * 17 = the kernel for at most 128 rows, by itself also taken for few outputs (weights streamed through a ring per wavefront; the accumulator dump not by name);
  * bits 16-23, when not zero, set the depth of the tile-order groups; bits 24-27 the tile order of the 256x256 kernels
  * (0 = by shape, 1 = groups of tile rows, 2 = banded patches of 8 x 4 tiles per XCD; every order computes every tile
  * once, the results are the same bits); bits 28-29 the treatment of the last, partial round of workgroups of a launch
@@ -320,7 +320,7 @@ int daxq_linear_e5m2_e4m3(const uint8_t* xq, int64_t ld_xq, const float* sx,
  * order and cut of the tiled kernel (one sequence of MFMAs per output element), so an output row does not depend on
  * how many rows the launch has; the generic kernel (every fp8 launch with n < 128, and launches of 33 to 127 rows with
  * n > 8192) adds in another order and agrees to fp32 rounding.  Every kernel writes bf16, fp16 and fp32; the accumulator dump of the tiled
- * kernels exists with bf16 outputs.  The choice is an argument of the call: the library keeps no process-wide
+ * kernels exists with bf16 outputs (with the others such a call takes the generic kernel).  The choice is an argument of the call: the library keeps no process-wide
  * selection.
  */
 int daxq_linear_w8a8(int x_fmt, int w_fmt, int out_dtype,

@@ -121,3 +121,31 @@ def test_fp8_rows_of_a_narrow_layer_do_not_depend_on_the_others(n, k, m):
     y = ops.linear_w8a8(x, sx, w, sw, None, "e4m3", "e4m3", torch.float32)
     for rows in (1, 16, 17, 128, 129, m // 2):
         assert torch.equal(ops.linear_w8a8(x[:rows], sx[:rows], w, sw, None, "e4m3", "e4m3", torch.float32), y[:rows]), rows
+
+
+@pytest.mark.parametrize("fmt", ["i8", "e4m3", "e5m2"])
+@pytest.mark.parametrize("n,k", [(130, 640), (264, 1408), (2052, 1152)])
+def test_accumulators_beside_the_outputs_of_few_rows(n, k, fmt):
+    """The form that returns the accumulators as well gives the outputs of the plain form, bit for bit, and the accumulators
+    they come from."""
+    import dax_amd.ops as ops
+
+    g = torch.Generator().manual_seed(n)
+    if fmt == "i8":
+        x, w = (torch.randint(-128, 128, s, generator=g, dtype=torch.int8).to("cuda") for s in ((300, k), (n, k)))
+    else:
+        f8 = {"e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}[fmt]
+        x, w = (torch.randn(*s, generator=g).to(f8).view(torch.uint8).to("cuda") for s in ((300, k), (n, k)))
+    sx, sw = torch.rand(300, generator=g).to("cuda"), torch.rand(n, generator=g).to("cuda")
+    for m in (1, 17, 64, 100, 127, 128, 300):
+        if m > 128 and n > 1000:  # (2000 blocks of 16 x 16 and more: the tiled kernels)
+            continue
+        for dtype in (torch.bfloat16, torch.float16, torch.float32):
+            bias = torch.randn(n, generator=g).to(dtype).to("cuda")
+            y = ops.linear_w8a8(x[:m], sx[:m], w, sw, bias, fmt, fmt, dtype)
+            ya, acc = ops.linear_w8a8_acc(x[:m], sx[:m], w, sw, bias, fmt, fmt, dtype)
+            assert torch.equal(y, ya), (m, dtype)
+            if dtype == torch.float32:
+                assert torch.equal(y, acc.float() * sx[:m, None] * sw + bias), m
+            if fmt == "i8":
+                assert torch.equal(acc.cpu(), O.int_mm(x[:m].cpu(), w.cpu()))
