@@ -256,6 +256,10 @@ static int launch_rows_one(const GemmArgs* args, hipStream_t st) {
 // Few workgroups (small n): cut K where the sums allow it, one row block per workgroup where they do not; many: two row
 // blocks, so that the activation is fetched half as often.  With more than 32 rows and N > 8192 the tiles, which fetch it
 // once per 128 columns, are as fast.
+// FP8 with more than 64 rows and many columns: four row blocks, 2,5,1 / 4,3,1 beside the tiles on 128 rows, us on weights out of
+// reach of the caches: N = 8192, K = 5120, m = 72 22.3 / 17.6, m = 128 30.2 / 22.0, 24.1; K = 13824, m = 128 85.2 / 69.4, 72.8;
+// N = 6144, K = 5120, m = 128 27.2 / 19.4, 26.8; at N = 5120 15.1 / 15.6 (m = 72) and 21.5 / 19.5 (128), at N = 3072 9.8 / 12.8 and
+// 14.3 / 14.7.
 // More than 128 rows (rows_applies says which): `blocks` of 16 x 16 outputs count the work.  us, 1,5,1 / 2,5,1 / 4,3,1 and for
 // INT8 2,3,4, beside the tiles (or, n < 128, the generic kernel):
 //   INT8  390 x 176, K = 3456 (275 blocks)  4.7 / 7.2 / - / 4.0, 11.9     543 x 254, K = 2688 (544)    4.4 / 6.3 / - / 5.0, 10.4
@@ -293,6 +297,9 @@ static int launch_rows_out(const GemmArgs* a, hipStream_t st) {
             if (a->m <= 64) return launch_rows_one<FP8, F8, 2, 3, 4, OUTK>(a, st);
             return launch_rows_one<FP8, F8, 4, 2, 4, OUTK>(a, st);
         }
+    }
+    if constexpr (FP8) {
+        if (a->m > 64 && a->n > 5120) return launch_rows_one<FP8, F8, 4, 3, 1, OUTK>(a, st);
     }
     if (a->m <= 16) return launch_rows_one<FP8, F8, 1, 10, 1, OUTK>(a, st);
     if (a->n <= 2048 || (a->m <= 32 && a->n <= 8192)) return launch_rows_one<FP8, F8, 1, 5, 1, OUTK>(a, st);

@@ -149,3 +149,21 @@ def test_accumulators_beside_the_outputs_of_few_rows(n, k, fmt):
                 assert torch.equal(y, acc.float() * sx[:m, None] * sw + bias), m
             if fmt == "i8":
                 assert torch.equal(acc.cpu(), O.int_mm(x[:m].cpu(), w.cpu()))
+
+
+@pytest.mark.parametrize("x_fmt,w_fmt", [("e4m3", "e4m3"), ("e5m2", "e4m3"), ("e4m3", "e5m2"), ("e5m2", "e5m2")])
+@pytest.mark.parametrize("n,k", [(5120, 640), (5121, 128), (5128, 512), (6000, 1408)])
+def test_fp8_bits_of_the_tiled_kernel_at_65_to_128_rows(select, n, k, x_fmt, w_fmt):
+    """Either side of the width from which four row blocks share a wavefront, K from one step to more than its ring holds."""
+    import dax_amd.ops as ops
+
+    g = torch.Generator().manual_seed(n * 3 + k)
+    f8 = {"e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}
+    xq = torch.randn(128, k, generator=g).to(f8[x_fmt]).view(torch.uint8).to("cuda")
+    wq = torch.randn(n, k, generator=g).to(f8[w_fmt]).view(torch.uint8).to("cuda")
+    sx, sw = torch.rand(128, generator=g).to("cuda"), torch.rand(n, generator=g).to("cuda")
+    select(11)
+    ref = ops.linear_w8a8(xq, sx, wq, sw, None, x_fmt, w_fmt, torch.float32)
+    select(0)
+    for m in (64, 65, 80, 113, 127, 128):
+        assert torch.equal(ops.linear_w8a8(xq[:m], sx[:m], wq, sw, None, x_fmt, w_fmt, torch.float32), ref[:m]), m
