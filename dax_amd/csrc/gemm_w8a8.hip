@@ -445,13 +445,28 @@ constexpr int64_t kMaxSplitTiles = kCounterBytes / 4;
 // least 1024 bytes of K deep and divide K / 128 evenly; 1 = no split.  Measured at N = K = 5120 (INT8, us, plain launch /
 // 2 / 4 ranges): M = 256 (80 tiles) 34 / 28 / 40, M = 512 (160 tiles) 24 / 35 / 52, M = 1024 52 / 71 / -: the partial
 // results make a round trip through device-coherent memory (about 10 us for 20 MB), which only idle CUs pay for.
+// Launches that the kernel for few rows is taken for leave their ranges alone, but not 65 to 128 rows against a large weight,
+// where the K ranges are as fast or faster from about 45 M weight bytes on (128 rows; that kernel / K ranges, us, weights out
+// of reach of the caches): N = 5120, K = 8960 30.2 / 27.9; 8192 x 5120 25.1 / 24.4; 6144 x 8960 34.2 / 28.6; 4096 x 13824
+// 34.5 / 31.1; 5120 x 13824 47.3 / 34.2; 8192 x 13824 68.5 / 40.3 (72 rows: 25.7, 22.4, 30.9, 30.1, 38.9, 59.6).
+constexpr int64_t kRowsBelowSplit = 45000000;
 static int splitk_choice(int64_t m, int64_t n, int64_t k) {
-    if (m < 128 || n < 128 || k % DAXQ_K_ALIGN || rows_applies(m, n, k, false)) return 1;
+    if (m < 128 || n < 128 || k % DAXQ_K_ALIGN) return 1;
+    if (rows_applies(m, n, k, false) && (m > 128 || n * k <= kRowsBelowSplit)) return 1;
     const int64_t tiles = splitk_tiles(m, n), units = k / DAXQ_K_ALIGN;
     int best = 1;
     for (int s = 2; s <= 8; ++s)
         if (units % s == 0 && k / s >= 1024 && tiles * s <= 256) best = s;
     return best;
+}
+
+// Rows that the GEMM of a linear runs on when the caller's buffers reach that far: m, or 128 where the tiled kernels (their
+// smallest tile) or, with a workspace, the K ranges are better than the kernel for few rows.  The rows beyond m hold
+// whatever the buffers held; an output row depends on its own operand row only.
+static int64_t gemm_rows(bool fp8, int64_t m, int64_t n, int64_t kp, bool splitk) {
+    if (m <= 0 || m >= 128 || n < 128) return m;
+    if (!rows_applies(m, n, kp, fp8)) return 128;
+    return splitk && !fp8 && m > 64 && splitk_choice(128, n, kp) > 1 ? 128 : m;
 }
 
 template <bool FP8>
@@ -647,6 +662,10 @@ int daxq_linear_w8a8(int x_fmt, int w_fmt, int out_dtype, const void* xq, int64_
     return fail(DAXQ_ERR_ARG, "linear: unsupported operand formats x=%d w=%d (int8 x int8, or fp8 x fp8)", x_fmt, w_fmt);
 }
 
+int64_t daxq_linear_rows(int x_fmt, int64_t m, int64_t n, int64_t k, int splitk) {
+    return daxq::gemm_rows(x_fmt != DAXQ_FMT_I8, m, n, (k + DAXQ_K_ALIGN - 1) / DAXQ_K_ALIGN * DAXQ_K_ALIGN, splitk != 0);
+}
+
 // ---- quantiser + GEMM behind one entry point --------------------------------------------------------------------
 int daxq_dynamic_linear(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int act_scale_round, const void* x, int64_t ld_x, void* xq,
                         int64_t ld_xq, float* sx, int64_t rows_alloc, const void* wq, int64_t ld_wq, const float* sw,
@@ -667,14 +686,13 @@ int daxq_dynamic_linear(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int ac
     // the quantiser zero-fills columns [k, kp) of the rows it writes
     const float qmax = x_fmt == DAXQ_FMT_I8 ? 127.0f : x_fmt == DAXQ_FMT_E4M3 ? 448.0f : 57344.0f;
     if (int rc = daxq_act_quant_rows_ex(x, x_dtype, x_fmt, m, k, ld_x, xq, ld_xq, sx, qmax, kEps, act_scale_round, stream)) return rc;
-    // Fewer rows than the smallest tile of the tiled kernels, and more columns than the kernel for few rows is taken for: run
-    // the tiled kernels on 128 rows of the caller's buffers when those reach that far (the rows beyond m hold whatever the buffers held; an output row depends on its own operand row only).
-    const bool rows = kernel == 0 && rows_applies(m, n, kp, fp8);
-    const int64_t mg = (!rows && m < 128 && rows_alloc >= 128 && n >= 128) ? 128 : m;
+    const bool may_split = !fp8 && workspace && out_dtype == DAXQ_BF16 && kernel == 0;
+    int64_t mg = kernel == 0 ? gemm_rows(fp8, m, n, kp, may_split) : m < 128 && n >= 128 ? 128 : m;
+    if (mg > rows_alloc) mg = m;
     hipStream_t st = (hipStream_t)stream;
     // INT8 launches with few tiles cut K into ranges when the caller brings a workspace (integer partial sums: the
     // same bits as the plain launch); FP8 sums would change with the number of rows, so they stay whole.
-    if (!fp8 && workspace && out_dtype == DAXQ_BF16 && kernel == 0 && !rows) {
+    if (may_split) {
         const int splits = splitk_choice(mg, n, kp);
         if (splits > 1 && workspace_bytes >= kCounterBytes + splitk_tiles(mg, n) * splits * kPartialBytes)
             return launch_gemm_splitk<false>(xq, ld_xq, sx, wq, ld_wq, sw, bias, out, ld_out, mg, n, kp, splits, workspace,

@@ -101,7 +101,8 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const int64_t ld_w = n > 1 ? wq->stride(0) : kp;
     if (ld_w < kp) Py_RETURN_NONE;
     // launches that take a split-K workspace, or 128 rows for the sake of the tiled kernels, keep those with the custom op
-    if (x_fmt == DAXQ_FMT_I8 && out_kind == DAXQ_BF16 && daxq_linear_splitk_choice(m, n, kp) > 1) Py_RETURN_NONE;
+    const int64_t split_rows = scheme == kToken ? daxq_linear_rows(x_fmt, m, n, k, 1) : m;
+    if (x_fmt == DAXQ_FMT_I8 && out_kind == DAXQ_BF16 && daxq_linear_splitk_choice(split_rows, n, kp) > 1) Py_RETURN_NONE;
     if (scheme == kToken && m > 32 && m < 128 && n > 8192) Py_RETURN_NONE;
 
     at::Tensor out;

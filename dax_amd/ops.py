@@ -114,7 +114,6 @@ def _rows_bf16(x: torch.Tensor, what: str) -> None:
 # written.
 Q_ROW_PAD = 128
 MIN_TILE_ROWS = 128  # rows of the smallest tile of the tiled GEMM kernels
-ROWS_KERNEL_MAX_N = 8192  # columns up to which 33 to 128 rows run in the kernel for few rows (fewer rows always do)
 
 
 def _row_pad(kp: int) -> int:
@@ -645,6 +644,7 @@ linear_e4m3_acc.register_fake(lambda xq, sx, wq, sw, bias: (
 _Q_DTYPE = {"i8": torch.int8, "e4m3": torch.uint8, "e5m2": torch.uint8}
 _W_FMT = {"i8": 0, "e4m3": 1, "e5m2": 1}  # the weight format each activation format is paired with here
 _splitk_memo = {}  # (rows, n, kp) -> daxq_linear_splitk_choice, host arithmetic asked once per shape
+_rows_memo = {}    # (m, n, kp, format) -> daxq_linear_rows
 _dyn_fn = None     # the bound daxq_dynamic_linear
 
 
@@ -672,10 +672,13 @@ def _dynamic_linear(x, wq, sw, bias, fmt: str, scale_fp32: bool = False):
         raise ValueError(f"daxq::dynamic_linear_{fmt}: sw must be contiguous fp32 [N]")
     if bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != n or not bias.is_contiguous()):
         raise ValueError(f"daxq::dynamic_linear_{fmt}: bias must be contiguous bfloat16 [N]")
-    # Fewer rows than one 128-row tile but more columns than the kernel for few rows is taken for: the buffers get 128
-    # rows and the tiled kernel runs on all of them; what the rows beyond M hold is never looked at, and their outputs are
-    # cut off.
-    rows = MIN_TILE_ROWS if 32 < m < MIN_TILE_ROWS and n > ROWS_KERNEL_MAX_N else m
+    # Fewer rows than one 128-row tile where the tiled kernel on all of 128 is still faster than the kernel for few rows: the
+    # buffers get 128 rows; what the rows beyond M hold is never looked at, and their outputs are cut off.
+    rows = m
+    if 0 < m < MIN_TILE_ROWS:
+        rows = _rows_memo.get((m, n, kp, fmt))
+        if rows is None:
+            rows = _rows_memo[m, n, kp, fmt] = _capi.lib().daxq_linear_rows(FMT[fmt], m, n, k, 1)
     ld_q = kp + (Q_ROW_PAD if kp % 1024 == 0 else 0)
     with _on_device(x):
         # quantised rows, then the fp32 scales (the row stride is a multiple of 128, so they are aligned)

@@ -341,9 +341,9 @@ int daxq_linear_w8a8(int x_fmt, int w_fmt, int out_dtype,
  * sx    scratch for the per-token scales, fp32 [rows_alloc]
  * wq    quantised weight [n, roundup(k, DAXQ_K_ALIGN)] (ld_wq), pad columns zero; sw fp32 [n]; bias [n] of out_dtype or NULL
  * out   [rows_alloc, n] of out_dtype elements (ld_out); rows [0, m) are the result
- * rows_alloc >= m: rows that xq, sx and out really hold.  With 32 < m < 128 <= rows_alloc and n > 8192 the tiled kernels
- *       run on 128 rows of those buffers (faster than the kernel that takes fewer rows); rows [m, 128) of out then hold
- *       unspecified values.  Fewer rows or columns have a kernel of their own and touch nothing beyond row m.
+ * rows_alloc >= m: rows that xq, sx and out really hold.  Where daxq_linear_rows says 128 and rows_alloc >= 128, the tiled
+ *       kernels run on 128 rows of those buffers (faster than the kernel that takes fewer rows); rows [m, 128) of out
+ *       then hold unspecified values.  Otherwise nothing beyond row m is touched.
  * workspace / workspace_bytes: optional split-K workspace as for daxq_linear_w8a8_splitk (counters zero), or NULL.
  *       INT8 launches with bf16 outputs and few tiles then cut K into ranges (same bits as the plain launch).
  * kernel: as for daxq_linear_w8a8 (0 = the library's choice).
@@ -375,6 +375,11 @@ int daxq_dynamic_linear_e5m2_e4m3(const void* x, int64_t ld_x, uint8_t* xq, int6
  * XCD more than 5 % over its share of the tiles).  For tests and diagnostics; no
  * counterpart in the reference, whose matmul comes from a vendor library. */
 int daxq_linear_tile_order_choice(int64_t m, int64_t n, int64_t k);
+
+/* Rows that xq, sx and out of daxq_dynamic_linear should hold (its rows_alloc) for the fastest launch the library has: m, or
+ * 128 where that many rows in the tiled kernels are faster than m in the kernel for few rows.  splitk: the caller brings a
+ * workspace (int8 with bf16 outputs).  Host arithmetic only. */
+int64_t daxq_linear_rows(int x_fmt, int64_t m, int64_t n, int64_t k, int splitk);
 
 /*
  * Split-K form of daxq_linear_w8a8 for launches with too few output tiles to fill the CUs (a few hundred rows: the

@@ -94,6 +94,25 @@ def test_tile_order_by_shape():
     assert f(512, 5120, 5120) == 1 and f(1, 8, 128) == 1 and f(0, 0, 0) == 1
 
 
+def test_rows_a_launch_wants():
+    """daxq_linear_rows / daxq_linear_splitk_choice (host arithmetic only): 128 rows for 33 to 127 of them against more than
+    8192 columns, and for 65 to 127 int8 rows against a large weight when K can be cut; m everywhere else."""
+    from dax_amd import _capi
+
+    rows, split = _capi.lib().daxq_linear_rows, _capi.lib().daxq_linear_splitk_choice
+    for fmt in (0, 1, 2):
+        for sk in (0, 1):
+            assert [rows(fmt, m, 13824, 5120, sk) for m in (0, 1, 32, 33, 127, 128, 500)] == [0, 1, 32, 128, 128, 128, 500]
+            assert [rows(fmt, m, 8192, 1536, sk) for m in (33, 64, 65, 127)] == [33, 64, 65, 127]
+            assert rows(fmt, 100, 100, 13824, sk) == 100   # fewer columns than a tile has
+            assert rows(fmt, 100, 8200, 100, sk) == 128    # any K: rounded up to whole slices
+        assert rows(fmt, 100, 5120, 13824, 0) == 100
+        assert rows(fmt, 100, 5120, 13824, 1) == (128 if fmt == 0 else 100)
+    assert rows(0, 64, 5120, 13824, 1) == 64 and rows(0, 65, 5120, 13824, 1) == 128
+    assert rows(0, 100, 8192, 5120, 1) == 100 and rows(0, 100, 5120, 8960, 1) == 128
+    assert split(128, 5120, 13824) > 1 and split(128, 8192, 13824) > 1 and split(128, 2048, 13824) == 1 and split(128, 5120, 5120) == 1
+
+
 def test_kernel_argument_fields():
     """The host-side selection (tests, comparisons) packs the fields of the `kernel` argument as include/daxq.h lays
     them out: implementation in the low 16 bits, group depth in bits 16-23, tile order in 24-27, treatment of the last

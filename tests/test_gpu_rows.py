@@ -167,3 +167,22 @@ def test_fp8_bits_of_the_tiled_kernel_at_65_to_128_rows(select, n, k, x_fmt, w_f
     select(0)
     for m in (64, 65, 80, 113, 127, 128):
         assert torch.equal(ops.linear_w8a8(xq[:m], sx[:m], wq, sw, None, x_fmt, w_fmt, torch.float32), ref[:m]), m
+
+
+@pytest.mark.parametrize("m", [64, 65, 100, 127, 128])
+@pytest.mark.parametrize("n,k", [(5120, 8960), (4104, 13704), (8192, 5632)])
+def test_int8_rows_against_a_large_weight(m, n, k):
+    """K cut into ranges on 128 rows of the op's own buffers: the outputs of the first m, bit for bit."""
+    import dax_amd.ops as ops
+
+    g = torch.Generator().manual_seed(m + n)
+    x = torch.randn(m, k, generator=g).bfloat16()
+    wq = torch.randint(-128, 128, (n, ops.pad_k(k)), generator=g, dtype=torch.int8)
+    wq[:, k:] = 0
+    sw, bias = torch.rand(n, generator=g) * 0.01, torch.randn(n, generator=g).bfloat16()
+    xq, sx = O.dynamic_quantize(x, (1, k), torch.int8, 127.0, ops.EPS_F32, torch.float32)
+    ref = O.epilogue_int8(O.int_mm(xq, wq[:, :k].contiguous()), sx.view(-1, 1), sw, bias)
+    args = [t.to("cuda") for t in (x, wq, sw, bias)]
+    for _ in range(2):  # (the second launch finds the workspace's counters as the first left them)
+        y = ops.dynamic_linear_i8(*args)
+        assert y.shape == (m, n) and torch.equal(y.cpu(), ref)
