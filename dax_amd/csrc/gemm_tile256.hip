@@ -13,8 +13,8 @@
 // activation rows and on different weight columns; the large launches take the banded one.
 //
 // Tiles at the M / N edge are shifted inwards (origin min(tile*BT, dim-BT)) instead of being predicated: the overlap
-// rows are computed twice with identical results.  Shapes with M < 128 or N < 128 take the generic kernel in
-// gemm_w8a8.hip.
+// rows are computed twice with identical results.  Shapes with M < 128 or N < 128 take the kernel in
+// gemm_rows.hip or the generic one in gemm_w8a8.hip.
 #include "gemm_tile.h"
 #include "gemm_tile256x128.h"
 

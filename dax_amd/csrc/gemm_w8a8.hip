@@ -379,13 +379,17 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
     switch (which) {
         case K_DEFAULT: {
             // (with the accumulator dump, too: the outputs beside it are the same bits as without)
-            if (rows_applies(m, n, k, FP8) && fits32) return launch_rows(a, FP8, f8, st);
+            // Fewer than 128 rows and no smaller tile: the kernel for few rows whatever the columns, so that an FP8 row's bits are
+            // those of the tiled kernels at any number of rows.  Beside the generic kernel, us (INT8 / e4m3): 33 x 13824, K = 5120
+            // 32.9 -> 23.0 / 32.5 -> 22.7, 127 rows 42.0 -> 40.6 / 41.7 -> 47.5, 127 x 8960, K = 13824 106 -> 83 / 106 -> 87; 128 rows of
+            // the caller's buffers in the tiled kernels, where they reach that far, take 24.6 / 22.9 and 75 / 74 (daxq_linear_rows).
+            if ((rows_applies(m, n, k, FP8) || (m < 128 && n >= 128)) && fits32) return launch_rows(a, FP8, f8, st);
             // fp16 / fp32 outputs together with the accumulator dump (tests): the generic kernel
             if (acc && out_kind != DAXQ_BF16)
                 return (m >= 256 && n >= 256) ? launch_generic<FP8, 256>(a, f8, st) : launch_generic<FP8, 128>(a, f8, st);
-            // library default: the kernel for few rows (rows_applies, gemm_rows.hip); the tiled kernel on 256x256 tiles once there is one for every second CU, on 128x128
-            // tiles (4x as many workgroups, two per CU) below that, and the generic kernel for operands smaller than
-            // one such tile.  Measured at N = K = 5120 (INT8, T-op/s, 128 / 256 tiles):
+            // library default: the kernel for few rows (above); the tiled kernel on 256x256 tiles once there is one for every
+            // second CU, on 128x128 tiles (4x as many workgroups, two per CU) below that, and the generic kernel for fewer
+            // columns than one such tile has.  Measured at N = K = 5120 (INT8, T-op/s, 128 / 256 tiles):
             // M = 512 -> 1127 / 551, M = 1024 (80 large tiles) -> 1275 / 1055, M = 2048 (160) -> 1542 / 1817;
             // 4096 x 1536 x 1536 (96) -> 1182 / 895, 8192 x 1536 x 1536 (192) -> 1517 / 1587.
             // Between a quarter and a half of the CUs' worth of large tiles, every tile runs as its two 256x128 halves with

@@ -100,10 +100,12 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     }
     const int64_t ld_w = n > 1 ? wq->stride(0) : kp;
     if (ld_w < kp) Py_RETURN_NONE;
-    // launches that take a split-K workspace, or 128 rows for the sake of the tiled kernels, keep those with the custom op
-    const int64_t split_rows = scheme == kToken ? daxq_linear_rows(x_fmt, m, n, k, 1) : m;
-    if (x_fmt == DAXQ_FMT_I8 && out_kind == DAXQ_BF16 && daxq_linear_splitk_choice(split_rows, n, kp) > 1) Py_RETURN_NONE;
-    if (scheme == kToken && m > 32 && m < 128 && n > 8192) Py_RETURN_NONE;
+    // launches that take a split-K workspace keep it with the custom op
+    const bool may_split = x_fmt == DAXQ_FMT_I8 && out_kind == DAXQ_BF16;
+    if (may_split && daxq_linear_splitk_choice(scheme == kToken ? daxq_linear_rows(x_fmt, m, n, k, 1) : m, n, kp) > 1) Py_RETURN_NONE;
+    // rows that the buffers hold: 128 where that many in the tiled kernels are faster than m (what the rows beyond m hold is
+    // never looked at, their outputs are cut off); a kernel chosen by name runs on the rows there are
+    const int64_t rows = kernel == 0 ? daxq_linear_rows(x_fmt, m, n, k, 0) : m;
 
     at::Tensor out;
     int rc = 0;
@@ -115,9 +117,9 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         const auto opt = at::TensorOptions().device(dev);
         const int64_t ld_q = kp + (kp % 1024 == 0 ? kRowPad : 0);
         // the quantised rows, their scales (the row length is a multiple of 128: aligned), 1 KiB for the abs-max of a tensor
-        const int64_t scales = m * ld_q, partial = (scales + 4 * m + 15) / 16 * 16;
+        const int64_t scales = rows * ld_q, partial = (scales + 4 * rows + 15) / 16 * 16;
         const at::Tensor scratch = at::empty({partial + (scheme == kTensor ? 1024 : 0)}, opt.dtype(at::kByte));
-        out = at::empty(shape, opt.dtype(out_type));
+        out = rows == m ? at::empty(shape, opt.dtype(out_type)) : at::empty({rows, n}, opt.dtype(out_type));
         uint8_t* q = static_cast<uint8_t*>(scratch.mutable_data_ptr());
         float* sx = reinterpret_cast<float*>(q + scales);
         void* st = c10::hip::getCurrentHIPStream(dev.index()).stream();
@@ -125,7 +127,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         const float* swp = sw->const_data_ptr<float>();
         void* op = out.mutable_data_ptr();
         if (scheme == kToken) {
-            rc = daxq_dynamic_linear(x_kind, x_fmt, w_fmt, out_kind, scale_fp32 ? 0 : 1, xp, ld_x, q, ld_q, sx, m, wp, ld_w, swp, bp, op, n, m,
+            rc = daxq_dynamic_linear(x_kind, x_fmt, w_fmt, out_kind, scale_fp32 ? 0 : 1, xp, ld_x, q, ld_q, sx, rows, wp, ld_w, swp, bp, op, n, m,
                                      n, k, nullptr, 0, kernel, st);
         } else {
             const float qmax = x_fmt == DAXQ_FMT_I8 ? 127.0f : x_fmt == DAXQ_FMT_E4M3 ? 448.0f : 57344.0f;
@@ -134,7 +136,11 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
             else
                 rc = daxq_quantize_tensor(xp, x_kind, x_fmt, m, k, ld_x, in_scale->const_data_ptr<float>(), q, ld_q, sx, st);
             if (!rc)
-                rc = daxq_linear_w8a8(x_fmt, w_fmt, out_kind, q, ld_q, sx, wp, ld_w, swp, bp, op, n, nullptr, n, m, n, kp, kernel, st);
+                rc = daxq_linear_w8a8(x_fmt, w_fmt, out_kind, q, ld_q, sx, wp, ld_w, swp, bp, op, n, nullptr, n, rows, n, kp, kernel, st);
+        }
+        if (rows != m) {
+            const at::AutoDispatchBelowADInplaceOrView below;  // (the cut is no view of another tensor for the caller)
+            out = out.narrow(0, 0, m).view(shape);
         }
     }
     if (rc) return PyLong_FromLong(rc);

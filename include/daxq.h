@@ -318,8 +318,8 @@ int daxq_linear_e5m2_e4m3(const uint8_t* xq, int64_t ld_xq, const float* sx,
  * 1 = never; 2 = whenever they number at most a quarter / half of the CUs).
  * int8 results are the same bits for every choice.  fp8 results are the same bits for every choice of tile size, tile
  * order and cut of the tiled kernel (one sequence of MFMAs per output element), so an output row does not depend on
- * how many rows the launch has; the generic kernel (every fp8 launch with n < 128, and launches of 33 to 127 rows with
- * n > 8192) adds in another order and agrees to fp32 rounding.  Every kernel writes bf16, fp16 and fp32; the accumulator dump of the tiled
+ * how many rows the launch has; the generic kernel (every fp8 launch with n < 128 and no other, row strides below 2^26)
+ * adds in another order and agrees to fp32 rounding.  Every kernel writes bf16, fp16 and fp32; the accumulator dump of the tiled
  * kernels exists with bf16 outputs (with the others such a call takes the generic kernel).  The choice is an argument of the call: the library keeps no process-wide
  * selection.
  */

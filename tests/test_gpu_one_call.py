@@ -151,3 +151,22 @@ def test_conversion_of_an_empty_weight(k, n):
     quantize_dynamic(model, {"": DYNAMIC["token_i8"]()})
     assert model[0].qweight.shape == (n, k) and model[0].weight_scale.shape == (1, n)
     assert bool((model[0].weight_scale == 1).all())
+
+
+@pytest.mark.parametrize("scheme", [*DYNAMIC, "static_e4m3", "static_e5m2"])
+@pytest.mark.parametrize("m", [33, 64, 127])
+@torch.no_grad()
+def test_buffers_of_more_rows_than_the_call_has(scheme, m):
+    """33 to 127 rows against more than 8192 columns run on buffers of 128: the bits of the general forward, for FP8 those of the
+    rows in a call of 128; the result has the call's shape and is nobody's view."""
+    dtype = torch.float16 if scheme == "token_i8" and m == 64 else torch.bfloat16
+    x = torch.randn(128, 520, device="cuda").to(dtype)
+    lin = _module(scheme, 520, 8208, dtype, True, x)
+    y = _native(lin, x[:m].view(1, m, 520))
+    assert y is not None and y.shape == (1, m, 8208) and y.is_contiguous() and not y._is_view()
+    assert torch.equal(y[0], _general(lin, x[:m]))
+    if not scheme.startswith("tensor"):
+        assert torch.equal(y[0], lin(x)[:m])
+    with torch.enable_grad():
+        y += torch.ones(8208, device="cuda", dtype=dtype, requires_grad=True)
+    assert y.requires_grad

@@ -186,3 +186,27 @@ def test_int8_rows_against_a_large_weight(m, n, k):
     for _ in range(2):  # (the second launch finds the workspace's counters as the first left them)
         y = ops.dynamic_linear_i8(*args)
         assert y.shape == (m, n) and torch.equal(y.cpu(), ref)
+
+
+@pytest.mark.parametrize("m", [33, 48, 64, 65, 100, 127])
+@pytest.mark.parametrize("n,k", [(8200, 1408), (13824, 640)])
+def test_33_to_127_rows_against_many_columns(m, n, k):
+    """The library's own choice on buffers of just m rows: INT8 against the oracle's epilogue, FP8 the bits of the first m rows
+    of a launch of 128, with and without the accumulators."""
+    import dax_amd.ops as ops
+
+    g = torch.Generator().manual_seed(m + n)
+    sx, sw = torch.rand(128, generator=g) * 0.01, torch.rand(n, generator=g) * 0.01
+    xq = torch.randint(-128, 128, (m, k), generator=g, dtype=torch.int8)
+    wq = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8)
+    sxd, swd = sx.to("cuda"), sw.to("cuda")
+    y = ops.linear_w8a8(xq.to("cuda"), sxd[:m], wq.to("cuda"), swd, None, "i8", "i8", torch.float16)
+    assert torch.equal(y.cpu(), O.epilogue_int8(O.int_mm(xq, wq), sx[:m, None], sw, None, out_dtype=torch.float16))
+    for x_fmt, w_fmt in (("e4m3", "e4m3"), ("e5m2", "e4m3"), ("e4m3", "e5m2"), ("e5m2", "e5m2")):
+        f8 = {"e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}
+        x = torch.randn(128, k, generator=g).to(f8[x_fmt]).view(torch.uint8).to("cuda")
+        w = torch.randn(n, k, generator=g).to(f8[w_fmt]).view(torch.uint8).to("cuda")
+        for dtype in (torch.bfloat16, torch.float16, torch.float32):
+            ref = ops.linear_w8a8(x, sxd, w, swd, None, x_fmt, w_fmt, dtype)
+            assert torch.equal(ops.linear_w8a8(x[:m], sxd[:m], w, swd, None, x_fmt, w_fmt, dtype), ref[:m]), (x_fmt, w_fmt, dtype)
+            assert torch.equal(ops.linear_w8a8_acc(x[:m], sxd[:m], w, swd, None, x_fmt, w_fmt, dtype)[0], ref[:m])
