@@ -42,11 +42,14 @@ int float_kind(at::ScalarType t) {
 const at::Tensor* unpack(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
 
 // The dispatcher would go to the plain CUDA kernel, and nobody differentiates through any of these tensors
-bool plain(std::initializer_list<const at::Tensor*> ts) {
+// (`detached` ones enter the general forward as plain values, too, whatever they require)
+bool plain(std::initializer_list<const at::Tensor*> ts, std::initializer_list<const at::Tensor*> detached) {
     if (at::impl::torch_function_mode_enabled() || at::hasCallbacks()) return false;
     const auto tls = c10::impl::tls_local_dispatch_key_set();
     c10::DispatchKeySet ks = tls.included_;
     for (auto* t : ts)
+        if (t) ks = ks | t->key_set();
+    for (auto* t : detached)
         if (t) ks = ks | t->key_set();
     const auto top = (ks - tls.excluded_).highestPriorityTypeId();
     if (top != c10::DispatchKey::AutogradCUDA && top != c10::DispatchKey::ADInplaceOrView && top != c10::DispatchKey::CUDA) return false;
@@ -55,14 +58,16 @@ bool plain(std::initializer_list<const at::Tensor*> ts) {
         if (!t) continue;
         if (grad && t->requires_grad()) return false;
         if (t->_fw_grad(0).defined()) return false;
-        // the dispatcher's fallbacks materialise these (their keys rank below autograd's); the bytes here are not the values
-        if (t->is_neg() || t->_is_zerotensor()) return false;
     }
+    // the dispatcher's fallbacks materialise these (their keys rank below autograd's); the bytes here are not the values
+    for (auto& list : {ts, detached})
+        for (auto* t : list)
+            if (t && (t->is_neg() || t->_is_zerotensor())) return false;
     return true;
 }
 
 // linear(x, wq, sw, bias, in_scale, k, x_fmt, w_fmt, out_kind, scheme, scale_fp32, kernel)
-//   x [..., k]; wq bytes [n, pad128(k)]; sw fp32 [n]; bias [n] of the output's type or None; in_scale fp32 [1] (static) or None
+//   x [..., k]; wq [n, pad128(k)] in its stored type or as bytes; sw fp32 [n], any shape; bias [n] of the output's type or None; in_scale fp32 [1] (static) or None
 // -> the output [..., n], None (not a plain call), or the non-zero status of a C entry point.
 PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
@@ -77,15 +82,16 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     const int x_fmt = (int)PyLong_AsLong(a[6]), w_fmt = (int)PyLong_AsLong(a[7]), out_kind = (int)PyLong_AsLong(a[8]);
     const int scheme = (int)PyLong_AsLong(a[9]), scale_fp32 = PyObject_IsTrue(a[10]), kernel = (int)PyLong_AsLong(a[11]);
     if (PyErr_Occurred()) return nullptr;
-    if (!plain({x, wq, sw, bias, in_scale})) Py_RETURN_NONE;
+    if (!plain({x, sw, in_scale}, {wq, bias})) Py_RETURN_NONE;
 
     const auto dev = x->device();
     const int x_kind = float_kind(x->scalar_type());
     if (!dev.is_cuda() || x_kind < 0 || x->layout() != at::kStrided || wq->device() != dev || sw->device() != dev) Py_RETURN_NONE;
     if ((bias && bias->device() != dev) || (scheme == kStatic) != (in_scale != nullptr)) Py_RETURN_NONE;
     const auto out_type = out_kind == DAXQ_BF16 ? at::kBFloat16 : out_kind == DAXQ_F16 ? at::kHalf : at::kFloat;
-    const auto q_type = x_fmt == DAXQ_FMT_I8 ? at::kChar : at::kByte;
-    if (wq->scalar_type() != q_type || wq->dim() != 2 || wq->stride(1) != 1) Py_RETURN_NONE;
+    const auto w_type = wq->scalar_type();  // the stored FP8 type, or its bytes
+    if (w_fmt == DAXQ_FMT_I8 ? w_type != at::kChar : w_type != at::kByte && w_type != (w_fmt == DAXQ_FMT_E4M3 ? at::kFloat8_e4m3fn : at::kFloat8_e5m2)) Py_RETURN_NONE;
+    if (wq->dim() != 2 || !wq->is_contiguous()) Py_RETURN_NONE;
     const int64_t n = wq->size(0), kp = wq->size(1);
     if (k <= 0 || n <= 0 || kp != (k + kAlign - 1) / kAlign * kAlign || x->dim() < 1 || x->size(-1) != k || x->numel() == 0) Py_RETURN_NONE;
     if (sw->scalar_type() != at::kFloat || sw->numel() != n || !sw->is_contiguous()) Py_RETURN_NONE;
@@ -98,8 +104,6 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         if (x->dim() != 2 || x->stride(1) != 1 || (m > 1 && x->stride(0) < k)) Py_RETURN_NONE;
         if (m > 1) ld_x = x->stride(0);
     }
-    const int64_t ld_w = n > 1 ? wq->stride(0) : kp;
-    if (ld_w < kp) Py_RETURN_NONE;
     // launches that take a split-K workspace keep it with the custom op
     const bool may_split = x_fmt == DAXQ_FMT_I8 && out_kind == DAXQ_BF16;
     if (may_split && daxq_linear_splitk_choice(scheme == kToken ? daxq_linear_rows(x_fmt, m, n, k, 1) : m, n, kp) > 1) Py_RETURN_NONE;
@@ -127,7 +131,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         const float* swp = sw->const_data_ptr<float>();
         void* op = out.mutable_data_ptr();
         if (scheme == kToken) {
-            rc = daxq_dynamic_linear(x_kind, x_fmt, w_fmt, out_kind, scale_fp32 ? 0 : 1, xp, ld_x, q, ld_q, sx, rows, wp, ld_w, swp, bp, op, n, m,
+            rc = daxq_dynamic_linear(x_kind, x_fmt, w_fmt, out_kind, scale_fp32 ? 0 : 1, xp, ld_x, q, ld_q, sx, rows, wp, kp, swp, bp, op, n, m,
                                      n, k, nullptr, 0, kernel, st);
         } else {
             const float qmax = x_fmt == DAXQ_FMT_I8 ? 127.0f : x_fmt == DAXQ_FMT_E4M3 ? 448.0f : 57344.0f;
@@ -136,7 +140,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
             else
                 rc = daxq_quantize_tensor(xp, x_kind, x_fmt, m, k, ld_x, in_scale->const_data_ptr<float>(), q, ld_q, sx, st);
             if (!rc)
-                rc = daxq_linear_w8a8(x_fmt, w_fmt, out_kind, q, ld_q, sx, wp, ld_w, swp, bp, op, n, nullptr, n, rows, n, kp, kernel, st);
+                rc = daxq_linear_w8a8(x_fmt, w_fmt, out_kind, q, ld_q, sx, wp, kp, swp, bp, op, n, nullptr, n, rows, n, kp, kernel, st);
         }
         if (rows != m) {
             const at::AutoDispatchBelowADInplaceOrView below;  // (the cut is no view of another tensor for the caller)

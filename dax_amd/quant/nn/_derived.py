@@ -8,6 +8,8 @@ never saved, rebuilt when the state changes, and built ahead of the first forwar
 """
 from __future__ import annotations
 
+import weakref
+
 import torch
 from torch import Tensor
 
@@ -22,68 +24,89 @@ def _refresh_after_load(module, incompatible_keys) -> None:
     module.refresh_derived()
 
 
+class _Derived(tuple):
+    """(what it was made from, tensor): a copy derived from a state tensor, good while that very tensor is still the module's
+    state, lives where it lived and has not been written to.  It does not keep the state tensor alive, and a copied or
+    unpickled module makes its own."""
+
+    __slots__ = ()
+
+    def __new__(cls, of: Tensor, made: Tensor):
+        return super().__new__(cls, ((weakref.ref(of), of.data_ptr(), of._version), made))
+
+    def is_from(self, t: Tensor) -> bool:
+        ref, ptr, version = self[0]
+        return ref() is t and t.data_ptr() == ptr and t._version == version
+
+    def __reduce__(self):
+        return type(None), ()
+
+
 class DerivedOperands:
     """Mixin for a module with ``qweight``, ``weight_scale`` and ``out_features``."""
 
-    # A module whose forward is quantiser + GEMM and whose state lives on the device keeps the arguments of that one call
-    # ready: every torch call in a forward costs the host a microsecond or two, and a small linear's time is the host's.
-    # The tensors alias the module's state (or are derived from it), so in-place updates of the aliased ones show through;
-    # the tuple also remembers which state tensors it was built from, where they lived and, where a derived copy stands
-    # for one, at which version, and a forward that finds anything else (a buffer or parameter replaced by assignment, by a
-    # hook of an off-loading framework, or through `.data`) rebuilds it.  Whatever sets the state afresh
-    # (conversion, load_state_dict, .to()) rebuilds it too.  Plain data only: a module must stay deep-copyable, and a
-    # copy finds the addresses changed and rebuilds.
-    _fast = None
+    # The forward of a module whose state lives on the device is one native call: every torch call in a forward costs the
+    # host a microsecond or two, and a small linear's time is the host's.  The state goes into that call as it stands at the
+    # time (a buffer or parameter replaced by assignment, by a hook of an off-loading framework, or through `.data`, and
+    # any update in place, show through, and nothing is kept alive); only copies derived from it are kept, and only the
+    # codes of the module's settings, with the settings they stand for beside them.
+    _fast = None  # (settings, codes or None: these settings need more than the one call)
 
-    def _fast_arguments(self):
+    def _fast_settings(self):
+        """The settings that the codes are made of."""
+        raise NotImplementedError
+
+    def _fast_codes(self):
         """(x_fmt, w_fmt, element type of the output, scheme) of the one call, or None where the module needs more."""
         raise NotImplementedError
 
     def _fast_state(self):
         raise NotImplementedError
 
-    def _build_fast(self) -> None:
-        object.__setattr__(self, "_fast", None)
-        args = self._fast_arguments()
-        qw, ws, bp, xs = self._fast_state()
-        if (args is None or qw.device.type != "cuda" or not qw.is_contiguous() or ops.is_tracing(qw)
-                or torch.cuda.is_current_stream_capturing()):
-            return
-        wq, sw = self._gemm_weight(), self._weight_scale_vector()
-        # (a tensor made in inference mode counts no versions: nothing can be derived from it that stays checkable)
-        derived = [t for t, of in ((qw, wq), (ws, sw)) if of.data_ptr() != t.data_ptr()]
-        if any(t.is_inference() for t in derived):
-            return
-        bias = None if bp is None else bp.detach()
-        in_scale = None if xs is None else xs.detach()
-        object.__setattr__(self, "_fast", (
-            (wq, sw, bias, in_scale, self.in_features, *args), qw.device.index, qw, ws, bp, xs, qw.data_ptr(), ws.data_ptr(),
-            0 if bp is None else bp.data_ptr(), 0 if xs is None else xs.data_ptr(),
-            tuple((t, t._version) for t in derived)))
-
     def _fast_forward(self, input: Tensor, scale_fp32: bool):
         """The output, or None where the general forward has to look at the call."""
-        f = self._fast
-        if f is None or input.__class__ is not Tensor or torch.compiler.is_compiling():
+        if input.__class__ is not Tensor or torch.compiler.is_compiling():
             return None
-        qw, ws, bp, xs = self._fast_state()
-        if (qw is not f[2] or ws is not f[3] or bp is not f[4] or xs is not f[5] or qw.data_ptr() != f[6] or ws.data_ptr() != f[7]
-                or (bp is not None and bp.data_ptr() != f[8]) or (xs is not None and xs.data_ptr() != f[9])
-                or any(t._version != v for t, v in f[10])):
-            self.refresh_derived()
-            f = self._fast
-            if f is None:
-                return None
-        if f[1] not in _capi._checked_devices:
-            _capi.require_gfx950(f[1])
-        out = _capi.native().linear(input, *f[0], scale_fp32, _capi.kernel_arg())
+        f, settings = self._fast, self._fast_settings()
+        if f is None:
+            f = (settings, self._fast_codes())
+            object.__setattr__(self, "_fast", f)
+        device = input.device.index
+        if f[1] is None or device is None:
+            return None
+        wq, sw, bias, in_scale = self._fast_state()
+        k = settings[0]
+        if k % ops.K_ALIGN:
+            d = self._packed
+            if d is None or not d.is_from(wq):
+                d = self._derive(wq, self._gemm_weight, "_packed")
+                if d is None:
+                    return None
+            wq = d[1]
+        if sw.numel() == 1:
+            d = self._sw_vec
+            if d is None or not d.is_from(sw):
+                d = self._derive(sw, self._weight_scale_vector, "_sw_vec")
+                if d is None:
+                    return None
+            sw = d[1]
+        if device not in _capi._checked_devices:
+            _capi.require_gfx950(device)
+        out = _capi.native().linear(input, wq, sw, bias, in_scale, k, *f[1], scale_fp32, _capi.kernel_arg())
         if out is not None and out.__class__ is int:
             _capi.check(out, "linear")
         return out
 
+    def _derive(self, of: Tensor, make, name: str):
+        """The copy derived from a state tensor, made now; None where none can be kept."""
+        if of.device.type != "cuda" or of.is_inference() or ops.is_tracing(of) or torch.cuda.is_current_stream_capturing():
+            return None
+        make()
+        return getattr(self, name)
+
     def _init_derived(self) -> None:
-        self._packed = None  # (key, K-padded byte view of qweight)
-        self._sw_vec = None  # (key, per-tensor weight scale once per output channel)
+        self._packed = None  # _Derived: K-padded byte copy of qweight
+        self._sw_vec = None  # _Derived: per-tensor weight scale once per output channel
         self.register_load_state_dict_post_hook(_refresh_after_load)
 
     def _apply(self, fn, recurse=True):
@@ -95,11 +118,10 @@ class DerivedOperands:
     def refresh_derived(self) -> None:
         """Builds the derived operands now, so that a forward launches nothing but its kernels.  A module that
         does not live on a ROCm device (yet) builds them at its first forward there."""
-        self._packed = self._sw_vec = None
+        self._packed = self._sw_vec = self._fast = None
         if self.qweight.device.type == "cuda":
             self._gemm_weight()
             self._weight_scale_vector()
-        self._build_fast()
 
     def _gemm_weight(self) -> Tensor:
         """qweight as the byte matrix [N, pad128(K)] the GEMM reads."""
@@ -113,15 +135,14 @@ class DerivedOperands:
         if ops.is_tracing(qw):
             # a traced graph cannot key a cache on the storage address: pad inside the graph
             return torch.nn.functional.pad(qw, (0, kp - k)).contiguous()
-        key = (self.qweight.data_ptr(), self.qweight._version, str(qw.device))
-        if self._packed is None or self._packed[0] != key:
+        if self._packed is None or not self._packed.is_from(self.qweight):
             buf = torch.zeros((qw.shape[0], kp), dtype=qw.dtype, device=qw.device)
             buf[:, :k] = qw
             if _capturing(qw):
                 # recorded, not executed: the buffer belongs to the graph's pool and holds data only after a
                 # replay, so it must not be kept for later eager calls
                 return buf
-            self._packed = (key, buf)
+            self._packed = _Derived(self.qweight, buf)
         return self._packed[1]
 
     def _weight_scale_vector(self) -> Tensor:
@@ -131,12 +152,11 @@ class DerivedOperands:
             return ws.view(-1)
         if ops.is_tracing(ws):
             return ops.broadcast_f32(ws.reshape(1).contiguous(), self.out_features)
-        key = (ws.data_ptr(), ws._version, str(ws.device))
-        if self._sw_vec is None or self._sw_vec[0] != key:
+        if self._sw_vec is None or not self._sw_vec.is_from(ws):
             vec = ops.broadcast_f32(ws.reshape(1).contiguous(), self.out_features)
             if _capturing(ws):
                 return vec
-            self._sw_vec = (key, vec)
+            self._sw_vec = _Derived(ws, vec)
         return self._sw_vec[1]
 
     def _check_device(self, dev) -> None:

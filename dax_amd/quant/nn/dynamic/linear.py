@@ -178,11 +178,12 @@ class Linear(DerivedOperands, nn.Module):
         return not (m > 16 and k % 8 == 0 and k > 0 and n % 8 == 0 and n > 0)
 
     # ------------------------------------------------------------------ the whole forward in one call
-    def _fast_arguments(self):
+    def _fast_settings(self):
+        return (self.in_features, self.out_dtype, self.input_dtype, self.weight_dtype, self.compute_dtype, self.input_qscheme)
+
+    def _fast_codes(self):
         if self.compute_dtype == "FP8" and self.input_qscheme == per_token_symmetric and self.out_dtype != torch.bfloat16:
             return None  # the row-wise matmul writes bf16, the result is cast afterwards
-        if self.bias is not None and self.bias.dtype != self.out_dtype:
-            return None
         return (ops.FMT[ops.FMT_OF_DTYPE[self.input_dtype]], ops.FMT[ops.FMT_OF_DTYPE[self.weight_dtype]],
                 ops.FLOAT_KIND[self.out_dtype], 0 if self.input_qscheme == per_token_symmetric else 1)
 

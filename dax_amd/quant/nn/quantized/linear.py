@@ -63,9 +63,12 @@ class Linear(DerivedOperands, nn.Module):
         """De-quantised weight in out_dtype (:87-89)."""
         return self.qweight.to(self.out_dtype) * self.weight_scale.reshape(-1, 1).to(self.out_dtype)
 
-    def _fast_arguments(self):
+    def _fast_settings(self):
+        return (self.in_features, self.out_dtype, self.input_dtype, self.weight_dtype, self.row_wise_scale)
+
+    def _fast_codes(self):
         mm_dtype = torch.bfloat16 if self.row_wise_scale else self.out_dtype
-        if mm_dtype != self.out_dtype or (self.bias is not None and self.bias.dtype != mm_dtype):
+        if mm_dtype != self.out_dtype:
             return None
         return (ops.FMT[ops.FMT_OF_DTYPE[self.input_dtype]], ops.FMT[ops.FMT_OF_DTYPE[self.weight_dtype]],
                 ops.FLOAT_KIND[mm_dtype], 2)

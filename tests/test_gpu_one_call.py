@@ -1,5 +1,9 @@
 """The forward of a quantised linear through the one native call (csrc/torch_linear.cpp): the bits of the general forward
 over every scheme, element type and layout it takes, and None wherever the dispatcher would do more than launch kernels."""
+import copy
+import io
+import weakref
+
 import pytest
 import torch
 from torch import nn
@@ -170,3 +174,64 @@ def test_buffers_of_more_rows_than_the_call_has(scheme, m):
     with torch.enable_grad():
         y += torch.ones(8208, device="cuda", dtype=dtype, requires_grad=True)
     assert y.requires_grad
+
+
+@pytest.mark.parametrize("scheme,dtype", [("token_i8", torch.bfloat16), ("token_i8", torch.float16), ("tensor_e4m3", torch.bfloat16),
+                                          ("static_e4m3", torch.bfloat16)])
+@torch.no_grad()
+def test_replaced_state_is_given_back(scheme, dtype):
+    """A hook that puts the state elsewhere between forwards (off-loading) gets its device memory back: nothing of the module
+    holds the tensors it had."""
+    x = torch.randn(32, 1024, device="cuda").to(dtype)
+    lin = _module(scheme, 1024, 2048, dtype, True, x)
+    want = lin(x)
+    assert _native(lin, x) is not None
+    kept = {name: t for name, t in (*lin._buffers.items(), *lin._parameters.items()) if t is not None}
+    homes = {name: t.detach().cpu() for name, t in kept.items()}
+    gone = [weakref.ref(t) for t in kept.values()]
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    for name, t in kept.items():
+        meta = t.to("meta")
+        if name in lin._buffers:
+            lin._buffers[name] = meta
+        else:
+            lin._parameters[name] = nn.Parameter(meta, requires_grad=False)
+    del kept, t
+    assert all(r() is None for r in gone)
+    assert before - torch.cuda.memory_allocated() >= 1024 * 2048
+    for name, t in homes.items():
+        if name in lin._buffers:
+            lin._buffers[name] = t.to("cuda")
+        else:
+            lin._parameters[name] = nn.Parameter(t.to("cuda"), requires_grad=False)
+    assert torch.equal(lin(x), want) and _native(lin, x) is not None
+
+
+@torch.no_grad()
+def test_state_of_another_module_at_the_same_address():
+    """K = 200: the zero-padded copy belongs to one tensor, not to the place it lay at; and a copied or unpickled module
+    makes its own."""
+    x = torch.randn(32, 200, device="cuda").bfloat16()
+    lin = _module("tensor_i8", 200, 512, torch.bfloat16, False, x)
+    lin(x)
+    at = lin.qweight.data_ptr()
+    content = -lin.qweight.cpu()
+    held = []
+    lin._buffers["qweight"] = torch.empty(0, dtype=torch.int8)
+    for _ in range(64):  # the allocator hands the freed block out again
+        t = torch.empty(content.shape, dtype=torch.int8, device="cuda")
+        if t.data_ptr() == at:
+            break
+        held.append(t)
+    t.copy_(content)
+    lin._buffers["qweight"] = t
+    for module in (lin, copy.deepcopy(lin)):
+        want = _general(module, x)
+        assert torch.equal(_native(module, x), want)
+        assert torch.equal(module._gemm_weight()[:, :200].cpu(), content)
+    buf = io.BytesIO()
+    torch.save(lin, buf)
+    buf.seek(0)
+    loaded = torch.load(buf, weights_only=False)
+    assert torch.equal(_native(loaded, x), want) and torch.equal(_general(loaded, x), want)
