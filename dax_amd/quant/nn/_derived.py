@@ -68,7 +68,7 @@ class DerivedOperands:
         if input.__class__ is not Tensor or torch.compiler.is_compiling():
             return None
         f, settings = self._fast, self._fast_settings()
-        if f is None:
+        if f is None or f[0] != settings:
             f = (settings, self._fast_codes())
             object.__setattr__(self, "_fast", f)
         device = input.device.index
@@ -118,7 +118,7 @@ class DerivedOperands:
     def refresh_derived(self) -> None:
         """Builds the derived operands now, so that a forward launches nothing but its kernels.  A module that
         does not live on a ROCm device (yet) builds them at its first forward there."""
-        self._packed = self._sw_vec = self._fast = None
+        self._packed = self._sw_vec = None
         if self.qweight.device.type == "cuda":
             self._gemm_weight()
             self._weight_scale_vector()

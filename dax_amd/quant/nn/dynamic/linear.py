@@ -179,9 +179,12 @@ class Linear(DerivedOperands, nn.Module):
 
     # ------------------------------------------------------------------ the whole forward in one call
     def _fast_settings(self):
-        return (self.in_features, self.out_dtype, self.input_dtype, self.weight_dtype, self.compute_dtype, self.input_qscheme)
+        return (self.in_features, self.out_dtype, self.input_dtype, self.weight_dtype, self.compute_dtype, self.input_qscheme,
+                getattr(self.quantize_activation, "__func__", None))
 
     def _fast_codes(self):
+        if getattr(self.quantize_activation, "__func__", None) is not _QUANTIZE_ACTIVATION:
+            return None  # a quantiser of the user's own: a subclass's, or one set on the module or the class
         if self.compute_dtype == "FP8" and self.input_qscheme == per_token_symmetric and self.out_dtype != torch.bfloat16:
             return None  # the row-wise matmul writes bf16, the result is cast afterwards
         return (ops.FMT[ops.FMT_OF_DTYPE[self.input_dtype]], ops.FMT[ops.FMT_OF_DTYPE[self.weight_dtype]],
@@ -333,3 +336,6 @@ class Linear(DerivedOperands, nn.Module):
             fresh = isinstance(mod.qconfig.weight, partial) and _is_per_channel_observer(mod.qconfig.weight.func)
             return cls.get_qlinear(mod, activation_post_process, weight_post_process, reserve_float_weight, fresh)
         return cls.get_qlinear(mod, activation_post_process, weight_post_process, reserve_float_weight)
+
+
+_QUANTIZE_ACTIVATION = Linear.quantize_activation

@@ -235,3 +235,52 @@ def test_state_of_another_module_at_the_same_address():
     buf.seek(0)
     loaded = torch.load(buf, weights_only=False)
     assert torch.equal(_native(loaded, x), want) and torch.equal(_general(loaded, x), want)
+
+
+@pytest.mark.parametrize("scheme,dtype", [("token_i8", torch.float16), ("tensor_i8", torch.bfloat16), ("tensor_e5m2", torch.bfloat16),
+                                          ("static_e4m3", torch.bfloat16), ("token_i8", torch.bfloat16)])
+@torch.no_grad()
+def test_settings_changed_after_conversion(scheme, dtype):
+    """The module computes with the settings it has when it is called, not with those it was converted with."""
+    x = torch.randn(24, 256, device="cuda").to(dtype)
+    lin = _module(scheme, 256, 64, dtype, False, x)
+    assert lin(x).dtype == dtype
+    for other in (torch.float32, torch.float16, dtype):
+        lin.out_dtype = other
+        assert lin(x).dtype == other and torch.equal(lin(x), _general(lin, x))
+    if scheme.startswith("static"):
+        lin.input_dtype = torch.float8_e5m2
+        assert torch.equal(lin(x), _general(lin, x))
+        lin.row_wise_scale = False
+        assert torch.equal(lin(x), _general(lin, x))
+
+
+@torch.no_grad()
+def test_a_quantiser_of_the_users_own_is_called():
+    """An override of quantize_activation by a subclass, on the module or on the class."""
+    from dax_amd.quant.nn.dynamic import Linear
+
+    x = torch.randn(24, 256, device="cuda").half()
+    plain = Linear.quantize_activation
+    calls = []
+
+    def own(self, input):
+        calls.append(input.shape)
+        return plain(self, input)
+
+    sub = type("Sub", (Linear,), {"quantize_activation": own})
+    lin = _module("token_i8", 256, 64, torch.float16, True, x)
+    want = lin(x)
+    assert not calls
+    lin.__class__ = sub
+    assert torch.equal(lin(x), want) and len(calls) == 1
+    lin.__class__ = Linear
+    lin.quantize_activation = own.__get__(lin)
+    assert torch.equal(lin(x), want) and len(calls) == 2
+    del lin.quantize_activation
+    Linear.quantize_activation = own
+    try:
+        assert torch.equal(lin(x), want) and len(calls) == 3
+    finally:
+        Linear.quantize_activation = plain
+    assert torch.equal(lin(x), want) and len(calls) == 3
