@@ -367,7 +367,7 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
     const int64_t kfill = fill_width(k, ld_q);
     if (((uintptr_t)x & (XB - 1)) != 0 || ((uintptr_t)scale & 3) != 0) return fail(DAXQ_ERR_ALIGN, "quant_rows: x must be element aligned and scale 4-byte aligned");
     uint8_t* qp = static_cast<uint8_t*>(q);
-    if (kfill <= 36 * 512) {
+    if (kfill <= DAXQ_MAX_TENSOR_K) {
         const QuantArgs a{static_cast<const char*>(x), m, ld_x, (int)k, (int)kfill, qp, ld_q, SCALE_IN ? t.scale_rows : scale, scale,
                     t.one_scale ? 0 : 1, t.partials, t.scale1, qmax, eps, round_x, t.partials || t.weight};
         const int cols = (int)((kfill + 511) / 512);
@@ -403,7 +403,7 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
         DAXQ_Q_CASE(9, 4)
 #undef DAXQ_Q_CASE
     }
-    if (t.one_scale || t.partials) return fail(DAXQ_ERR_ARG, "quant_rows: one scale for the tensor is taken for rows of at most %d columns", 36 * 512);
+    if (t.one_scale || t.partials) return fail(DAXQ_ERR_ARG, "quant_rows: one scale for the tensor is taken for rows of at most %d columns", DAXQ_MAX_TENSOR_K);
     if (m > 0x7fffffff) return fail(DAXQ_ERR_ARG, "quant_rows: too many rows");
     hipLaunchKernelGGL((quant_rows_block<FMT, SCALE_IN, XT>), dim3((unsigned)m), dim3(256), 0, st, x, m, k, ld_x, qp,
                        ld_q, kfill, scale, qmax, eps, round_x);
@@ -670,8 +670,8 @@ int daxq_quantize_rows(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t
 int daxq_act_quant_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int64_t k, int64_t ld_x, void* q, int64_t ld_q,
                           float* scale_rows, float* scale1, void* scratch, float quant_max, float eps, int scale_round, daxq_stream_t stream) {
     using namespace daxq;
-    if (m < 0 || k <= 0 || ld_x < k || ld_q < k || m > 0x7fffffff || k > 36 * 512)
-        return fail(DAXQ_ERR_ARG, "act_quant_tensor: bad shape m=%lld k=%lld (at most %d columns)", (long long)m, (long long)k, 36 * 512);
+    if (m < 0 || k <= 0 || ld_x < k || ld_q < k || m > 0x7fffffff || k > DAXQ_MAX_TENSOR_K)
+        return fail(DAXQ_ERR_ARG, "act_quant_tensor: bad shape m=%lld k=%lld (at most %d columns)", (long long)m, (long long)k, DAXQ_MAX_TENSOR_K);
     if (scale_round != DAXQ_SCALE_ROUND_X && scale_round != DAXQ_SCALE_ROUND_NONE)
         return fail(DAXQ_ERR_ARG, "act_quant_tensor: unknown scale rounding %d", scale_round);
     if (!(quant_max > 0.0f) || !(eps >= 0.0f)) return fail(DAXQ_ERR_ARG, "act_quant_tensor: quant_max must be positive and eps not negative");

@@ -30,7 +30,6 @@ namespace {
 
 constexpr int64_t kAlign = DAXQ_K_ALIGN;
 constexpr int64_t kRowPad = 128;          // as Q_ROW_PAD of ops.py: rows of whole kilobytes are kept a line apart
-constexpr int64_t kMaxTensorQuantK = 18432;  // longest row of the per-tensor quantisers
 constexpr float kEps = 1.1920928955078125e-07f;
 
 enum Scheme { kToken = 0, kTensor = 1, kStatic = 2 };
@@ -97,7 +96,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (sw->scalar_type() != at::kFloat || sw->numel() != n || !sw->is_contiguous()) Py_RETURN_NONE;
     if (bias && (bias->scalar_type() != out_type || bias->numel() != n || !bias->is_contiguous())) Py_RETURN_NONE;
     if (in_scale && (in_scale->device() != dev || in_scale->scalar_type() != at::kFloat || in_scale->numel() != 1)) Py_RETURN_NONE;
-    if (scheme != kToken && k > kMaxTensorQuantK) Py_RETURN_NONE;
+    if (scheme != kToken && k > DAXQ_MAX_TENSOR_K) Py_RETURN_NONE;
     // rows: a matrix of contiguous rows at any distance, or a contiguous tensor of any shape
     int64_t m = x->numel() / k, ld_x = k;
     if (!x->is_contiguous()) {
@@ -160,4 +159,14 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_daxq_torch", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__daxq_torch() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__daxq_torch() {
+    PyObject* m = PyModule_Create(&module);
+    if (!m) return nullptr;
+    // the rules that ops.py applies as well
+    if (PyModule_AddIntConstant(m, "K_ALIGN", kAlign) || PyModule_AddIntConstant(m, "ROW_PAD", kRowPad) ||
+        PyModule_AddIntConstant(m, "MAX_TENSOR_K", DAXQ_MAX_TENSOR_K) || PyModule_AddObject(m, "EPS", PyFloat_FromDouble(kEps))) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

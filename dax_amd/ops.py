@@ -337,7 +337,7 @@ quantize_rows_e4m3.register_fake(
 
 
 # ----------------------------------------------------------------------------- one scale for the whole tensor
-MAX_TENSOR_QUANT_K = 18432  # longest row daxq_act_quant_tensor / daxq_quantize_tensor take
+MAX_TENSOR_QUANT_K = 18432  # DAXQ_MAX_TENSOR_K: longest row daxq_act_quant_tensor / daxq_quantize_tensor take
 
 
 def _tensor_q(m: int, k: int, fmt: str, padded: bool, device) -> torch.Tensor:
@@ -679,7 +679,7 @@ def _dynamic_linear(x, wq, sw, bias, fmt: str, scale_fp32: bool = False):
         rows = _rows_memo.get((m, n, kp, fmt))
         if rows is None:
             rows = _rows_memo[m, n, kp, fmt] = _capi.lib().daxq_linear_rows(FMT[fmt], m, n, k, 1)
-    ld_q = kp + (Q_ROW_PAD if kp % 1024 == 0 else 0)
+    ld_q = kp + _row_pad(kp)
     with _on_device(x):
         # quantised rows, then the fp32 scales (the row stride is a multiple of 128, so they are aligned)
         scratch = torch.empty((rows * (ld_q + 4),), dtype=torch.uint8, device=dev)

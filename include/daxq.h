@@ -39,6 +39,8 @@ extern "C" {
  * (ld_q may be smaller); a row stride ld_q beyond that keeps rows apart, or makes
  * q a column slice of a wider buffer, and those bytes are not touched. */
 #define DAXQ_K_ALIGN 128
+/* longest row of the entry points that take one scale for the whole tensor in place of its rows' own */
+#define DAXQ_MAX_TENSOR_K 18432
 
 /* quantised formats (one byte per element) */
 #define DAXQ_FMT_I8 0   /* two's-complement int8 */
@@ -223,7 +225,7 @@ int daxq_tensor_minmax_update(const float* row_min, const float* row_max, int64_
 int daxq_broadcast_f32(const float* src, float* dst, int64_t n, daxq_stream_t stream);
 
 /*
- * The same two schemes without the statistics per row, for rows of at most 18432 columns (any alignment):
+ * The same two schemes without the statistics per row, for rows of at most DAXQ_MAX_TENSOR_K columns (any alignment):
  * daxq_act_quant_tensor: dynamic per-tensor quantisation in two passes over x -- the abs-max of the tensor into `scratch`
  *   (1 KiB, 16-byte aligned, contents unspecified before and after), then scale and bytes.  Arguments and arithmetic as for
  *   daxq_act_quant_rows_ex with the whole matrix as one row; scale_rows [m] receives the one scale once per row (the vector

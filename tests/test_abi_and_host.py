@@ -554,6 +554,20 @@ def test_module_forward_traces_with_fake_tensors(dtype, k):
             assert y.shape == (2, 300, 520) and y.dtype == torch.bfloat16 and y.device.type == "cuda"
 
 
+def test_constants_of_the_python_and_the_native_forward_agree():
+    """The one native call of a forward lays its buffers out and draws the line of the per-tensor quantisers as the custom ops
+    and the C library do."""
+    from dax_amd import _capi, ops
+
+    native = _capi.native()
+    assert (native.K_ALIGN, native.ROW_PAD, native.MAX_TENSOR_K, native.EPS) == (
+        ops.K_ALIGN, ops.Q_ROW_PAD, ops.MAX_TENSOR_QUANT_K, ops.EPS_F32)
+    lib, p = _capi.lib(), 4096  # (refused by shape, before any pointer is looked at or anything launched)
+    for k, said in ((native.MAX_TENSOR_K, "null pointer"), (native.MAX_TENSOR_K + 1, "at most 18432 columns")):
+        assert lib.daxq_act_quant_tensor(p, 0, 0, 1, k, k, 0, k, p, p, p, 127.0, ops.EPS_F32, 0, 0) != 0
+        assert said in _capi.last_error()
+
+
 def test_product_never_touches_the_oracle_or_a_cpu_path():
     """The oracle is test infrastructure: no file of the package names it, and every custom op is registered for
     the GPU only."""
