@@ -192,7 +192,10 @@ class Linear(DerivedOperands, nn.Module):
 
     def _fast_state(self):
         b = self._buffers
-        return b["qweight"], b["weight_scale"], self._parameters["bias"], None
+        try:
+            return b["qweight"], b["weight_scale"], self._parameters["bias"], None
+        except KeyError:  # (state that a wrapper keeps as plain attributes or computes)
+            return self.qweight, self.weight_scale, self.bias, None
 
     def forward(self, input) -> Tensor:
         if not self.uncompiled_small_shape_fallback:

@@ -75,7 +75,10 @@ class Linear(DerivedOperands, nn.Module):
 
     def _fast_state(self):
         p, b = self._parameters, self._buffers
-        return p["qweight"], b["weight_scale"], p["bias"], b["input_scale"]
+        try:
+            return p["qweight"], b["weight_scale"], p["bias"], b["input_scale"]
+        except KeyError:  # (state that a wrapper keeps as plain attributes or computes)
+            return self.qweight, self.weight_scale, self.bias, self.input_scale
 
     def forward(self, input: Tensor) -> Tensor:
         out = self._fast_forward(input, False)

@@ -568,6 +568,25 @@ def test_constants_of_the_python_and_the_native_forward_agree():
         assert said in _capi.last_error()
 
 
+def test_state_that_is_no_parameter_or_buffer_is_found():
+    """What the native call of a forward is handed: also where a wrapper keeps the state as plain attributes."""
+    from dax_amd.quant.nn.dynamic import Linear as Dynamic
+    from dax_amd.quant.nn.quantized import Linear as Static
+    from dax_amd.quant.qscheme import per_channel_symmetric, per_token_symmetric
+
+    for lin in (Static(32, 16, row_wise_scale=True),
+                Dynamic(32, 16, weight_dtype=torch.int8, input_dtype=torch.int8, weight_qscheme=per_channel_symmetric,
+                        input_qscheme=per_token_symmetric)):
+        want = lin._fast_state()
+        for name in ("qweight", "weight_scale", "bias", "input_scale"):
+            if hasattr(lin, name):
+                t = getattr(lin, name)
+                delattr(lin, name)
+                lin.__dict__[name] = t
+        assert not lin._parameters and not lin._buffers
+        assert all(a is b for a, b in zip(lin._fast_state(), want))
+
+
 def test_product_never_touches_the_oracle_or_a_cpu_path():
     """The oracle is test infrastructure: no file of the package names it, and every custom op is registered for
     the GPU only."""

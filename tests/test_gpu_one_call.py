@@ -284,3 +284,20 @@ def test_a_quantiser_of_the_users_own_is_called():
     finally:
         Linear.quantize_activation = plain
     assert torch.equal(lin(x), want) and len(calls) == 3
+
+
+@pytest.mark.parametrize("scheme,k", [("token_i8", 256), ("tensor_i8", 200), ("static_e4m3", 256), ("static_e4m3", 200)])
+@torch.no_grad()
+def test_state_that_is_no_parameter_or_buffer(scheme, k):
+    """A wrapper may keep the state as plain attributes (a sharding framework's flat parameter) or compute it
+    (torch.nn.utils.parametrize): the module reads it by name."""
+    x = torch.randn(24, k, device="cuda").bfloat16()
+    lin = _module(scheme, k, 64, torch.bfloat16, True, x)
+    want = lin(x)
+    for name in ("qweight", "weight_scale", "bias", "input_scale"):
+        if name in lin._parameters or name in lin._buffers:
+            t = getattr(lin, name).detach()
+            delattr(lin, name)
+            setattr(lin, name, t)
+    assert "qweight" not in lin._parameters and "qweight" not in lin._buffers
+    assert torch.equal(lin(x), want) and torch.equal(_native(lin, x), want)
