@@ -71,11 +71,11 @@ class DerivedOperands:
         if f is None or f[0] != settings:
             f = (settings, self._fast_codes())
             object.__setattr__(self, "_fast", f)
-        device = input.device.index
-        if f[1] is None or device is None:
+        device = input.get_device()
+        if f[1] is None or device < 0:
             return None
         wq, sw, bias, in_scale = self._fast_state()
-        k = settings[0]
+        k = self.in_features
         if k % ops.K_ALIGN:
             d = self._packed
             if d is None or not d.is_from(wq):
@@ -83,18 +83,20 @@ class DerivedOperands:
                 if d is None:
                     return None
             wq = d[1]
-        if sw.numel() == 1:
-            d = self._sw_vec
-            if d is None or not d.is_from(sw):
-                d = self._derive(sw, self._weight_scale_vector, "_sw_vec")
-                if d is None:
-                    return None
-            sw = d[1]
+        d = self._sw_vec  # (per channel there is none)
+        if d is not None:
+            if not d.is_from(sw):
+                self._sw_vec = None
+                d = self._derive(sw, self._weight_scale_vector, "_sw_vec") if sw.numel() == 1 else None
+            if d is not None:
+                sw = d[1]
         if device not in _capi._checked_devices:
             _capi.require_gfx950(device)
         out = _capi.native().linear(input, wq, sw, bias, in_scale, k, *f[1], scale_fp32, _capi.kernel_arg())
-        if out is not None and out.__class__ is int:
+        if out.__class__ is int:
             _capi.check(out, "linear")
+        if out is None and d is None and sw.numel() == 1 and self._derive(sw, self._weight_scale_vector, "_sw_vec") is not None:
+            return self._fast_forward(input, scale_fp32)  # (a scalar scale whose vector did not exist yet)
         return out
 
     def _derive(self, of: Tensor, make, name: str):

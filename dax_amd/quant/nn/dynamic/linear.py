@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import logging
 from functools import partial
+from operator import itemgetter
 
 import torch
 from torch import Tensor, nn
@@ -64,6 +65,10 @@ def _is_per_channel_observer(cls) -> bool:
     from ...quantization.observer import PerChannelMinMaxObserver  # (that package imports this module)
 
     return cls is PerChannelMinMaxObserver
+
+
+_SETTING_NAMES = ("out_dtype", "input_dtype", "weight_dtype", "compute_dtype", "input_qscheme")
+_SETTINGS = itemgetter(*_SETTING_NAMES)  # (of a module's __dict__: a third of the time that the attributes take one by one)
 
 
 class Linear(DerivedOperands, nn.Module):
@@ -179,12 +184,17 @@ class Linear(DerivedOperands, nn.Module):
 
     # ------------------------------------------------------------------ the whole forward in one call
     def _fast_settings(self):
-        return (self.in_features, self.out_dtype, self.input_dtype, self.weight_dtype, self.compute_dtype, self.input_qscheme,
-                getattr(self.quantize_activation, "__func__", None))
+        d = self.__dict__
+        try:
+            settings = _SETTINGS(d)
+        except KeyError:  # (one that a subclass computes)
+            settings = tuple(getattr(self, name) for name in _SETTING_NAMES)
+        # (and whether the quantiser is the user's own: a subclass's, or one set on the module or the class)
+        return settings, "quantize_activation" not in d and self.__class__.quantize_activation is _QUANTIZE_ACTIVATION
 
     def _fast_codes(self):
-        if getattr(self.quantize_activation, "__func__", None) is not _QUANTIZE_ACTIVATION:
-            return None  # a quantiser of the user's own: a subclass's, or one set on the module or the class
+        if not self._fast_settings()[1]:
+            return None
         if self.compute_dtype == "FP8" and self.input_qscheme == per_token_symmetric and self.out_dtype != torch.bfloat16:
             return None  # the row-wise matmul writes bf16, the result is cast afterwards
         return (ops.FMT[ops.FMT_OF_DTYPE[self.input_dtype]], ops.FMT[ops.FMT_OF_DTYPE[self.weight_dtype]],

@@ -301,3 +301,36 @@ def test_state_that_is_no_parameter_or_buffer(scheme, k):
             setattr(lin, name, t)
     assert "qweight" not in lin._parameters and "qweight" not in lin._buffers
     assert torch.equal(lin(x), want) and torch.equal(_native(lin, x), want)
+
+
+@torch.no_grad()
+def test_a_scale_of_the_other_form():
+    """A per-tensor weight scale replaced by one per channel and back: the vector made from the scalar does not stay."""
+    x = torch.randn(24, 256, device="cuda").bfloat16()
+    lin = _module("tensor_i8", 256, 64, torch.bfloat16, True, x)
+    scalar, per_channel = lin.weight_scale, torch.rand(1, 64, device="cuda") + 0.5
+    for s in (scalar, per_channel, scalar, scalar * 2, per_channel):
+        lin.weight_scale = s
+        got = _native(lin, x)
+        assert got is not None and torch.equal(got, _general(lin, x))
+        vector = lin._weight_scale_vector()
+        assert torch.equal(vector, s.reshape(-1).expand(64))
+
+
+@torch.no_grad()
+def test_settings_that_a_subclass_computes():
+    """An out_dtype that is a property, and a module saved with a quantiser of the user's own."""
+    from dax_amd.quant.nn.dynamic import Linear
+
+    x = torch.randn(24, 256, device="cuda").half()
+    lin = _module("token_i8", 256, 64, torch.float16, False, x)
+    want = lin(x)
+    del lin.out_dtype
+    lin.__class__ = type("Sub", (Linear,), {"out_dtype": property(lambda self: torch.float16)})
+    assert torch.equal(lin(x), want) and torch.equal(_native(lin, x), want)
+    lin.__class__ = type("Own", (Linear,), {"out_dtype": torch.float16, "quantize_activation": lambda self, x: Linear.quantize_activation(self, x)})
+    assert torch.equal(lin(x), want) and _native(lin, x) is None
+    lin.__class__ = Linear
+    lin.out_dtype = torch.float16
+    buf = io.BytesIO()
+    torch.save(lin, buf)
