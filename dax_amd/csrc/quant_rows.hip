@@ -78,9 +78,10 @@ __device__ __forceinline__ void chunk_values(const Chunk<XT>& v, float (&f)[8]) 
 //              range of either format, have at most five significant bits, i.e. zeros in the low 19 bits of the fp32
 //              pattern, so a product within three steps of such a pattern sends the wavefront's chunks through the
 //              division (seven patterns in 2^19, 13 elements in 10^6 under an arbitrary scale; zeros and infinities
-//              too).  A NaN does as well: a bf16 NaN has zeros in 16 low bits only, the rest of its payload lies in
-//              those 19, so it is looked for by itself.  Measured with a scale from the
-//              caller, 4096 x 5120 e5m2: 18.9 us dividing every element (26 VALU issue slots), 11.6 us here.
+//              too).  A NaN need not be near: a bf16 NaN has zeros in 16 low bits only, the rest of its payload lies in
+//              those 19.  The clamp keeps it instead (v_maximum3 / v_minimum3 return a NaN, fmed3 its lower bound; a
+//              compare per element beside the fmed3 cost 32 rows of 13824 0.2 us).  Measured with a scale from the
+//              caller, 4096 x 5120 e5m2: 18.9 us dividing every element (26 VALU issue slots), 11.5 us here.
 //   kExact     FP8 under a power of two: x * inv is the quotient
 //   kShort     bf16 elements under a bf16 scale from the caller (a per-tensor scale): their quotients hit such values all
 //              the time; the sequence of kOwn, clamped, and the division for chunks that hold an infinity or a NaN
@@ -119,8 +120,12 @@ __device__ __forceinline__ uint2 quant8(const float (&f)[8], float s, float inv)
                     const uint32_t d = (__float_as_uint(q0) << 13) + (3u << 13);
                     near = d < near ? d : near;
                 }
-                nan |= q0 != q0;
-                v[i] = __builtin_amdgcn_fmed3f(q0, -kMax, kMax);
+                if constexpr (FORM == kNear) {  // a NaN stays one
+                    v[i] = __builtin_elementwise_minimum(__builtin_elementwise_maximum(q0, -kMax), kMax);
+                } else {
+                    nan |= q0 != q0;
+                    v[i] = __builtin_amdgcn_fmed3f(q0, -kMax, kMax);
+                }
             }
             if (__ballot((FORM == kNear && near <= (6u << 13)) || nan)) {
 #pragma unroll
