@@ -156,6 +156,7 @@ _kernel_choice = 0
 _tile_group = 0
 _tile_order = 0
 _tail = 0
+_kernel_arg = 0  # all four, as the calls take them
 
 
 def debug_select_gemm(v: int) -> None:
@@ -164,7 +165,7 @@ def debug_select_gemm(v: int) -> None:
     (1000 = default); 2000 + o = tile order of the 256x256 kernels (2000 = by shape, 2001 = groups of tile rows,
     2002 = banded patches); 3000 + t = the last partial round of a 256x256 launch as 128x128 quadrants or 256x128 halves
     (3000 = by shape, 3001 = never, 3002 = whenever every such tile gets a CU)."""
-    global _kernel_choice, _tile_group, _tile_order, _tail
+    global _kernel_choice, _tile_group, _tile_order, _tail, _kernel_arg
     v = int(v)
     if 1000 <= v < 1064:
         _tile_group = v - 1000
@@ -176,7 +177,8 @@ def debug_select_gemm(v: int) -> None:
         _kernel_choice = v
     else:
         raise DaxqError(f"unknown gemm kernel choice {v}")
+    _kernel_arg = _kernel_choice | (_tile_group << 16) | (_tile_order << 24) | (_tail << 28)
 
 
 def kernel_arg() -> int:
-    return _kernel_choice | (_tile_group << 16) | (_tile_order << 24) | (_tail << 28)
+    return _kernel_arg

@@ -92,7 +92,7 @@ class DerivedOperands:
                 sw = d[1]
         if device not in _capi._checked_devices:
             _capi.require_gfx950(device)
-        out = _capi.native().linear(input, wq, sw, bias, in_scale, k, *f[1], scale_fp32, _capi.kernel_arg())
+        out = (_capi._native or _capi.native()).linear(input, wq, sw, bias, in_scale, k, *f[1], scale_fp32, _capi._kernel_arg)
         if out.__class__ is int:
             _capi.check(out, "linear")
         if out is None and d is None and sw.numel() == 1 and self._derive(sw, self._weight_scale_vector, "_sw_vec") is not None:
