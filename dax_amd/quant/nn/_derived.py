@@ -118,12 +118,13 @@ class DerivedOperands:
         return out
 
     def refresh_derived(self) -> None:
-        """Builds the derived operands now, so that a forward launches nothing but its kernels.  A module that
-        does not live on a ROCm device (yet) builds them at its first forward there."""
+        """Builds the derived operands and the codes of the native call now, so that a forward launches nothing but its
+        kernels.  A module that does not live on a ROCm device (yet) builds them at its first forward there."""
         self._packed = self._sw_vec = None
         if self.qweight.device.type == "cuda":
             self._gemm_weight()
             self._weight_scale_vector()
+            object.__setattr__(self, "_fast", (self._fast_settings(), self._fast_codes()))
 
     def _gemm_weight(self) -> Tensor:
         """qweight as the byte matrix [N, pad128(K)] the GEMM reads."""

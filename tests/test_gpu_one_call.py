@@ -334,3 +334,15 @@ def test_settings_that_a_subclass_computes():
     lin.out_dtype = torch.float16
     buf = io.BytesIO()
     torch.save(lin, buf)
+
+
+@pytest.mark.parametrize("scheme", ["token_i8", "tensor_e4m3", "static_e4m3"])
+@torch.no_grad()
+def test_conversion_prepares_the_first_forward(scheme):
+    """What the native call needs besides the state is there before the first forward, and that forward makes nothing anew."""
+    x = torch.randn(24, 200, device="cuda").bfloat16()
+    lin = _module(scheme, 200, 64, torch.bfloat16, True, x)
+    ready = lin._fast, lin._packed, lin._sw_vec
+    assert ready[0] is not None and ready[1] is not None
+    lin(x)
+    assert all(a is b for a, b in zip(ready, (lin._fast, lin._packed, lin._sw_vec)))
