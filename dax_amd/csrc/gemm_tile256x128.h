@@ -202,9 +202,8 @@ __device__ __forceinline__ void gemm_tile256x128_body(const GemmArgs& p, const i
 // the fragments of pair q+1 are read during the MFMAs of pair q, the LDS holds three pairs (48 KB each: pair q+1
 // landed, q+2 in flight, and the slot of pair q, which was read a pair ago, taking the loads of q+3), one barrier per pair.
 namespace h2f {
-constexpr int BKS = 64, BM = 256, BN = 128, T = 256;
-constexpr int A_HALF = BM * BKS, B_HALF = BN * BKS;          // one slice of an operand: 16 KB / 8 KB
-constexpr int A_PART = 2 * A_HALF, SLOT = A_PART + 2 * B_HALF;  // a pair: 32 KB of activation rows, 16 KB of weight rows
+constexpr int BKP = 128, BM = 256, BN = 128, T = 256;
+constexpr int A_PART = BM * BKP, SLOT = A_PART + BN * BKP;  // a pair: 32 KB of activation rows, 16 KB of weight rows
 constexpr int NBI = 8, NBJ = 4, NREG = NBI * NBJ;
 constexpr int A_LOADS = 8, B_LOADS = 4, PAIR_LOADS = A_LOADS + B_LOADS;
 constexpr int SMEM = 3 * SLOT;
@@ -223,42 +222,38 @@ __device__ __forceinline__ void gemm_tile256x128_fp8_body(const GemmArgs& p, con
     m0 = m0 + 256 <= p.m ? m0 : p.m - 256;
     n0 = (n0 + 256 <= p.n ? n0 : p.n - 256) + (half_id & 1) * 128;
 
-    const uint32_t gsw = (uint32_t)(((t & 3) ^ ((t >> 3) & 3)) << 4);
-    uint32_t voff_a = (uint32_t)(t >> 2) * (uint32_t)p.lda + gsw;
-    uint32_t voff_b = (uint32_t)(t >> 2) * (uint32_t)p.ldb + gsw;
-    uint32_t voff_a1 = voff_a + BKS, voff_b1 = voff_b + BKS;  // second half of the 128-byte line
+    const uint32_t gsw = (uint32_t)(((t & 7) ^ ((t >> 3) & 7)) << 4);
+    uint32_t voff_a = (uint32_t)(t >> 3) * (uint32_t)p.lda + gsw;
+    uint32_t voff_b = (uint32_t)(t >> 3) * (uint32_t)p.ldb + gsw;
     const uint8_t* abase = p.a + (int64_t)m0 * p.lda;
     const uint8_t* bbase = p.b + (int64_t)n0 * p.ldb;
-    const int64_t a_step = 64 * p.lda, b_step = 64 * p.ldb;
+    const int64_t a_step = 32 * p.lda, b_step = 32 * p.ldb;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(DAXQ_LDS uint8_t*)smem;
     const uint32_t wave_lds = lds0 + (uint32_t)__builtin_amdgcn_readfirstlane(wave * 1024);
-    // load g of a pair (12): 0-7 activation rows, 8-11 weight rows; 64-row block, then slice g%2 of the pair (the two
-    // halves of a 128-byte line by consecutive instructions).  Address = uniform row-block base (SGPR pair) + per-lane
-    // 32-bit offset: no VALU work per load.
+    // load g of a pair (12): 0-7 activation rows, 8-11 weight rows; 32 rows x 128 bytes of the workgroup, 8 of the wavefront.
+    // Address = uniform row-block base (SGPR pair) + per-lane 32-bit offset: no VALU work per load.
     auto issue_one = [&](uint32_t slot, int g) {
-        const int opnd = g >= A_LOADS, gg = opnd ? g - A_LOADS : g, j = gg >> 1, half = gg & 1;
+        const int opnd = g >= A_LOADS, j = opnd ? g - A_LOADS : g;
         const uint8_t* src = opnd ? bbase + j * b_step : abase + j * a_step;
-        const uint32_t voff = opnd ? (half ? voff_b1 : voff_b) : (half ? voff_a1 : voff_a);
-        const uint32_t dst = wave_lds + slot + (opnd ? A_PART + half * B_HALF : half * A_HALF) + j * 4096;
-        __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(src + voff), (DAXQ_LDS void*)(uintptr_t)dst, 16, 0, 0);
+        const uint32_t dst = wave_lds + slot + opnd * A_PART + j * 4096;
+        __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(src + (opnd ? voff_b : voff_a)), (DAXQ_LDS void*)(uintptr_t)dst, 16, 0, 0);
     };
     auto advance = [&]() {
-        voff_a += 2 * BKS;
-        voff_b += 2 * BKS;
-        voff_a1 += 2 * BKS;
-        voff_b1 += 2 * BKS;
+        voff_a += BKP;
+        voff_b += BKP;
     };
 
     const int lr = lane & 15, kg = lane >> 4;
-    const int xo = (kg ^ ((lr >> 1) & 3)) << 4;
-    const uint8_t* a_rd = smem + (wm * 128 + lr) * BKS + xo;
-    const uint8_t* b_rd = smem + A_PART + (wn * 64 + lr) * BKS + xo;
+    const int xo = (kg ^ (lr & 7)) << 4;
+    const uint8_t* a_rd = smem + (wm * 128 + lr) * BKP + xo;
+    const uint8_t* b_rd = smem + A_PART + (wn * 64 + lr) * BKP + xo;
+    const int to_up = 64 - 2 * (xo & 64);  // from a lane's chunk of the first slice to its chunk of the second
     // fragment f of a pair: 0-7 activation block f, 8-11 weight block f-8; registers 0-3 the first slice, 4-7 the second
     auto read_frag = [&](uint32_t slot, int f, v8i (&af)[NBI], v8i (&bf)[NBJ]) __attribute__((always_inline)) {
         const bool w = f >= NBI;
-        const uint8_t* pr = (w ? b_rd + (f - NBI) * 16 * BKS : a_rd + f * 16 * BKS) + slot;
+        const uint8_t* pr = (w ? b_rd + (f - NBI) * 16 * BKP : a_rd + f * 16 * BKP) + slot;
         const v4i lo = *reinterpret_cast<const v4i*>(pr);
-        const v4i up = *reinterpret_cast<const v4i*>(pr + (w ? B_HALF : A_HALF));
+        const v4i up = *reinterpret_cast<const v4i*>(pr + to_up);
         const v8i v = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
         if (w) bf[f - NBI] = v;
         else af[f] = v;
@@ -283,7 +278,7 @@ __device__ __forceinline__ void gemm_tile256x128_fp8_body(const GemmArgs& p, con
         }
     };
 
-    const int Q = p.k / (2 * BKS);  // pairs; K is a multiple of 128
+    const int Q = p.k / BKP;  // pairs; K is a multiple of 128
     uint32_t s0 = 0, s1 = SLOT, s2 = 2 * SLOT;  // slots of pairs q (read a pair ago), q+1, q+2
     // One pair.  PAR: which register set it consumes.  ISSUE: pair q+3 exists, its loads go into the slot of pair q.
     // NEXT: pair q+1 exists, its fragments are read into the other set.  YOUNG: tile loads behind those of pair q+1 that
@@ -293,11 +288,9 @@ __device__ __forceinline__ void gemm_tile256x128_fp8_body(const GemmArgs& p, con
         __builtin_amdgcn_s_barrier();  // pair q+1 has landed for everyone, and everyone has read pair q out of its slot
 #pragma unroll
         for (int g = 0; g < NREG; ++g) {
-            // Two loads per region, the two halves of a 128-byte line: the activation rows' four lines in regions 0, 8,
-            // 16, 24, the weight rows' two in regions 4 and 20.  (One load per region in twelve regions, between the
-            // regions that read fragments, ran the pair in 0.70 us instead of 0.56: 80.3 against 65.3 us at 1024 x 5120,
-            // K = 13824; three or four loads per region 67 to 68 us, all twelve at once 92.7.  The other tiled kernels
-            // were tried with their loads in twos as well and are as fast or 1 to 2 % faster with single ones.)
+            // Two loads per region, those of the activation rows in regions 0, 8, 16, 24, those of the weight rows in regions 4
+            // and 20.  (While a load took half lines, one load per region ran the pair in 0.70 us instead of 0.56; with whole
+            // lines the two differ by less than 1 %.)
             if constexpr (ISSUE.value) {
                 if (g % 8 == 0) {
                     issue_one(s0, g / 4);

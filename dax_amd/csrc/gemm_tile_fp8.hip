@@ -19,15 +19,17 @@
 //                                          j is dead after its NB MFMAs and is refilled in place for the next pair
 //                                          right behind them; the last block, which is in use until the pair ends, has
 //                                          a second register set
-// LDS: five parts, each ONE operand of ONE pair, [slice of the pair][BT rows][64 B] with the 16-byte chunk swizzle
-// chunk ^ ((row >> 1) & 3) (a fragment read takes 16 rows x 4 chunks and is conflict free).  They form a ring in the
+// LDS: five parts, each ONE operand of ONE pair, [BT rows][128 B] with the 16-byte chunk swizzle chunk ^ (row & 7) (a
+// fragment read takes 16 rows x 4 chunks and is conflict free).  They form a ring in the
 // order the loads are issued, ... B(q+1), A(q+1), B(q+2), A(q+2), B(q+3) ...:
 //   pair q, even half   MFMAs of the first half of the B blocks; DMA loads of A(q+2) into the part B(q) has left
 //   pair q, odd half    MFMAs of the other B blocks; DMA loads of B(q+3) into the part A(q) has left; reads all of A
 //                       of pair q+1
 // One barrier per half: at the first B(q+1) has landed, at the second A(q+1); every load has two to three slice
 // times to land.  Loads are global_load_lds_dwordx4 straight into LDS, addressed as SGPR row-block base + 32-bit lane
-// offset, the two halves of a 128-byte line by consecutive instructions.
+// offset, 8 rows x 128 bytes an instruction.  16 rows x 64 bytes, the two halves of a line by consecutive instructions -> this,
+// us: 512 x 5120 x 5120 20.9 -> 19.4 (weights out of reach of the caches 29.6 -> 28.0), 1024 x 5120 x 5120 29.1 -> 27.2 (halves),
+// 4096 x 1536 x 1536 15.7 -> 15.1, 9450 x 13824, K = 5120 480 -> 468, 75600 x 5120 x 5120 1371 -> 1359.
 // A and B of a lane hold the same K bytes (chunk l/16 of the pair's first slice, then of its second), which is all
 // the MFMA needs: the order of K inside an instruction is free as long as both operands agree.
 // K shorter than four pairs (K < 512) takes a plain loop of the same MFMAs: load a pair, wait, multiply.
@@ -37,7 +39,7 @@
 namespace daxq {
 
 namespace f16 {
-constexpr int BKS = 64, T = 256, NPART = 5;
+constexpr int BKP = 128, T = 256, NPART = 5;
 }  // namespace f16
 
 template <bool DUMP, int F8, int BT = 256, int OUTK = DAXQ_BF16>
@@ -47,8 +49,7 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
     static_assert(OUTK == DAXQ_BF16 || !DUMP, "the accumulator dump exists with bf16 outputs");
     constexpr int NB = BT / 32;             // 16x16 blocks per operand and wavefront
     constexpr int WT = BT / 2;              // edge of a wavefront's outputs
-    constexpr int HALF = BT * BKS;          // one slice of one operand: 16 / 8 KB
-    constexpr int PART = 2 * HALF;          // one operand of one pair
+    constexpr int PART = BT * BKP;          // one operand of one pair: 32 / 16 KB
     constexpr int LPO = BT / 32;            // DMA loads per thread, operand and pair
     constexpr int NREG = NB * NB;           // MFMAs = scheduling regions per pair
     constexpr int HREG = NREG / 2;          // ... per half
@@ -60,51 +61,46 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
     int m0, n0;
     if (!tile_origin<BT>(p, block, m0, n0)) return;  // padding slot (before any barrier)
 
-    // ---- HBM side: one wave instruction fills 1 KB of LDS = 16 rows x 64 B; lane l -> row l/4, stored chunk l%4,
-    //      i.e. global chunk (l%4) ^ ((row >> 1) & 3).  Load g of an operand and pair: row block g/2 (64 rows, of which
-    //      this wave fills 16), slice g%2 of the pair (the two halves of a 128-byte line, adjacent instructions).
-    const uint32_t gsw = (uint32_t)(((t & 3) ^ ((t >> 3) & 3)) << 4);
-    uint32_t voff_a = (uint32_t)(t >> 2) * (uint32_t)p.lda + gsw;
-    uint32_t voff_b = (uint32_t)(t >> 2) * (uint32_t)p.ldb + gsw;
-    uint32_t voff_a1 = voff_a + BKS, voff_b1 = voff_b + BKS;
+    // ---- HBM side: one wave instruction fills 1 KB of LDS = 8 rows x 128 B (whole lines: what a CU gets through its load path
+    //      is bound by the lines an instruction touches, gemm_tile256.hip); lane l -> row l/8, stored chunk l%8, i.e. global
+    //      chunk (l%8) ^ (row&7).  Load g of an operand and pair: rows 32 g .. 32 g + 31, of which this wave fills 8.
+    const uint32_t gsw = (uint32_t)(((t & 7) ^ ((t >> 3) & 7)) << 4);
+    uint32_t voff_a = (uint32_t)(t >> 3) * (uint32_t)p.lda + gsw;
+    uint32_t voff_b = (uint32_t)(t >> 3) * (uint32_t)p.ldb + gsw;
     const uint8_t* abase = p.a + (int64_t)m0 * p.lda;
     const uint8_t* bbase = p.b + (int64_t)n0 * p.ldb;
-    const int64_t a_step = 64 * p.lda, b_step = 64 * p.ldb;
+    const int64_t a_step = 32 * p.lda, b_step = 32 * p.ldb;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(DAXQ_LDS uint8_t*)smem;
     const uint32_t wave_lds = lds0 + (uint32_t)__builtin_amdgcn_readfirstlane(wave * 1024);
     auto issue_a = [&](uint32_t part, int g) {
-        const int j = g >> 1, half = g & 1;
-        const uint32_t dst = wave_lds + part + half * HALF + j * 4096;
-        __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(abase + j * a_step + (half ? voff_a1 : voff_a)),
-                                         (DAXQ_LDS void*)(uintptr_t)dst, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(abase + g * a_step + voff_a),
+                                         (DAXQ_LDS void*)(uintptr_t)(wave_lds + part + g * 4096), 16, 0, 0);
     };
     auto issue_b = [&](uint32_t part, int g) {
-        const int j = g >> 1, half = g & 1;
-        const uint32_t dst = wave_lds + part + half * HALF + j * 4096;
-        __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(bbase + j * b_step + (half ? voff_b1 : voff_b)),
-                                         (DAXQ_LDS void*)(uintptr_t)dst, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(bbase + g * b_step + voff_b),
+                                         (DAXQ_LDS void*)(uintptr_t)(wave_lds + part + g * 4096), 16, 0, 0);
     };
     auto advance_a = [&]() {
-        voff_a += 2 * BKS;
-        voff_a1 += 2 * BKS;
+        voff_a += BKP;
     };
     auto advance_b = [&]() {
-        voff_b += 2 * BKS;
-        voff_b1 += 2 * BKS;
+        voff_b += BKP;
     };
 
-    // ---- LDS side: row (w*WT + i*16 + l%16), K chunk l/16 of either slice, stored at chunk (l/16) ^ ((l%16 >> 1) & 3)
+    // ---- LDS side: row (w*WT + i*16 + l%16), K chunk l/16 of either slice, chunk c of the line stored at c ^ (row&7)
     const int lr = lane & 15, kg = lane >> 4;
-    const int xo = (kg ^ ((lr >> 1) & 3)) << 4;
-    const uint8_t* a_rd = smem + (wm * WT + lr) * BKS + xo;
-    const uint8_t* b_rd = smem + (wn * WT + lr) * BKS + xo;
+    const int xo = (kg ^ (lr & 7)) << 4;
+    const uint8_t* a_rd = smem + (wm * WT + lr) * BKP + xo;
+    const uint8_t* b_rd = smem + (wn * WT + lr) * BKP + xo;
+    const int to_up = 64 - 2 * (xo & 64);  // from a lane's chunk of the first slice to its chunk of the second
+    const uint8_t *a_up = a_rd + to_up, *b_up = b_rd + to_up;
     // A fragment is refilled as two updates of half of its registers: the register allocator then keeps the
     // fragment where it is (a fresh 8-register value per refill made it rotate the fragment sets through one
     // another with copies and spills).
-    auto read_into = [&](v8i& dst, const uint8_t* base, uint32_t part, int blk) __attribute__((always_inline)) {
-        const uint8_t* pr = base + part + blk * 16 * BKS;
-        const v4i lo = *reinterpret_cast<const v4i*>(pr);
-        const v4i up = *reinterpret_cast<const v4i*>(pr + HALF);
+    auto read_into = [&](v8i& dst, bool w, uint32_t part, int blk) __attribute__((always_inline)) {
+        const uint32_t at = part + blk * 16 * BKP;
+        const v4i lo = *reinterpret_cast<const v4i*>((w ? b_rd : a_rd) + at);
+        const v4i up = *reinterpret_cast<const v4i*>((w ? b_up : a_up) + at);
         const v8i lo8 = __builtin_shufflevector(lo, lo, 0, 1, 2, 3, -1, -1, -1, -1);  // (widened; the upper lanes are never taken)
         const v8i up8 = __builtin_shufflevector(up, up, 0, 1, 2, 3, -1, -1, -1, -1);
         dst = __builtin_shufflevector(lo8, dst, 0, 1, 2, 3, 12, 13, 14, 15);
@@ -142,7 +138,7 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
         }
     };
 
-    const int Q = p.k / (2 * BKS);  // pairs; K is a multiple of 128
+    const int Q = p.k / BKP;  // pairs; K is a multiple of 128
     // the ring, oldest part first: at the start of pair q it holds B(q), A(q) (both read already), B(q+1), A(q+1), B(q+2)
     uint32_t r0 = 0, r1 = PART, r2 = 2 * PART, r3 = 3 * PART, r4 = 4 * PART;
 
@@ -169,11 +165,11 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
                 __builtin_amdgcn_s_waitcnt(vmcnt_imm((ISSUE_A.value ? 2 * LPO : 0) + EXTRA.value));
                 __builtin_amdgcn_s_barrier();
             }
-            // 128 tiles issue their loads in twos (both halves of a 128-byte line in one region): with a load in every other
+            // 128 tiles issue their loads in twos: with a load in every other
             // region of so short a pair nearly every MFMA has a memory instruction in front of it; +2.5 % on launches with
             // a CU per workgroup and long K (512 x 5120 x 5120: 21.0 -> 20.5 us), nothing elsewhere.  The 256 tiles, a
             // load every fourth region, lose 1 % that way.
-            constexpr bool twos = BT == 128;
+                        constexpr bool twos = BT == 128;
             if constexpr (ISSUE_A.value) {
                 if constexpr (twos) {
                     if (g < HREG && g % (2 * DMA_EVERY) == 0) {
@@ -197,11 +193,11 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
             if constexpr (nxt) {
                 // the last B block of the next pair into the set this pair does not use
                 if (g == (NB == 8 ? 2 : 1)) {
-                    if constexpr (par) read_into(fbl_0, b_rd, r2, NB - 1);
-                    else read_into(fbl_1, b_rd, r2, NB - 1);
+                    if constexpr (par) read_into(fbl_0, true, r2, NB - 1);
+                    else read_into(fbl_1, true, r2, NB - 1);
                 }
                 // B block j right behind its last MFMA of this pair
-                if (g >= NB && g % NB == 0) read_into(fb[g / NB - 1], b_rd, r2, g / NB - 1);
+                if (g >= NB && g % NB == 0) read_into(fb[g / NB - 1], true, r2, g / NB - 1);
                 // all of A of the next pair during the odd half, between the B refills
                 if (g > HREG) {
                     const int o = g - HREG;  // 1 .. HREG-1
@@ -218,8 +214,8 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
                             if (o == at[x]) i = x;
                     }
                     if (i >= 0) {
-                        if constexpr (par) read_into(fa0[i], a_rd, r3, i);
-                        else read_into(fa1[i], a_rd, r3, i);
+                        if constexpr (par) read_into(fa0[i], false, r3, i);
+                        else read_into(fa1[i], false, r3, i);
                     }
                 }
             }
@@ -277,10 +273,10 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * LPO));
         __builtin_amdgcn_s_barrier();
 #pragma unroll
-        for (int j = 0; j < NB - 1; ++j) read_into(fb[j], b_rd, r0, j);
+        for (int j = 0; j < NB - 1; ++j) read_into(fb[j], true, r0, j);
 #pragma unroll
-        for (int i = 0; i < NB; ++i) read_into(fa0[i], a_rd, r1, i);
-        read_into(fbl_0, b_rd, r0, NB - 1);
+        for (int i = 0; i < NB; ++i) read_into(fa0[i], false, r1, i);
+        read_into(fbl_0, true, r0, NB - 1);
 
         // Pair q consumes register set q % 2 and fills the other one.  Pair 0, then the steady pairs 1 .. Q-4 two at a
         // time (odd, even), then one more if their number is odd.  The three pairs of the tail are code paths of their
@@ -321,10 +317,10 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
             __builtin_amdgcn_s_barrier();
 #pragma unroll
-            for (int j = 0; j < NB - 1; ++j) read_into(fb[j], b_rd, r0, j);
-            read_into(fbl_0, b_rd, r0, NB - 1);
+            for (int j = 0; j < NB - 1; ++j) read_into(fb[j], true, r0, j);
+            read_into(fbl_0, true, r0, NB - 1);
 #pragma unroll
-            for (int i = 0; i < NB; ++i) read_into(fa0[i], a_rd, r1, i);
+            for (int i = 0; i < NB; ++i) read_into(fa0[i], false, r1, i);
             __builtin_amdgcn_s_waitcnt(lgkmcnt0_mask() & vmcnt_imm(63));
             __builtin_amdgcn_sched_barrier(0);
             if (q == 0) {
@@ -385,7 +381,7 @@ __global__ __launch_bounds__(256) void gemm_tile_fp8_then_quadrants_kernel(const
 template <bool DUMP, int F8, int BT, int OUTK>
 static int prepare_fp8() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK>), f16::NPART * 2 * BT * f16::BKS, lds_set);
+    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK>), f16::NPART * BT * f16::BKP, lds_set);
 }
 
 template <bool DUMP, int F8, int BT, int OUTK>
@@ -393,7 +389,7 @@ static int launch_fp8_impl(const GemmArgs& a, hipStream_t st) {
     if (int rc = prepare_fp8<DUMP, F8, BT, OUTK>()) return rc;
     const int64_t nt = grid_of_order(a);
     if (nt > 0x7fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
-    hipLaunchKernelGGL((gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK>), dim3((unsigned)nt), dim3(f16::T), f16::NPART * 2 * BT * f16::BKS, st, a);
+    hipLaunchKernelGGL((gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK>), dim3((unsigned)nt), dim3(f16::T), f16::NPART * BT * f16::BKP, st, a);
     return check_launch("gemm_tile_fp8");
 }
 
@@ -424,13 +420,13 @@ static const void* fp8_then_kernel() {
 template <bool QUADS, bool DUMP, int F8, int OUTK>
 static int prepare_fp8_then() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    return ensure_dynamic_lds(fp8_then_kernel<QUADS, DUMP, F8, OUTK>(), f16::NPART * 2 * 256 * f16::BKS, lds_set);
+    return ensure_dynamic_lds(fp8_then_kernel<QUADS, DUMP, F8, OUTK>(), f16::NPART * 256 * f16::BKP, lds_set);
 }
 
 template <bool QUADS, bool DUMP, int F8, int OUTK>
 static int launch_fp8_then_impl(const GemmArgs& a, int64_t nt, hipStream_t st) {
     if (int rc = prepare_fp8_then<QUADS, DUMP, F8, OUTK>()) return rc;
-    constexpr int SMEM = f16::NPART * 2 * 256 * f16::BKS;
+    constexpr int SMEM = f16::NPART * 256 * f16::BKP;
     if constexpr (QUADS) hipLaunchKernelGGL((gemm_tile_fp8_then_quadrants_kernel<DUMP, F8, OUTK>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
     else hipLaunchKernelGGL((gemm_tile_fp8_then_halves_kernel<DUMP, F8, OUTK>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
     return check_launch(QUADS ? "gemm_tile_fp8_then_quadrants" : "gemm_tile_fp8_then_halves");
