@@ -22,25 +22,21 @@ namespace daxq {
 
 // ZERO: the block's first MFMA of a tile, which starts from zero instead of the accumulator
 // F8: FP8 operand formats (kF8XE5 / kF8WE5: e5m2 activation / weight bytes)
-template <bool FP8, int F8, bool ZERO = false, int NB = 4>
-__device__ __forceinline__ void mfma_one(typename AccT<FP8>::type (&acc)[NB][NB], int g, const typename Frag<FP8>::type (&af)[4],
-                                         const typename Frag<FP8>::type (&bf)[4]) {
+template <int F8, bool ZERO = false, int NB = 4>
+__device__ __forceinline__ void mfma_one(v16f (&acc)[NB][NB], int g, const v8i (&af)[4], const v8i (&bf)[4]) {
     const int j = g / NB, i = g % NB;
-    typename AccT<FP8>::type c = {};
+    v16f c = {};
     if constexpr (!ZERO) c = acc[j][i];
-    if constexpr (!FP8)
-        acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], af[i], c, 0, 0, 0);
-    else
-        acc[j][i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af[i], c, (F8 & kF8WE5) ? 1 : 0, (F8 & kF8XE5) ? 1 : 0, 0, 0, 0, 0);
+    acc[j][i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af[i], c, (F8 & kF8WE5) ? 1 : 0, (F8 & kF8XE5) ? 1 : 0, 0, 0, 0, 0);
 }
 
-// Epilogue.  In a 32x32 block a lane owns output row m = l%32 and, in registers 4q..4q+3, the
+// Epilogue of the FP8 split-K form.  In a 32x32 block a lane owns output row m = l%32 and, in registers 4q..4q+3, the
 // columns n = 8q + 4*(l/32) + {0..3}.  Two v_permlane32_swap per pair of q give each lane 8
 // consecutive columns, stored as one 16-byte write.  The tile's scales and bias are staged in LDS.
 // pre_*: this thread's element (index t) of the tile's sx / sw / bias, already loaded by the caller.
-// NB: 32x32 blocks per operand and wavefront (4: 256x256 tile, 2: 128x128 tile); the tile edge is 64 * NB.
-template <bool FP8, bool DUMP, int NB = 4>
-__device__ __forceinline__ void tile256_epilogue(const GemmArgs& p, typename AccT<FP8>::type (&acc)[NB][NB], uint8_t* smem,
+// NB: 32x32 blocks per operand and wavefront; the tile edge is 64 * NB.
+template <int NB>
+__device__ __forceinline__ void tile256_epilogue(const GemmArgs& p, v16f (&acc)[NB][NB], uint8_t* smem,
                                                  int m0, int n0, int t, int wm, int wn, int l31, int hi, float pre_sx,
                                                  float pre_sw, float pre_bias) {
     constexpr int BT = 64 * NB, WT = 32 * NB;
@@ -53,23 +49,6 @@ __device__ __forceinline__ void tile256_epilogue(const GemmArgs& p, typename Acc
         s_bias[t] = pre_bias;
     }
     __syncthreads();
-
-    if constexpr (DUMP) {
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                const int64_t m = m0 + wm * WT + i * 32 + l31;
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int n = n0 + wn * WT + j * 32 + 8 * (v >> 2) + 4 * hi + (v & 3);
-                    if constexpr (!FP8)
-                        static_cast<int32_t*>(p.acc)[m * p.ldacc + n] = acc[j][i][v];
-                    else
-                        static_cast<float*>(p.acc)[m * p.ldacc + n] = acc[j][i][v];
-                }
-            }
-    }
 
     // every scale and bias value this lane needs goes into registers in one burst of LDS reads
     // (the fragment registers of the main loop are free now): 4 x sx, 16 x 4 sw, 16 x 4 bias
@@ -102,21 +81,8 @@ __device__ __forceinline__ void tile256_epilogue(const GemmArgs& p, typename Acc
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {  // two columns at a time: v_cvt_pk_bf16_f32 rounds a pair (RNE)
                     const int r = 2 * h;
-                    if constexpr (!FP8) {
-                        float y0 = (float)acc[j][i][q * 4 + r];  // v_cvt_f32_i32, round to nearest even
-                        float y1 = (float)acc[j][i][q * 4 + r + 1];
-                        y0 = y0 * sxv;
-                        y1 = y1 * sxv;
-                        y0 = y0 * sws[r];
-                        y1 = y1 * sws[r + 1];
-                        const uint32_t o1 = pack_bf16_rne(y0, y1);
-                        // second rounding: the bias is added to the bf16 value
-                        pk[q][h] = pack_bf16_rne(__uint_as_float(o1 << 16) + bs[r],
-                                                 __uint_as_float(o1 & 0xffff0000u) + bs[r + 1]);
-                    } else {
-                        pk[q][h] = pack_bf16_rne(acc[j][i][q * 4 + r] * sxv * sws[r] + bs[r],
-                                                 acc[j][i][q * 4 + r + 1] * sxv * sws[r + 1] + bs[r + 1]);
-                    }
+                    pk[q][h] = pack_bf16_rne(acc[j][i][q * 4 + r] * sxv * sws[r] + bs[r],
+                                             acc[j][i][q * 4 + r + 1] * sxv * sws[r + 1] + bs[r + 1]);
                 }
             }
 #pragma unroll
@@ -132,22 +98,27 @@ __device__ __forceinline__ void tile256_epilogue(const GemmArgs& p, typename Acc
 }
 
 // ---------------------------------------------------------------------------------------------
-// K in 64-byte slices through five 32 KB LDS stages (all 160 KB): the LDS holds the slice being read plus four more,
-// and the load stream is even: 8 loads per 64-byte slice, one every eighth MFMA (INT8).
-//   * loads are issued in pairs of slices (2q, 2q+1) so that the two 64-byte halves of a 128-byte
-//     line are requested by adjacent instructions (the second hits L1: measured at the full-line
-//     rate, whereas half lines requested a slice apart run at half of it);
+// K in pairs of 64-byte slices through five 32 KB LDS parts (all 160 KB), each ONE operand of ONE pair: the LDS holds the
+// pair being read plus one and a half more, and the load stream is even: 8 loads per 64-byte slice, one every eighth
+// MFMA (INT8).
+//   * a load instruction takes 8 rows x 128 bytes, i.e. whole lines.  What a CU gets through its load path is bound by the
+//     lines an instruction touches (loads into LDS alone, rows 20 KB apart, cycles per 32 KB: 16 rows x 64 bytes, both halves of
+//     a line by consecutive instructions, 840 to 970; 8 rows x 128 bytes 710 to 750; 1 KB in one piece 670); a 128 tile needs
+//     32 KB per 512 MFMA cycles and a 256 tile 64 KB per 2048;
 //   * the A loads of pair q+2 go out during slice 2q, its B loads during slice 2q+1; the pair has to
 //     have landed at the barrier of slice 2q+3;
-//   * fragments of slice s+1 are read during slice s into the other of two register sets.
-// LDS layout of an operand part: [256 rows][64 B], 16-byte chunk c of row r stored at chunk
-// c ^ ((r >> 2) & 3) (32x32 MFMA forms) or c ^ ((r >> 1) & 3) (16x16 form): the ds_read_b128 of either form
-// then runs at the full LDS rate.
+//   * fragments of slice s+1 are read during slice s into the other of two register sets.  One barrier per pair, at its
+//     odd slice: there pair q+1 has landed and everyone has read pair q out of its parts.
+// LDS layout of a part: [256 rows][128 B], 16-byte chunk c of row r stored at chunk c ^ (r & 7): a ds_read_b128 of 16 rows
+// then takes 4.8 cycles of the LDS (with ((r >> 1) & 3) or (r & 7) ^ ((r >> 3) & 1) 8.0, in plain order 16).
+// Half lines and a barrier per slice -> this, us, weights of three launches in turn: 512 x 5120 x 5120 (128 tiles) 22.0 -> 20.3,
+// with weights out of reach of the caches 30.8 -> 28.6; 4096 x 1536 x 1536 (128 tiles) 17.4 -> 15.6; 9450 x 13824, K = 5120 503 ->
+// 495; 32760 x 4608, K = 1536 221 -> 216; 75600 x 5120 x 5120 1391 -> 1375 (the board's power, not the load path).
 //
 // BT: tile edge.  256 is the form described above; 128 (wavefronts of 64 x 64, five 16 KB stages, two workgroups
 // per CU) is the same pipeline for launches with too few 256-tiles to fill the CUs.
 namespace t5 {
-constexpr int BKS = 64, NST = 5, T = 256;
+constexpr int BKS = 64, BKP = 2 * BKS, T = 256;
 }  // namespace t5
 
 // accumulators of a wavefront's 128 x 128 outputs
@@ -178,17 +149,15 @@ __device__ __forceinline__ void gemm_tile256s5_body(const GemmArgs& p, const int
     static_assert(FP8 ? SPLITK : N16, "INT8 runs the 16x16 form; FP8 comes here for split-K only");
     static_assert(BT == 256 || BT == 128, "tile edge");
     static_assert(D == 2 || (D == 4 && BT == 128 && !SPLITK), "the deep ring exists on 128 tiles (nine 16 KB stages)");
-    constexpr int NSTG = 2 * D + 1;                   // LDS stages: the slice being read plus D pairs in flight
+    constexpr int NPART = 2 * D + 1;                  // LDS parts: the pair being read, D - 1 more and the one being loaded
     typedef typename Frag<FP8>::type frag_t;
     constexpr int WT = BT / 2;                        // edge of a wavefront's outputs
-    constexpr int NB = WT / (N16 ? 16 : 32);          // MFMA blocks per operand and wavefront: 8 / 4 (256), 4 / 2 (128)
-    constexpr int A_BYTES = BT * BKS, STAGE = 2 * A_BYTES;
+    constexpr int NB = WT / (N16 ? 16 : 32);          // MFMA blocks per operand and wavefront: 8 / 4 (16x16, 256 / 128 tile), 2 (32x32)
+    constexpr int PART = BT * BKP;                    // one operand of one pair
     constexpr int PAIR_LOADS = BT / 16;               // DMA loads per thread and pair of slices
-    constexpr int JB = BT / 64;                       // 64-row blocks of an operand part (one DMA instruction each)
-    constexpr int STEPS = FP8 ? 1 : 2;               // MFMA steps per 64-byte slice (32x32 form)
-    constexpr int NREG = N16 ? NB * NB : NB * NB * STEPS;  // MFMAs = scheduling regions per slice
+    constexpr int NREG = NB * NB;                     // MFMAs = scheduling regions per slice
     constexpr int DMA_EVERY = NREG / (PAIR_LOADS / 2);     // regions per DMA load
-    constexpr int READ_EVERY = NREG >= 48 ? 3 : NREG / (2 * NB);  // N16: regions per fragment read (2 * NB reads)
+    constexpr int READ_EVERY = NREG >= 48 ? 3 : NREG / (2 * NB);  // regions per fragment read (2 * NB reads)
 
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
@@ -210,129 +179,99 @@ __device__ __forceinline__ void gemm_tile256s5_body(const GemmArgs& p, const int
         if (!tile_origin<BT>(p, tile_id, m0, n0)) return;  // padding slot (before any barrier)
     }
 
-    // ---- HBM side.  One wave instruction fills 1 KB of LDS = 16 rows x 64 B: lane l -> row l/4,
-    //      stored chunk l%4, i.e. global chunk (l%4) ^ ((row>>2)&3).  Instruction j of a thread
-    //      covers tile rows j*64 + t/4.
-    //      N16 swizzles with (row>>1)&3 instead: its fragment reads (16 rows x 4 chunks per instruction) are
-    //      conflict free with that one and lose a fifth of the LDS rate with (row>>2)&3 (measured).
-    const uint32_t gsw = (uint32_t)(((t & 3) ^ ((N16 ? t >> 3 : t >> 4) & 3)) << 4);
-    uint32_t voff_a = (uint32_t)(t >> 2) * (uint32_t)p.lda + gsw;
-    uint32_t voff_b = (uint32_t)(t >> 2) * (uint32_t)p.ldb + gsw;
-    uint32_t voff_a1 = voff_a + BKS, voff_b1 = voff_b + BKS;  // second half of the 128-byte line
+    // ---- HBM side.  One wave instruction fills 1 KB of LDS = 8 rows x 128 B: lane l -> row l/8, stored chunk l%8, i.e.
+    //      global chunk (l%8) ^ (row&7).  Instruction j of a thread covers tile rows j*32 + t/8.
+    const uint32_t gsw = (uint32_t)(((t & 7) ^ ((t >> 3) & 7)) << 4);
+    uint32_t voff_a = (uint32_t)(t >> 3) * (uint32_t)p.lda + gsw;
+    uint32_t voff_b = (uint32_t)(t >> 3) * (uint32_t)p.ldb + gsw;
     const uint8_t* abase = p.a + (int64_t)m0 * p.lda + (int64_t)split * klen;
     const uint8_t* bbase = p.b + (int64_t)n0 * p.ldb + (int64_t)split * klen;
-    const int64_t a_step = 64 * p.lda, b_step = 64 * p.ldb;
+    const int64_t a_step = 32 * p.lda, b_step = 32 * p.ldb;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(DAXQ_LDS uint8_t*)smem;
     const uint32_t wave_lds = lds0 + (uint32_t)__builtin_amdgcn_readfirstlane(wave * 1024);
-    // load g of a pair (16 for a 256 tile): first half of them operand A, row block (g/2) % JB, half g%2 -> stage o0 / o1.
+    // load g of a pair (16 for a 256 tile): first half of them operand A, row block g % (PAIR_LOADS / 2) -> the part at `part`.
     // Address = uniform row-block base (SGPR pair) + per-lane 32-bit offset: no VALU work per load.
-    auto issue_one = [&](uint32_t o0, uint32_t o1, int g) {
-        const int opnd = g / (PAIR_LOADS / 2), j = (g >> 1) % JB, half = g & 1;
+    auto issue_one = [&](uint32_t part, int g) {
+        const int opnd = g / (PAIR_LOADS / 2), j = g % (PAIR_LOADS / 2);
         const uint8_t* src = opnd ? bbase + j * b_step : abase + j * a_step;
-        const uint32_t voff = opnd ? (half ? voff_b1 : voff_b) : (half ? voff_a1 : voff_a);
-        const uint32_t dst = wave_lds + (half ? o1 : o0) + opnd * A_BYTES + j * 4096;
-        __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(src + voff), (DAXQ_LDS void*)(uintptr_t)dst, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const DAXQ_GLOBAL void*)(src + (opnd ? voff_b : voff_a)),
+                                         (DAXQ_LDS void*)(uintptr_t)(wave_lds + part + j * 4096), 16, 0, 0);
     };
-    auto advance_a = [&]() {
-        voff_a += 2 * BKS;
-        voff_a1 += 2 * BKS;
-    };
-    auto advance_b = [&]() {
-        voff_b += 2 * BKS;
-        voff_b1 += 2 * BKS;
-    };
+    auto advance_a = [&]() { voff_a += BKP; };
+    auto advance_b = [&]() { voff_b += BKP; };
     auto advance = [&]() {
         advance_a();
         advance_b();
     };
 
-    // ---- LDS side: row (w*128 + i*32 + l%32), chunk c of the slice at (c ^ g) * 16, g = (l%32 >> 2) & 3
-    //      N16: row (w*128 + i*16 + l%16), the lane's K chunk is l/16
+    // ---- LDS side: row r of a wavefront's block, lane l on row l%16 (16x16 form: its K chunk is l/16 of the slice, i.e. chunk
+    //      l/16 + 4h of the line in slice h of the pair) or l%32 (32x32 form: chunks 2 (l/32) + {0, 1} + 4h)
     const int l31 = lane & 31, hi = lane >> 5;
     const int lr = N16 ? (lane & 15) : l31;  // row of the lane inside an MFMA block
-    const int gq = ((N16 ? lr >> 1 : lr >> 2)) & 3;
-    const uint8_t* a_rd = smem + (wm * WT + lr) * BKS;
-    const uint8_t* b_rd = smem + A_BYTES + (wn * WT + lr) * BKS;
-    // one fragment: f = 0..3 A block f, 4..7 B block f-4; step ks of the slice in the stage at offset o
-    // (N16: ks selects the upper four of the eight 16-row blocks; every fragment spans the whole slice)
-    auto read_frag = [&](uint32_t o, int ks, int f, frag_t (&af)[4], frag_t (&bf)[4]) {
+    const int c0 = ((N16 ? lane >> 4 : 2 * hi) ^ (lr & 7)) << 4;
+    const int to_odd = 64 - 2 * (c0 & 64);   // from the lane's chunk of the even slice to that of the odd one
+    const uint8_t* a_rd = smem + (wm * WT + lr) * BKP + c0;
+    const uint8_t* b_rd = smem + (wn * WT + lr) * BKP + c0;
+    const uint8_t *a_rd1 = a_rd + to_odd, *b_rd1 = b_rd + to_odd;
+    // one fragment: f = 0..3 A block f, 4..7 B block f-4, of the slice H of the pair whose part lies at offset o
+    // (16x16 form: ks selects the upper four of the eight 16-row blocks)
+    auto read_frag = [&](auto H, uint32_t o, int ks, int f, frag_t (&af)[4], frag_t (&bf)[4]) __attribute__((always_inline)) {
+        const uint8_t* pr = (f < 4 ? (H.value ? a_rd1 : a_rd) : (H.value ? b_rd1 : b_rd)) + o;
         if constexpr (N16) {
-            const uint8_t* pr = (f < 4 ? a_rd : b_rd) + o + (ks * 4 + (f & 3)) * 16 * BKS;
-            (f < 4 ? af[f & 3] : bf[f & 3]) = *reinterpret_cast<const v4i*>(pr + (((lane >> 4) ^ gq) << 4));
-            return;
-        }
-        if ((f & 3) >= NB) return;  // 128 tile: two 32-row blocks per operand
-        const uint8_t* pr = (f < 4 ? a_rd : b_rd) + o + (f & 3) * 32 * BKS;
-        if constexpr (!FP8) {
-            const int xo = ((ks * 2 + hi) ^ gq) << 4;
-            (f < 4 ? af[f & 3] : bf[f & 3]) = *reinterpret_cast<const v4i*>(pr + xo);
+            (f < 4 ? af[f & 3] : bf[f & 3]) = *reinterpret_cast<const v4i*>(pr + (ks * 4 + (f & 3)) * 16 * BKP);
         } else {
-            const int xo0 = ((hi * 2) ^ gq) << 4, xo1 = ((hi * 2 + 1) ^ gq) << 4;
-            v4i lo = *reinterpret_cast<const v4i*>(pr + xo0);
-            v4i up = *reinterpret_cast<const v4i*>(pr + xo1);
+            if ((f & 3) >= NB) return;  // two 32-row blocks per operand
+            const v4i lo = *reinterpret_cast<const v4i*>(pr + (f & 3) * 32 * BKP);
+            const v4i up = *reinterpret_cast<const v4i*>(pr + (f & 3) * 32 * BKP + (16 - 2 * (c0 & 16)));
             (f < 4 ? af[f & 3] : bf[f & 3]) = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
         }
     };
 
     typename TileAcc<FP8, N16>::type acc[NB][NB];
 
-    // fragment sets: [slice parity][MFMA step] (N16: [slice parity][blocks 0-3 / 4-7])
+    // fragment sets: [slice parity][16x16 form: blocks 0-3 / 4-7]
     frag_t fa00[4] = {}, fb00[4] = {}, fa01[4] = {}, fb01[4] = {}, fa10[4] = {}, fb10[4] = {}, fa11[4] = {}, fb11[4] = {};
 
-    const int S = klen / BKS;  // slices; even because K (and each split range) is a multiple of 128
-    // stage offsets of slices s .. s+2D-1 and, last, of slice s-1 (s = the even slice of the current pair)
-    uint32_t st[NSTG];
+    const int Q = klen / BKP;  // pairs
+    // parts of A(q), B(q), ... A(q+D-1), B(q+D-1) and, last, of A(q+D) (q = the current pair)
+    uint32_t st[NPART];
 #pragma unroll
-    for (int i = 0; i < NSTG; ++i) st[i] = i * STAGE;
+    for (int i = 0; i < NPART; ++i) st[i] = i * PART;
 
-    // One slice.  ODD: slice parity (which register set is consumed).  At its barrier slice s+1 has
-    // landed for every wave and every wave has the fragments of slice s in registers.
-    //   ISSUE  start half of pair (s+2D, s+2D+1) (s even: the A loads; s odd: the B loads of the same
-    //          pair) into the stages o_ld0 / o_ld1 that slices s-1 and s have left
+    // One slice.  ODD: slice parity (which register set is consumed).
+    //   ISSUE  even: start the A loads of pair q+D into the part that B of pair q-1 has left (everyone has been past its reads
+    //          since the barrier of the last odd slice); odd: its B loads into the part that A of pair q has left
     //   NEXT   slice s+1 exists: read its fragments into the other set
-    //   YOUNG  number of loads issued after those of slice s+1 that may stay in flight: D-1 whole pairs at
-    //          an even slice, D-2 pairs and the A half of the newest pair at an odd one (vmcnt retires in order)
+    //   YOUNG  odd: number of loads issued after those of pair q+1 that may stay in flight: D-2 pairs and the A half of the
+    //          newest pair (vmcnt retires in order)
     //   EXTRA  younger loads that are not tile loads (the epilogue's scales) and may stay in flight
     //   FIRST  slice 0 of the tile: its MFMAs start from zero, the accumulators need no clearing
-    auto slice = [&](auto ODD, auto ISSUE, auto NEXT, auto YOUNG, auto EXTRA, auto FIRST, uint32_t o_next, uint32_t o_ld0, uint32_t o_ld1)
+    auto slice = [&](auto ODD, auto ISSUE, auto NEXT, auto YOUNG, auto EXTRA, auto FIRST, uint32_t o_a, uint32_t o_b, uint32_t o_ld)
                      __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(YOUNG.value + EXTRA.value) & lgkmcnt0_mask());
-        __builtin_amdgcn_s_barrier();
+        if constexpr (ODD.value) {
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(YOUNG.value + EXTRA.value) & lgkmcnt0_mask());
+            __builtin_amdgcn_s_barrier();
+        } else {
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(63) & lgkmcnt0_mask());
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int g = 0; g < NREG; ++g) {
             if constexpr (ISSUE.value) {
-                if (g % DMA_EVERY == 0) issue_one(o_ld0, o_ld1, g / DMA_EVERY + (ODD.value ? PAIR_LOADS / 2 : 0));
+                if (g % DMA_EVERY == 0) issue_one(o_ld, g / DMA_EVERY + (ODD.value ? PAIR_LOADS / 2 : 0));
             }
-            if constexpr (NEXT.value && N16) {  // 2 * NB reads, one every READ_EVERY regions
+            if constexpr (NEXT.value) {  // 2 * NB reads, one every READ_EVERY regions
                 if (g % READ_EVERY == 0 && g / READ_EVERY < 2 * NB) {
-                    // NB = 8: blocks 0-3 of A and B, then blocks 4-7; NB = 4: blocks 0-3 of A and B
-                    const int idx = NB == 8 ? g / READ_EVERY : (g / READ_EVERY < NB ? g / READ_EVERY : 4 + g / READ_EVERY - NB);
+                    const int r = g / READ_EVERY;
+                    // NB = 8: blocks 0-3 of A and B, then blocks 4-7; else the blocks of A, then those of B
+                    const int idx = NB == 8 ? r : (r < NB ? r : 4 + r - NB);
+                    const uint32_t o = idx % 8 < 4 ? o_a : o_b;
                     if constexpr (ODD.value) {
-                        if (idx < 8) read_frag(o_next, 0, idx, fa00, fb00);
-                        else read_frag(o_next, 1, idx - 8, fa01, fb01);
+                        if (idx < 8) read_frag(No{}, o, 0, idx, fa00, fb00);
+                        else read_frag(No{}, o, 1, idx - 8, fa01, fb01);
                     } else {
-                        if (idx < 8) read_frag(o_next, 0, idx, fa10, fb10);
-                        else read_frag(o_next, 1, idx - 8, fa11, fb11);
-                    }
-                }
-            } else if constexpr (NEXT.value) {
-                // fragment fi of a step: the NB blocks of A, then the NB blocks of B (slot 4 + block in read_frag)
-                if constexpr (!FP8) {  // 2 * NB reads of step 0 in the first regions, then those of step 1
-                    if (g < 4 * NB) {
-                        const int fi = g % (2 * NB), f = fi < NB ? fi : 4 + fi - NB;
-                        if (g < 2 * NB) {
-                            if constexpr (ODD.value) read_frag(o_next, 0, f, fa00, fb00);
-                            else read_frag(o_next, 0, f, fa10, fb10);
-                        } else {
-                            if constexpr (ODD.value) read_frag(o_next, 1, f, fa01, fb01);
-                            else read_frag(o_next, 1, f, fa11, fb11);
-                        }
-                    }
-                } else {
-                    if (g < 2 * NB) {
-                        const int f = g < NB ? g : 4 + g - NB;
-                        if constexpr (ODD.value) read_frag(o_next, 0, f, fa00, fb00);
-                        else read_frag(o_next, 0, f, fa10, fb10);
+                        if (idx < 8) read_frag(Yes{}, o, 0, idx, fa10, fb10);
+                        else read_frag(Yes{}, o, 1, idx - 8, fa11, fb11);
                     }
                 }
             }
@@ -348,21 +287,13 @@ __device__ __forceinline__ void gemm_tile256s5_body(const GemmArgs& p, const int
                     asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, 0" : "=a"(acc[j][i]) : "v"(bfr), "v"(afr));
                 else
                     asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(acc[j][i]) : "v"(bfr), "v"(afr));
-            } else if constexpr (!FP8) {
-                if constexpr (ODD.value) {
-                    if (g < NB * NB) mfma_one<FP8, F8, false, NB>(acc, g, fa10, fb10);
-                    else mfma_one<FP8, F8, false, NB>(acc, g - NB * NB, fa11, fb11);
-                } else {
-                    if (g < NB * NB) mfma_one<FP8, F8, FIRST.value, NB>(acc, g, fa00, fb00);
-                    else mfma_one<FP8, F8, false, NB>(acc, g - NB * NB, fa01, fb01);
-                }
             } else {
-                if constexpr (ODD.value) mfma_one<FP8, F8, false, NB>(acc, g, fa10, fb10);
-                else mfma_one<FP8, F8, FIRST.value, NB>(acc, g, fa00, fb00);
+                if constexpr (ODD.value) mfma_one<F8, false, NB>(acc, g, fa10, fb10);
+                else mfma_one<F8, FIRST.value, NB>(acc, g, fa00, fb00);
             }
             // loop bookkeeping inside the last regions, in the issue slots an MFMA leaves free, instead of
-            // in a block of its own behind the slice: lane offsets of the operand this slice loaded, and
-            // (odd slice) the rotation of the stage offsets by one pair
+            // in a block of its own behind the slice: lane offset of the operand this slice loaded, and
+            // (odd slice) the rotation of the parts by one pair
             if constexpr (ISSUE.value) {
                 // behind the slice's last load (with a load in every region that is the last region)
                 if (g == (DMA_EVERY == 1 ? NREG - 1 : NREG - 2)) {
@@ -374,67 +305,62 @@ __device__ __forceinline__ void gemm_tile256s5_body(const GemmArgs& p, const int
                 if (g == NREG - 1) {
                     const uint32_t r0 = st[0], r1 = st[1];
 #pragma unroll
-                    for (int i = 0; i + 2 < NSTG; ++i) st[i] = st[i + 2];
-                    st[NSTG - 2] = r0;
-                    st[NSTG - 1] = r1;
+                    for (int i = 0; i + 2 < NPART; ++i) st[i] = st[i + 2];
+                    st[NPART - 2] = r0;
+                    st[NPART - 1] = r1;
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // a pair of slices (s, s+1), s even.  The stage offsets are passed by value: the odd slice rotates them in its
-    // last region.
-    auto pair = [&](auto ISSUE, auto YOUNG_E, auto YOUNG_O, auto NEXT_O, auto EXTRA, auto FIRST) __attribute__((always_inline)) {
-        slice(No{}, ISSUE, Yes{}, YOUNG_E, EXTRA, FIRST, st[1], st[NSTG - 1], st[0]);
-        slice(Yes{}, ISSUE, NEXT_O, YOUNG_O, EXTRA, No{}, st[2], st[NSTG - 1], st[0]);
+    // a pair of slices: the even one reads the odd one's fragments, the odd one those of the next pair's even slice.
+    // The offsets are passed by value: the odd slice rotates them in its last region.
+    auto pair = [&](auto ISSUE, auto YOUNG, auto NEXT, auto EXTRA, auto FIRST) __attribute__((always_inline)) {
+        slice(No{}, ISSUE, Yes{}, Int<0>{}, EXTRA, FIRST, st[0], st[1], st[NPART - 1]);
+        slice(Yes{}, ISSUE, NEXT, YOUNG, EXTRA, No{}, st[2], st[3], st[0]);
     };
     // a pair of the steady state (it starts pair q+D), and tail pair TL of the D pairs behind the last loads
-    typedef Int<(D - 1) * PAIR_LOADS> SteadyE;
-    typedef Int<(D - 2) * PAIR_LOADS + PAIR_LOADS / 2> SteadyO;
+    typedef Int<(D - 2) * PAIR_LOADS + PAIR_LOADS / 2> Steady;
     auto tail_pair = [&](auto TL) __attribute__((always_inline)) {
         constexpr int t = decltype(TL)::value;
-        pair(No{}, Int<(D - 1 - t) * PAIR_LOADS>{}, Int<(D - 2 - t > 0 ? D - 2 - t : 0) * PAIR_LOADS>{}, Int<(t < D - 1)>{}, Int<3>{}, No{});
+        pair(No{}, Int<(D - 2 - t > 0 ? D - 2 - t : 0) * PAIR_LOADS>{}, Int<(t < D - 1)>{}, Int<3>{}, No{});
     };
 
     // ---- prologue: pairs 0 .. D-1 in flight, pair 0 landed, fragments of slice 0 in set 0
+    auto issue_pair = [&](int d) __attribute__((always_inline)) {
 #pragma unroll
-    for (int g = 0; g < PAIR_LOADS; ++g) issue_one(0, STAGE, g);
-    advance();
+        for (int g = 0; g < PAIR_LOADS; ++g) issue_one((2 * d + g / (PAIR_LOADS / 2)) * PART, g);
+        advance();
+    };
+    issue_pair(0);
     if constexpr (D == 2) {
-        if (S >= 4) {
-#pragma unroll
-            for (int g = 0; g < PAIR_LOADS; ++g) issue_one(2 * STAGE, 3 * STAGE, g);
-            advance();
+        if (Q >= 2) {
+            issue_pair(1);
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(PAIR_LOADS));
         } else {
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         }
     } else {  // the launcher sends only K of at least 2 D pairs here
 #pragma unroll
-        for (int d = 1; d < D; ++d) {
-#pragma unroll
-            for (int g = 0; g < PAIR_LOADS; ++g) issue_one(2 * d * STAGE, (2 * d + 1) * STAGE, g);
-            advance();
-        }
+        for (int d = 1; d < D; ++d) issue_pair(d);
         __builtin_amdgcn_s_waitcnt(vmcnt_imm((D - 1) * PAIR_LOADS));
     }
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int f = 0; f < 8; ++f) {
-        read_frag(0, 0, f, fa00, fb00);
-        if constexpr (!FP8 && !(N16 && NB == 4)) read_frag(0, 1, f, fa01, fb01);  // 16x16 form: blocks 4-7 exist for NB = 8
+        read_frag(No{}, f < 4 ? 0 : PART, 0, f, fa00, fb00);
+        if constexpr (N16 && NB == 8) read_frag(No{}, f < 4 ? 0 : PART, 1, f, fa01, fb01);
     }
 
-    const int Q = S >> 1;  // pairs
     if (D > 2 || Q >= 3) {
-        pair(Yes{}, SteadyE{}, SteadyO{}, Yes{}, Int<0>{}, Yes{});
+        pair(Yes{}, Steady{}, Yes{}, Int<0>{}, Yes{});
     } else {  // short K: no pair to peel, clear the accumulators instead
 #pragma unroll
         for (int j = 0; j < NB; ++j)
 #pragma unroll
             for (int i = 0; i < NB; ++i) acc[j][i] = typename TileAcc<FP8, N16>::type{};
     }
-    for (int q = 1; q + D < Q; ++q) pair(Yes{}, SteadyE{}, SteadyO{}, Yes{}, Int<0>{}, No{});
+    for (int q = 1; q + D < Q; ++q) pair(Yes{}, Steady{}, Yes{}, Int<0>{}, No{});
 
     // The epilogue's scales and bias are requested here, behind the last tile loads, so that their
     // latency is covered by the remaining two pairs of slices.  Always three loads (a missing bias
@@ -561,7 +487,7 @@ __device__ __forceinline__ void gemm_tile256s5_body(const GemmArgs& p, const int
         tile_epilogue16<DUMP, NB, NB, false, OUTK>(p, acc, smem, m0, n0, t, wm, wn, lr, lane >> 4, pre_sx, pre_sw,
                                                   !p.bias ? -0.0f : OUTK == DAXQ_F32 ? __uint_as_float(pre_b) : OUTK == DAXQ_F16 ? f16_bits_to_f32((uint16_t)pre_b) : bf16_bits_to_f32(pre_b));
     else
-        tile256_epilogue<FP8, DUMP, NB>(p, acc, smem, m0, n0, t, wm, wn, l31, hi, pre_sx, pre_sw,
+        tile256_epilogue<NB>(p, acc, smem, m0, n0, t, wm, wn, l31, hi, pre_sx, pre_sw,
                                         p.bias ? bf16_bits_to_f32(pre_b) : -0.0f);
 }
 
@@ -591,14 +517,14 @@ template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, bool SPLI
 static int prepare_tile256s5() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
     return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256s5_kernel<FP8, DUMP, F8, N16, BT, SPLITK, D, OUTK>),
-                              (2 * D + 1) * 2 * BT * t5::BKS, lds_set);
+                              (2 * D + 1) * BT * t5::BKP, lds_set);
 }
 
 // split-K launch on 128 tiles: a.splits ranges of K, a.counters zero, a.partials large enough (checked by the caller)
 template <bool FP8, int F8>
 static int launch_splitk_impl(const GemmArgs& a, hipStream_t st) {
     using namespace t5;
-    constexpr int SMEM = NST * 2 * 128 * BKS;
+    constexpr int SMEM = 5 * 128 * BKP;
     auto kern = gemm_tile256s5_kernel<FP8, false, F8, !FP8, 128, true>;
     if (int rc = prepare_tile256s5<FP8, false, F8, !FP8, 128, true>()) return rc;
     const int64_t nt = (int64_t)a.tiles_m * a.tiles_n * a.splits;
@@ -630,7 +556,7 @@ template int launch_tile128_splitk<true>(const GemmArgs&, int, hipStream_t);
 template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, int D = 2, int OUTK = DAXQ_BF16>
 static int launch_tile256s5_impl(const GemmArgs& a, hipStream_t st) {
     using namespace t5;
-    constexpr int SMEM = (2 * D + 1) * 2 * BT * BKS;  // 160 KB (256 tile), 80 KB (128 tile), 144 KB (128 tile, nine stages)
+    constexpr int SMEM = (2 * D + 1) * BT * BKP;  // 160 KB (256 tile), 80 KB (128 tile), 144 KB (128 tile, nine stages)
     if (a.out_kind != OUTK) return fail(DAXQ_ERR_ARG, "gemm: this kernel writes output type %d, not %d", OUTK, a.out_kind);
     auto kern = gemm_tile256s5_kernel<FP8, DUMP, F8, N16, BT, false, D, OUTK>;
     if (int rc = prepare_tile256s5<FP8, DUMP, F8, N16, BT, false, D, OUTK>()) return rc;
@@ -677,13 +603,13 @@ static int launch_i8_one(const GemmArgs& a, bool small, hipStream_t st) {
 template <bool DUMP, int OUTK>
 static int prepare_then_halves() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256_then_halves_kernel<DUMP, OUTK>), 5 * 2 * 256 * t5::BKS, lds_set);
+    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256_then_halves_kernel<DUMP, OUTK>), 5 * 256 * t5::BKP, lds_set);
 }
 
 template <bool DUMP, int OUTK>
 static int launch_then_halves_impl(const GemmArgs& a, int64_t nt, hipStream_t st) {
     if (int rc = prepare_then_halves<DUMP, OUTK>()) return rc;
-    hipLaunchKernelGGL((gemm_tile256_then_halves_kernel<DUMP, OUTK>), dim3((unsigned)nt), dim3(t5::T), 5 * 2 * 256 * t5::BKS, st, a);
+    hipLaunchKernelGGL((gemm_tile256_then_halves_kernel<DUMP, OUTK>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
     return check_launch("gemm_tile256_then_halves");
 }
 
@@ -703,13 +629,13 @@ static int launch_then_halves(const GemmArgs& a0, int whole, int halves, hipStre
 template <bool DUMP, int OUTK, int D>
 static int prepare_then_quadrants() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D>), 5 * 2 * 256 * t5::BKS, lds_set);
+    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D>), 5 * 256 * t5::BKP, lds_set);
 }
 
 template <bool DUMP, int OUTK, int D>
 static int launch_then_quadrants_impl(const GemmArgs& a, int64_t nt, hipStream_t st) {
     if (int rc = prepare_then_quadrants<DUMP, OUTK, D>()) return rc;
-    hipLaunchKernelGGL((gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D>), dim3((unsigned)nt), dim3(t5::T), 5 * 2 * 256 * t5::BKS, st, a);
+    hipLaunchKernelGGL((gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
     return check_launch("gemm_tile256_then_quadrants");
 }
 

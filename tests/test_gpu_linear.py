@@ -386,6 +386,27 @@ def test_fp8_16x16x128_form_every_count_of_slice_pairs(ops, k, variant):
     assert torch.equal(acc, acc2) and torch.equal(out, out2), "every tile size must give the same FP8 bits"
 
 
+@pytest.mark.parametrize("variant", [8, 11, 14])
+@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 768, 896, 1152])
+def test_int8_every_count_of_slice_pairs(ops, k, variant):
+    """Every number of 128-byte pairs of K slices that takes another path through the INT8 pipeline (one and two pairs, the
+    peeled first one, steady ones) on the three tile sizes: accumulators and outputs against the integer oracle, ragged edges."""
+    from dax_amd import _capi
+
+    m, n = 300, 700
+    g = torch.Generator("cpu").manual_seed(k)
+    xq = torch.randint(-128, 128, (m, k), generator=g, dtype=torch.int32).to(torch.int8)
+    wq = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int32).to(torch.int8)
+    sx, sw = torch.rand(m, generator=g) * 0.02 + 1e-3, torch.rand(n, generator=g) * 0.002 + 1e-4
+    b = torch.randn(n, generator=g).bfloat16()
+    want = O.int_mm(xq, wq)
+    _capi.debug_select_gemm(variant)
+    out, acc = ops.linear_i8_acc(dev(xq), dev(sx), dev(wq), dev(sw), dev(b))
+    assert torch.equal(acc.cpu(), want)
+    np.testing.assert_array_equal(bf16_bits(out), bf16_bits(O.epilogue_int8(want, sx.view(-1, 1), sw.view(1, -1), b)))
+    np.testing.assert_array_equal(bf16_bits(ops.linear_i8(dev(xq), dev(sx), dev(wq), dev(sw), dev(b))), bf16_bits(out))
+
+
 @pytest.mark.parametrize("k", [3968, 4096, 4224, 4352, 4480, 5120, 13824])
 def test_nine_stage_128_tile_form_every_count_of_slice_pairs(ops, k):
     """Launches of at most 256 tiles of 128x128 with K >= 4096 run the five-stage pipeline with nine stages (four pairs
