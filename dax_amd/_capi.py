@@ -57,6 +57,8 @@ SIGNATURES = {
     "daxq_linear_e5m2_e4m3": [_P, _I64, _P, _P, _I64, _P, _P, _P, _I64, _P, _I64, _I64, _I64, _I64, _P],
     "daxq_linear_splitk_choice": [_I64, _I64, _I64],
     "daxq_linear_rows": [_INT, _I64, _I64, _I64, _INT],
+    "daxq_linear_launch_rows": [_INT, _I64, _I64, _I64],
+    "daxq_linear_launch_splits": [_I64, _I64, _I64],
     "daxq_linear_tile_order_choice": [_I64, _I64, _I64],
     "daxq_linear_splitk_workspace_bytes": [_I64, _I64, _INT],
     "daxq_linear_w8a8_splitk": [_INT, _INT, _P, _I64, _P, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _INT, _P, _I64, _P],
@@ -88,7 +90,7 @@ def lib() -> C.CDLL:
                     fn = getattr(L, name)
                     fn.argtypes = args
                     fn.restype = (C.c_char_p if name == "daxq_last_error" else
-                                  _I64 if name in ("daxq_linear_splitk_workspace_bytes", "daxq_linear_rows") else _INT)
+                                  _I64 if name in ("daxq_linear_splitk_workspace_bytes", "daxq_linear_rows", "daxq_linear_launch_rows") else _INT)
                 got = L.daxq_abi_version()
                 if got != ABI_VERSION:
                     raise RuntimeError(f"libdaxq ABI {got} != expected {ABI_VERSION}; rebuild the library")

@@ -337,23 +337,33 @@ int prepare_rows_kernels() {
     return rc;
 }
 
-// Launches this kernel is the library's choice for.  At most 128 rows: see above.  More rows, where 128x128 tiles are few or
-// do not exist: such a tile takes 0.16 to 0.2 us per 64 bytes of K on its CU (its LDS traffic, 48 KB) while the CUs without
-// a tile idle, here every 16 x 16 outputs or a few of them are a wavefront.  A tile in five CUs is where the two meet
-// (2048 blocks of 16 x 16; e4m3 217 x 2391, K = 1408, 2100 blocks: 7.2 against 8.8 us, 418 x 1558, K = 3840, 2646: 13.8 / 14.9,
-// 784 x 1360, K = 384, 4165: 5.2 / 5.7, 291 x 3671, K = 2176, 4370: 14.7 / 11.3); INT8 launches of long K have split-K
-// beside them (450 x 1137, K = 12800: 32 against 27 us).  Fewer than 128 columns leave only the generic kernel (INT8, 9191 x 79, K = 512:
-// 15.4 -> 6.9 us, 2404 x 74, K = 3072: 25.6 -> 8.2), which is as fast from about 4000 blocks at K = 4096 on.
+// Launches this kernel is the library's choice for: those of so few outputs that it has more wavefronts to put on them than fitted
+// tiles have workgroups (gemm_tile_fit.hip), and all of fewer rows than such a tile has.  `blocks` of 16 x 16 outputs; us, here /
+// 64 x 64 tiles (64 x 96 where marked):
+//   INT8  66 x 976, K = 3072 (305) 5.0 / 5.9            179 x 448, K = 7168 (336) 6.8 / 12.0          87 x 1224, K = 4608 (462) 6.7 / 8.1
+//         235 x 512, K = 5120 (480) 5.6 / 9.8           99 x 1536, K = 13824 (672) 13.6 / 19.9        106 x 1536, K = 8960 (672) 10.0 / 14.0
+//         717 x 296, K = 6272 (855) 12.1 / 10.7         71 x 2928, K = 9856 (915) 17.3 / 15.3         164 x 1536, K = 4608 (1056) 9.6 / 8.7
+//         219 x 1536, K = 4096 (1344) 12.6 / 8.1        71 x 4608, K = 7296 (1440) 19.1 / 12.7        111 x 4608 x 4608 (2016) 14.3 / 9.1
+//   e4m3  102 x 952, K = 8064 (420) 9.4 / 12.7          107 x 1080, K = 6656 (476) 8.2 / 11.0         66 x 1760, K = 4352 (550) 7.4 / 8.2
+//         79 x 1840, K = 13824 (575) 21.9 / 19.7        95 x 1712, K = 6784 (642) 13.2 / 11.1         101 x 4608, K = 1536 (2016) 6.6 / 5.3 *
+//         289 x 760, K = 6016 (912) 9.3 / 10.3          224 x 1048, K = 8960 (924) 12.7 / 14.1        158 x 1920, K = 10112 (1200) 14.4 / 15.4
+//         198 x 1264, K = 15360 (1027) 27.7 / 22.2      247 x 1536, K = 5120 (1536) 11.5 / 9.7        574 x 1536, K = 3968 (3456) 14.8 / 8.7
+// (more than 128 rows against 64 to 128 of them: FP8 runs its wider forms there).  INT8 launches of long K stop at 131072 block-steps
+// of 128 K bytes.  Fewer than 64 columns leave only the generic kernel (INT8, 9191 x 79, K = 512: 15.4 -> 6.9 us, 2404 x 74, K = 3072:
+// 25.6 -> 8.2), which is as fast from about 4000 blocks at K = 4096 on.
 // FP8 with fewer than 128 columns keeps the generic kernel at any number of rows: it adds in another order, and beyond a few
 // thousand blocks this kernel is too slow to be the only one (e4m3 75600 x 64, K = 5120: 212 against 125 us), so a
 // line between the two would change a row's bits with the rows around it.
-bool rows_applies(int64_t m, int64_t n, int64_t k, bool fp8) {
+// acc: the launch asks for its accumulators, which the fitted tiles do not write (beside 128x128 tiles the line lies at 2048 blocks).
+bool rows_applies(int64_t m, int64_t n, int64_t k, bool fp8, bool acc) {
     if (fp8 && n < 128) return false;
-    if (m <= 128) return m <= (n > 8192 ? 32 : 128);
+    if (m < 64) return m <= (n > 8192 ? 32 : 63);
     if (m > (1 << 20) || n > (1 << 20)) return false;
     const int64_t blocks = row_blocks(m, n), work = blocks * (k / 128);
+    if (m <= 128 && (n < 128 || (acc && n <= 8192))) return true;
     if (n < 128) return work <= 65536;
-    return blocks <= 2048 && (fp8 || work <= 131072);
+    if (m <= 128) return blocks <= (fp8 ? 600 : 768);
+    return blocks <= (acc ? 2048 : fp8 ? 1280 : 768) && (fp8 || work <= 131072);
 }
 
 // 32-bit row offsets

@@ -27,9 +27,13 @@ struct Int {
     static constexpr int value = N;
 };
 
-// sched_group_barrier masks
-#define DAXQ_SG_MFMA 0x008
-#define DAXQ_SG_DS_RD 0x100
+template <int I, int N, typename F>
+__device__ __forceinline__ void for_up(F&& f) {
+    if constexpr (I < N) {
+        f(Int<I>{});
+        for_up<I + 1, N>(f);
+    }
+}
 
 // GemmArgs::order
 constexpr int kOrderRowGroups = 0, kOrderBanded = 1;
@@ -78,28 +82,37 @@ struct Acc16<true> {
     typedef v4f type;
 };
 
+// Behind the last MFMA of a path.  The MFMAs are inline asm, so the compiler cannot count the wait states between one of them and
+// another instruction that reads its result: idle cycles first.  It stands in front of a join of control flow, not behind it: where
+// two paths hold an accumulator in different registers, the compiler copies it at the end of a path, and a copy in front of the idle
+// cycles reads a result that is not there yet (found in a kernel with the accumulator dump: the halves' sums were off by 3 %).
+__device__ __forceinline__ void mfma_settle() {
+    asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 7");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 // The epilogue of a wavefront's accumulators held as NBJ x NBI blocks of 16x16 (v_mfma_i32_16x16x64_i8,
 // v_mfma_f32_16x16x128_f8f6f4): acc[j][i] is weight block j (16 output columns) and activation block i (16 output rows)
-// of the wavefront's part of a tile of 32 NBI rows x 32 NBJ columns (four wavefronts, 2 x 2).
+// of the wavefront's part of a tile of WM x WN wavefronts.
 // In a block a lane owns output row m = l%16 and the columns n = 4*(l/16) + {0..3}.  One
 // v_permlane16_swap per word over two neighbouring blocks gives each lane 8 consecutive columns of one
 // of them: lanes 0-15 block 2jp columns 0-7, lanes 16-31 block 2jp+1 columns 0-7, lanes 32-47 block
 // 2jp columns 8-15, lanes 48-63 block 2jp+1 columns 8-15.
-// NBJ, NBI: 8, 8 for a 256x256 tile, 4, 4 for a 128x128 tile, 4, 8 for a half tile of 256 rows x 128 columns.
+// (an odd NBJ leaves a block without a partner: its lanes store their own four columns).
 // OUTK: element type of out and bias, DAXQ_BF16 / DAXQ_F16 / DAXQ_F32.  A template argument, i.e. a kernel
 // of its own per type: with all three forms inside one kernel behind uniform branches its code grew from 27 to 44 KB
 // and the bf16 launches at K = 1536, which change between main loop and epilogue every 24 slices, lost 2.7 %; with
 // the choice inside the loops they lost 2 to 11 % everywhere.
-template <bool DUMP, int NBJ, int NBI, bool FP8 = false, int OUTK = DAXQ_BF16>
+template <bool DUMP, int NBJ, int NBI, bool FP8 = false, int OUTK = DAXQ_BF16, int WM = 2, int WN = 2>
 __device__ __forceinline__ void tile_epilogue16(const GemmArgs& p, typename Acc16<FP8>::type (&acc)[NBJ][NBI], uint8_t* smem, int m0, int n0, int t,
                                                 int wm, int wn, int l15, int g4, float pre_sx, float pre_sw,
                                                 float pre_bias) {
-    constexpr int BM = 32 * NBI, BN = 32 * NBJ, WTM = 16 * NBI, WTN = 16 * NBJ;
+    constexpr int WTM = 16 * NBI, WTN = 16 * NBJ, BM = WM * WTM, BN = WN * WTN, T = 64 * WM * WN;
     float* s_sx = reinterpret_cast<float*>(smem);
     float* s_sw = s_sx + BM;
     float* s_bias = s_sw + BN;
-    if (BM == 256 || t < BM) s_sx[t] = pre_sx;
-    if (BN == 256 || t < BN) {
+    if (BM == T || t < BM) s_sx[t] = pre_sx;
+    if (BN == T || t < BN) {
         s_sw[t] = pre_sw;
         s_bias[t] = pre_bias;
     }
@@ -163,13 +176,14 @@ __device__ __forceinline__ void tile_epilogue16(const GemmArgs& p, typename Acc1
     for (int i = 0; i < NBI; ++i) {
         const int ml = wm * WTM + i * 16 + l15;
         const float sxv = sxr[i];
-        uint16_t* orow = p.out + (int64_t)(m0 + ml) * p.ldo + n0 + wn * WTN + (g4 & 1) * 16 + (g4 >> 1) * 8;
+        uint16_t* orow = p.out + (int64_t)(m0 + ml) * p.ldo + n0 + wn * WTN;
 #pragma unroll
-        for (int jp = 0; jp < NBJ / 2; ++jp) {
+        for (int jp = 0; jp < (NBJ + 1) / 2; ++jp) {
             uint32_t pk[2][2];
 #pragma unroll
             for (int jj = 0; jj < 2; ++jj) {
                 const int j = 2 * jp + jj;
+                if (j >= NBJ) continue;
                 const float sws[4] = {swr[j].x, swr[j].y, swr[j].z, swr[j].w};
                 const float bs[4] = {br[j].x, br[j].y, br[j].z, br[j].w};
 #pragma unroll
@@ -206,9 +220,13 @@ __device__ __forceinline__ void tile_epilogue16(const GemmArgs& p, typename Acc1
                     }
                 }
             }
+            if (2 * jp + 1 == NBJ) {
+                *reinterpret_cast<uint2*>(orow + jp * 32 + 4 * g4) = make_uint2(pk[0][0], pk[0][1]);
+                continue;
+            }
             v2u s0 = __builtin_amdgcn_permlane16_swap(pk[0][0], pk[1][0], false, false);
             v2u s1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
-            *reinterpret_cast<uint4*>(orow + jp * 32) = make_uint4(s0.x, s1.x, s0.y, s1.y);
+            *reinterpret_cast<uint4*>(orow + jp * 32 + (g4 & 1) * 16 + (g4 >> 1) * 8) = make_uint4(s0.x, s1.x, s0.y, s1.y);
         }
     }
     }

@@ -16,7 +16,7 @@
 // rows are computed twice with identical results.  Shapes with M < 128 or N < 128 take the kernel in
 // gemm_rows.hip or the generic one in gemm_w8a8.hip.
 #include "gemm_tile.h"
-#include "gemm_tile256x128.h"
+#include "gemm_tile_fit.h"
 
 namespace daxq {
 
@@ -385,11 +385,9 @@ __device__ __forceinline__ void gemm_tile256s5_body(const GemmArgs& p, const int
     }
 
     if constexpr (N16) {
-        // The 16x16 MFMAs are inline asm, so the compiler cannot count the wait states between one of them and a
-        // VALU read of its result, and it places such reads right behind the MFMA if nothing stops it.  Volatile
-        // asm statements keep their order: 24 idle cycles first, then every accumulator is passed through an empty
-        // statement, which no read of it can move above.
-        asm volatile("s_nop 15\n\ts_nop 7");
+        // (the compiler places reads of an accumulator right behind its last MFMA if nothing stops it; volatile asm statements keep
+        // their order: every accumulator is passed through an empty statement, which no read of it can move above)
+        mfma_settle();
 #pragma unroll
         for (int j = 0; j < NB; j += 2) {
             if constexpr (NB == 8) {
@@ -502,7 +500,7 @@ __global__ __launch_bounds__(256) void gemm_tile256s5_kernel(const GemmArgs p) {
 template <bool DUMP, int OUTK>
 __global__ __launch_bounds__(256) void gemm_tile256_then_halves_kernel(const GemmArgs p) {
     if ((int)blockIdx.x < p.grid) gemm_tile256s5_body<false, DUMP, 0, true, 256, false, 2, OUTK>(p, (int)blockIdx.x);
-    else gemm_tile256x128_body<DUMP, OUTK>(p, (int)blockIdx.x - p.grid);
+    else gemm_half_body<false, 0, DUMP, OUTK>(p, (int)blockIdx.x - p.grid);
 }
 
 // The same for left-over tiles that run as 128x128 quadrants (tail_tiles): workgroups 0 .. p.grid - 1 compute whole

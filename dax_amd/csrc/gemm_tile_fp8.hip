@@ -34,7 +34,7 @@
 // the MFMA needs: the order of K inside an instruction is free as long as both operands agree.
 // K shorter than four pairs (K < 512) takes a plain loop of the same MFMAs: load a pair, wait, multiply.
 #include "gemm_tile.h"
-#include "gemm_tile256x128.h"
+#include "gemm_tile_fit.h"
 
 namespace daxq {
 
@@ -302,6 +302,7 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
 
         pair(Yes{}, No{}, No{}, Yes{}, Int<3>{}, No{});  // pair Q-2 (odd)
         pair(No{}, No{}, No{}, No{}, Int<3>{}, No{});    // pair Q-1 (even)
+        mfma_settle();
     } else {
         // ---- short K (one to three pairs): load a pair, wait for it, multiply.  The same MFMAs on the same fragments
         // as above, so the sums are the same bits as the pipelined path would give.
@@ -332,13 +333,11 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        mfma_settle();
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     }
 
-    // The MFMAs are inline asm, so the compiler cannot count the wait states between one of them and a VALU read of
-    // its result: idle cycles first, then every accumulator is passed through an empty statement, which no read of
-    // it can move above.
-    asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 7");
+    // ... and every accumulator is passed through an empty statement, which no read of it can move above
 #pragma unroll
     for (int j = 0; j < NB; j += 2) {
         if constexpr (NB == 8) {
@@ -367,7 +366,7 @@ __global__ __launch_bounds__(256) void gemm_tile_fp8_kernel(const GemmArgs p) {
 template <bool DUMP, int F8, int OUTK>
 __global__ __launch_bounds__(256) void gemm_tile_fp8_then_halves_kernel(const GemmArgs p) {
     if ((int)blockIdx.x < p.grid) gemm_tile_fp8_body<DUMP, F8, 256, OUTK>(p, (int)blockIdx.x);
-    else gemm_tile256x128_fp8_body<DUMP, F8, OUTK>(p, (int)blockIdx.x - p.grid);
+    else gemm_half_body<true, F8, DUMP, OUTK>(p, (int)blockIdx.x - p.grid);
 }
 
 // The same for left-over tiles that run as 128x128 quadrants (tail_tiles): workgroups 0 .. p.grid - 1 compute whole

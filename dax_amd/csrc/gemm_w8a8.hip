@@ -246,7 +246,10 @@ int launch_tile_fp8(const GemmArgs& a, int f8, bool small, int tail, hipStream_t
 int launch_halves_i8(const GemmArgs& a, hipStream_t st);                                // gemm_tile256.hip
 int launch_halves_fp8(const GemmArgs& a, int f8, hipStream_t st);                       // gemm_tile_fp8.hip
 int launch_rows(const GemmArgs& a, bool fp8, int f8, hipStream_t st);                    // gemm_rows.hip
-bool rows_applies(int64_t m, int64_t n, int64_t k, bool fp8);
+int launch_fit_i8(const GemmArgs& a, int tile, hipStream_t st);                          // gemm_tile_fit.hip
+int launch_fit_fp8(const GemmArgs& a, int tile, int f8, hipStream_t st);                 // gemm_tile_fit.hip
+int fit_choice(int64_t m, int64_t n, int64_t k, bool fp8);                               // gemm_tile_fit.hip
+bool rows_applies(int64_t m, int64_t n, int64_t k, bool fp8, bool acc = false);
 template <bool FP8>
 int launch_tile128_splitk(const GemmArgs& a, int f8, hipStream_t st);
 
@@ -262,6 +265,15 @@ static int launch_halves(const GemmArgs& a, int f8, hipStream_t st) {
     else return launch_halves_i8(a, st);
 }
 
+template <bool FP8>
+static int launch_fitted(const GemmArgs& a, int f8, int tile, hipStream_t st) {
+    if (a.lda >= (1 << 26) || a.ldb >= (1 << 26)) return fail(DAXQ_ERR_ARG, "linear: the fitted tiles take row strides below 2^26");
+    if constexpr (FP8) return launch_fit_fp8(a, tile, f8, st);
+    else return launch_fit_i8(a, tile, st);
+}
+
+int prepare_fit_i8_kernels();
+int prepare_fit_fp8_kernels();
 int prepare_tile_fp8_kernels();
 int prepare_rows_kernels();
 int prepare_tile256_kernels();
@@ -304,7 +316,7 @@ static int launch_generic(const GemmArgs& a, int f8, hipStream_t st) {
 
 // Kernel choices of the `kernel` argument (daxq_linear_w8a8): low 16 bits pick the implementation, bits 16-23 the
 // depth of the tile-order groups (0 = 4 tile rows).
-enum { K_DEFAULT = 0, K_GENERIC256 = 2, K_GENERIC128 = 5, K_TILED_256 = 8, K_TILED_128 = 11, K_TILED_HALVES = 14, K_ROWS = 17 };
+enum { K_DEFAULT = 0, K_GENERIC256 = 2, K_GENERIC128 = 5, K_TILED_256 = 8, K_TILED_128 = 11, K_TILED_HALVES = 14, K_ROWS = 17, K_FIT = 32 };
 
 // Tile order a launch of 256x256 tiles takes when the caller names none.  The banded order (tile_order.h: patches of
 // 8 x 4 tiles per XCD, the eight XCDs of a round on the same activation rows and on different weight bands) reads the
@@ -378,31 +390,23 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
         return fail(DAXQ_ERR_ARG, "linear: the tiled kernels dump their accumulators with bf16 outputs only");
     switch (which) {
         case K_DEFAULT: {
-            // (with the accumulator dump, too: the outputs beside it are the same bits as without)
-            // Fewer than 128 rows and no smaller tile: the kernel for few rows whatever the columns, so that an FP8 row's bits are
+            // One round of workgroups or less: tiles fitted to the launch (gemm_tile_fit.hip; not with the accumulator dump, whose
+            // outputs are the same bits either way), but for the few outputs that the kernel for few rows is faster at.
+            const bool rows = rows_applies(m, n, k, FP8, acc != nullptr);
+            if (!rows && !acc && fits32) {
+                const int tile = fit_choice(m, n, k, FP8);
+                if (tile >= 0) return launch_fitted<FP8>(a, f8, tile, st);
+            }
+            // Fewer than 128 rows and no tile that small: the kernel for few rows whatever the columns, so that an FP8 row's bits are
             // those of the tiled kernels at any number of rows.  Beside the generic kernel, us (INT8 / e4m3): 33 x 13824, K = 5120
-            // 32.9 -> 23.0 / 32.5 -> 22.7, 127 rows 42.0 -> 40.6 / 41.7 -> 47.5, 127 x 8960, K = 13824 106 -> 83 / 106 -> 87; 128 rows of
-            // the caller's buffers in the tiled kernels, where they reach that far, take 24.6 / 22.9 and 75 / 74 (daxq_linear_rows).
-            if ((rows_applies(m, n, k, FP8) || (m < 128 && n >= 128)) && fits32) return launch_rows(a, FP8, f8, st);
+            // 32.9 -> 23.0 / 32.5 -> 22.7.
+            if ((rows || (m < 128 && n >= 128)) && fits32) return launch_rows(a, FP8, f8, st);
             // fp16 / fp32 outputs together with the accumulator dump (tests): the generic kernel
             if (acc && out_kind != DAXQ_BF16)
                 return (m >= 256 && n >= 256) ? launch_generic<FP8, 256>(a, f8, st) : launch_generic<FP8, 128>(a, f8, st);
-            // library default: the kernel for few rows (above); the tiled kernel on 256x256 tiles once there is one for every
-            // second CU, on 128x128 tiles (4x as many workgroups, two per CU) below that, and the generic kernel for fewer
-            // columns than one such tile has.  Measured at N = K = 5120 (INT8, T-op/s, 128 / 256 tiles):
-            // M = 512 -> 1127 / 551, M = 1024 (80 large tiles) -> 1275 / 1055, M = 2048 (160) -> 1542 / 1817;
-            // 4096 x 1536 x 1536 (96) -> 1182 / 895, 8192 x 1536 x 1536 (192) -> 1517 / 1587.
-            // Between a quarter and a half of the CUs' worth of large tiles, every tile runs as its two 256x128 halves with
-            // a CU each (K >= 2048), unless the 128x128 tiles get a CU each as well.  Measured against what these launches took
-            // before (128x128 tiles up to 127 large
-            // tiles, whole 256x256 tiles at 128), INT8 / e4m3, us: 1024 x 5120 x 5120 (80 tiles) 38.7 -> 31.0 / 37.7 -> 29.6,
-            // 1536 x 5120 x 5120 (120) 41.1 -> 35.0 / 40.3 -> 35.3, 1100 x 4352 x 5120 (85) 42.4 -> 31.6 / 41.1 -> 31.1,
-            // 2048 x 4096 x 4096 (128) 39.6 -> 30.7 / 38.7 -> 31.2, 1024 x 5120, K = 13824 95.9 -> 69.3 / 93.1 -> 66.8,
-            // 4096 x 1536, K = 8960 62.3 -> 50.7 / 60.5 -> 50.3; with 60 tiles (768 x 5120 x 5120) the quadrants' 23.8 us
-            // become 30.5, and ragged ones (3312 x 1070, K = 7424: 65 large tiles or 234 small ones) lose as much: 28.2 / 39.6;
-            // 5588 x 584, K = 6272 (66 / 220) 23.8 / 35.3.  Below K = 2048 a repeated launch gains 5 to 10 % (4096 x 1536 x 1536
-            // 16.7 -> 15.4), but behind its quantiser and on other operands each time, as in a model, it loses 10 (23.2 -> 26.0
-            // for the pair).
+            // More than one round: 256x256 tiles once there is one for every second CU and the 128x128 tiles need a second round at
+            // two per CU, those below that, and the generic kernel for fewer columns than one such tile has.  Measured at N = K = 5120
+            // (INT8, T-op/s, 128 / 256 tiles): M = 2048 (160 large tiles) -> 1542 / 1817; 8192 x 1536 x 1536 (192) -> 1517 / 1587.
             // A launch whose 128x128 tiles all fit at two per CU takes them although its large tiles number 128 and more
             // (ragged edges: 2358 x 3239 is 130 large tiles or 494 small ones).  256x256 -> 128x128 tiles, INT8 / e4m3: that shape
             // at K = 256 16.9 -> 11.3 / 17.6 -> 11.4, K = 1536 26.4 -> 20.5 / 26.4 -> 19.4 (behind its quantiser 34.0 -> 27.1),
@@ -412,7 +416,6 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
             const int64_t tiles256 = ((m + 255) / 256) * ((n + 255) / 256);
             const int cus = cu_count();
             const int64_t tiles128 = ((m + 127) / 128) * ((n + 127) / 128);
-            if (tile256_applies(a) && k >= 2048 && cus >= 8 && 4 * tiles256 > cus && 2 * tiles256 <= cus && tiles128 > cus) return launch_halves<FP8>(a, f8, st);
             if (tile256_applies(a) && tiles256 >= 128 && tiles128 > 2 * cus) return launch_tiled<FP8>(a, f8, false, tail, st);
             if (m >= 128 && n >= 128 && fits32) return launch_tiled<FP8>(a, f8, true, 1, st);
             return launch_generic<FP8, 128>(a, f8, st);
@@ -431,7 +434,9 @@ static int launch_gemm(const void* xq, int64_t ld_xq, const float* sx, const voi
         case K_ROWS:
             if (m > 128 || acc) return fail(DAXQ_ERR_ARG, "linear: the kernel for few rows takes at most 128, and no accumulator dump, by name");
             return launch_rows(a, FP8, f8, st);
-        default: return fail(DAXQ_ERR_ARG, "linear: unknown kernel choice %d", which);
+        default:
+            if (which >= K_FIT && !acc) return launch_fitted<FP8>(a, f8, which - K_FIT, st);
+            return fail(DAXQ_ERR_ARG, "linear: unknown kernel choice %d", which);
     }
 }
 
@@ -449,14 +454,16 @@ constexpr int64_t kMaxSplitTiles = kCounterBytes / 4;
 // least 1024 bytes of K deep and divide K / 128 evenly; 1 = no split.  Measured at N = K = 5120 (INT8, us, plain launch /
 // 2 / 4 ranges): M = 256 (80 tiles) 34 / 28 / 40, M = 512 (160 tiles) 24 / 35 / 52, M = 1024 52 / 71 / -: the partial
 // results make a round trip through device-coherent memory (about 10 us for 20 MB), which only idle CUs pay for.
-// Launches that the kernel for few rows is taken for leave their ranges alone, but not 65 to 128 rows against a large weight,
+// (That was beside 128x128 tiles; a linear's forward takes a fitted tile first, launch_splits.)
+// Launches of few rows or outputs leave their ranges alone, but not 65 to 128 rows against a large weight,
 // where the K ranges are as fast or faster from about 45 M weight bytes on (128 rows; that kernel / K ranges, us, weights out
 // of reach of the caches): N = 5120, K = 8960 30.2 / 27.9; 8192 x 5120 25.1 / 24.4; 6144 x 8960 34.2 / 28.6; 4096 x 13824
 // 34.5 / 31.1; 5120 x 13824 47.3 / 34.2; 8192 x 13824 68.5 / 40.3 (72 rows: 25.7, 22.4, 30.9, 30.1, 38.9, 59.6).
 constexpr int64_t kRowsBelowSplit = 45000000;
 static int splitk_choice(int64_t m, int64_t n, int64_t k) {
     if (m < 128 || n < 128 || k % DAXQ_K_ALIGN) return 1;
-    if (rows_applies(m, n, k, false) && (m > 128 || n * k <= kRowsBelowSplit)) return 1;
+    const int64_t blocks = ((m + 15) / 16) * ((n + 15) / 16);
+    if (m <= 128 ? n <= 8192 && n * k <= kRowsBelowSplit : blocks <= 2048 && blocks * (k / 128) <= 131072) return 1;
     const int64_t tiles = splitk_tiles(m, n), units = k / DAXQ_K_ALIGN;
     int best = 1;
     for (int s = 2; s <= 8; ++s)
@@ -464,13 +471,29 @@ static int splitk_choice(int64_t m, int64_t n, int64_t k) {
     return best;
 }
 
-// Rows that the GEMM of a linear runs on when the caller's buffers reach that far: m, or 128 where the tiled kernels (their
-// smallest tile) or, with a workspace, the K ranges are better than the kernel for few rows.  The rows beyond m hold
-// whatever the buffers held; an output row depends on its own operand row only.
-static int64_t gemm_rows(bool fp8, int64_t m, int64_t n, int64_t kp, bool splitk) {
+// Rows that the caller's buffers may hold for the widest choice of launches (daxq_linear_rows): m, or 128 with 33 to 127 rows
+// against more than 8192 columns, or where K ranges would run on 128 rows.
+static int64_t buffer_rows(bool fp8, int64_t m, int64_t n, int64_t kp, bool splitk) {
     if (m <= 0 || m >= 128 || n < 128) return m;
-    if (!rows_applies(m, n, kp, fp8)) return 128;
+    if (m > 32 && n > 8192) return 128;
     return splitk && !fp8 && m > 64 && splitk_choice(128, n, kp) > 1 ? 128 : m;
+}
+
+// Rows that the GEMM of a linear runs on when the caller's buffers reach that far: m where the kernel for few rows or a fitted tile
+// takes the launch; 64, the smallest fitted tile, or 128 where the kernel for few rows would only be the last resort (33 to 127 rows
+// against more than 8192 columns).  The rows beyond m hold whatever the buffers held; an output row depends on its own operand
+// row only.
+static int64_t gemm_rows(bool fp8, int64_t m, int64_t n, int64_t kp) {
+    if (m <= 0 || m >= 128 || n < 128 || rows_applies(m, n, kp, fp8) || fit_choice(m, n, kp, fp8) >= 0) return m;
+    return m < 64 && fit_choice(64, n, kp, fp8) >= 0 ? 64 : 128;
+}
+
+// Ranges of K that an INT8 launch with a workspace takes: none where the kernel for few rows or a fitted tile does it at once.  us, in
+// as many ranges as splitk_choice says / fitted tile: 256 x 5120 x 5120 21.0 / 12.8, 128 x 5120, K = 13824 28.8 / 21.0, 128 x 8192, K =
+// 13824 38.6 / 36.1, 371 x 1536, K = 13824 26.9 / 21.2, 512 x 1536 x 5120 22.2 / 10.3, 450 x 1137, K = 12800 26.1 / 20.1.
+static int launch_splits(int64_t m, int64_t n, int64_t kp) {
+    if (rows_applies(m, n, kp, false) || fit_choice(m, n, kp, false) >= 0) return 1;
+    return splitk_choice(m, n, kp);
 }
 
 template <bool FP8>
@@ -630,6 +653,8 @@ int daxq_init(void) {
     int rc = prepare_tile256_kernels();
     if (!rc) rc = prepare_tile_fp8_kernels();
     if (!rc) rc = prepare_rows_kernels();
+    if (!rc) rc = prepare_fit_i8_kernels();
+    if (!rc) rc = prepare_fit_fp8_kernels();
 #define DAXQ_PREP_ALL(FP8, BT, WN)                                        \
     if (!rc) rc = prepare_cfg<FP8, BT, BT, 128, 2, WN, true, 0>();
     DAXQ_PREP_ALL(false, 128, 2)
@@ -667,7 +692,15 @@ int daxq_linear_w8a8(int x_fmt, int w_fmt, int out_dtype, const void* xq, int64_
 }
 
 int64_t daxq_linear_rows(int x_fmt, int64_t m, int64_t n, int64_t k, int splitk) {
-    return daxq::gemm_rows(x_fmt != DAXQ_FMT_I8, m, n, (k + DAXQ_K_ALIGN - 1) / DAXQ_K_ALIGN * DAXQ_K_ALIGN, splitk != 0);
+    return daxq::buffer_rows(x_fmt != DAXQ_FMT_I8, m, n, (k + DAXQ_K_ALIGN - 1) / DAXQ_K_ALIGN * DAXQ_K_ALIGN, splitk != 0);
+}
+
+int64_t daxq_linear_launch_rows(int x_fmt, int64_t m, int64_t n, int64_t k) {
+    return daxq::gemm_rows(x_fmt != DAXQ_FMT_I8, m, n, (k + DAXQ_K_ALIGN - 1) / DAXQ_K_ALIGN * DAXQ_K_ALIGN);
+}
+
+int daxq_linear_launch_splits(int64_t m, int64_t n, int64_t k) {
+    return daxq::launch_splits(m, n, (k + DAXQ_K_ALIGN - 1) / DAXQ_K_ALIGN * DAXQ_K_ALIGN);
 }
 
 // ---- quantiser + GEMM behind one entry point --------------------------------------------------------------------
@@ -691,13 +724,13 @@ int daxq_dynamic_linear(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int ac
     const float qmax = x_fmt == DAXQ_FMT_I8 ? 127.0f : x_fmt == DAXQ_FMT_E4M3 ? 448.0f : 57344.0f;
     if (int rc = daxq_act_quant_rows_ex(x, x_dtype, x_fmt, m, k, ld_x, xq, ld_xq, sx, qmax, kEps, act_scale_round, stream)) return rc;
     const bool may_split = !fp8 && workspace && out_dtype == DAXQ_BF16 && kernel == 0;
-    int64_t mg = kernel == 0 ? gemm_rows(fp8, m, n, kp, may_split) : m < 128 && n >= 128 ? 128 : m;
+    int64_t mg = kernel == 0 ? gemm_rows(fp8, m, n, kp) : m < 128 && n >= 128 ? 128 : m;
     if (mg > rows_alloc) mg = m;
     hipStream_t st = (hipStream_t)stream;
     // INT8 launches with few tiles cut K into ranges when the caller brings a workspace (integer partial sums: the
     // same bits as the plain launch); FP8 sums would change with the number of rows, so they stay whole.
     if (may_split) {
-        const int splits = splitk_choice(mg, n, kp);
+        const int splits = launch_splits(mg, n, kp);
         if (splits > 1 && workspace_bytes >= kCounterBytes + splitk_tiles(mg, n) * splits * kPartialBytes)
             return launch_gemm_splitk<false>(xq, ld_xq, sx, wq, ld_wq, sw, bias, out, ld_out, mg, n, kp, splits, workspace,
                                              workspace_bytes, st, 0);

@@ -105,10 +105,10 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     }
     // launches that take a split-K workspace keep it with the custom op
     const bool may_split = x_fmt == DAXQ_FMT_I8 && out_kind == DAXQ_BF16;
-    if (may_split && daxq_linear_splitk_choice(scheme == kToken ? daxq_linear_rows(x_fmt, m, n, k, 1) : m, n, kp) > 1) Py_RETURN_NONE;
-    // rows that the buffers hold: 128 where that many in the tiled kernels are faster than m (what the rows beyond m hold is
+    if (may_split && daxq_linear_launch_splits(m, n, k) > 1) Py_RETURN_NONE;
+    // rows that the buffers hold: 64 or 128 where that many in a tiled kernel are faster than m (what the rows beyond m hold is
     // never looked at, their outputs are cut off); a kernel chosen by name runs on the rows there are
-    const int64_t rows = kernel == 0 ? daxq_linear_rows(x_fmt, m, n, k, 0) : m;
+    const int64_t rows = kernel == 0 ? daxq_linear_launch_rows(x_fmt, m, n, k) : m;
 
     at::Tensor out;
     int rc = 0;

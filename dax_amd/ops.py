@@ -494,7 +494,7 @@ def _auto_splits(m: int, n: int, k: int, out_dtype, want_acc: bool, fp8: bool) -
     # the same whatever the batch it arrives in; FP8 sums would change in the last bits with the number of rows
     if not SPLITK_AUTO or fp8 or want_acc or out_dtype != torch.bfloat16 or _capi.kernel_arg() != 0:
         return 1
-    return _capi.lib().daxq_linear_splitk_choice(m, n, k)
+    return _capi.lib().daxq_linear_launch_splits(m, n, k)
 
 
 def _linear(xq, sx, wq, sw, bias, fp8: bool, want_acc: bool, x_e5m2: bool = False, w_e5m2: bool = False,

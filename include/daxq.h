@@ -309,6 +309,8 @@ int daxq_linear_e5m2_e4m3(const uint8_t* xq, int64_t ld_xq, const float* sx,
  * bits 2 / 5 = the generic kernel on 256x256 / 128x128 tiles (an implementation of its own, any shape), 8 / 11 / 14 =
  * the tiled kernel on 256x256 / 128x128 / 256x128 tiles (int8: 16x16x64 MFMAs; fp8: 16x16x128 MFMAs; needs m, n >= the
  * tile edge, 256 for the 256x128 tiles);
+ * 32 + i = tile i of those fitted to launches of one round of workgroups (csrc/gemm_tile_fit.hip; needs m, n >= the tile; no
+ * accumulator dump);
  * 17 = the kernel for at most 128 rows, by itself also taken for few outputs (weights streamed through a ring per wavefront; the accumulator dump not by name);
  * bits 16-23, when not zero, set the depth of the tile-order groups; bits 24-27 the tile order of the 256x256 kernels
  * (0 = by shape, 1 = groups of tile rows, 2 = banded patches of 8 x 4 tiles per XCD; every order computes every tile
@@ -382,6 +384,11 @@ int daxq_linear_tile_order_choice(int64_t m, int64_t n, int64_t k);
  * 128 where that many rows in the tiled kernels are faster than m in the kernel for few rows.  splitk: the caller brings a
  * workspace (int8 with bf16 outputs).  Host arithmetic only. */
 int64_t daxq_linear_rows(int x_fmt, int64_t m, int64_t n, int64_t k, int splitk);
+
+/* What daxq_dynamic_linear does with such buffers and such a workspace: the rows its GEMM runs on (m, 64 or 128; at most those the
+ * buffers hold), and the ranges of K it takes with a workspace (1: none).  Host arithmetic only. */
+int64_t daxq_linear_launch_rows(int x_fmt, int64_t m, int64_t n, int64_t k);
+int daxq_linear_launch_splits(int64_t m, int64_t n, int64_t k);
 
 /*
  * Split-K form of daxq_linear_w8a8 for launches with too few output tiles to fill the CUs (a few hundred rows: the
