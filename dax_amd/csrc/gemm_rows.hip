@@ -17,26 +17,9 @@
 // output element is then the same sequence of MFMAs over the same K bytes in the same register positions as in
 // gemm_tile_fp8.hip, and an output row does not depend on how many rows the launch has.
 // Rows and columns beyond the matrix repeat its last row / column and are not stored.
-#include "gemm_tile.h"
+#include "gemm_rows.h"
 
 namespace daxq {
-
-// FP8 formats as in the tiled kernels: the weight is the MFMA "A" operand (cbsz), the activations the "B" operand (blgp)
-template <bool FP8, int F8>
-__device__ __forceinline__ typename Acc16<FP8>::type mfma_step(v8i w, v8i x, typename Acc16<FP8>::type c) {
-    if constexpr (FP8) {
-        return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, x, c, (F8 & kF8WE5) ? 1 : 0, (F8 & kF8XE5) ? 1 : 0, 0, 0, 0, 0);
-    } else {
-        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_shufflevector(w, w, 0, 1, 2, 3), __builtin_shufflevector(x, x, 0, 1, 2, 3), c, 0, 0, 0);
-        return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_shufflevector(w, w, 4, 5, 6, 7), __builtin_shufflevector(x, x, 4, 5, 6, 7), c, 0, 0, 0);
-    }
-}
-
-template <int T, typename F>
-__device__ __forceinline__ void for_down(F&& f) {
-    f(Int<T>{});
-    if constexpr (T > 0) for_down<T - 1>(f);
-}
 
 constexpr int rows_step_bytes(int mb) { return 2048 * (1 + mb); }  // LDS of a step: 16 weight rows, then MB x 16 activation rows
 
@@ -151,16 +134,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_rows_kernel(const GemmArgs p) {
 
     // ---- epilogue (the arithmetic of tile_epilogue16): a lane owns output row l % 16 of a block and 4 consecutive columns
     const int nc = n0 + 4 * g4;
-    float sw[4], bias[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int c = nc + e < p.n ? nc + e : p.n - 1;
-        sw[e] = p.sw[c];
-        if (!p.bias) bias[e] = -0.0f;  // x + (-0.0) == x bit for bit
-        else if constexpr (OUTK == DAXQ_F32) bias[e] = reinterpret_cast<const float*>(p.bias)[c];
-        else if constexpr (OUTK == DAXQ_F16) bias[e] = f16_bits_to_f32(p.bias[c]);
-        else bias[e] = bf16_bits_to_f32(p.bias[c]);
-    }
+    const ColumnBits<OUTK> cols(p, nc);
     v4i* s_part = reinterpret_cast<v4i*>(smem);
     if constexpr (KS > 1) {
         __syncthreads();  // every wavefront is done with the ring
@@ -188,45 +162,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_rows_kernel(const GemmArgs p) {
                 else static_cast<int32_t*>(p.acc)[(int64_t)m * p.ldacc + nc + e] = acc[i][e];
             }
         }
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float y = (float)acc[i][e];  // (int8: v_cvt_f32_i32, round to nearest even)
-            y = y * sxv;
-            y = y * sw[e];
-            if constexpr (OUTK == DAXQ_F32 || FP8) {
-                o[e] = y + bias[e];
-                if constexpr (OUTK == DAXQ_F16) asm("" : "+v"(o[e]));  // the sum is rounded to fp32 before the cast to fp16
-            } else if constexpr (OUTK == DAXQ_F16) {
-                asm("" : "+v"(y));
-                float z = (float)(_Float16)y + bias[e];
-                asm("" : "+v"(z));
-                o[e] = z;
-            } else {
-                o[e] = bf16_bits_to_f32(pack_bf16_rne(y, 0.0f) & 0xffffu) + bias[e];
-            }
-        }
-        const int64_t at = (int64_t)m * p.ldo + nc;
-        if constexpr (OUTK == DAXQ_F32) {
-            float* dst = reinterpret_cast<float*>(p.out) + at;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (nc + e < p.n) dst[e] = o[e];
-        } else {
-            uint32_t lo, hi;
-            if constexpr (OUTK == DAXQ_F16) lo = pack_f16_rne(o[0], o[1]), hi = pack_f16_rne(o[2], o[3]);
-            else lo = pack_bf16_rne(o[0], o[1]), hi = pack_bf16_rne(o[2], o[3]);
-            typedef v2u loose __attribute__((aligned(2)));
-            uint16_t* dst = p.out + at;
-            if (nc + 4 <= p.n) {
-                *reinterpret_cast<loose*>(dst) = v2u{lo, hi};
-            } else {
-                const uint32_t w[4] = {lo & 0xffffu, lo >> 16, hi & 0xffffu, hi >> 16};
-#pragma unroll
-                for (int e = 0; e < 3; ++e)
-                    if (nc + e < p.n) dst[e] = (uint16_t)w[e];
-            }
-        }
+        store_columns<FP8, OUTK>(p, acc[i], sxv, cols, m, nc);
     }
 }
 

@@ -276,6 +276,7 @@ int prepare_fit_i8_kernels();
 int prepare_fit_fp8_kernels();
 int prepare_tile_fp8_kernels();
 int prepare_rows_kernels();
+int prepare_few_kernels();
 int prepare_tile256_kernels();
 
 template <bool FP8, int BM, int BN, int BK, int WM, int WN, bool DIRECT, int F8 = 0>
@@ -653,6 +654,7 @@ int daxq_init(void) {
     int rc = prepare_tile256_kernels();
     if (!rc) rc = prepare_tile_fp8_kernels();
     if (!rc) rc = prepare_rows_kernels();
+    if (!rc) rc = prepare_few_kernels();
     if (!rc) rc = prepare_fit_i8_kernels();
     if (!rc) rc = prepare_fit_fp8_kernels();
 #define DAXQ_PREP_ALL(FP8, BT, WN)                                        \

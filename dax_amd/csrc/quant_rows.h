@@ -3,6 +3,8 @@
 // leaf quantisers for int8 / OCP e4m3fn / OCP e5m2.
 #pragma once
 
+#include <type_traits>
+
 #include "daxq_common.h"
 
 namespace daxq {
@@ -216,6 +218,154 @@ __device__ __forceinline__ uint4 load_stream_16(const uint4* p) {
 __device__ __forceinline__ void store_stream_8(uint2* p, uint2 v) {
     const daxq_v2u t = {v.x, v.y};
     __builtin_nontemporal_store(t, reinterpret_cast<daxq_v2u*>(p));
+}
+
+// A row is cut into chunks of 8 elements.  Any alignment is taken: the loads and stores are the same 16- and 8-byte
+// instructions whatever the address (gfx950 runs them on any byte address of global memory).
+template <int XT>
+struct Chunk {
+    daxq_v4u w[XT == DAXQ_F32 ? 2 : 1];
+};
+
+template <int XT>
+__device__ __forceinline__ void load_chunk(Chunk<XT>& v, const char* p) {
+    typedef daxq_v4u loose __attribute__((aligned(2)));
+#pragma unroll
+    for (int h = 0; h < (XT == DAXQ_F32 ? 2 : 1); ++h) v.w[h] = __builtin_nontemporal_load(reinterpret_cast<const loose*>(p) + h);
+}
+
+__device__ __forceinline__ void store_chunk(uint8_t* p, uint2 v) {
+    typedef daxq_v2u loose __attribute__((aligned(1)));
+    const daxq_v2u t = {v.x, v.y};
+    __builtin_nontemporal_store(t, reinterpret_cast<loose*>(p));
+}
+
+// running abs-max of chunks: packed 16-bit magnitudes or 32-bit ones
+template <int XT>
+__device__ __forceinline__ uint32_t chunk_amax(uint32_t mx, const Chunk<XT>& v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (XT != DAXQ_F32) {
+            mx = pk_max_u16(mx, v.w[0][i] & 0x7fff7fffu);
+        } else {
+            const uint32_t a = v.w[0][i] & 0x7fffffffu, b = v.w[1][i] & 0x7fffffffu;
+            mx = a > mx ? a : mx;
+            mx = b > mx ? b : mx;
+        }
+    }
+    return mx;
+}
+template <int XT>
+__device__ __forceinline__ uint32_t amax_of_lane(uint32_t mx) {
+    if constexpr (XT == DAXQ_F32) return mx;
+    return (mx & 0xffffu) > (mx >> 16) ? (mx & 0xffffu) : (mx >> 16);
+}
+
+template <int XT>
+__device__ __forceinline__ void chunk_values(const Chunk<XT>& v, float (&f)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if constexpr (XT == DAXQ_F32) f[i] = __uint_as_float(v.w[i >> 2][i & 3]);
+        else if constexpr (XT == DAXQ_BF16) f[i] = __uint_as_float(i & 1 ? v.w[0][i >> 1] & 0xffff0000u : v.w[0][i >> 1] << 16);
+        else f[i] = x_bits_to_f32<XT>(i & 1 ? v.w[0][i >> 1] >> 16 : v.w[0][i >> 1] & 0xffffu);
+    }
+}
+
+// How the elements of a row become bytes, one choice per row:
+//   kOwn       a bf16 row under its own scale at no more than the format's maximum: no clamp (dead code there,
+//              quant_rows.h), for FP8 the reciprocal sequence verified exhaustively for bf16 elements under bf16 scales
+//   kDivide    x / s by IEEE division (int8: x * inv), clamped
+//   kNear      FP8 under any other scale: x * inv, whose error is at most 1.5 steps of fp32, rounds to the byte of x / s
+//              unless it lies that close to a value where the byte changes.  Those values, in the normal and the subnormal
+//              range of either format, have at most five significant bits, i.e. zeros in the low 19 bits of the fp32
+//              pattern, so a product within three steps of such a pattern sends the wavefront's chunks through the
+//              division (seven patterns in 2^19, 13 elements in 10^6 under an arbitrary scale; zeros and infinities
+//              too).  A NaN need not be near: a bf16 NaN has zeros in 16 low bits only, the rest of its payload lies in
+//              those 19.  The clamp keeps it instead (v_maximum3 / v_minimum3 return a NaN, fmed3 its lower bound; a
+//              compare per element beside the fmed3 cost 32 rows of 13824 0.2 us).  Measured with a scale from the
+//              caller, 4096 x 5120 e5m2: 18.9 us dividing every element (26 VALU issue slots), 11.5 us here.
+//   kExact     FP8 under a power of two: x * inv is the quotient
+//   kShort     bf16 elements under a bf16 scale from the caller (a per-tensor scale): their quotients hit such values all
+//              the time; the sequence of kOwn, clamped, and the division for chunks that hold an infinity or a NaN
+enum { kOwn = 0, kDivide = 1, kNear = 2, kExact = 3, kShort = 4 };
+
+template <int FMT, int XT>
+__device__ __forceinline__ int form_of_scale(float s) {
+    if constexpr (FMT == 0) return kDivide;
+    const uint32_t b = __float_as_uint(s);
+    if (!(s >= 0x1p-100f && s <= 0x1p100f)) return kDivide;  // (NaN too)
+    if ((b & 0x7fffffu) == 0) return kExact;
+    return XT == DAXQ_BF16 && (b & 0xffffu) == 0 ? kShort : kNear;
+}
+
+template <int FMT, int FORM, int XT>
+__device__ __forceinline__ uint2 quant8(const float (&f)[8], float s, float inv) {
+    uint32_t o[2];
+    if constexpr (FMT == 0) {
+        constexpr bool CLAMP = FORM != kOwn;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {  // byte 0 of each of the four words: three v_perm_b32
+            const uint32_t p01 = __builtin_amdgcn_perm(q_i8_bits<CLAMP>(f[4 * h + 1], inv), q_i8_bits<CLAMP>(f[4 * h], inv), 0x0c0c0400u);
+            const uint32_t p23 = __builtin_amdgcn_perm(q_i8_bits<CLAMP>(f[4 * h + 3], inv), q_i8_bits<CLAMP>(f[4 * h + 2], inv), 0x0c0c0400u);
+            o[h] = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+        }
+    } else {
+        constexpr float kMax = FMT == 2 ? 57344.0f : 448.0f;
+        float v[8];
+        if constexpr (FORM == kNear || FORM == kExact || FORM == kShort) {
+            uint32_t near = 0xffffffffu;
+            bool nan = false;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float q0 = FORM == kShort ? q_f8_pre<FMT, false, false>(f[i], s, inv) : f[i] * inv;
+                if constexpr (FORM == kNear) {
+                    const uint32_t d = (__float_as_uint(q0) << 13) + (3u << 13);
+                    near = d < near ? d : near;
+                }
+                if constexpr (FORM == kNear) {  // a NaN stays one
+                    v[i] = __builtin_elementwise_minimum(__builtin_elementwise_maximum(q0, -kMax), kMax);
+                } else {
+                    nan |= q0 != q0;
+                    v[i] = __builtin_amdgcn_fmed3f(q0, -kMax, kMax);
+                }
+            }
+            if (__ballot((FORM == kNear && near <= (6u << 13)) || nan)) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = q_f8_pre<FMT, true>(f[i], s, inv);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = q_f8_pre<FMT, FORM != kOwn, FORM != kOwn>(f[i], s, inv);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int p = cvt_pk_f8<FMT>(v[4 * h], v[4 * h + 1], 0, false);
+            o[h] = (uint32_t)cvt_pk_f8<FMT>(v[4 * h + 2], v[4 * h + 3], p, true);
+        }
+    }
+    return make_uint2(o[0], o[1]);
+}
+
+// Calls f with the form (a compile-time constant) that the elements of a row take under scale s.  scale_in: the scale is the
+// caller's; round_x: a dynamic scale was rounded to the element type; leaf: the scale is a tensor's or a weight's, and the leaf
+// quantiser's bytes are wanted also where it is not finite (under an infinite scale a finite element is x / inf = 0, which the
+// reciprocal sequence gives as NaN, and an infinity is inf / inf, whose int8 byte depends on the clamp; so does that of a NaN)
+template <int FMT, int XT, typename F>
+__device__ __forceinline__ void with_form(float s, float qmax, bool scale_in, int round_x, int leaf, F&& f) {
+    constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
+    if (XT == DAXQ_BF16 && !scale_in && qmax <= kFmtMax && (FMT == 0 || round_x) && (!leaf || s < __builtin_inff())) {
+        f(std::integral_constant<int, kOwn>{});
+    } else if constexpr (FMT == 0) {
+        f(std::integral_constant<int, kDivide>{});
+    } else {
+        // (fp16 rows under their own fp16 scale: both have few significant bits, the products hit the values that need the
+        // division all the time)
+        const int form = XT == DAXQ_F16 && !scale_in && round_x ? kDivide : form_of_scale<FMT, XT>(s);
+        if (form == kNear) f(std::integral_constant<int, kNear>{});
+        else if (XT == DAXQ_BF16 && form == kShort) f(std::integral_constant<int, XT == DAXQ_BF16 ? kShort : kDivide>{});
+        else if (form == kExact) f(std::integral_constant<int, kExact>{});
+        else f(std::integral_constant<int, kDivide>{});
+    }
 }
 
 }  // namespace daxq

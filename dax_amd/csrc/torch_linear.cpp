@@ -103,9 +103,11 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         if (x->dim() != 2 || x->stride(1) != 1 || (m > 1 && x->stride(0) < k)) Py_RETURN_NONE;
         if (m > 1) ld_x = x->stride(0);
     }
+    // a handful of rows: one launch that quantises for itself
+    const bool few = kernel == 0 && daxq_linear_few_applies(x_kind, x_fmt, w_fmt, out_kind, scheme, scale_fp32 ? 0 : 1, m, n, k);
     // launches that take a split-K workspace keep it with the custom op
     const bool may_split = x_fmt == DAXQ_FMT_I8 && out_kind == DAXQ_BF16;
-    if (may_split && daxq_linear_launch_splits(m, n, k) > 1) Py_RETURN_NONE;
+    if (!few && may_split && daxq_linear_launch_splits(m, n, k) > 1) Py_RETURN_NONE;
     // rows that the buffers hold: 64 or 128 where that many in a tiled kernel are faster than m (what the rows beyond m hold is
     // never looked at, their outputs are cut off); a kernel chosen by name runs on the rows there are
     const int64_t rows = kernel == 0 ? daxq_linear_launch_rows(x_fmt, m, n, k) : m;
@@ -118,30 +120,38 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         auto shape = x->sizes().vec();
         shape.back() = n;
         const auto opt = at::TensorOptions().device(dev);
-        const int64_t ld_q = kp + (kp % 1024 == 0 ? kRowPad : 0);
-        // the quantised rows, their scales (the row length is a multiple of 128: aligned), 1 KiB for the abs-max of a tensor
-        const int64_t scales = rows * ld_q, partial = (scales + 4 * rows + 15) / 16 * 16;
-        const at::Tensor scratch = at::empty({partial + (scheme == kTensor ? 1024 : 0)}, opt.dtype(at::kByte));
-        out = rows == m ? at::empty(shape, opt.dtype(out_type)) : at::empty({rows, n}, opt.dtype(out_type));
-        uint8_t* q = static_cast<uint8_t*>(scratch.mutable_data_ptr());
-        float* sx = reinterpret_cast<float*>(q + scales);
-        void* st = c10::hip::getCurrentHIPStream(dev.index()).stream();
-        const void *xp = x->const_data_ptr(), *wp = wq->const_data_ptr(), *bp = bias ? bias->const_data_ptr() : nullptr;
-        const float* swp = sw->const_data_ptr<float>();
-        void* op = out.mutable_data_ptr();
-        if (scheme == kToken) {
-            rc = daxq_dynamic_linear(x_kind, x_fmt, w_fmt, out_kind, scale_fp32 ? 0 : 1, xp, ld_x, q, ld_q, sx, rows, wp, kp, swp, bp, op, n, m,
-                                     n, k, nullptr, 0, kernel, st);
+        if (few) {
+            out = at::empty(shape, opt.dtype(out_type));
+            rc = daxq_linear_few(x_kind, x_fmt, w_fmt, out_kind, scheme, scale_fp32 ? 0 : 1, x->const_data_ptr(), ld_x,
+                                 in_scale ? in_scale->const_data_ptr<float>() : nullptr, wq->const_data_ptr(), kp, sw->const_data_ptr<float>(),
+                                 bias ? bias->const_data_ptr() : nullptr, out.mutable_data_ptr(), n, m, n, k,
+                                 c10::hip::getCurrentHIPStream(dev.index()).stream());
         } else {
-            const float qmax = x_fmt == DAXQ_FMT_I8 ? 127.0f : x_fmt == DAXQ_FMT_E4M3 ? 448.0f : 57344.0f;
-            if (scheme == kTensor)
-                rc = daxq_act_quant_tensor(xp, x_kind, x_fmt, m, k, ld_x, q, ld_q, sx, nullptr, q + partial, qmax, kEps, scale_fp32 ? 0 : 1, st);
-            else
-                rc = daxq_quantize_tensor(xp, x_kind, x_fmt, m, k, ld_x, in_scale->const_data_ptr<float>(), q, ld_q, sx, st);
-            if (!rc)
-                rc = daxq_linear_w8a8(x_fmt, w_fmt, out_kind, q, ld_q, sx, wp, kp, swp, bp, op, n, nullptr, n, rows, n, kp, kernel, st);
+            const int64_t ld_q = kp + (kp % 1024 == 0 ? kRowPad : 0);
+            // the quantised rows, their scales (the row length is a multiple of 128: aligned), 1 KiB for the abs-max of a tensor
+            const int64_t scales = rows * ld_q, partial = (scales + 4 * rows + 15) / 16 * 16;
+            const at::Tensor scratch = at::empty({partial + (scheme == kTensor ? 1024 : 0)}, opt.dtype(at::kByte));
+            out = rows == m ? at::empty(shape, opt.dtype(out_type)) : at::empty({rows, n}, opt.dtype(out_type));
+            uint8_t* q = static_cast<uint8_t*>(scratch.mutable_data_ptr());
+            float* sx = reinterpret_cast<float*>(q + scales);
+            void* st = c10::hip::getCurrentHIPStream(dev.index()).stream();
+            const void *xp = x->const_data_ptr(), *wp = wq->const_data_ptr(), *bp = bias ? bias->const_data_ptr() : nullptr;
+            const float* swp = sw->const_data_ptr<float>();
+            void* op = out.mutable_data_ptr();
+            if (scheme == kToken) {
+                rc = daxq_dynamic_linear(x_kind, x_fmt, w_fmt, out_kind, scale_fp32 ? 0 : 1, xp, ld_x, q, ld_q, sx, rows, wp, kp, swp, bp, op, n, m,
+                                         n, k, nullptr, 0, kernel, st);
+            } else {
+                const float qmax = x_fmt == DAXQ_FMT_I8 ? 127.0f : x_fmt == DAXQ_FMT_E4M3 ? 448.0f : 57344.0f;
+                if (scheme == kTensor)
+                    rc = daxq_act_quant_tensor(xp, x_kind, x_fmt, m, k, ld_x, q, ld_q, sx, nullptr, q + partial, qmax, kEps, scale_fp32 ? 0 : 1, st);
+                else
+                    rc = daxq_quantize_tensor(xp, x_kind, x_fmt, m, k, ld_x, in_scale->const_data_ptr<float>(), q, ld_q, sx, st);
+                if (!rc)
+                    rc = daxq_linear_w8a8(x_fmt, w_fmt, out_kind, q, ld_q, sx, wp, kp, swp, bp, op, n, nullptr, n, rows, n, kp, kernel, st);
+            }
         }
-        if (rows != m) {
+        if (!few && rows != m) {
             const at::AutoDispatchBelowADInplaceOrView below;  // (the cut is no view of another tensor for the caller)
             out = out.narrow(0, 0, m).view(shape);
         }

@@ -374,6 +374,18 @@ int daxq_dynamic_linear_e5m2_e4m3(const void* x, int64_t ld_x, uint8_t* xq, int6
                                   const uint8_t* wq, int64_t ld_wq, const float* sw, const void* bias,
                                   void* out, int64_t ld_out, int64_t m, int64_t n, int64_t k, daxq_stream_t stream);
 
+/* The forward of a linear of at most eight rows in one launch, without scratch memory: x [m, k] (ld_x) is quantised inside the kernel.
+ * daxq_linear_few_applies says which calls it takes (1 / 0, host arithmetic only): int8 x int8 with bf16, fp16 or fp32 x, e4m3 / e5m2 x e4m3
+ * with bf16 x (n >= 128), out of x's type, k a multiple of 8, and so little of x that quantising it in every workgroup pays (csrc/gemm_few.hip); others are refused.
+ * scheme 0: a dynamic scale per row, 1: one dynamic scale for x, 2: the caller's, in_scale fp32 [1] on the device (NULL otherwise).  Outputs are
+ * the bits of the quantisers (daxq_act_quant_rows_ex / _tensor, daxq_quantize_tensor) followed by daxq_linear_w8a8; the other arguments as for
+ * daxq_dynamic_linear.  (dax/quant/nn/dynamic/linear.py:146-228, dax/quant/nn/quantized/linear.py) */
+int daxq_linear_few_applies(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme, int act_scale_round, int64_t m, int64_t n, int64_t k);
+int daxq_linear_few(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme, int act_scale_round,
+                    const void* x, int64_t ld_x, const float* in_scale,
+                    const void* wq, int64_t ld_wq, const float* sw, const void* bias,
+                    void* out, int64_t ld_out, int64_t m, int64_t n, int64_t k, daxq_stream_t stream);
+
 /* The tile order daxq_linear_w8a8 takes for a launch of 256x256 tiles when bits 24-27 of `kernel` are 0, as the value
  * of those bits: 1 = groups of tile rows, 2 = banded patches (large launches: K >= 2048, N >= 5120, M >= 7937 and no
  * XCD more than 5 % over its share of the tiles).  For tests and diagnostics; no
