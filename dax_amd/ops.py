@@ -438,8 +438,7 @@ def scale_from_minmax(min_val: torch.Tensor, max_val: torch.Tensor, qmax: float,
 scale_from_minmax.register_fake(lambda min_val, max_val, qmax, eps=EPS_F32: torch.empty_like(min_val))
 
 
-@torch.library.custom_op("daxq::weight_quant", mutates_args=(), device_types="cuda")
-def weight_quant(w: torch.Tensor, fmt: str, quant_max: float, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
+def weight_quant_rows(w: torch.Tensor, fmt: str, quant_max: float, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
     """Symmetric per-row (per-output-channel) quantisation of a bf16 / fp16 / fp32 weight in one pass: (bytes [N, K] without
     padding, fp32 scale [N]).  The same bits as row_minmax, scale_from_minmax and quantize_rows: the row's abs-max is the
     larger of -min and max, and the scale is not rounded."""
@@ -455,6 +454,12 @@ def weight_quant(w: torch.Tensor, fmt: str, quant_max: float, eps: float) -> Tup
             _capi.check(_capi.lib().daxq_weight_quant_rows(w.data_ptr(), kind, FMT[fmt], n, k, w.stride(0) if n > 1 else k, q.data_ptr(), k,
                                                            s.data_ptr(), quant_max, eps, _stream(w)), name)
     return q, s
+
+
+@torch.library.custom_op("daxq::weight_quant", mutates_args=(), device_types="cuda")
+def weight_quant(w: torch.Tensor, fmt: str, quant_max: float, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``weight_quant_rows`` as an op that modes and traces see (which costs a call 8 us of the host)."""
+    return weight_quant_rows(w, fmt, quant_max, eps)
 
 
 weight_quant.register_fake(lambda w, fmt, quant_max, eps: (

@@ -121,9 +121,12 @@ class DerivedOperands:
         """Builds the derived operands and the codes of the native call now, so that a forward launches nothing but its
         kernels.  A module that does not live on a ROCm device (yet) builds them at its first forward there."""
         self._packed = self._sw_vec = None
-        if self.qweight.device.type == "cuda":
-            self._gemm_weight()
-            self._weight_scale_vector()
+        qw, ws = self.qweight, self.weight_scale
+        if qw.device.type == "cuda":
+            if qw.shape[1] % ops.K_ALIGN or not qw.is_contiguous():
+                self._gemm_weight()
+            if ws.numel() == 1:
+                self._weight_scale_vector()
             object.__setattr__(self, "_fast", (self._fast_settings(), self._fast_codes()))
 
     def _gemm_weight(self) -> Tensor:

@@ -15,6 +15,7 @@ calibration diagnostic that writes plots) is not built.
 """
 from __future__ import annotations
 
+from collections import namedtuple
 from functools import partial
 
 import torch
@@ -24,6 +25,8 @@ from ... import ops
 from ..qscheme import per_channel_symmetric, per_tensor_symmetric, per_token_symmetric
 
 ALLOWED_DTYPES = (torch.float8_e4m3fn, torch.float8_e5m2, torch.int8)
+_QUANT_MAX = {dt: float(torch.iinfo(dt).max if dt == torch.int8 else torch.finfo(dt).max) for dt in ALLOWED_DTYPES}
+_EPS = torch.finfo(torch.float32).eps
 
 
 class UniformQuantizationObserverBase(nn.Module):
@@ -170,3 +173,23 @@ class DynamicObserverPlaceholder(UniformQuantizationObserverBase):
 
     def calculate_qparams(self):
         pass
+
+
+# What a conversion needs to know of an observer that it would only build to ask.
+PlainSettings = namedtuple("PlainSettings", ["dtype", "qscheme", "quant_max", "eps"])
+_PLAIN_ARGUMENTS = {"dtype", "qscheme", "is_dynamic"}
+
+
+def plain_settings(factory, weight: bool):
+    """The settings of the object that ``factory`` makes, where that is exactly this file's per-channel weight observer
+    (``weight``) or activation placeholder with no arguments but those that the qconfig factories give; None otherwise, and
+    where the constructor would refuse them."""
+    if (factory.__class__ is not partial or factory.func is not (PerChannelMinMaxObserver if weight else DynamicObserverPlaceholder)
+            or factory.args or not factory.keywords.keys() <= _PLAIN_ARGUMENTS):
+        return None
+    dtype, qscheme = factory.keywords.get("dtype", torch.float8_e4m3fn), factory.keywords.get("qscheme", per_tensor_symmetric)
+    if dtype not in ALLOWED_DTYPES or qscheme not in ((per_channel_symmetric,) if weight else
+                                                      (per_tensor_symmetric, per_channel_symmetric, per_token_symmetric)):
+        return None
+    # (the constructor keeps the floor of the scales in the default element type; a power of two is the same in all of them)
+    return PlainSettings(dtype, qscheme, _QUANT_MAX[dtype], _EPS)
