@@ -54,7 +54,9 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
     __shared__ uint32_t s_max[4];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t row0 = (int64_t)blockIdx.x * (4 / W) + wave / W;
+    // behind tensor_amax_kernel: the rows that it read last first, each on the XCD that read it
+    const int64_t unit = W > 1 && !PLAIN && !SCALE_IN && a.partials ? (int64_t)((gridDim.x >> 3) - 1 - (blockIdx.x >> 3)) * 8 + (blockIdx.x & 7) : blockIdx.x;
+    const int64_t row0 = unit * (4 / W) + wave / W;
     if (W == 1 && row0 >= a.m) return;
     const int64_t row = row0 < a.m ? row0 : a.m - 1;  // (rows beyond the last: the wavefront still reaches the barrier)
     const int part = wave % W, nch = a.k >> 3, npad = a.kfill >> 3;
@@ -206,6 +208,14 @@ struct ScaleKind {
     bool weight = false;                 // rows of a weight: the leaf quantiser's bytes also under a scale that is not finite
 };
 
+// Rows that a workgroup of quant_rows_kernel takes where a row has more than one wavefront (the instantiations that
+// launch_quant_rows_t goes through), else 0.
+static int quant_unit(int x_dtype, int64_t kfill) {
+    const int64_t cols = (kfill + 511) / 512;
+    if (x_dtype == DAXQ_F32) return cols <= 2 ? 0 : 1;
+    return cols <= 4 ? 0 : cols <= 6 ? 2 : 1;
+}
+
 // at most `count` rows of `a` from row r on
 template <int XB>
 static QuantArgs rows_from(const QuantArgs& a, int64_t r, int64_t count) {
@@ -244,7 +254,8 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
         constexpr int64_t kRows = 4 / W, kSlab = kRows << 23;                                                              \
         for (int64_t r = 0; r < m; r += kSlab) {                                                                           \
             const QuantArgs b = rows_from<XB>(a, r, kSlab);                                                                \
-            const dim3 grid((unsigned)((b.m + kRows - 1) / kRows));                                                        \
+            const unsigned groups = (unsigned)((b.m + kRows - 1) / kRows);                                                 \
+            const dim3 grid(W > 1 && a.partials ? (groups + 7) / 8 * 8 : groups);                                          \
             if (plain) hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain>), grid, dim3(256), 0, st, b); \
             else hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false>), grid, dim3(256), 0, st, b);        \
         }                                                                                                                  \
@@ -300,46 +311,95 @@ static int launch_quant_rows_fmt(int q_fmt, const void* x, int x_dtype, int64_t 
 }
 
 // Abs-max of a whole matrix as kPartials bit patterns (sign cleared; their maximum is the abs-max, NaN above infinity):
-// one workgroup of sixteen wavefronts per CU, four 16-byte loads per lane in flight.
+// one workgroup of sixteen wavefronts per CU, U chunks per lane in flight (2 to 4 of 16 bytes are level, 6 and 8 slower by 1 to 10 %:
+// the last turns of the loop are emptier).
+// It is bound by memory, and what it reads the quantiser reads again right behind it.  With a row or two to a workgroup of the
+// quantiser (unit > 0: the rows of one, K > 2048), workgroup i here takes the rows of the quantiser's workgroups i, i + 256, ...,
+// which run on the same XCD, and the quantiser begins with the rows that were read last, out of that XCD's L2.  Both launches, us,
+// matrix read as it lies -> this (bf16, e5m2): 4096 x 5120 21.3 -> 19.9, 4725 x 13824 55.2 -> 53.8, 12000 x 4608 46.2 -> 44.6, 1000 x 8960
+// 12.2 -> 10.8, 300 x 5120 6.7 -> 6.5; shorter rows lose what they gain to the row arithmetic (16000 x 1536 23.7 -> 24.9).
+struct AmaxArgs {
+    const char* x;
+    int64_t m, ld_x;
+    int k;
+    int unit;  // rows that a workgroup of the quantiser takes, or 0: the matrix is read as it lies
+    uint32_t* partials;
+};
 template <int XT>
-__global__ __launch_bounds__(1024) void tensor_amax_kernel(const char* __restrict__ x, int64_t m, int k, int64_t ld_x, uint32_t* __restrict__ partials) {
-    constexpr int XB = XT == DAXQ_F32 ? 4 : 2, U = XT == DAXQ_F32 ? 2 : 4;
+__global__ __launch_bounds__(1024) void tensor_amax_kernel(const AmaxArgs a) {
+    constexpr int XB = XT == DAXQ_F32 ? 4 : 2, U = XT == DAXQ_F32 ? 2 : 3;
     constexpr uint32_t kAbs = XT == DAXQ_F32 ? 0x7fffffffu : 0x7fffu;
     __shared__ uint32_t s_max[16];
-    int64_t len = k;
-    if (ld_x == k || m == 1) {  // one long row
-        len = (int64_t)k * m;
-        m = 1;
-    }
-    const int64_t nch = len >> 3;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t mx = 0, tl = 0;
-    // a long row is spread over the grid, rows of a strided matrix are dealt to the workgroups
-    const int64_t first = m == 1 ? (int64_t)blockIdx.x * 1024 : 0, step = m == 1 ? (int64_t)kPartials * 1024 : 1024;
-    for (int64_t r = m == 1 ? 0 : blockIdx.x; r < m; r += kPartials) {
-        const char* xr = x + r * ld_x * XB;
-        for (int64_t c = first + threadIdx.x; c < nch; c += U * step) {
+    auto element = [&](const char* xr, int64_t e) __attribute__((always_inline)) {
+        const uint32_t t = (XT == DAXQ_F32 ? reinterpret_cast<const uint32_t*>(xr)[e] : reinterpret_cast<const uint16_t*>(xr)[e]) & kAbs;
+        tl = t > tl ? t : tl;
+    };
+    if (a.unit) {
+        // a wavefront takes every sixteenth piece (64 chunks of a row) of the workgroup's rows
+        const int nch = a.k >> 3, pieces = (nch + 63) >> 6;
+        const int64_t rows = a.m;
+        int64_t row = (int64_t)blockIdx.x * a.unit;
+        int in = 0, c = 0;  // row of the unit, piece of the row
+        auto advance = [&](int by) __attribute__((always_inline)) {
+            c += by;
+            while (c >= pieces) {
+                c -= pieces;
+                if (++in == a.unit) in = 0, row += (int64_t)kPartials * a.unit;
+            }
+        };
+        advance(wave);
+        while (row < rows) {
             Chunk<XT> v[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int64_t cu = c + u * step;
-                load_chunk<XT>(v[u], xr + (cu < nch ? cu : c) * (8 * XB));  // (beyond the end: the lane's first chunk again)
+                if (row + in < rows) {
+                    const char* xr = a.x + (row + in) * a.ld_x * XB;
+                    const int at = c * 64 + lane;
+                    load_chunk<XT>(v[u], xr + (uint32_t)(at < nch ? at : nch - 1) * (8u * XB));
+                    if (c == pieces - 1 && lane < (a.k & 7)) element(xr, nch * 8 + lane);
+                } else {
+                    v[u] = Chunk<XT>{};
+                }
+                advance(16);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) mx = chunk_amax<XT>(mx, v[u]);
         }
-        const int64_t e = (nch << 3) + threadIdx.x;
-        if (e < len) {
-            const uint32_t t = (XT == DAXQ_F32 ? reinterpret_cast<const uint32_t*>(xr)[e] : reinterpret_cast<const uint16_t*>(xr)[e]) & kAbs;
-            tl = t > tl ? t : tl;
+    } else {
+        int64_t len = a.k, m = a.m;
+        if (a.ld_x == a.k || m == 1) {  // one long row
+            len *= m;
+            m = 1;
+        }
+        const int64_t nch = len >> 3;
+        // a long row is spread over the grid, rows of a strided matrix are dealt to the workgroups
+        const int64_t first = m == 1 ? (int64_t)blockIdx.x * 1024 : 0, step = m == 1 ? (int64_t)kPartials * 1024 : 1024;
+        for (int64_t r = m == 1 ? 0 : blockIdx.x; r < m; r += kPartials) {
+            const char* xr = a.x + r * a.ld_x * XB;
+            for (int64_t c = first + threadIdx.x; c < nch; c += U * step) {
+                Chunk<XT> v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int64_t cu = c + u * step;
+                    load_chunk<XT>(v[u], xr + (cu < nch ? cu : c) * (8 * XB));  // (beyond the end: the lane's first chunk again)
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) mx = chunk_amax<XT>(mx, v[u]);
+            }
+            const int64_t e = (nch << 3) + threadIdx.x;
+            if (e < len) element(xr, e);
         }
     }
     mx = amax_of_lane<XT>(mx);
     mx = wave_max_u32(tl > mx ? tl : mx);
-    if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = mx;
+    if (lane == 0) s_max[wave] = mx;
     __syncthreads();
     if (threadIdx.x < 64) {
         mx = wave_max_u32(threadIdx.x < 16 ? s_max[threadIdx.x] : 0u);
-        if (threadIdx.x == 0) partials[blockIdx.x] = mx;
+        if (threadIdx.x == 0) a.partials[blockIdx.x] = mx;
     }
 }
 
@@ -545,12 +605,12 @@ int daxq_act_quant_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int6
     if ((uintptr_t)x & (x_dtype == DAXQ_F32 ? 3 : 1)) return fail(DAXQ_ERR_ALIGN, "act_quant_tensor: x must be element aligned");
     hipStream_t st = (hipStream_t)stream;
     uint32_t* part = static_cast<uint32_t*>(scratch);
-    const char* xp = static_cast<const char*>(x);
+    const AmaxArgs a{static_cast<const char*>(x), m, ld_x, (int)k, quant_unit(x_dtype, fill_width(k, ld_q)), part};
     const dim3 grid(kPartials), block(1024);
     switch (x_dtype) {
-        case DAXQ_BF16: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_BF16>, grid, block, 0, st, xp, m, (int)k, ld_x, part); break;
-        case DAXQ_F16: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_F16>, grid, block, 0, st, xp, m, (int)k, ld_x, part); break;
-        case DAXQ_F32: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_F32>, grid, block, 0, st, xp, m, (int)k, ld_x, part); break;
+        case DAXQ_BF16: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_BF16>, grid, block, 0, st, a); break;
+        case DAXQ_F16: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_F16>, grid, block, 0, st, a); break;
+        case DAXQ_F32: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_F32>, grid, block, 0, st, a); break;
         default: return fail(DAXQ_ERR_ARG, "act_quant_tensor: unknown element type %d", x_dtype);
     }
     if (int rc = check_launch("tensor_amax")) return rc;

@@ -118,6 +118,25 @@ def test_one_scale_for_the_tensor(ops, dtype, m, k, pitch):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k,pad", [(897, 0), (1024, 8), (1921, 3), (2049, 0), (3072, 0), (3073, 8), (16384, 0)])
+@pytest.mark.parametrize("m", [1, 2, 9, 511, 514, 1031])
+def test_one_scale_found_by_the_rows_of_the_quantiser(ops, dtype, k, pad, m):
+    """Rows of one to four wavefronts, units of one and two rows, row counts around whole groups of units and of eight units,
+    with the largest element anywhere: one reading order for both launches changes neither scale nor bytes."""
+    g = torch.Generator("cuda").manual_seed(m + k)
+    base = torch.randn(m, k + pad, device="cuda", generator=g).to(dtype)
+    s0 = torch.zeros(1, device="cuda")
+    for at in ((m - 1, k - 1), (0, 0), (m // 2, k // 2), (max(0, m - 2), 511), (m // 3, k - k % 8 - 1)):
+        x = base.clone()
+        x[at] = -9.5
+        q, s, s1 = ops.act_quant_tensor(x[:, :k], "e4m3", 448.0, ops.EPS_F32, True, True)
+        s0.copy_((torch.tensor(9.5).to(dtype) / 448.0).to(torch.float32))
+        assert torch.equal(s1, s0) and torch.equal(s, s0.expand(m))
+        q1, _ = ops.quantize_tensor(x[:, :k], s0, "e4m3", True)
+        assert torch.equal(q, q1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("n,k,pitch", [(1, 1, 1), (5, 7, 9), (3, 8, 8), (4, 2047, 2047), (3, 2048, 2051), (7, 8193, 8193), (2, 20001, 20001)])
 def test_row_statistics_and_weights_in_one_pass(ops, dtype, n, k, pitch):
     """Row minima and maxima with 16-byte loads (chunks, leftover elements, rows that start anywhere; all-negative, zero and
