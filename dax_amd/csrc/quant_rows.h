@@ -275,27 +275,39 @@ __device__ __forceinline__ void chunk_values(const Chunk<XT>& v, float (&f)[8]) 
 //   kOwn       a bf16 row under its own scale at no more than the format's maximum: no clamp (dead code there,
 //              quant_rows.h), for FP8 the reciprocal sequence verified exhaustively for bf16 elements under bf16 scales
 //   kDivide    x / s by IEEE division (int8: x * inv), clamped
-//   kNear      FP8 under any other scale: x * inv, whose error is at most 1.5 steps of fp32, rounds to the byte of x / s
+//   kNear      FP8 and fp32 elements: x * inv, whose error is at most 1.5 steps of fp32, rounds to the byte of x / s
 //              unless it lies that close to a value where the byte changes.  Those values, in the normal and the subnormal
 //              range of either format, have at most five significant bits, i.e. zeros in the low 19 bits of the fp32
 //              pattern, so a product within three steps of such a pattern sends the wavefront's chunks through the
 //              division (seven patterns in 2^19, 13 elements in 10^6 under an arbitrary scale; zeros and infinities
-//              too).  A NaN need not be near: a bf16 NaN has zeros in 16 low bits only, the rest of its payload lies in
-//              those 19.  The clamp keeps it instead (v_maximum3 / v_minimum3 return a NaN, fmed3 its lower bound; a
-//              compare per element beside the fmed3 cost 32 rows of 13824 0.2 us).  Measured with a scale from the
-//              caller, 4096 x 5120 e5m2: 18.9 us dividing every element (26 VALU issue slots), 11.5 us here.
+//              too).  A NaN need not be near (some of its payload lies in those 19 bits): the clamp keeps it instead
+//              (v_maximum3 / v_minimum3 return a NaN, fmed3 its lower bound; a compare per element beside the fmed3 cost
+//              32 rows of 13824 0.2 us).
 //   kExact     FP8 under a power of two: x * inv is the quotient
-//   kShort     bf16 elements under a bf16 scale from the caller (a per-tensor scale): their quotients hit such values all
-//              the time; the sequence of kOwn, clamped, and the division for chunks that hold an infinity or a NaN
+//   kShort     FP8 and 16-bit elements under any other scale: the sequence of kOwn, clamped, and the division for chunks
+//              that hold an infinity or a NaN.  Quotients of such elements hit values where the byte changes all the time
+//              (an abs-max of 8 bits over 448 = 7 x 64 is the scale of a calibrated or a weight's row: every element with the
+//              abs-max's significand does), so that kNear divides nearly every chunk: e4m3 under such a scale, us, kNear ->
+//              kShort: 4725 x 5120 17.5 -> 13.6, a weight of 13824 x 5120 47.9 -> 34.8, 9000 x 1536 11.3 -> 9.4; fp16 rows
+//              under their own fp16 scale, which divided every element, 4725 x 5120 19.8 -> 14.9.
+//              Its bytes are those of the division: with u the step of the quotient, the corrected quotient is x / s,
+//              off by less than 6 x 2^-24 u (reciprocal and residual are rounded once each, the first quotient is off
+//              by at most 3 u), rounded.  Another byte than that of RN(x / s) needs a midpoint m, half a step from a value of five bits, inside
+//              that error.  In units of u / 2, m = +-1 mod 2^20 and x / s = X / S with the significand S of s and X a multiple of 2^36
+//              (x has at most 11 bits), so |X - m S| is at least the distance of S from a multiple of 2^20, not zero (m is odd
+//              and longer than x), and would have to be below 12: scales that close to a significand of four bits, but not one
+//              themselves, divide.
 enum { kOwn = 0, kDivide = 1, kNear = 2, kExact = 3, kShort = 4 };
 
 template <int FMT, int XT>
 __device__ __forceinline__ int form_of_scale(float s) {
     if constexpr (FMT == 0) return kDivide;
     const uint32_t b = __float_as_uint(s);
-    if (!(s >= 0x1p-100f && s <= 0x1p100f)) return kDivide;  // (NaN too)
+    // (NaN too; from 2^-80 on the residual of a quotient that is not rounded to zero is a normal number)
+    if (!(s >= (XT == DAXQ_F32 ? 0x1p-100f : 0x1p-80f) && s <= 0x1p100f)) return kDivide;
     if ((b & 0x7fffffu) == 0) return kExact;
-    return XT == DAXQ_BF16 && (b & 0xffffu) == 0 ? kShort : kNear;
+    if constexpr (XT == DAXQ_F32) return kNear;
+    return ((b + 16u) & 0xfffffu) <= 32u && (b & 0xfffffu) != 0 ? kDivide : kShort;
 }
 
 template <int FMT, int FORM, int XT>
@@ -317,7 +329,9 @@ __device__ __forceinline__ uint2 quant8(const float (&f)[8], float s, float inv)
             bool nan = false;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float q0 = FORM == kShort ? q_f8_pre<FMT, false, false>(f[i], s, inv) : f[i] * inv;
+                float q0 = f[i] * inv;
+                // (the negated residual: +0 where there is none, so that a -0 stays one; a NaN's sign is the division's)
+                if constexpr (FORM == kShort) q0 = __builtin_fmaf(-__builtin_fmaf(q0, s, -f[i]), inv, q0);
                 if constexpr (FORM == kNear) {
                     const uint32_t d = (__float_as_uint(q0) << 13) + (3u << 13);
                     near = d < near ? d : near;
@@ -358,11 +372,9 @@ __device__ __forceinline__ void with_form(float s, float qmax, bool scale_in, in
     } else if constexpr (FMT == 0) {
         f(std::integral_constant<int, kDivide>{});
     } else {
-        // (fp16 rows under their own fp16 scale: both have few significant bits, the products hit the values that need the
-        // division all the time)
-        const int form = XT == DAXQ_F16 && !scale_in && round_x ? kDivide : form_of_scale<FMT, XT>(s);
-        if (form == kNear) f(std::integral_constant<int, kNear>{});
-        else if (XT == DAXQ_BF16 && form == kShort) f(std::integral_constant<int, XT == DAXQ_BF16 ? kShort : kDivide>{});
+        const int form = form_of_scale<FMT, XT>(s);
+        constexpr int kMost = XT == DAXQ_F32 ? kNear : kShort;
+        if (form == kMost) f(std::integral_constant<int, kMost>{});
         else if (form == kExact) f(std::integral_constant<int, kExact>{});
         else f(std::integral_constant<int, kDivide>{});
     }

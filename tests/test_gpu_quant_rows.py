@@ -117,6 +117,30 @@ def test_one_scale_for_the_tensor(ops, dtype, m, k, pitch):
     assert bool(torch.isnan(s).all()) and bool(torch.isnan(s1).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+def test_every_element_under_scales_near_short_significands(ops, dtype, fmt):
+    """All 65536 elements of a 16-bit type: under quotients of short numbers and the format's maximum (calibrated scales), scales
+    of any bits, and scales around those with a significand of four bits, where the corrected reciprocal gives way to the
+    division.  The bytes are those of an IEEE division."""
+    g = torch.Generator().manual_seed(3)
+    qmax = torch.tensor(ops.QMAX[fmt])
+    bits = [torch.randint(0x3b000000, 0x41000000, (60,), generator=g)]                      # any
+    bits.append((torch.rand(40, generator=g) * 90 + 0.01).to(dtype).float().div(qmax).view(torch.int32).long())
+    short = 0x3c000000 + torch.randint(0, 80, (12,), generator=g) * (1 << 20)
+    bits += [(short[:, None] + torch.tensor([-17, -16, -12, -6, -3, -2, -1, 0, 1, 2, 3, 6, 12, 16, 17])).reshape(-1)]
+    bits.append(torch.tensor([2.0 ** -130, 2.0 ** -101, 1.1 * 2.0 ** -90, 1.3 * 2.0 ** -80, 1.7 * 2.0 ** -79, 1.9 * 2.0 ** 99,
+                              1.1 * 2.0 ** 100]).view(torch.int32).long())
+    scales = torch.cat(bits).to(torch.int32).view(torch.float32)
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype).reshape(4, 16384)
+    xs, sc = x.repeat(len(scales), 1), scales.repeat_interleave(4)
+    q = getattr(ops, "quantize_rows_" + fmt)(xs.to("cuda"), sc.to("cuda"))
+    ref = O.quantize_to_fp8(xs, sc[:, None], FP8[fmt])
+    nan = torch.isnan(xs)
+    np.testing.assert_array_equal(_bytes(q)[~nan.numpy()], _bytes(ref)[~nan.numpy()])
+    assert bool(torch.isnan(q.cpu().view(FP8[fmt]).float()[nan]).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("k,pad", [(897, 0), (1024, 8), (1921, 3), (2049, 0), (3072, 0), (3073, 8), (16384, 0)])
 @pytest.mark.parametrize("m", [1, 2, 9, 511, 514, 1031])
