@@ -497,7 +497,7 @@ static int launch_ln_rows(const char* what, const uint16_t* x, int64_t m, int64_
     }
     const int64_t rpg = rows_per_group < m ? rows_per_group : m, qpg = (rpg + 3) / 4, quads = (m / rpg) * qpg + (m % rpg + 3) / 4;
     const int64_t want = (int64_t)cus * per_cu;
-    hipLaunchKernelGGL((ln_rows<NCOL, FMT>), dim3((unsigned)(quads < want ? quads : want)), dim3(256), lds, st, x, m, (int)k, ld_x, mul,
+    launch_kernel((ln_rows<NCOL, FMT>), dim3((unsigned)(quads < want ? quads : want)), dim3(256), lds, st, x, m, (int)k, ld_x, mul,
                        add, rpg, qpg, quads, eps, q, ld_q, (int)kfill, scale, qmax);
     return check_launch(what);
 }
@@ -556,7 +556,7 @@ static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t
             switch (k / 512) {
 #define DAXQ_GELU_EXACT(N)                                                                                                        \
     case N:                                                                                                                       \
-        hipLaunchKernelGGL((gelu_rows_exact<N, FMT>), grid, dim3(256), 0, st, xp, m, ld_x, qp, ld_q, scale, qmax);                 \
+        launch_kernel((gelu_rows_exact<N, FMT>), grid, dim3(256), 0, st, xp, m, ld_x, qp, ld_q, scale, qmax);                 \
         return check_launch(what);
                 DAXQ_GELU_EXACT(12)
                 DAXQ_GELU_EXACT(16)
@@ -593,10 +593,10 @@ static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t
         }                                                                                                                \
         const dim3 grid((unsigned)(quads < want ? quads : want));                                                        \
         if (yp)                                                                                                          \
-            hipLaunchKernelGGL((fused_rows_wave<N, FMT, PRE, true>), grid, block, lds, st, xp, m, (int)k, ld_x, mul, add, \
+            launch_kernel((fused_rows_wave<N, FMT, PRE, true>), grid, block, lds, st, xp, m, (int)k, ld_x, mul, add, \
                                rows_per_group, eps, yp, ld_y, qp, ld_q, (int)kfill, scale, qmax);                                    \
         else                                                                                                             \
-            hipLaunchKernelGGL((fused_rows_wave<N, FMT, PRE, false>), grid, block, lds, st, xp, m, (int)k, ld_x, mul, add, \
+            launch_kernel((fused_rows_wave<N, FMT, PRE, false>), grid, block, lds, st, xp, m, (int)k, ld_x, mul, add, \
                                rows_per_group, eps, yp, ld_y, qp, ld_q, (int)kfill, scale, qmax);                                    \
         return check_launch(what);                                                                                       \
     }

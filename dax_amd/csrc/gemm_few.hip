@@ -224,7 +224,7 @@ static int launch_few_one(const FewArgs* a, hipStream_t st) {
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), most, lds_set)) return rc;
     if (!a) return DAXQ_OK;
     const int lds = ring + MR * (a->g.k + 16) + (kFewWaves + MR) * 4;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((a->g.n + 16 * CG - 1) / (16 * CG))), dim3(64 * kFewWaves), lds, st, *a);
+    launch_kernel(kern, dim3((unsigned)((a->g.n + 16 * CG - 1) / (16 * CG))), dim3(64 * kFewWaves), lds, st, *a);
     return check_launch("gemm_few");
 }
 

@@ -175,7 +175,7 @@ static int launch_rows_one(const GemmArgs* args, hipStream_t st) {
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_set)) return rc;
     if (!args) return DAXQ_OK;
     const dim3 grid((unsigned)((args->n + 15) / 16), (unsigned)((args->m + 16 * MB - 1) / (16 * MB)));
-    hipLaunchKernelGGL(kern, grid, dim3(64 * KS), lds, st, *args);
+    launch_kernel(kern, grid, dim3(64 * KS), lds, st, *args);
     return check_launch("gemm_rows");
 }
 

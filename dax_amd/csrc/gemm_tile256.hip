@@ -527,7 +527,7 @@ static int launch_splitk_impl(const GemmArgs& a, hipStream_t st) {
     if (int rc = prepare_tile256s5<FP8, false, F8, !FP8, 128, true>()) return rc;
     const int64_t nt = (int64_t)a.tiles_m * a.tiles_n * a.splits;
     if (nt > 0x7fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many workgroups");
-    hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(T), SMEM, st, a);
+    launch_kernel(kern, dim3((unsigned)nt), dim3(T), SMEM, st, a);
     return check_launch("gemm_tile128_splitk");
 }
 
@@ -560,7 +560,7 @@ static int launch_tile256s5_impl(const GemmArgs& a, hipStream_t st) {
     if (int rc = prepare_tile256s5<FP8, DUMP, F8, N16, BT, false, D, OUTK>()) return rc;
     const int64_t nt = grid_of_order(a);
     if (nt > 0x7fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
-    hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(T), SMEM, st, a);
+    launch_kernel(kern, dim3((unsigned)nt), dim3(T), SMEM, st, a);
     return check_launch("gemm_tile256s5");
 }
 
@@ -607,7 +607,7 @@ static int prepare_then_halves() {
 template <bool DUMP, int OUTK>
 static int launch_then_halves_impl(const GemmArgs& a, int64_t nt, hipStream_t st) {
     if (int rc = prepare_then_halves<DUMP, OUTK>()) return rc;
-    hipLaunchKernelGGL((gemm_tile256_then_halves_kernel<DUMP, OUTK>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
+    launch_kernel((gemm_tile256_then_halves_kernel<DUMP, OUTK>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
     return check_launch("gemm_tile256_then_halves");
 }
 
@@ -633,7 +633,7 @@ static int prepare_then_quadrants() {
 template <bool DUMP, int OUTK, int D>
 static int launch_then_quadrants_impl(const GemmArgs& a, int64_t nt, hipStream_t st) {
     if (int rc = prepare_then_quadrants<DUMP, OUTK, D>()) return rc;
-    hipLaunchKernelGGL((gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
+    launch_kernel((gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
     return check_launch("gemm_tile256_then_quadrants");
 }
 

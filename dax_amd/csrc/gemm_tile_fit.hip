@@ -50,7 +50,7 @@ static int launch_fit_one(const GemmArgs* args, hipStream_t st) {
     a.tiles_n = (a.n + TILE::BN - 1) / TILE::BN;
     const int64_t nt = (int64_t)a.tiles_m * a.tiles_n;
     if (nt > 0x7fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
-    hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(TILE::T), TILE::SMEM, st, a);
+    launch_kernel(kern, dim3((unsigned)nt), dim3(TILE::T), TILE::SMEM, st, a);
     return check_launch("gemm_fit");
 }
 

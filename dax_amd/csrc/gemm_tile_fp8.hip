@@ -388,7 +388,7 @@ static int launch_fp8_impl(const GemmArgs& a, hipStream_t st) {
     if (int rc = prepare_fp8<DUMP, F8, BT, OUTK>()) return rc;
     const int64_t nt = grid_of_order(a);
     if (nt > 0x7fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
-    hipLaunchKernelGGL((gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK>), dim3((unsigned)nt), dim3(f16::T), f16::NPART * BT * f16::BKP, st, a);
+    launch_kernel((gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK>), dim3((unsigned)nt), dim3(f16::T), f16::NPART * BT * f16::BKP, st, a);
     return check_launch("gemm_tile_fp8");
 }
 
@@ -426,8 +426,8 @@ template <bool QUADS, bool DUMP, int F8, int OUTK>
 static int launch_fp8_then_impl(const GemmArgs& a, int64_t nt, hipStream_t st) {
     if (int rc = prepare_fp8_then<QUADS, DUMP, F8, OUTK>()) return rc;
     constexpr int SMEM = f16::NPART * 256 * f16::BKP;
-    if constexpr (QUADS) hipLaunchKernelGGL((gemm_tile_fp8_then_quadrants_kernel<DUMP, F8, OUTK>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
-    else hipLaunchKernelGGL((gemm_tile_fp8_then_halves_kernel<DUMP, F8, OUTK>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
+    if constexpr (QUADS) launch_kernel((gemm_tile_fp8_then_quadrants_kernel<DUMP, F8, OUTK>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
+    else launch_kernel((gemm_tile_fp8_then_halves_kernel<DUMP, F8, OUTK>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
     return check_launch(QUADS ? "gemm_tile_fp8_then_quadrants" : "gemm_tile_fp8_then_halves");
 }
 

@@ -296,7 +296,7 @@ static int launch_cfg(const GemmArgs& a0, hipStream_t st) {
     if (int rc = prepare_cfg<FP8, BM, BN, BK, WM, WN, DIRECT, F8>()) return rc;
     const int64_t nt = (int64_t)a.tiles_m * a.tiles_n;
     if (nt > 0x7fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
-    hipLaunchKernelGGL(kern, dim3((unsigned)nt), dim3(WM * WN * 64), smem, st, a);
+    launch_kernel(kern, dim3((unsigned)nt), dim3(WM * WN * 64), smem, st, a);
     return check_launch("gemm_w8a8");
 }
 

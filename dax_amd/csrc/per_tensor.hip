@@ -92,7 +92,7 @@ int daxq_tensor_scale(const float* row_min, const float* row_max, int64_t m, flo
     using namespace daxq;
     if (m <= 0 || n_expand < 0 || !(qmax > 0.0f) || !(eps >= 0.0f)) return fail(DAXQ_ERR_ARG, "tensor_scale: bad argument m=%lld n_expand=%lld", (long long)m, (long long)n_expand);
     if (!row_min || !row_max || !scale1 || (n_expand > 0 && !expand)) return fail(DAXQ_ERR_ARG, "tensor_scale: null pointer");
-    hipLaunchKernelGGL(tensor_scale_kernel, dim3(1), dim3(kRedThreads), 0, (hipStream_t)stream, row_min, row_max, m, qmax,
+    launch_kernel(tensor_scale_kernel, dim3(1), dim3(kRedThreads), 0, (hipStream_t)stream, row_min, row_max, m, qmax,
                        eps, round_bf16, scale1, expand, n_expand);
     return check_launch("tensor_scale");
 }
@@ -102,7 +102,7 @@ int daxq_tensor_minmax_update(const float* row_min, const float* row_max, int64_
     using namespace daxq;
     if (m <= 0) return fail(DAXQ_ERR_ARG, "tensor_minmax_update: bad argument m=%lld", (long long)m);
     if (!row_min || !row_max || !min_inout || !max_inout) return fail(DAXQ_ERR_ARG, "tensor_minmax_update: null pointer");
-    hipLaunchKernelGGL(tensor_minmax_kernel, dim3(1), dim3(kRedThreads), 0, (hipStream_t)stream, row_min, row_max, m,
+    launch_kernel(tensor_minmax_kernel, dim3(1), dim3(kRedThreads), 0, (hipStream_t)stream, row_min, row_max, m,
                        min_inout, max_inout);
     return check_launch("tensor_minmax_update");
 }
@@ -112,7 +112,7 @@ int daxq_broadcast_f32(const float* src, float* dst, int64_t n, daxq_stream_t st
     if (n < 0) return fail(DAXQ_ERR_ARG, "broadcast_f32: bad argument");
     if (n == 0) return DAXQ_OK;
     if (!src || !dst) return fail(DAXQ_ERR_ARG, "broadcast_f32: null pointer");
-    hipLaunchKernelGGL(broadcast_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, src, dst, n);
+    launch_kernel(broadcast_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, src, dst, n);
     return check_launch("broadcast_f32");
 }
 

@@ -160,8 +160,8 @@ int daxq_block_scale(const void* x, int x_dtype, int nd, const int64_t* view_sha
     const dim3 grid((unsigned)n_kept), block(256);
     hipStream_t st = (hipStream_t)stream;
 #define DAXQ_BS(XT)                                                                                             \
-    if (round_to_x) hipLaunchKernelGGL((block_scale_kernel<XT, true>), grid, block, 0, st, x, v, n_red, qmax, eps, scale); \
-    else hipLaunchKernelGGL((block_scale_kernel<XT, false>), grid, block, 0, st, x, v, n_red, qmax, eps, scale)
+    if (round_to_x) launch_kernel((block_scale_kernel<XT, true>), grid, block, 0, st, x, v, n_red, qmax, eps, scale); \
+    else launch_kernel((block_scale_kernel<XT, false>), grid, block, 0, st, x, v, n_red, qmax, eps, scale)
     switch (x_dtype) {
         case DAXQ_BF16: DAXQ_BS(DAXQ_BF16); break;
         case DAXQ_F16: DAXQ_BS(DAXQ_F16); break;
@@ -191,9 +191,9 @@ int daxq_block_quantize(const void* x, int x_dtype, int q_fmt, int nd, const int
     uint8_t* qp = static_cast<uint8_t*>(q);
 #define DAXQ_BQ(XT)                                                                                                   \
     switch (q_fmt) {                                                                                                  \
-        case DAXQ_FMT_I8: hipLaunchKernelGGL((block_quantize_kernel<XT, 0>), grid, block, 0, st, x, v, total, scale, qp, sk, ct); break;   \
-        case DAXQ_FMT_E4M3: hipLaunchKernelGGL((block_quantize_kernel<XT, 1>), grid, block, 0, st, x, v, total, scale, qp, sk, ct); break; \
-        case DAXQ_FMT_E5M2: hipLaunchKernelGGL((block_quantize_kernel<XT, 2>), grid, block, 0, st, x, v, total, scale, qp, sk, ct); break; \
+        case DAXQ_FMT_I8: launch_kernel((block_quantize_kernel<XT, 0>), grid, block, 0, st, x, v, total, scale, qp, sk, ct); break;   \
+        case DAXQ_FMT_E4M3: launch_kernel((block_quantize_kernel<XT, 1>), grid, block, 0, st, x, v, total, scale, qp, sk, ct); break; \
+        case DAXQ_FMT_E5M2: launch_kernel((block_quantize_kernel<XT, 2>), grid, block, 0, st, x, v, total, scale, qp, sk, ct); break; \
         default: return fail(DAXQ_ERR_ARG, "block_quantize: unknown quantised format %d", q_fmt);                    \
     }
     switch (x_dtype) {

@@ -256,8 +256,8 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
             const QuantArgs b = rows_from<XB>(a, r, kSlab);                                                                \
             const unsigned groups = (unsigned)((b.m + kRows - 1) / kRows);                                                 \
             const dim3 grid(W > 1 && a.partials ? (groups + 7) / 8 * 8 : groups);                                          \
-            if (plain) hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain>), grid, dim3(256), 0, st, b); \
-            else hipLaunchKernelGGL((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false>), grid, dim3(256), 0, st, b);        \
+            if (plain) launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain>), grid, dim3(256), 0, st, b); \
+            else launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false>), grid, dim3(256), 0, st, b);        \
         }                                                                                                                  \
         return check_launch("quant_rows");                                                                                 \
     }
@@ -280,7 +280,7 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
     }
     if (t.one_scale || t.partials) return fail(DAXQ_ERR_ARG, "quant_rows: one scale for the tensor is taken for rows of at most %d columns", DAXQ_MAX_TENSOR_K);
     if (m > 0x7fffffff) return fail(DAXQ_ERR_ARG, "quant_rows: too many rows");
-    hipLaunchKernelGGL((quant_rows_block<FMT, SCALE_IN, XT>), dim3((unsigned)m), dim3(256), 0, st, x, m, k, ld_x, qp,
+    launch_kernel((quant_rows_block<FMT, SCALE_IN, XT>), dim3((unsigned)m), dim3(256), 0, st, x, m, k, ld_x, qp,
                        ld_q, kfill, scale, qmax, eps, round_x);
     return check_launch("quant_rows_block");
 }
@@ -545,9 +545,9 @@ int daxq_row_minmax_t(const void* x, int x_dtype, int64_t m, int64_t k, int64_t 
     const char* xp = static_cast<const char*>(x);
     auto launch = [&](auto XT) {
         constexpr int X = decltype(XT)::value;
-        if (k <= 2048) hipLaunchKernelGGL((row_minmax_kernel<X, 1>), grid, block, 0, st, xp, k, ld_x, min_out, max_out);
-        else if (k <= 4096 || X == DAXQ_F32) hipLaunchKernelGGL((row_minmax_kernel<X, 2>), grid, block, 0, st, xp, k, ld_x, min_out, max_out);
-        else hipLaunchKernelGGL((row_minmax_kernel<X, 4>), grid, block, 0, st, xp, k, ld_x, min_out, max_out);
+        if (k <= 2048) launch_kernel((row_minmax_kernel<X, 1>), grid, block, 0, st, xp, k, ld_x, min_out, max_out);
+        else if (k <= 4096 || X == DAXQ_F32) launch_kernel((row_minmax_kernel<X, 2>), grid, block, 0, st, xp, k, ld_x, min_out, max_out);
+        else launch_kernel((row_minmax_kernel<X, 4>), grid, block, 0, st, xp, k, ld_x, min_out, max_out);
     };
     switch (x_dtype) {
         case DAXQ_BF16: launch(std::integral_constant<int, DAXQ_BF16>{}); break;
@@ -608,9 +608,9 @@ int daxq_act_quant_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int6
     const AmaxArgs a{static_cast<const char*>(x), m, ld_x, (int)k, quant_unit(x_dtype, fill_width(k, ld_q)), part};
     const dim3 grid(kPartials), block(1024);
     switch (x_dtype) {
-        case DAXQ_BF16: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_BF16>, grid, block, 0, st, a); break;
-        case DAXQ_F16: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_F16>, grid, block, 0, st, a); break;
-        case DAXQ_F32: hipLaunchKernelGGL(tensor_amax_kernel<DAXQ_F32>, grid, block, 0, st, a); break;
+        case DAXQ_BF16: launch_kernel(tensor_amax_kernel<DAXQ_BF16>, grid, block, 0, st, a); break;
+        case DAXQ_F16: launch_kernel(tensor_amax_kernel<DAXQ_F16>, grid, block, 0, st, a); break;
+        case DAXQ_F32: launch_kernel(tensor_amax_kernel<DAXQ_F32>, grid, block, 0, st, a); break;
         default: return fail(DAXQ_ERR_ARG, "act_quant_tensor: unknown element type %d", x_dtype);
     }
     if (int rc = check_launch("tensor_amax")) return rc;
@@ -640,7 +640,7 @@ int daxq_scale_from_minmax_eps(const float* min_in, const float* max_in, int64_t
     if (n < 0 || !(qmax > 0.0f) || eps != eps) return fail(DAXQ_ERR_ARG, "scale_from_minmax: bad argument");
     if (n == 0) return DAXQ_OK;
     if (!min_in || !max_in || !scale) return fail(DAXQ_ERR_ARG, "scale_from_minmax: null pointer");
-    hipLaunchKernelGGL(scale_from_minmax_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+    launch_kernel(scale_from_minmax_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                        min_in, max_in, n, qmax, eps, scale);
     return check_launch("scale_from_minmax");
 }
