@@ -34,6 +34,7 @@ struct QuantArgs {
     int leaf;                 // the scale is a tensor's or a weight's: the leaf quantiser's bytes also where it is not finite
 };
 constexpr int kPartials = 256;  // workgroups of tensor_amax_kernel, one per CU
+constexpr int kTensorQuantPieces = 128;  // pieces of 64 chunks that tensor_quant_kernel has in flight: 8 in each of 16 wavefronts
 
 // W wavefronts share a row (4 / W rows per workgroup), lane l of wavefront w holding chunks (i W + w) 64 + l.  One
 // wavefront per row for short rows, four for long ones: the chunks of a row then arrive in a quarter of the instructions,
@@ -403,6 +404,113 @@ __global__ __launch_bounds__(1024) void tensor_amax_kernel(const AmaxArgs a) {
     }
 }
 
+// Dynamic per-tensor quantisation of a small matrix in one launch: every workgroup finds the abs-max of the whole matrix for
+// itself and quantises one row, which it requested first.
+// What bounds it: latency.  The abs-max launch that it saves costs the host 2.2 us and the GPU a launch that the next one waits
+// for; against that, sixteen wavefronts read the matrix out of their XCD's L2, 64 chunks of a row (a piece) per instruction, all
+// of their U pieces in flight at once.  Forwards, us, GPU alone (back to back), two launches and GEMM -> this and GEMM:
+//   9 x 1536 x 1536 8.3 -> 6.9 e5m2 (11.7 -> 8.5)    40 x 1536 x 1536 8.6 -> 7.8 int8 (12.0 -> 9.0)     64 x 256, N = 1536 7.6 -> 7.0 (12.3 -> 9.0)
+//   12 x 5120 x 5120 10.8 -> 10.3 int8 (12.1 -> 10.4)  21 x 3072 x 3072 9.8 -> 8.8 int8 (12.6 -> 9.1)  40 x 1536 x 1536 fp32 8.2 -> 8.1 (12.5 -> 9.1)
+template <int FMT, int XT>
+__global__ __launch_bounds__(1024) void tensor_quant_kernel(const QuantArgs a) {
+    constexpr int XB = XT == DAXQ_F32 ? 4 : 2, U = kTensorQuantPieces / 16, NCH = (DAXQ_MAX_TENSOR_K / 8 + 1023) / 1024;
+    constexpr uint32_t kAbs = XT == DAXQ_F32 ? 0x7fffffffu : 0x7fffu;
+    typedef daxq_v4u loose __attribute__((aligned(2)));
+    __shared__ uint32_t s_max[16];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nch = a.k >> 3, npad = a.kfill >> 3, rest = a.k & 7, pieces = (nch + 63) >> 6;  // (nch > 0: tensor_quant_applies)
+    const bool ragged = ((a.k | a.kfill) & 7) != 0;  // as in quant_rows_kernel
+    auto element = [&](const char* xr) __attribute__((always_inline)) -> uint32_t {
+        if constexpr (XT == DAXQ_F32) return reinterpret_cast<const uint32_t*>(xr)[nch * 8 + lane];
+        else return reinterpret_cast<const uint16_t*>(xr)[nch * 8 + lane];
+    };
+    const char* xr = a.x + (int64_t)blockIdx.x * a.ld_x * XB;
+    Chunk<XT> v[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int c = i * 1024 + t;
+        if (i * 1024 < nch) load_chunk<XT>(v[i], xr + (uint32_t)(c < nch ? c : nch - 1) * (8u * XB));
+        else v[i] = Chunk<XT>{};
+    }
+    const uint32_t tail = wave == 0 && lane < rest ? element(xr) : 0;
+
+    // the wavefront's pieces: the first, then every sixteenth (pieces <= 36: products with 2^16 / pieces, rounded up, give whole
+    // quotients)
+    const int inv_pieces = (65536 + pieces - 1) / pieces, rows16 = (16 * inv_pieces) >> 16, c16 = 16 - rows16 * pieces;
+    int row = (wave * inv_pieces) >> 16, c = wave - row * pieces;
+    uint32_t mx = 0, tl = 0;
+    Chunk<XT> w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (row < a.m) {
+            const char* wr = a.x + row * a.ld_x * XB;
+            const int at = c * 64 + lane;
+            // (not load_chunk: what its hint evicts the XCD's other workgroups read again; 12 x 5120 fp32 15.1 -> 11.1 us)
+            const loose* wp = reinterpret_cast<const loose*>(wr + (uint32_t)(at < nch ? at : nch - 1) * (8u * XB));
+#pragma unroll
+            for (int h = 0; h < XB / 2; ++h) w[u].w[h] = wp[h];
+            if (c == pieces - 1 && lane < rest) {
+                const uint32_t e = element(wr) & kAbs;
+                tl = e > tl ? e : tl;
+            }
+        } else {
+            w[u] = Chunk<XT>{};
+        }
+        row += rows16, c += c16;
+        if (c >= pieces) c -= pieces, ++row;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) mx = chunk_amax<XT>(mx, w[u]);
+    mx = amax_of_lane<XT>(mx);
+    mx = wave_max_u32(tl > mx ? tl : mx);
+    if (lane == 0) s_max[wave] = mx;
+    __syncthreads();
+    const uint32_t amax = wave_max_u32(s_max[lane & 15]);
+    const float s = scale_from_amax_bits_rt<XT>(amax, a.qmax, a.eps, a.round_x);
+    if (t == 0) {
+        a.scale[blockIdx.x] = s;
+        if (a.scale1 && blockIdx.x == 0) a.scale1[0] = s;
+    }
+    const float inv = 1.0f / s;  // IEEE division, not v_rcp_f32
+    uint8_t* qr = a.q + (int64_t)blockIdx.x * a.ld_q;
+    with_form<FMT, XT>(s, a.qmax, false, a.round_x, 1, [&](auto FORM) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            if (i * 1024 >= npad) continue;
+            const int at = i * 1024 + t;
+            float f[8];
+            chunk_values<XT>(v[i], f);
+            const uint2 o = quant8<FMT, decltype(FORM)::value, XT>(f, s, inv);
+            if (at < nch) store_chunk(qr + (uint32_t)at * 8u, o);
+            else if (!ragged && at < npad) store_chunk(qr + (uint32_t)at * 8u, make_uint2(0, 0));
+        }
+    });
+    if (ragged && wave == 0) {
+        const float f = x_bits_to_f32<XT>(tail);
+        uint8_t o;
+        if constexpr (FMT == 0) o = (uint8_t)q_i8_bits(f, inv);
+        else o = (uint8_t)cvt_pk_f8<FMT>(q_f8_pre<FMT, true>(f, s, inv), 0.0f, 0, false);
+        for (int at = nch * 8 + lane; at < a.kfill; at += 64) qr[at] = at < a.k ? o : 0;
+    }
+}
+
+// Which matrices: those whose pieces are all in flight at once.  With more of them the loads take turns and the GPU loses what the
+// host gains: 17 x 5120 bf16 (170 pieces) 11.7 -> 12.2 us with the GEMM, 64 x 1536 (192) 8.8 -> 9.3, 250 x 256 8.4 -> 9.9.
+static bool tensor_quant_applies(int64_t m, int64_t k) {
+    return k >= 64 && m <= kTensorQuantPieces && m * ((k / 8 + 63) / 64) <= kTensorQuantPieces;
+}
+
+template <int FMT>
+static bool launch_tensor_quant(const QuantArgs& a, int x_dtype, hipStream_t st) {
+    const dim3 grid((unsigned)a.m), block(1024);
+    if (x_dtype == DAXQ_BF16) launch_kernel((tensor_quant_kernel<FMT, DAXQ_BF16>), grid, block, 0, st, a);
+    else if (x_dtype == DAXQ_F16) launch_kernel((tensor_quant_kernel<FMT, DAXQ_F16>), grid, block, 0, st, a);
+    else if (x_dtype == DAXQ_F32) launch_kernel((tensor_quant_kernel<FMT, DAXQ_F32>), grid, block, 0, st, a);
+    else return false;
+    return true;
+}
+
 // Per-row min and max of a bf16 / fp16 / fp32 matrix in fp32 (observer statistics), one workgroup per row, 16-byte loads.
 // The bit patterns are compared as two's-complement integers (magnitude bits of negative values flipped), two 16-bit
 // values per instruction; a NaN sorts beyond either infinity and makes both results NaN.  HBM-bound; measured against two-byte
@@ -604,6 +712,14 @@ int daxq_act_quant_tensor(const void* x, int x_dtype, int q_fmt, int64_t m, int6
     if ((uintptr_t)scratch & 15) return fail(DAXQ_ERR_ALIGN, "act_quant_tensor: the scratch must be 16-byte aligned");
     if ((uintptr_t)x & (x_dtype == DAXQ_F32 ? 3 : 1)) return fail(DAXQ_ERR_ALIGN, "act_quant_tensor: x must be element aligned");
     hipStream_t st = (hipStream_t)stream;
+    if (tensor_quant_applies(m, k) && ((uintptr_t)scale_rows & 3) == 0) {
+        const QuantArgs a{static_cast<const char*>(x), m, ld_x, (int)k, (int)fill_width(k, ld_q), static_cast<uint8_t*>(q), ld_q, scale_rows, nullptr,
+                          0, nullptr, scale1, quant_max, eps, scale_round == DAXQ_SCALE_ROUND_X, 1};
+        if (q_fmt == DAXQ_FMT_I8 ? launch_tensor_quant<0>(a, x_dtype, st)
+                                 : q_fmt == DAXQ_FMT_E4M3 ? launch_tensor_quant<1>(a, x_dtype, st)
+                                                          : q_fmt == DAXQ_FMT_E5M2 && launch_tensor_quant<2>(a, x_dtype, st))
+            return check_launch("tensor_quant");
+    }
     uint32_t* part = static_cast<uint32_t*>(scratch);
     const AmaxArgs a{static_cast<const char*>(x), m, ld_x, (int)k, quant_unit(x_dtype, fill_width(k, ld_q)), part};
     const dim3 grid(kPartials), block(1024);

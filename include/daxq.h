@@ -227,7 +227,8 @@ int daxq_broadcast_f32(const float* src, float* dst, int64_t n, daxq_stream_t st
 /*
  * The same two schemes without the statistics per row, for rows of at most DAXQ_MAX_TENSOR_K columns (any alignment):
  * daxq_act_quant_tensor: dynamic per-tensor quantisation in two passes over x -- the abs-max of the tensor into `scratch`
- *   (1 KiB, 16-byte aligned, contents unspecified before and after), then scale and bytes.  Arguments and arithmetic as for
+ *   (1 KiB, 16-byte aligned, contents unspecified before and after), then scale and bytes.  Matrices of at most 128 pieces of
+ *   512 columns, rows cut one by one, take one launch that leaves `scratch` alone.  Arguments and arithmetic as for
  *   daxq_act_quant_rows_ex with the whole matrix as one row; scale_rows [m] receives the one scale once per row (the vector
  *   the GEMM reads), scale1 [1] once more, or NULL.
  * daxq_quantize_tensor: daxq_quantize_rows with the one scale scale1[0] for every row; scale_rows [m] receives it once per

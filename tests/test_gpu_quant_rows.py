@@ -117,6 +117,36 @@ def test_one_scale_for_the_tensor(ops, dtype, m, k, pitch):
     assert bool(torch.isnan(s).all()) and bool(torch.isnan(s1).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,k,pitch", [(128, 512, 512), (129, 512, 512), (2, 64, 64), (2, 63, 63), (128, 65, 67), (64, 513, 515), (42, 1535, 1537),
+                                       (43, 1536, 1536), (12, 5115, 5121), (13, 5120, 5120), (3, 18432, 18432), (4, 18431, 18433)])
+def test_one_scale_for_a_small_tensor(ops, dtype, m, k, pitch):
+    """On either side of 128 pieces of 512 columns, up to which every workgroup takes the abs-max of the matrix itself: the largest
+    element in the first and last piece of rows, whole chunks and what they leave over; scale, bytes and padding against the
+    oracle's quantiser of the flattened tensor, exactly; an infinity or a NaN in the last element."""
+    g = torch.Generator().manual_seed(m + k)
+    base = torch.randn(m, pitch, generator=g).to(dtype)
+    for n, at in enumerate(((0, 0), (0, k - 1), (m // 2, k // 2), (m - 1, k // 8 * 8 - 1), (m - 1, k - 1))):
+        x = base.clone()
+        x[at] = -9.5
+        x[m - 1, k:] = 100.0  # beyond the rows
+        fmt = ("i8", "e4m3", "e5m2")[n % 3]
+        target = torch.int8 if fmt == "i8" else FP8[fmt]
+        qo, so = O.dynamic_quantize(x[:, :k].reshape(1, -1), (1, m * k), target, ops.QMAX[fmt], ops.EPS_F32, torch.float32)
+        q, s, s1 = ops.act_quant_tensor(x.to("cuda")[:, :k], fmt, ops.QMAX[fmt], ops.EPS_F32, True, True)
+        assert torch.equal(s1.cpu(), so.view(1)) and torch.equal(s.cpu(), so.view(1).expand(m))
+        np.testing.assert_array_equal(_bytes(q[:, :k]), _bytes(qo).reshape(m, k))
+        assert q.shape[1] == ops.pad_k(k) and not q[:, k:].any()
+    for bad in (float("inf"), float("nan")):
+        x[m - 1, k - 1] = bad
+        for fmt in ("i8", "e4m3"):
+            q, s, s1 = ops.act_quant_tensor(x.to("cuda")[:, :k], fmt, ops.QMAX[fmt], ops.EPS_F32, True, True)
+            ref = O.quantize_to_int8 if fmt == "i8" else lambda t, sc: O.quantize_to_fp8(t, sc, FP8["e4m3"])
+            assert not bool(torch.isfinite(s).any()) and not bool(torch.isfinite(s1).any())
+            if bad == float("inf"):
+                np.testing.assert_array_equal(_bytes(q[:, :k])[:-1], _bytes(ref(x[:-1, :k].contiguous(), s1.cpu())))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
 def test_every_element_under_scales_near_short_significands(ops, dtype, fmt):
