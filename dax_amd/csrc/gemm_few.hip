@@ -3,7 +3,7 @@
 //
 // What bounds it: the launches.  The quantiser and the GEMM of such a call take 2 and 3 to 7 us, their launches cost the host 2.8 to
 // 3.6 us each (a per-tensor scale is a third one), and the second one starts when the first has ended and drained.  The quantised rows
-// are few (m x K <= 20 KB), so that quantising them once per workgroup costs about what waiting for the weight does anyway.
+// are few (m x K <= 40 KB), so that quantising them once per workgroup costs about what waiting for the weight does anyway.
 // Forwards back to back, us, separate launches -> this: 1 x 1536 x 1536 8.2 -> 5.5, 4 x 1536 x 1536 e5m2 under a per-tensor scale
 // 10.9 -> 5.7, 1 x 5120 x 5120 e4m3 8.2 -> 7.9 (its kernel).
 //
@@ -32,19 +32,21 @@ struct FewArgs {
 enum { kFewToken = 0, kFewTensor = 1, kFewStatic = 2 };
 
 constexpr int kFewWaves = 8;
-constexpr int kFewMaxK = 16384, kFewMaxBytes = 20480;  // columns; quantised bytes in LDS, rows counted as they are dealt out
+// columns; quantised bytes in LDS, rows counted as they are dealt out.  WIDE: twice as many, in kernels of their own (the longer
+// code of more chunks per lane costs the smaller calls 0.25 us)
+constexpr int kFewMaxK = 16384, kFewMaxBytes = 20480, kFewWideBytes = 40960;
 // chunks of 8 elements per lane: 8 / rows wavefronts share a row of what those bytes leave it
-constexpr int few_chunks(int rows) {
-    return ((rows > 1 ? kFewMaxBytes : kFewMaxK) + kFewWaves * 512 - 1) / (kFewWaves * 512);
+constexpr int few_chunks(int rows, bool wide) {
+    return ((rows == 1 ? kFewMaxK : wide ? kFewWideBytes : kFewMaxBytes) + kFewWaves * 512 - 1) / (kFewWaves * 512);
 }
 
 // MR: rows the wavefronts are dealt to (1, 2, 4, 8).  ONE: one scale for the tensor (dynamic or the caller's) instead of one per row
-template <bool FP8, int F8, int XT, bool ONE, int MR, int CG, int KS, int R>
+template <bool FP8, int F8, int XT, bool ONE, int MR, bool WIDE, int CG, int KS, int R>
 __global__ __launch_bounds__(64 * kFewWaves) void gemm_few_kernel(const FewArgs a) {
     typedef typename Acc16<FP8>::type acc_t;
     constexpr int XB = XT == DAXQ_F32 ? 4 : 2, OUTK = XT, FMT = !FP8 ? 0 : (F8 & kF8XE5) ? 2 : 1;
     constexpr float kMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
-    constexpr int NCH = few_chunks(MR), WPR = kFewWaves / MR;  // wavefronts per row
+    constexpr int NCH = few_chunks(MR, WIDE), WPR = kFewWaves / MR;  // wavefronts per row
     constexpr int STEP = 2048, L = 2;  // LDS of a step: 16 weight rows of 128 bytes, two load instructions
     static_assert(CG * KS <= kFewWaves && R * L < 64, "wavefronts, load counter");
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -65,7 +67,7 @@ __global__ __launch_bounds__(64 * kFewWaves) void gemm_few_kernel(const FewArgs 
     for (int i = 0; i < NCH; ++i) {
         if (i * WPR * 64 < nch) {
             const int c = (i * WPR + rpart) * 64 + lane;
-            load_chunk<XT>(v[i], xrow + (uint32_t)(c < nch ? c : nch - 1) * (8u * XB));
+            load_chunk_shared<XT>(v[i], xrow + (uint32_t)(c < nch ? c : nch - 1) * (8u * XB));
         }
     }
     // ---- the weight's first steps (gemm_rows.hip)
@@ -215,12 +217,12 @@ __global__ __launch_bounds__(64 * kFewWaves) void gemm_few_kernel(const FewArgs 
 }
 
 // args null: only raises the kernel's LDS limit on the current device
-template <bool FP8, int F8, int XT, bool ONE, int MR>
+template <bool FP8, int F8, int XT, bool ONE, int MR, bool WIDE = false>
 static int launch_few_one(const FewArgs* a, hipStream_t st) {
     constexpr int CG = 2, KS = FP8 ? 1 : 4, R = FP8 ? 10 : 4;  // (rings of 15 and 20 steps: 0 to 3 % slower, a CU then has room for fewer workgroups)
-    auto kern = gemm_few_kernel<FP8, F8, XT, ONE, MR, CG, KS, R>;
+    auto kern = gemm_few_kernel<FP8, F8, XT, ONE, MR, WIDE, CG, KS, R>;
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    constexpr int ring = CG * KS * R * 2048, most = ring + kFewMaxBytes + MR * 16 + (kFewWaves + MR) * 4;
+    constexpr int ring = CG * KS * R * 2048, most = ring + (WIDE ? kFewWideBytes : kFewMaxBytes) + MR * 16 + (kFewWaves + MR) * 4;
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), most, lds_set)) return rc;
     if (!a) return DAXQ_OK;
     const int lds = ring + MR * (a->g.k + 16) + (kFewWaves + MR) * 4;
@@ -229,7 +231,8 @@ static int launch_few_one(const FewArgs* a, hipStream_t st) {
 }
 
 template <bool FP8, int F8, int XT, bool ONE>
-static int launch_few_rows(const FewArgs* a, int m, hipStream_t st) {
+static int launch_few_rows(const FewArgs* a, int m, bool wide, hipStream_t st) {
+    if (wide) return m <= 4 ? launch_few_one<FP8, F8, XT, ONE, 4, true>(a, st) : launch_few_one<FP8, F8, XT, ONE, 8, true>(a, st);
     if (m <= 1) return launch_few_one<FP8, F8, XT, ONE, 1>(a, st);
     if (m <= 2) return launch_few_one<FP8, F8, XT, ONE, 2>(a, st);
     if (m <= 4) return launch_few_one<FP8, F8, XT, ONE, 4>(a, st);
@@ -237,26 +240,31 @@ static int launch_few_rows(const FewArgs* a, int m, hipStream_t st) {
 }
 
 template <bool ONE>
-static int launch_few(const FewArgs* a, int m, int x_fmt, int x_dtype, hipStream_t st) {
-    if (x_fmt == DAXQ_FMT_E4M3) return launch_few_rows<true, 0, DAXQ_BF16, ONE>(a, m, st);
-    if (x_fmt == DAXQ_FMT_E5M2) return launch_few_rows<true, kF8XE5, DAXQ_BF16, ONE>(a, m, st);
-    if (x_dtype == DAXQ_F16) return launch_few_rows<false, 0, DAXQ_F16, ONE>(a, m, st);
-    if (x_dtype == DAXQ_F32) return launch_few_rows<false, 0, DAXQ_F32, ONE>(a, m, st);
-    return launch_few_rows<false, 0, DAXQ_BF16, ONE>(a, m, st);
+static int launch_few(const FewArgs* a, int m, bool wide, int x_fmt, int x_dtype, hipStream_t st) {
+    if (x_fmt == DAXQ_FMT_E4M3) return launch_few_rows<true, 0, DAXQ_BF16, ONE>(a, m, wide, st);
+    if (x_fmt == DAXQ_FMT_E5M2) return launch_few_rows<true, kF8XE5, DAXQ_BF16, ONE>(a, m, wide, st);
+    if (x_dtype == DAXQ_F16) return launch_few_rows<false, 0, DAXQ_F16, ONE>(a, m, wide, st);
+    if (x_dtype == DAXQ_F32) return launch_few_rows<false, 0, DAXQ_F32, ONE>(a, m, wide, st);
+    return launch_few_rows<false, 0, DAXQ_BF16, ONE>(a, m, wide, st);
 }
 
 int prepare_few_kernels() {
     int rc = 0;
-    auto prepare = [&](int m, int fmt, int x) {
-        if (!rc) rc = launch_few<false>(nullptr, m, fmt, x, nullptr);
-        if (!rc) rc = launch_few<true>(nullptr, m, fmt, x, nullptr);
+    auto prepare = [&](int m, bool wide, int fmt, int x) {
+        if (!rc) rc = launch_few<false>(nullptr, m, wide, fmt, x, nullptr);
+        if (!rc) rc = launch_few<true>(nullptr, m, wide, fmt, x, nullptr);
     };
-    for (int m : {1, 2, 4, 8}) {
-        for (int x : {DAXQ_BF16, DAXQ_F16, DAXQ_F32}) prepare(m, DAXQ_FMT_I8, x);
-        for (int f : {DAXQ_FMT_E4M3, DAXQ_FMT_E5M2}) prepare(m, f, DAXQ_BF16);
-    }
+    for (int m : {1, 2, 4, 8})
+        for (bool wide : {false, true}) {
+            if (wide && m < 4) continue;
+            for (int x : {DAXQ_BF16, DAXQ_F16, DAXQ_F32}) prepare(m, wide, DAXQ_FMT_I8, x);
+            for (int f : {DAXQ_FMT_E4M3, DAXQ_FMT_E5M2}) prepare(m, wide, f, DAXQ_BF16);
+        }
     return rc;
 }
+
+// rows as the wavefronts are dealt to them
+static inline int64_t few_dealt(int64_t m) { return m <= 2 ? m : m <= 4 ? 4 : 8; }
 
 }  // namespace daxq
 
@@ -271,14 +279,21 @@ int daxq_linear_few_applies(int x_dtype, int x_fmt, int w_fmt, int out_dtype, in
     const bool f8 = (x_fmt == DAXQ_FMT_E4M3 || x_fmt == DAXQ_FMT_E5M2) && w_fmt == DAXQ_FMT_E4M3 && x_dtype == DAXQ_BF16;
     if ((!i8 && !f8) || x_dtype != out_dtype || x_dtype < DAXQ_BF16 || x_dtype > DAXQ_F32) return 0;
     if (m < 1 || m > 8 || k < 8 || k % 8 || k > kFewMaxK || n < (f8 ? 128 : 1) || n > (1 << 20)) return 0;
-    // What it costs to quantise in every workgroup grows with rows x K, what it saves does not.  us on the GPU, separate launches / one
-    // (a forward of separate launches takes the host 8.2 besides, one of a single launch 5.5), INT8; e4m3:
-    //   8 x 1536, K = 1536 5.2 / 4.2; 5.9 / 5.2     2 x 5120 x 5120 9.3 / 8.1; 9.3 / 8.4      1 x 1536 x 1536 4.8 / 3.6; 5.4 / 3.8
-    //   8 x 15360, K = 1536 8.8 / 8.5; 9.0 / 8.6    4 x 5120 x 5120 9.5 / 9.1; 9.4 / 9.5      1 x 15360, K = 13824 42.6 / 39.8; 42.7 / 40.4
-    //   8 x 5120 x 5120 9.7 / 10.6; 9.6 / 11.2      4 x 15360, K = 5120 16.1 / 18.7; 16.1 / 15.4  1 x 1536, K = 13824 9.4 / 9.8; 14.1 / 12.5
-    //   3 x 15360, K = 10240 33.2 / 36.5; 33.3 / 37.4   4 x 1536, K = 5120 6.2 / 5.7 to 7.0; 8.0 / 8.5
-    const int64_t kp = (k + DAXQ_K_ALIGN - 1) / DAXQ_K_ALIGN * DAXQ_K_ALIGN, rows = m <= 2 ? m : m <= 4 ? 4 : 8;
-    return rows * kp <= 12288 || (rows * kp <= kFewMaxBytes && n >= 4096 && (m == 1 || n <= 8192));
+    // What it costs to quantise in every workgroup grows with rows x K, what it saves does not: more of it is taken where a launch
+    // has a workgroup for most CUs (N from 4096) and all of them run at once (to 8192; fp8, whose rings are smaller, two to a CU).
+    // Below 4096 columns the other kernels cut a long K of int8 over more wavefronts than this one.  us per call on the GPU, weights
+    // out of reach of the caches, separate launches / one, INT8; e4m3; e5m2 under a per-tensor scale (two launches or this):
+    //   5 x 1536, K = 3072 6.1 / 5.8; 7.0 / 6.1; 8.0 / 6.6      4 x 5120, K = 8960 14.8 / 13.8; 14.9 / 14.0; 16.0 / 13.9   8 x 15360, K = 2048 10.8 / 12.1; 10.8 / 8.7; 11.8 / 9.4
+    //   3 x 1536, K = 5120 7.7 / 8.1; 8.4 / 8.2; 9.4 / 8.1      8 x 4096 x 4096 8.8 / 8.4; 8.8 / 8.8; 10.2 / 9.3           3 x 13824, K = 5120 19.0 / 19.4; 19.1 / 16.0; 20.0 / 15.9
+    //   2 x 1536, K = 8192 8.8 / 9.3; 10.5 / 9.5; 11.5 / 9.6    8 x 5120 x 5120 11.1 / 10.4; 11.3 / 10.2; 12.4 / 10.9      2 x 13824, K = 8192 27.1 / 25.2; 27.1 / 25.9; 28.0 / 26.2
+    //   1 x 1536, K = 13824 11.7 / 13.3; 14.7 / 13.1; 15.1 / 13.2  3 x 8192, K = 5120 12.2 / 11.7; 12.4 / 11.8; 12.3 / 11.8  8 x 13824, K = 5120 19.5 / 21.8; 19.5 / 22.2; 20.7 / 22.9
+    //   8 x 1536, K = 5120 8.2 / 9.2; 8.6 / 9.1; 9.9 / 9.6      8 x 8192, K = 4608 12.4 / 11.9; 12.1 / 11.6; 13.3 / 11.9
+    // (forwards back to back besides save what the host takes for a launch: 5 x 1536, K = 3072 9.1 -> 6.0, 8 x 5120 x 5120 11.0 -> 10.1.)
+    const int64_t kp = (k + DAXQ_K_ALIGN - 1) / DAXQ_K_ALIGN * DAXQ_K_ALIGN, bytes = few_dealt(m) * kp;
+    if (bytes <= 12288) return 1;
+    if (n < 4096) return bytes <= (m > 2 ? 24576 : kFewMaxBytes) && (f8 || kp <= 4096);
+    if (n <= 8192) return bytes <= (m > 2 ? kFewWideBytes : kFewMaxBytes);
+    return bytes <= kFewMaxBytes && (f8 || m <= 2);
 }
 
 int daxq_linear_few(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme, int act_scale_round, const void* x, int64_t ld_x,
@@ -314,8 +329,9 @@ int daxq_linear_few(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme
     a.kx = (int)k;
     a.round_x = act_scale_round == DAXQ_SCALE_ROUND_X;
     a.scheme = scheme;
-    if (scheme == kFewToken) return launch_few<false>(&a, (int)m, x_fmt, x_dtype, (hipStream_t)stream);
-    return launch_few<true>(&a, (int)m, x_fmt, x_dtype, (hipStream_t)stream);
+    const bool wide = m > 2 && few_dealt(m) * kp > kFewMaxBytes;
+    if (scheme == kFewToken) return launch_few<false>(&a, (int)m, wide, x_fmt, x_dtype, (hipStream_t)stream);
+    return launch_few<true>(&a, (int)m, wide, x_fmt, x_dtype, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -234,6 +234,14 @@ __device__ __forceinline__ void load_chunk(Chunk<XT>& v, const char* p) {
     for (int h = 0; h < (XT == DAXQ_F32 ? 2 : 1); ++h) v.w[h] = __builtin_nontemporal_load(reinterpret_cast<const loose*>(p) + h);
 }
 
+// for what other workgroups of the XCD read, too: the hint above would evict it from the L2 that they share
+template <int XT>
+__device__ __forceinline__ void load_chunk_shared(Chunk<XT>& v, const char* p) {
+    typedef daxq_v4u loose __attribute__((aligned(2)));
+#pragma unroll
+    for (int h = 0; h < (XT == DAXQ_F32 ? 2 : 1); ++h) v.w[h] = reinterpret_cast<const loose*>(p)[h];
+}
+
 __device__ __forceinline__ void store_chunk(uint8_t* p, uint2 v) {
     typedef daxq_v2u loose __attribute__((aligned(1)));
     const daxq_v2u t = {v.x, v.y};

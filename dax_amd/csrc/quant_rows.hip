@@ -415,7 +415,6 @@ template <int FMT, int XT>
 __global__ __launch_bounds__(1024) void tensor_quant_kernel(const QuantArgs a) {
     constexpr int XB = XT == DAXQ_F32 ? 4 : 2, U = kTensorQuantPieces / 16, NCH = (DAXQ_MAX_TENSOR_K / 8 + 1023) / 1024;
     constexpr uint32_t kAbs = XT == DAXQ_F32 ? 0x7fffffffu : 0x7fffu;
-    typedef daxq_v4u loose __attribute__((aligned(2)));
     __shared__ uint32_t s_max[16];
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -446,10 +445,8 @@ __global__ __launch_bounds__(1024) void tensor_quant_kernel(const QuantArgs a) {
         if (row < a.m) {
             const char* wr = a.x + row * a.ld_x * XB;
             const int at = c * 64 + lane;
-            // (not load_chunk: what its hint evicts the XCD's other workgroups read again; 12 x 5120 fp32 15.1 -> 11.1 us)
-            const loose* wp = reinterpret_cast<const loose*>(wr + (uint32_t)(at < nch ? at : nch - 1) * (8u * XB));
-#pragma unroll
-            for (int h = 0; h < XB / 2; ++h) w[u].w[h] = wp[h];
+            // (load_chunk instead: 12 x 5120 fp32 11.1 -> 15.1 us)
+            load_chunk_shared<XT>(w[u], wr + (uint32_t)(at < nch ? at : nch - 1) * (8u * XB));
             if (c == pieces - 1 && lane < rest) {
                 const uint32_t e = element(wr) & kAbs;
                 tl = e > tl ? e : tl;

@@ -74,7 +74,8 @@ def test_outputs_are_the_bits_of_the_separate_launches(fmt, dtype, scheme):
     against the 32 columns of a workgroup; rows at a distance; no bias."""
     for m in range(1, 9):
         rows = m if m <= 2 else 4 if m <= 4 else 8
-        for n, k in ((130, 8), (1000, 520), (257, 1536), (128, 12288 // rows), (4100, min(20480 // rows, 16384))):
+        wide = ((4097, 20488 // rows // 8 * 8), (4100, 40960 // rows - 8), (4100, 40960 // rows), (1000, 24576 // 8)) if m > 2 else ()
+        for n, k in ((130, 8), (1000, 520), (257, 1536), (128, 12288 // rows), (4100, min(20480 // rows, 16384)), *wide):
             got, want, _ = _case(fmt, dtype, scheme, m, n, k, pad=8 * (m % 3), bias=m % 4 != 3)
             assert torch.equal(got, want), (m, n, k)
 
@@ -103,9 +104,12 @@ def test_calls_that_are_not_taken():
     L = _capi.lib()
     takes = L.daxq_linear_few_applies
     assert takes(0, 0, 0, 0, 0, 1, 8, 1, 1536) == 1 and takes(0, 0, 0, 0, 0, 1, 8, 4096, 2560) == 1 and takes(0, 0, 0, 0, 0, 1, 1, 1, 8) == 1
-    assert takes(0, 0, 0, 0, 0, 1, 8, 4095, 1544) == 0 and takes(0, 0, 0, 0, 0, 1, 8, 8193, 1544) == 0
+    # int8 beyond 12 KB of rows: of at most 4096 columns against few outputs, at most two rows against many
+    assert takes(0, 0, 0, 0, 0, 1, 8, 4095, 3072) == 1 and takes(0, 0, 0, 0, 0, 1, 8, 4095, 3080) == 0 and takes(0, 0, 0, 0, 0, 1, 3, 4095, 4104) == 0
+    assert takes(0, 0, 0, 0, 0, 1, 8, 8192, 5120) == 1 and takes(0, 0, 0, 0, 0, 1, 8, 8193, 1544) == 0 and takes(0, 0, 0, 0, 0, 1, 2, 8193, 10240) == 1
+    assert takes(0, 1, 1, 0, 0, 1, 3, 4095, 6144) == 1 and takes(0, 1, 1, 0, 0, 1, 8, 8193, 2560) == 1 and takes(0, 1, 1, 0, 0, 1, 2, 4095, 10248) == 0
     for bad in ((0, 0, 0, 0, 0, 1, 9, 1536, 1536), (0, 0, 0, 0, 0, 1, 0, 1536, 1536), (0, 0, 0, 0, 0, 1, 1, 1536, 1540),
-                (0, 0, 0, 0, 0, 1, 1, 8192, 16392), (0, 0, 0, 0, 0, 1, 5, 4096, 2568), (0, 0, 0, 1, 0, 1, 1, 1536, 1536),
+                (0, 0, 0, 0, 0, 1, 1, 8192, 16392), (0, 0, 0, 0, 0, 1, 5, 4096, 5128), (0, 0, 0, 1, 0, 1, 1, 1536, 1536),
                 (1, 1, 1, 1, 0, 1, 1, 1536, 1536), (0, 1, 2, 0, 0, 1, 1, 1536, 1536), (0, 1, 1, 0, 0, 1, 1, 127, 1536),
                 (0, 1, 1, 0, 0, 0, 1, 1536, 1536), (0, 0, 1, 0, 0, 1, 1, 1536, 1536), (0, 0, 0, 0, 3, 1, 1, 1536, 1536)):
         assert takes(*bad) == 0, bad
