@@ -319,6 +319,9 @@ static int launch_quant_rows_fmt(int q_fmt, const void* x, int x_dtype, int64_t 
 // which run on the same XCD, and the quantiser begins with the rows that were read last, out of that XCD's L2.  Both launches, us,
 // matrix read as it lies -> this (bf16, e5m2): 4096 x 5120 21.3 -> 19.9, 4725 x 13824 55.2 -> 53.8, 12000 x 4608 46.2 -> 44.6, 1000 x 8960
 // 12.2 -> 10.8, 300 x 5120 6.7 -> 6.5; shorter rows lose what they gain to the row arithmetic (16000 x 1536 23.7 -> 24.9).
+// The loads carry no hint for data that is read once (load_chunk), which would evict what the quantiser reads next, bf16; fp32:
+// 4096 x 5120 20.0 -> 17.2; 36.0 -> 28.6, 4725 x 13824 53.2 -> 48.8; 103.6 -> 86.7, 12000 x 4608 45.6 -> 41.8; 88.5 -> 72.0, 16000 x 1536
+// 24.4 -> 22.5; 42.7 -> 35.5, 500 x 1536 6.3 -> 5.8; 6.3 -> 6.3, 4096 x 1536 9.7 -> 9.8; 14.7 -> 13.1, 12000 x 15360 143 -> 140; 283 -> 265.
 struct AmaxArgs {
     const char* x;
     int64_t m, ld_x;
@@ -359,7 +362,7 @@ __global__ __launch_bounds__(1024) void tensor_amax_kernel(const AmaxArgs a) {
                 if (row + in < rows) {
                     const char* xr = a.x + (row + in) * a.ld_x * XB;
                     const int at = c * 64 + lane;
-                    load_chunk<XT>(v[u], xr + (uint32_t)(at < nch ? at : nch - 1) * (8u * XB));
+                    load_chunk_shared<XT>(v[u], xr + (uint32_t)(at < nch ? at : nch - 1) * (8u * XB));
                     if (c == pieces - 1 && lane < (a.k & 7)) element(xr, nch * 8 + lane);
                 } else {
                     v[u] = Chunk<XT>{};
@@ -385,7 +388,7 @@ __global__ __launch_bounds__(1024) void tensor_amax_kernel(const AmaxArgs a) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const int64_t cu = c + u * step;
-                    load_chunk<XT>(v[u], xr + (cu < nch ? cu : c) * (8 * XB));  // (beyond the end: the lane's first chunk again)
+                    load_chunk_shared<XT>(v[u], xr + (cu < nch ? cu : c) * (8 * XB));  // (beyond the end: the lane's first chunk again)
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) mx = chunk_amax<XT>(mx, v[u]);
@@ -445,7 +448,7 @@ __global__ __launch_bounds__(1024) void tensor_quant_kernel(const QuantArgs a) {
         if (row < a.m) {
             const char* wr = a.x + row * a.ld_x * XB;
             const int at = c * 64 + lane;
-            // (load_chunk instead: 12 x 5120 fp32 11.1 -> 15.1 us)
+            // (with load_chunk: 12 x 5120 fp32 11.1 -> 15.1 us)
             load_chunk_shared<XT>(w[u], wr + (uint32_t)(at < nch ? at : nch - 1) * (8u * XB));
             if (c == pieces - 1 && lane < rest) {
                 const uint32_t e = element(wr) & kAbs;
