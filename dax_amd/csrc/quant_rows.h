@@ -207,8 +207,8 @@ __device__ __forceinline__ uint32_t chunk_absmax(uint32_t mx, const uint4& v) {
 }
 
 // Streaming accesses of the row kernels: the bf16 row is read once and the quantised row is written once, so both
-// go past the caches with the non-temporal hint (measured: the per-token quantiser runs 6 - 11 % faster, the GEMM
-// that reads the result afterwards is unchanged).
+// go past the caches with the non-temporal hint (measured at 75600 rows: the per-token quantiser runs 6 - 11 % faster, the GEMM
+// that reads the result afterwards is unchanged; store_chunk and quant_rows.hip for bytes that the caches hold).
 typedef unsigned daxq_v4u __attribute__((ext_vector_type(4)));
 typedef unsigned daxq_v2u __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint4 load_stream_16(const uint4* p) {
@@ -242,10 +242,13 @@ __device__ __forceinline__ void load_chunk_shared(Chunk<XT>& v, const char* p) {
     for (int h = 0; h < (XT == DAXQ_F32 ? 2 : 1); ++h) v.w[h] = reinterpret_cast<const loose*>(p)[h];
 }
 
+// KEEP: an ordinary store, whose bytes the GEMM behind the quantiser finds in the caches; else past them
+template <bool KEEP>
 __device__ __forceinline__ void store_chunk(uint8_t* p, uint2 v) {
     typedef daxq_v2u loose __attribute__((aligned(1)));
     const daxq_v2u t = {v.x, v.y};
-    __builtin_nontemporal_store(t, reinterpret_cast<loose*>(p));
+    if constexpr (KEEP) *reinterpret_cast<loose*>(p) = t;
+    else __builtin_nontemporal_store(t, reinterpret_cast<loose*>(p));
 }
 
 // running abs-max of chunks: packed 16-bit magnitudes or 32-bit ones

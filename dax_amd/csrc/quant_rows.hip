@@ -49,7 +49,8 @@ constexpr int kTensorQuantPieces = 128;  // pieces of 64 chunks that tensor_quan
 // stores then sit in one straight piece of code; with the other forms' branches between them a wavefront issues later, which
 // short rows feel most.  us, all forms in one / PLAIN, INT8 (e4m3): 32760 x 1536 26.0 / 24.3 (26.2 / 24.5), 4096 x 2048 6.2 / 6.0
 // (6.3 / 6.2), 9450 x 5120 24.2 / 23.4 (24.4 / 23.8), 516 x 5120 3.4 / 3.2 (3.6 / 3.4); none of eighteen slower.
-template <int NCH, int W, int FMT, bool SCALE_IN, int XT, bool PLAIN>
+// KEEP: the bytes stay in the caches (kKeepBytes)
+template <int NCH, int W, int FMT, bool SCALE_IN, int XT, bool PLAIN, bool KEEP>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
     constexpr int XB = XT == DAXQ_F32 ? 4 : 2;
     __shared__ uint32_t s_max[4];
@@ -128,8 +129,8 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
             float f[8];
             chunk_values<XT>(v[i], f);
             const uint2 o = quant8<FMT, F, XT>(f, s, inv);
-            if (c < nch) store_chunk(qr + (uint32_t)c * 8u, o);
-            else if (!ragged && c < npad) store_chunk(qr + (uint32_t)c * 8u, make_uint2(0, 0));
+            if (c < nch) store_chunk<KEEP>(qr + (uint32_t)c * 8u, o);
+            else if (!ragged && c < npad) store_chunk<KEEP>(qr + (uint32_t)c * 8u, make_uint2(0, 0));
         }
     };
     if constexpr (PLAIN) store(std::integral_constant<int, kOwn>{});
@@ -209,6 +210,13 @@ struct ScaleKind {
     bool weight = false;                 // rows of a weight: the leaf quantiser's bytes also under a scale that is not finite
 };
 
+// Activations of at most this many quantised bytes are stored where the GEMM finds them again, in the caches (the Infinity Cache
+// holds 256 MB), larger ones past them.  Forwards, us, past the caches -> kept: 512 x 5120 x 5120 25.5 -> 22.4, 4096 x 1536 x 1536
+// 21.9 -> 19.8, 2900 x 1000 x 3080 fp16 20.4 -> 19.7, 4725 x 5120 x 5120 static e4m3 104.8 -> 102.6, 32760 x 4608, K = 1536 238.6 -> 229.9,
+// 75600 x 5120 x 5120 e4m3 1498 -> 1505; converting a weight of 13824 x 5120 37.0 -> 38.3.  (The rows' own loads without the hint as
+// well: 512 x 5120 22.2, 4096 x 1536 19.6, but 4725 x 5120 105.2 and 32760 x 1536 234.8.)
+constexpr int64_t kKeepBytes = (int64_t)128 << 20;
+
 // Rows that a workgroup of quant_rows_kernel takes where a row has more than one wavefront (the instantiations that
 // launch_quant_rows_t goes through), else 0.
 static int quant_unit(int x_dtype, int64_t kfill) {
@@ -249,6 +257,8 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
         constexpr bool kMayBePlain = !SCALE_IN && XT == DAXQ_BF16;
         constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
         const bool plain = kMayBePlain && ((k | kfill) & 7) == 0 && !a.leaf && qmax <= kFmtMax && (FMT == 0 || round_x);
+        // (the rows of a weight, and those under a scale each from the caller, have no GEMM behind them)
+        const bool keep = m * kfill <= kKeepBytes && !t.weight && (!SCALE_IN || t.one_scale);
         // A launch holds fewer than 2^32 work items, i.e. 2^24 workgroups: more rows are as many launches as they need
 #define DAXQ_Q_CASE(N, W)                                                                                                  \
     if (cols <= N * W) {                                                                                                   \
@@ -257,8 +267,10 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
             const QuantArgs b = rows_from<XB>(a, r, kSlab);                                                                \
             const unsigned groups = (unsigned)((b.m + kRows - 1) / kRows);                                                 \
             const dim3 grid(W > 1 && a.partials ? (groups + 7) / 8 * 8 : groups);                                          \
-            if (plain) launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain>), grid, dim3(256), 0, st, b); \
-            else launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false>), grid, dim3(256), 0, st, b);        \
+            if (plain && keep) launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain, true>), grid, dim3(256), 0, st, b); \
+            else if (plain) launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain, false>), grid, dim3(256), 0, st, b); \
+            else if (keep) launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false, true>), grid, dim3(256), 0, st, b); \
+            else launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false, false>), grid, dim3(256), 0, st, b);        \
         }                                                                                                                  \
         return check_launch("quant_rows");                                                                                 \
     }
@@ -482,8 +494,8 @@ __global__ __launch_bounds__(1024) void tensor_quant_kernel(const QuantArgs a) {
             float f[8];
             chunk_values<XT>(v[i], f);
             const uint2 o = quant8<FMT, decltype(FORM)::value, XT>(f, s, inv);
-            if (at < nch) store_chunk(qr + (uint32_t)at * 8u, o);
-            else if (!ragged && at < npad) store_chunk(qr + (uint32_t)at * 8u, make_uint2(0, 0));
+            if (at < nch) store_chunk<true>(qr + (uint32_t)at * 8u, o);
+            else if (!ragged && at < npad) store_chunk<true>(qr + (uint32_t)at * 8u, make_uint2(0, 0));
         }
     });
     if (ragged && wave == 0) {
