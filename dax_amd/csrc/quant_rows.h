@@ -242,12 +242,15 @@ __device__ __forceinline__ void load_chunk_shared(Chunk<XT>& v, const char* p) {
     for (int h = 0; h < (XT == DAXQ_F32 ? 2 : 1); ++h) v.w[h] = reinterpret_cast<const loose*>(p)[h];
 }
 
-// KEEP: an ordinary store, whose bytes the GEMM behind the quantiser finds in the caches; else past them
-template <bool KEEP>
+// Where the stored bytes go: past the caches (non-temporal), into them for the GEMM behind the quantiser, or into them and through
+// the L2 to memory at once (a device-coherent store; p is a multiple of 8 then)
+enum { kStorePast = 0, kStoreKeep = 1, kStoreThrough = 2 };
+template <int STORE>
 __device__ __forceinline__ void store_chunk(uint8_t* p, uint2 v) {
     typedef daxq_v2u loose __attribute__((aligned(1)));
     const daxq_v2u t = {v.x, v.y};
-    if constexpr (KEEP) *reinterpret_cast<loose*>(p) = t;
+    if constexpr (STORE == kStoreThrough) __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else if constexpr (STORE == kStoreKeep) *reinterpret_cast<loose*>(p) = t;
     else __builtin_nontemporal_store(t, reinterpret_cast<loose*>(p));
 }
 

@@ -36,6 +36,12 @@ struct QuantArgs {
 constexpr int kPartials = 256;  // workgroups of tensor_amax_kernel, one per CU
 constexpr int kTensorQuantPieces = 128;  // pieces of 64 chunks that tensor_quant_kernel has in flight: 8 in each of 16 wavefronts
 
+// Workgroup b of n as its XCD's (b mod 8) next one of a contiguous range
+__device__ __forceinline__ uint32_t xcd_range(uint32_t b, uint32_t n) {
+    const uint32_t x = b & 7, q = n >> 3, r = n & 7;
+    return x * q + (x < r ? x : r) + (b >> 3);
+}
+
 // W wavefronts share a row (4 / W rows per workgroup), lane l of wavefront w holding chunks (i W + w) 64 + l.  One
 // wavefront per row for short rows, four for long ones: the chunks of a row then arrive in a quarter of the instructions,
 // which is what a launch of few rows waits for (512 x 5120: 4.1 -> 3.0 us, 17 x 5120 3.5 -> 2.4 us; a wavefront alone on
@@ -49,15 +55,20 @@ constexpr int kTensorQuantPieces = 128;  // pieces of 64 chunks that tensor_quan
 // stores then sit in one straight piece of code; with the other forms' branches between them a wavefront issues later, which
 // short rows feel most.  us, all forms in one / PLAIN, INT8 (e4m3): 32760 x 1536 26.0 / 24.3 (26.2 / 24.5), 4096 x 2048 6.2 / 6.0
 // (6.3 / 6.2), 9450 x 5120 24.2 / 23.4 (24.4 / 23.8), 516 x 5120 3.4 / 3.2 (3.6 / 3.4); none of eighteen slower.
-// KEEP: the bytes stay in the caches (kKeepBytes)
-template <int NCH, int W, int FMT, bool SCALE_IN, int XT, bool PLAIN, bool KEEP>
+// STORE: where the bytes go (store_of)
+// Rows of one wavefront whose bytes stay in the caches are dealt out in ranges, an eighth of the matrix to each XCD, as the tiled GEMMs'
+// row groups take them: what the consumer's own L2 holds it need not fetch, and no L2 has to give up lines that the next pass rewrites.
+// Quantiser + GEMM, us, rows dealt round the XCDs / in ranges, INT8: 11732 x 304, K = 1536 23.0 / 20.4, 4096 x 1536 x 1536 20.0 / 19.2,
+// 4412 x 1056, K = 920 14.6 / 13.9, 33629 x 504, K = 552 33.1 / 32.2, 32760 x 2728, K = 1536 152.5 / 150.7.  Longer rows are level (0.2 %).
+template <int NCH, int W, int FMT, bool SCALE_IN, int XT, bool PLAIN, int STORE>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
     constexpr int XB = XT == DAXQ_F32 ? 4 : 2;
     __shared__ uint32_t s_max[4];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // behind tensor_amax_kernel: the rows that it read last first, each on the XCD that read it
-    const int64_t unit = W > 1 && !PLAIN && !SCALE_IN && a.partials ? (int64_t)((gridDim.x >> 3) - 1 - (blockIdx.x >> 3)) * 8 + (blockIdx.x & 7) : blockIdx.x;
+    const int64_t unit = W > 1 && !PLAIN && !SCALE_IN && a.partials ? (int64_t)((gridDim.x >> 3) - 1 - (blockIdx.x >> 3)) * 8 + (blockIdx.x & 7)
+                         : W == 1 && STORE != kStorePast ? xcd_range(blockIdx.x, gridDim.x) : blockIdx.x;
     const int64_t row0 = unit * (4 / W) + wave / W;
     if (W == 1 && row0 >= a.m) return;
     const int64_t row = row0 < a.m ? row0 : a.m - 1;  // (rows beyond the last: the wavefront still reaches the barrier)
@@ -129,8 +140,8 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const QuantArgs a) {
             float f[8];
             chunk_values<XT>(v[i], f);
             const uint2 o = quant8<FMT, F, XT>(f, s, inv);
-            if (c < nch) store_chunk<KEEP>(qr + (uint32_t)c * 8u, o);
-            else if (!ragged && c < npad) store_chunk<KEEP>(qr + (uint32_t)c * 8u, make_uint2(0, 0));
+            if (c < nch) store_chunk<STORE>(qr + (uint32_t)c * 8u, o);
+            else if (!ragged && c < npad) store_chunk<STORE>(qr + (uint32_t)c * 8u, make_uint2(0, 0));
         }
     };
     if constexpr (PLAIN) store(std::integral_constant<int, kOwn>{});
@@ -216,6 +227,20 @@ struct ScaleKind {
 // 75600 x 5120 x 5120 e4m3 1498 -> 1505; converting a weight of 13824 x 5120 37.0 -> 38.3.  (The rows' own loads without the hint as
 // well: 512 x 5120 22.2, 4096 x 1536 19.6, but 4725 x 5120 105.2 and 32760 x 1536 234.8.)
 constexpr int64_t kKeepBytes = (int64_t)128 << 20;
+// Kept bytes that only lie in the L2s are written back when the kernel has ended, and the GEMM waits for that: it starts 1.5 us
+// behind the last acknowledged store with nothing to write back, 3.1 us with 2.6 MB (512 x 5120), 4.5 us with 6.3 MB (4096 x 1536).
+// Stores through the L2 write while the kernel runs.  Quantiser + GEMM, us, kept / through (rows of one wavefront in ranges):
+//   134 x 3472, K = 5120 (0.65 MB) 12.5 / 12.5    17 x 5120 x 5120 e4m3 (0.1) 9.05 / 9.22    64 x 5120 x 5120 (0.3) 12.1 / 12.4
+//   512 x 5120 x 5120 (2.5) 22.3 / 22.0    2900 x 3080, K = 1000 (2.8) 19.7 / 19.4    313 x 4608, K = 13824 (4.1) 31.9 / 31.3
+//   1024 x 5120 x 5120 e4m3 (5) 29.8 / 29.2    1230 x 2712, K = 5120 (6) 26.5 / 25.8    887 x 5120, K = 8960 e4m3 (7.6) 40.9 / 40.3
+//   2225 x 5120, K = 4608 (9.8) 51.1 / 51.3    1003 x 4608, K = 13824 (13) 60.5 / 61.0    2358 x 5120, K = 8960 (20) 92.7 / 93.0
+//   4071 x 5120, K = 13824 (54) 216.7 / 216.2  13198 x 1536, K = 5120 (64) 111.8 / 109.2   16034 x 5120, K = 5160 e4m3 (80) 320 / 312
+constexpr int64_t kThroughFrom = (int64_t)1 << 20, kThroughTo = (int64_t)8 << 20, kThroughAgain = (int64_t)32 << 20;
+static int store_of(int64_t bytes, const void* q, int64_t ld_q) {
+    if (bytes > kKeepBytes) return kStorePast;
+    const bool aligned = (((uintptr_t)q | (uintptr_t)ld_q) & 7) == 0;
+    return aligned && bytes >= kThroughFrom && (bytes <= kThroughTo || bytes >= kThroughAgain) ? kStoreThrough : kStoreKeep;
+}
 
 // Rows that a workgroup of quant_rows_kernel takes where a row has more than one wavefront (the instantiations that
 // launch_quant_rows_t goes through), else 0.
@@ -258,7 +283,7 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
         constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
         const bool plain = kMayBePlain && ((k | kfill) & 7) == 0 && !a.leaf && qmax <= kFmtMax && (FMT == 0 || round_x);
         // (the rows of a weight, and those under a scale each from the caller, have no GEMM behind them)
-        const bool keep = m * kfill <= kKeepBytes && !t.weight && (!SCALE_IN || t.one_scale);
+        const int to = t.weight || (SCALE_IN && !t.one_scale) ? kStorePast : store_of(m * kfill, q, ld_q);
         // A launch holds fewer than 2^32 work items, i.e. 2^24 workgroups: more rows are as many launches as they need
 #define DAXQ_Q_CASE(N, W)                                                                                                  \
     if (cols <= N * W) {                                                                                                   \
@@ -267,10 +292,14 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
             const QuantArgs b = rows_from<XB>(a, r, kSlab);                                                                \
             const unsigned groups = (unsigned)((b.m + kRows - 1) / kRows);                                                 \
             const dim3 grid(W > 1 && a.partials ? (groups + 7) / 8 * 8 : groups);                                          \
-            if (plain && keep) launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain, true>), grid, dim3(256), 0, st, b); \
-            else if (plain) launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain, false>), grid, dim3(256), 0, st, b); \
-            else if (keep) launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false, true>), grid, dim3(256), 0, st, b); \
-            else launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false, false>), grid, dim3(256), 0, st, b);        \
+            auto launch = [&](auto STORE) {                                                                                \
+                constexpr int S = decltype(STORE)::value;                                                                  \
+                if (plain) launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, kMayBePlain, S>), grid, dim3(256), 0, st, b); \
+                else launch_kernel((quant_rows_kernel<N, W, FMT, SCALE_IN, XT, false, S>), grid, dim3(256), 0, st, b);     \
+            };                                                                                                             \
+            if (to == kStoreThrough) launch(std::integral_constant<int, kStoreThrough>{});                                 \
+            else if (to == kStoreKeep) launch(std::integral_constant<int, kStoreKeep>{});                                  \
+            else launch(std::integral_constant<int, kStorePast>{});                                                        \
         }                                                                                                                  \
         return check_launch("quant_rows");                                                                                 \
     }
@@ -494,8 +523,8 @@ __global__ __launch_bounds__(1024) void tensor_quant_kernel(const QuantArgs a) {
             float f[8];
             chunk_values<XT>(v[i], f);
             const uint2 o = quant8<FMT, decltype(FORM)::value, XT>(f, s, inv);
-            if (at < nch) store_chunk<true>(qr + (uint32_t)at * 8u, o);
-            else if (!ragged && at < npad) store_chunk<true>(qr + (uint32_t)at * 8u, make_uint2(0, 0));
+            if (at < nch) store_chunk<kStoreKeep>(qr + (uint32_t)at * 8u, o);
+            else if (!ragged && at < npad) store_chunk<kStoreKeep>(qr + (uint32_t)at * 8u, make_uint2(0, 0));
         }
     });
     if (ragged && wave == 0) {

@@ -351,3 +351,50 @@ def test_bytes_over_the_rows_they_are_made_from(ops, dtype, fmt, m, k):
         assert bool((scratch != 0).any()) == (i == 1)
         if i == 1:
             assert torch.equal(q[:, :k], apart[:, :k]) and torch.equal(scale[0], scale[1])
+
+
+@pytest.mark.parametrize("k,m", [(1536, 681), (1536, 683), (1537, 5041), (5120, 205), (5120, 1639), (2560, 3277), (5120, 6557), (1536, 21847)])
+@pytest.mark.parametrize("form", ["token", "one_scale", "tensor"])
+def test_matrices_whose_bytes_are_stored_through_the_l2(form, k, m):
+    """On either side of the lines between the ways of storing the bytes (1, 8 and 32 MB), numbers of rows that leave the XCDs' ranges
+    uneven: the bytes and scales of the whole matrix are those of slices of a few rows, at an address that is a multiple of 8 and at one
+    that is not, and nothing around them is written."""
+    from dax_amd import _capi
+
+    L = _capi.lib()
+    st = torch.cuda.current_stream().cuda_stream
+    kp = (k + 127) // 128 * 128
+    g = torch.Generator("cuda").manual_seed(k + m)
+    x = (torch.randn(m, k, generator=g, device="cuda") * torch.rand(m, 1, generator=g, device="cuda")).to(torch.bfloat16)
+    part = torch.empty(256, dtype=torch.int32, device="cuda")
+    s1 = torch.tensor([0.0123], device="cuda")
+
+    def quantise(xs, q, sx):
+        rows = xs.shape[0]
+        if form == "token":
+            rc = L.daxq_act_quant_rows(xs.data_ptr(), 0, 0, rows, k, k, q, kp, sx.data_ptr(), st)
+        elif form == "one_scale":
+            rc = L.daxq_quantize_tensor(xs.data_ptr(), 0, 1, rows, k, k, s1.data_ptr(), q, kp, sx.data_ptr(), st)
+        else:
+            rc = L.daxq_act_quant_tensor(xs.data_ptr(), 0, 2, rows, k, k, q, kp, sx.data_ptr(), None, part.data_ptr(), 57344.0, 2.0 ** -23, 1, st)
+        _capi.check(rc, "quantiser")
+
+    want = torch.zeros(m, kp, dtype=torch.uint8, device="cuda")
+    want_s = torch.zeros(m, device="cuda")
+    if form == "tensor":  # one scale: the leaf quantiser's bytes under it, in slices
+        scale = (x.float().abs().max() / 57344.0).to(torch.bfloat16).float().clamp_min(2.0 ** -23)
+        want_s.fill_(scale.item())
+        for r in range(0, m, 160):
+            n = min(160, m - r)
+            _capi.check(L.daxq_quantize_rows(x[r:].data_ptr(), 0, 2, n, k, k, want_s[r:].data_ptr(), want[r:].data_ptr(), kp, st), "rows")
+    else:
+        for r in range(0, m, 160):
+            quantise(x[r:r + 160], want[r:].data_ptr(), want_s[r:])
+    for shift in (8, 3):
+        buf = torch.full((m * kp + 32,), 0x5A, dtype=torch.uint8, device="cuda")
+        sx = torch.full((m + 1,), 7.0, device="cuda")
+        quantise(x, buf.data_ptr() + shift, sx)
+        torch.cuda.synchronize()
+        assert torch.equal(buf[shift:shift + m * kp].view(m, kp), want)
+        assert torch.equal(sx[:m], want_s) and sx[m].item() == 7.0
+        assert bool((buf[:shift] == 0x5A).all()) and bool((buf[shift + m * kp:] == 0x5A).all())
