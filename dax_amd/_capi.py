@@ -61,6 +61,8 @@ SIGNATURES = {
     "daxq_linear_launch_splits": [_I64, _I64, _I64],
     "daxq_linear_few_applies": [_INT, _INT, _INT, _INT, _INT, _INT, _I64, _I64, _I64],
     "daxq_linear_few": [_INT, _INT, _INT, _INT, _INT, _INT, _P, _I64, _P, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _P],
+    "daxq_linear_short_rows_applies": [_INT, _INT, _INT, _INT, _INT, _INT, _I64, _I64, _I64],
+    "daxq_linear_short_rows": [_INT, _INT, _INT, _INT, _INT, _INT, _P, _I64, _P, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _P],
     "daxq_linear_kernel_choice": [_INT, _I64, _I64, _I64],
     "daxq_linear_tile_order_choice": [_I64, _I64, _I64],
     "daxq_linear_splitk_workspace_bytes": [_I64, _I64, _INT],

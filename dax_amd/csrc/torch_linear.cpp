@@ -103,8 +103,8 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         if (x->dim() != 2 || x->stride(1) != 1 || (m > 1 && x->stride(0) < k)) Py_RETURN_NONE;
         if (m > 1) ld_x = x->stride(0);
     }
-    // a handful of rows: one launch that quantises for itself
-    const bool few = kernel == 0 && daxq_linear_few_applies(x_kind, x_fmt, w_fmt, out_kind, scheme, scale_fp32 ? 0 : 1, m, n, k);
+    // a handful of rows, or some more short ones: one launch that quantises for itself
+    const bool few = kernel == 0 && m <= 64 && (m <= 8 ? daxq_linear_few_applies : daxq_linear_short_rows_applies)(x_kind, x_fmt, w_fmt, out_kind, scheme, scale_fp32 ? 0 : 1, m, n, k);
     // rows that the buffers hold: 64 or 128 where that many in a tiled kernel are faster than m (what the rows beyond m hold is
     // never looked at, their outputs are cut off); a kernel chosen by name runs on the rows there are
     const int64_t rows = kernel == 0 ? daxq_linear_launch_rows(x_fmt, m, n, k) : m;
@@ -119,7 +119,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         const auto opt = at::TensorOptions().device(dev);
         if (few) {
             out = at::empty(shape, opt.dtype(out_type));
-            rc = daxq_linear_few(x_kind, x_fmt, w_fmt, out_kind, scheme, scale_fp32 ? 0 : 1, x->const_data_ptr(), ld_x,
+            rc = (m <= 8 ? daxq_linear_few : daxq_linear_short_rows)(x_kind, x_fmt, w_fmt, out_kind, scheme, scale_fp32 ? 0 : 1, x->const_data_ptr(), ld_x,
                                  in_scale ? in_scale->const_data_ptr<float>() : nullptr, wq->const_data_ptr(), kp, sw->const_data_ptr<float>(),
                                  bias ? bias->const_data_ptr() : nullptr, out.mutable_data_ptr(), n, m, n, k,
                                  c10::hip::getCurrentHIPStream(dev.index()).stream());

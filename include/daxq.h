@@ -387,6 +387,13 @@ int daxq_linear_few(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme
                     const void* wq, int64_t ld_wq, const float* sw, const void* bias,
                     void* out, int64_t ld_out, int64_t m, int64_t n, int64_t k, daxq_stream_t stream);
 
+/* The same for 9 to 64 rows so short that quantising all of them in every workgroup pays. */
+int daxq_linear_short_rows_applies(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme, int act_scale_round, int64_t m, int64_t n, int64_t k);
+int daxq_linear_short_rows(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme, int act_scale_round,
+                           const void* x, int64_t ld_x, const float* in_scale,
+                           const void* wq, int64_t ld_wq, const float* sw, const void* bias,
+                           void* out, int64_t ld_out, int64_t m, int64_t n, int64_t k, daxq_stream_t stream);
+
 /* The implementation that daxq_linear_w8a8 takes on the current device when the low 16 bits of `kernel` are 0 (row strides below 2^26, no
  * accumulator dump), as the value of those bits.  Host arithmetic only; for tests and diagnostics. */
 int daxq_linear_kernel_choice(int x_fmt, int64_t m, int64_t n, int64_t k);
