@@ -29,9 +29,19 @@ constexpr float kEps = 1.1920928955078125e-07f;  // 2^-23 = torch.finfo(float32)
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
-// two floats rounded to fp16 (nearest even; overflow gives infinity, as a cast does), lo in the low half
+// two floats rounded to fp16 (nearest even; overflow gives infinity, as a cast does), lo in the low half: v_cvt_pk_f16_f32
+typedef _Float16 daxq_f16x2 __attribute__((ext_vector_type(2)));
+typedef float daxq_f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_f16_rne(float lo, float hi) {
-    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((daxq_f32x2{lo, hi}), daxq_f16x2));
+}
+// the fp16 value in half `HI` of h plus b, rounded to fp32 once: the widening rides in the add (h * 1 is exact)
+template <int HI>
+__device__ __forceinline__ float add_f16_half(uint32_t h, float b) {
+    float z;
+    if constexpr (HI) asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(z) : "v"(h), "v"(b));
+    else asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(z) : "v"(h), "v"(b));
+    return z;
 }
 
 // max / min that give NaN when either operand is NaN, like torch.max / torch.min / torch.clamp on tensors
@@ -48,7 +58,6 @@ __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
 
 // two f32 -> two bf16 in one word (lo = first), round to nearest even: v_cvt_pk_bf16_f32
 typedef __bf16 daxq_bf16x2 __attribute__((ext_vector_type(2)));
-typedef float daxq_f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16_rne(float lo, float hi) {
     daxq_f32x2 v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, daxq_bf16x2));

@@ -14,6 +14,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 #define DAXQ_LDS __attribute__((address_space(3)))
 #define DAXQ_GLOBAL __attribute__((address_space(1)))

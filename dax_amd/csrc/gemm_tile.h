@@ -91,9 +91,69 @@ __device__ __forceinline__ void mfma_settle() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// Four outputs of a row as 16-bit values (OUTK: DAXQ_BF16 / DAXQ_F16)
+template <bool FP8, int OUTK>
+__device__ __forceinline__ uint2 outputs4(const typename Acc16<FP8>::type& acc, float sx, const v4f& sw, const v4f& bias) {
+    uint32_t pk[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int r = 2 * h;
+        if constexpr (FP8) {
+            float z0 = acc[r] * sx * sw[r] + bias[r], z1 = acc[r + 1] * sx * sw[r + 1] + bias[r + 1];
+            if constexpr (OUTK == DAXQ_F16) {  // one rounding, to fp16 (kept apart from the add: no mixed-precision fold)
+                asm("" : "+v"(z0), "+v"(z1));
+                pk[h] = pack_f16_rne(z0, z1);
+            } else {
+                pk[h] = pack_bf16_rne(z0, z1);
+            }
+        } else {
+            float y0 = (float)acc[r];  // v_cvt_f32_i32, round to nearest even
+            float y1 = (float)acc[r + 1];
+            y0 = y0 * sx;
+            y1 = y1 * sx;
+            y0 = y0 * sw[r];
+            y1 = y1 * sw[r + 1];
+            if constexpr (OUTK == DAXQ_F16) {  // fp16 module: the same two roundings, to fp16
+                // (the products and sums pass through empty asm statements: the compiler otherwise folds
+                // a multiply or add and the conversion behind it into one mixed-precision instruction
+                // that rounds once, where the reference rounds to fp32 first)
+                asm("" : "+v"(y0), "+v"(y1));
+                const uint32_t o1 = pack_f16_rne(y0, y1);
+                pk[h] = pack_f16_rne(add_f16_half<0>(o1, bias[r]), add_f16_half<1>(o1, bias[r + 1]));
+            } else {
+                // second rounding: the bias is added to the bf16 value, which the first leaves in the upper half of a word
+                const float o0 = __uint_as_float(pack_bf16_rne(0.0f, y0)), o1 = __uint_as_float(pack_bf16_rne(0.0f, y1));
+                pk[h] = pack_bf16_rne(o0 + bias[r], o1 + bias[r + 1]);
+            }
+        }
+    }
+    return make_uint2(pk[0], pk[1]);
+}
+
+// 16 bytes at any address, into the L2 and through it to memory at once (a device-coherent store)
+__device__ __forceinline__ void store_through(uint8_t* p, v4u v) {
+    __builtin_amdgcn_global_store_b128((DAXQ_GLOBAL v4u*)p, v, "agent");
+}
+
+// Accumulators as they are (tests): int32 / fp32 [m, ldacc]
+template <int NBJ, int NBI, bool FP8>
+__device__ __forceinline__ void dump_tile16(const GemmArgs& p, typename Acc16<FP8>::type (&acc)[NBJ][NBI], int m0, int n0, int l15, int g4) {
+#pragma unroll
+    for (int j = 0; j < NBJ; ++j)
+#pragma unroll
+        for (int i = 0; i < NBI; ++i) {
+            const int64_t m = m0 + i * 16 + l15;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if constexpr (FP8) static_cast<float*>(p.acc)[m * p.ldacc + n0 + j * 16 + 4 * g4 + v] = acc[j][i][v];
+                else static_cast<int32_t*>(p.acc)[m * p.ldacc + n0 + j * 16 + 4 * g4 + v] = acc[j][i][v];
+            }
+        }
+}
+
 // The epilogue of a wavefront's accumulators held as NBJ x NBI blocks of 16x16 (v_mfma_i32_16x16x64_i8,
 // v_mfma_f32_16x16x128_f8f6f4): acc[j][i] is weight block j (16 output columns) and activation block i (16 output rows)
-// of the wavefront's part of a tile of WM x WN wavefronts.
+// of the wavefront's outputs, whose first is (m0, n0).
 // In a block a lane owns output row m = l%16 and the columns n = 4*(l/16) + {0..3}.  One
 // v_permlane16_swap per word over two neighbouring blocks gives each lane 8 consecutive columns of one
 // of them: lanes 0-15 block 2jp columns 0-7, lanes 16-31 block 2jp+1 columns 0-7, lanes 32-47 block
@@ -103,6 +163,62 @@ __device__ __forceinline__ void mfma_settle() {
 // of its own per type: with all three forms inside one kernel behind uniform branches its code grew from 27 to 44 KB
 // and the bf16 launches at K = 1536, which change between main loop and epilogue every 24 slices, lost 2.7 %; with
 // the choice inside the loops they lost 2 to 11 % everywhere.
+// sx, sw, bias: the scales of the lane's output row in each block of rows, scales and bias of its four columns in each block of columns.
+template <bool DUMP, int NBJ, int NBI, bool FP8, int OUTK>
+__device__ __forceinline__ void tile_outputs16(const GemmArgs& p, typename Acc16<FP8>::type (&acc)[NBJ][NBI], int m0, int n0, int l15, int g4,
+                                               const float (&sx)[NBI], const v4f (&sw)[NBJ], const v4f (&bias)[NBJ]) {
+    if constexpr (DUMP) dump_tile16<NBJ, NBI, FP8>(p, acc, m0, n0, l15, g4);
+    // a lane's place in the first block of rows; the others lie a uniform step apart, the blocks of columns at constant offsets
+    constexpr int XB = OUTK == DAXQ_F32 ? 4 : 2;
+    const int64_t step = 16 * p.ldo * XB;
+    uint8_t* row = reinterpret_cast<uint8_t*>(p.out) + ((int64_t)(m0 + l15) * p.ldo + n0) * XB;
+
+    // fp32 module: one rounding less and four-byte outputs, a lane's four columns of a block as one store
+    if constexpr (OUTK == DAXQ_F32) {
+        row += 16 * g4;
+#pragma unroll
+        for (int i = 0; i < NBI; ++i) {
+#pragma unroll
+            for (int j = 0; j < NBJ; ++j) {
+                float o[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float y = (float)acc[j][i][r];  // (int8: v_cvt_f32_i32, round to nearest even)
+                    y = y * sx[i];
+                    y = y * sw[j][r];
+                    o[r] = y + bias[j][r];
+                }
+                *reinterpret_cast<float4*>(row + j * 64) = make_float4(o[0], o[1], o[2], o[3]);
+            }
+            row += step;
+        }
+    } else {
+        uint8_t* last = row + 8 * g4;  // (of a block without a partner)
+        row += (g4 & 1) * 32 + (g4 >> 1) * 16;
+#pragma unroll
+        for (int i = 0; i < NBI; ++i) {
+#pragma unroll
+            for (int jp = 0; jp < (NBJ + 1) / 2; ++jp) {
+                const int j = 2 * jp;
+                const uint2 lo = outputs4<FP8, OUTK>(acc[j][i], sx[i], sw[j], bias[j]);
+                if (j + 1 == NBJ) {
+                    *reinterpret_cast<uint2*>(last + jp * 64) = lo;
+                    continue;
+                }
+                const int pj = j + 1 < NBJ ? j + 1 : j;
+                const uint2 up = outputs4<FP8, OUTK>(acc[pj][i], sx[i], sw[pj], bias[pj]);
+                v2u s0 = __builtin_amdgcn_permlane16_swap(lo.x, up.x, false, false);
+                v2u s1 = __builtin_amdgcn_permlane16_swap(lo.y, up.y, false, false);
+                *reinterpret_cast<uint4*>(row + jp * 64) = make_uint4(s0.x, s1.x, s0.y, s1.y);
+            }
+            row += step;
+            last += step;
+        }
+    }
+}
+
+// The same for kernels that have no registers for the scales beside their main loop: a thread has requested one of each, and they
+// pass through the LDS.
 template <bool DUMP, int NBJ, int NBI, bool FP8 = false, int OUTK = DAXQ_BF16, int WM = 2, int WN = 2>
 __device__ __forceinline__ void tile_epilogue16(const GemmArgs& p, typename Acc16<FP8>::type (&acc)[NBJ][NBI], uint8_t* smem, int m0, int n0, int t,
                                                 int wm, int wn, int l15, int g4, float pre_sx, float pre_sw,
@@ -117,119 +233,18 @@ __device__ __forceinline__ void tile_epilogue16(const GemmArgs& p, typename Acc1
         s_bias[t] = pre_bias;
     }
     __syncthreads();
-
-    if constexpr (DUMP) {
+    float sx[NBI];
+    v4f sw[NBJ], bias[NBJ];
 #pragma unroll
-        for (int j = 0; j < NBJ; ++j)
-#pragma unroll
-            for (int i = 0; i < NBI; ++i) {
-                const int64_t m = m0 + wm * WTM + i * 16 + l15;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    if constexpr (FP8) static_cast<float*>(p.acc)[m * p.ldacc + n0 + wn * WTN + j * 16 + 4 * g4 + v] = acc[j][i][v];
-                    else static_cast<int32_t*>(p.acc)[m * p.ldacc + n0 + wn * WTN + j * 16 + 4 * g4 + v] = acc[j][i][v];
-                }
-            }
-    }
-
-    float sxr[NBI];
-    float4 swr[NBJ], br[NBJ];
-#pragma unroll
-    for (int i = 0; i < NBI; ++i) sxr[i] = s_sx[wm * WTM + i * 16 + l15];
+    for (int i = 0; i < NBI; ++i) sx[i] = s_sx[wm * WTM + i * 16 + l15];
 #pragma unroll
     for (int j = 0; j < NBJ; ++j) {
         const int nl = wn * WTN + j * 16 + 4 * g4;
-        swr[j] = *reinterpret_cast<const float4*>(s_sw + nl);
-        br[j] = *reinterpret_cast<const float4*>(s_bias + nl);
+        sw[j] = *reinterpret_cast<const v4f*>(s_sw + nl);
+        bias[j] = *reinterpret_cast<const v4f*>(s_bias + nl);
     }
     __builtin_amdgcn_sched_barrier(0);
-
-    // fp32 module: one rounding less and four-byte outputs, a lane's four columns of a block as one store
-    if constexpr (OUTK == DAXQ_F32) {
-        {
-#pragma unroll
-            for (int i = 0; i < NBI; ++i) {
-                const float sxv = sxr[i];
-                float* orow = reinterpret_cast<float*>(p.out) + (int64_t)(m0 + wm * WTM + i * 16 + l15) * p.ldo + n0 + wn * WTN + 4 * g4;
-#pragma unroll
-                for (int j = 0; j < NBJ; ++j) {
-                    const float sws[4] = {swr[j].x, swr[j].y, swr[j].z, swr[j].w};
-                    const float bs[4] = {br[j].x, br[j].y, br[j].z, br[j].w};
-                    float o[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        float y = (float)acc[j][i][r];  // (int8: v_cvt_f32_i32, round to nearest even)
-                        y = y * sxv;
-                        y = y * sws[r];
-                        o[r] = y + bs[r];
-                    }
-                    *reinterpret_cast<float4*>(orow + j * 16) = make_float4(o[0], o[1], o[2], o[3]);
-                }
-            }
-        }
-        return;
-    }
-    // out and bias are fp16 instead of bf16
-    constexpr bool f16 = OUTK == DAXQ_F16;
-    {
-#pragma unroll
-    for (int i = 0; i < NBI; ++i) {
-        const int ml = wm * WTM + i * 16 + l15;
-        const float sxv = sxr[i];
-        uint16_t* orow = p.out + (int64_t)(m0 + ml) * p.ldo + n0 + wn * WTN;
-#pragma unroll
-        for (int jp = 0; jp < (NBJ + 1) / 2; ++jp) {
-            uint32_t pk[2][2];
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj) {
-                const int j = 2 * jp + jj;
-                if (j >= NBJ) continue;
-                const float sws[4] = {swr[j].x, swr[j].y, swr[j].z, swr[j].w};
-                const float bs[4] = {br[j].x, br[j].y, br[j].z, br[j].w};
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int r = 2 * h;
-                    if constexpr (FP8) {
-                        float z0 = acc[j][i][r] * sxv * sws[r] + bs[r], z1 = acc[j][i][r + 1] * sxv * sws[r + 1] + bs[r + 1];
-                        if constexpr (f16) {  // one rounding, to fp16 (kept apart from the add: no mixed-precision fold)
-                            asm("" : "+v"(z0), "+v"(z1));
-                            pk[jj][h] = pack_f16_rne(z0, z1);
-                        } else {
-                            pk[jj][h] = pack_bf16_rne(z0, z1);
-                        }
-                    } else {
-                        float y0 = (float)acc[j][i][r];  // v_cvt_f32_i32, round to nearest even
-                        float y1 = (float)acc[j][i][r + 1];
-                        y0 = y0 * sxv;
-                        y1 = y1 * sxv;
-                        y0 = y0 * sws[r];
-                        y1 = y1 * sws[r + 1];
-                        if constexpr (f16) {  // fp16 module: the same two roundings, to fp16
-                            // (the products and sums pass through empty asm statements: the compiler otherwise folds
-                            // a multiply or add and the conversion behind it into one mixed-precision instruction
-                            // that rounds once, where the reference rounds to fp32 first)
-                            asm("" : "+v"(y0), "+v"(y1));
-                            float z0 = (float)(_Float16)y0 + bs[r], z1 = (float)(_Float16)y1 + bs[r + 1];
-                            asm("" : "+v"(z0), "+v"(z1));
-                            pk[jj][h] = pack_f16_rne(z0, z1);
-                        } else {
-                            const uint32_t o1 = pack_bf16_rne(y0, y1);
-                            // second rounding: the bias is added to the bf16 value
-                            pk[jj][h] = pack_bf16_rne(__uint_as_float(o1 << 16) + bs[r], __uint_as_float(o1 & 0xffff0000u) + bs[r + 1]);
-                        }
-                    }
-                }
-            }
-            if (2 * jp + 1 == NBJ) {
-                *reinterpret_cast<uint2*>(orow + jp * 32 + 4 * g4) = make_uint2(pk[0][0], pk[0][1]);
-                continue;
-            }
-            v2u s0 = __builtin_amdgcn_permlane16_swap(pk[0][0], pk[1][0], false, false);
-            v2u s1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
-            *reinterpret_cast<uint4*>(orow + jp * 32 + (g4 & 1) * 16 + (g4 >> 1) * 8) = make_uint4(s0.x, s1.x, s0.y, s1.y);
-        }
-    }
-    }
+    tile_outputs16<DUMP, NBJ, NBI, FP8, OUTK>(p, acc, m0 + wm * WTM, n0 + wn * WTN, l15, g4, sx, sw, bias);
 }
 
 // CUs of the current device (0 if the query fails), asked once per device

@@ -24,8 +24,16 @@ struct FitTile {
     static constexpr int SLOT = (BM + BN) * BKP, SMEM = NS * SLOT;
     static constexpr int ROWS = T / 8;  // rows a load instruction of the workgroup takes
     static constexpr int A_LOADS = BM / ROWS, B_LOADS = BN / ROWS, PAIR_LOADS = A_LOADS + B_LOADS;
+    // the way of 16-bit outputs to memory (tile_lines): groups of G blocks of rows per wavefront, so that the stores of one run beside
+    // the arithmetic of the next (256 rows in two groups of four: 2000 x 4608 22.5 instead of 22.2 us); chunks of 16 bytes
+    static constexpr int G = 2, GROUPS = NBI / G, GROUP_ROWS = 16 * G * WM;
+    static constexpr int CHUNKS = BN / 8, STEPS = GROUP_ROWS * CHUNKS / T;  // of a row; stores of a group
+    static constexpr int PERIOD = CHUNKS % 7 == 0 ? 7 : CHUNKS % 5 == 0 ? 5 : CHUNKS % 3 == 0 ? 3 : 1, PERIOD_ROWS = PERIOD * T / CHUNKS;
+    static constexpr int OUT_ROW = 2 * BN + 16;  // bytes: 4 banks times an odd number
+    static_assert(NBI % G == 0 && GROUP_ROWS * CHUNKS % T == 0 && PERIOD * T % CHUNKS == 0 && GROUP_ROWS % PERIOD_ROWS == 0, "whole stores");
+    static_assert((16 * G) % PERIOD_ROWS == 0 || PERIOD_ROWS % (16 * G) == 0, "a step's rows are a lane's and a constant");
+    static_assert(GROUPS * GROUP_ROWS * OUT_ROW <= SMEM, "the outputs fit into the LDS of the pairs");
     static_assert(BM % ROWS == 0 && BN % ROWS == 0, "whole load instructions");
-    static_assert(T >= BM && T >= BN, "a scale per thread");
     static_assert(NS >= 3 && SMEM <= 160 * 1024 && NS * PAIR_LOADS < 60, "LDS and load counter");
 };
 typedef FitTile<2, 2, 8, 4, 3> HalfTile;  // 256 x 128
@@ -161,17 +169,48 @@ __device__ __forceinline__ void gemm_fit_body(const GemmArgs& p, const int m0, c
         }
     };
 
-    // the epilogue's scales and bias, requested behind the last tile loads: always three loads per thread (a missing bias reads a
-    // scale instead and is replaced by -0.0: x + (-0.0) == x bit for bit), so that the counts of the waits hold
-    const int tm = t < BM ? t : BM - 1, tn = t < BN ? t : BN - 1;
-    float pre_sx, pre_sw;
-    uint32_t pre_b;  // the bias element's bits: bf16 / fp16, or fp32
+    // the epilogue's scales and bias, requested behind the last tile loads, each lane its own outputs': always NBI + 2 NBJ loads (a missing
+    // bias reads a scale instead and is replaced by -0.0: x + (-0.0) == x bit for bit), so that the counts of the waits hold
+    constexpr int SCALE_LOADS = NBI + 2 * NBJ;
+    typedef v4f loose_v4f __attribute__((aligned(4)));
+    typedef v2u loose_v2u __attribute__((aligned(2)));
+    const int mw = m0 + wm * 16 * NBI, nw = n0 + wn * 16 * NBJ;
+    float sx[NBI];
+    v4f sw[NBJ], bias[NBJ];
+    v2u bias_bits[NBJ];  // bf16 / fp16
     auto request_scales = [&]() __attribute__((always_inline)) {
-        pre_sx = p.sx[m0 + tm];
-        pre_sw = p.sw[n0 + tn];
-        if constexpr (OUTK == DAXQ_F32) pre_b = __float_as_uint((p.bias ? reinterpret_cast<const float*>(p.bias) : p.sw)[n0 + tn]);
-        else pre_b = (p.bias ? p.bias : reinterpret_cast<const uint16_t*>(p.sw))[n0 + tn];
+#pragma unroll
+        for (int i = 0; i < NBI; ++i) sx[i] = p.sx[mw + 16 * i + lr];
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j) {
+            const int n = nw + 16 * j + 4 * kg;
+            sw[j] = *reinterpret_cast<const loose_v4f*>(p.sw + n);
+            if constexpr (OUTK == DAXQ_F32) bias[j] = *reinterpret_cast<const loose_v4f*>((p.bias ? reinterpret_cast<const float*>(p.bias) : p.sw) + n);
+            else bias_bits[j] = *reinterpret_cast<const loose_v2u*>((p.bias ? p.bias : reinterpret_cast<const uint16_t*>(p.sw)) + n);
+        }
         __builtin_amdgcn_sched_barrier(0);
+    };
+    // Outputs of 16 bits leave by way of the LDS, as rows of the tile, and through the L2 to memory (store_through).  A launch of one
+    // round writes all its outputs at its end.  Stored straight from the registers, 16 rows x 64 bytes an instruction, they took a CU 36
+    // cycles per KB, and what lay in the L2s was written back behind the kernel, 2.4 us of nothing else at 4096 x 1536; whole rows take 17
+    // cycles per KB, and half lines stored through the L2 are slower than ones that stay in it.  us, straight / rows / rows and
+    // through, INT8 forwards: 4096 x 1536 x 1536 20.7 / 20.3 / 19.5, 2900 x 3080, K = 1000 fp16 20.0 / 20.2 / 19.1, 2000 x 4608, K = 1536
+    // 22.7 / 22.7 / 21.4, 512 x 5120 x 5120 22.7 / 22.6 / 22.0, 4096 x 1537, K = 1536 24.3 / 20.8 / 20.0 (rows that start anywhere);
+    // none of 25 launches slower by more than 0.5 %.
+    // Chunk s T + t of a group of rows is the thread's at step s: its row and column repeat every PERIOD steps, PERIOD_ROWS rows further.
+    // (put together here, where the first loads are waited for, and kept in registers)
+    typedef TILE L;
+    constexpr bool LINES = OUTK != DAXQ_F32;
+    int64_t line_out[L::PERIOD];   // bytes from the tile's first output
+    uint32_t line_lds[L::PERIOD];  // bytes from the group's first output in the LDS
+    auto tile_lines = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < L::PERIOD; ++s) {
+            const int c = s * L::T + t, r = c / L::CHUNKS, col = c - r * L::CHUNKS;  // row r of the group's, wavefront row by wavefront row
+            line_out[s] = ((int64_t)(r / (16 * L::G) * (16 * NBI) + r % (16 * L::G)) * p.ldo + col * 8) * 2;
+            line_lds[s] = (uint32_t)(r * L::OUT_ROW + col * 16);
+            asm volatile("" : "+v"(line_out[s]), "+v"(line_lds[s]));
+        }
     };
     auto issue_pair = [&](uint32_t slot) __attribute__((always_inline)) {
 #pragma unroll
@@ -183,6 +222,7 @@ __device__ __forceinline__ void gemm_fit_body(const GemmArgs& p, const int m0, c
         // ---- prologue: pairs 0 .. NS-1 in flight, pair 0 landed, its fragments in set 0
 #pragma unroll
         for (int s = 0; s < NS; ++s) issue_pair(st[s]);
+        if constexpr (LINES) tile_lines();
         __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 1) * PAIR_LOADS));
         __builtin_amdgcn_s_barrier();
 #pragma unroll
@@ -206,7 +246,7 @@ __device__ __forceinline__ void gemm_fit_body(const GemmArgs& p, const int m0, c
         request_scales();
         auto tail = [&](auto T) __attribute__((always_inline)) {
             constexpr int n = decltype(T)::value;  // of NS
-            pair(Int<n % 2 == 0>{}, No{}, Int<(n < NS - 1)>{}, Int<(n < NS - 2 ? NS - 2 - n : 0) * PAIR_LOADS>{}, Int<3>{}, No{});
+            pair(Int<n % 2 == 0>{}, No{}, Int<(n < NS - 1)>{}, Int<(n < NS - 2 ? NS - 2 - n : 0) * PAIR_LOADS>{}, Int<SCALE_LOADS>{}, No{});
         };
         for_up<0, NS>(tail);
         mfma_settle();
@@ -214,6 +254,7 @@ __device__ __forceinline__ void gemm_fit_body(const GemmArgs& p, const int m0, c
         // ---- short K: every pair has a slot
         for (int q = 0; q < Q; ++q) issue_pair(q * SLOT);
         request_scales();
+        if constexpr (LINES) tile_lines();
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         __builtin_amdgcn_s_barrier();
         for (int q = 0; q < Q; ++q) {
@@ -230,6 +271,7 @@ __device__ __forceinline__ void gemm_fit_body(const GemmArgs& p, const int m0, c
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        __syncthreads();  // (the outputs go where other wavefronts may still read fragments)
         mfma_settle();
     }
 
@@ -239,10 +281,48 @@ __device__ __forceinline__ void gemm_fit_body(const GemmArgs& p, const int m0, c
 #pragma unroll
         for (int i = 0; i < NBI; ++i) asm volatile("" : "+a"(acc[j][i]));
 
-    __syncthreads();  // every wavefront is past its last fragment read (the short-K loop has no barrier behind its reads)
-    tile_epilogue16<DUMP, NBJ, NBI, FP8, OUTK, TILE::WM, TILE::WN>(
-        p, acc, smem, m0, n0, t, wm, wn, lr, kg, pre_sx, pre_sw,
-        !p.bias ? -0.0f : OUTK == DAXQ_F32 ? __uint_as_float(pre_b) : OUTK == DAXQ_F16 ? f16_bits_to_f32((uint16_t)pre_b) : bf16_bits_to_f32(pre_b));
+#pragma unroll
+    for (int j = 0; j < NBJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (OUTK != DAXQ_F32) {
+                const uint32_t w = bias_bits[j][r >> 1], b = r & 1 ? w >> 16 : w & 0xffffu;
+                bias[j][r] = OUTK == DAXQ_F16 ? f16_bits_to_f32((uint16_t)b) : bf16_bits_to_f32(b);
+            }
+            if (!p.bias) bias[j][r] = -0.0f;
+        }
+    if constexpr (!LINES) {
+        tile_outputs16<DUMP, NBJ, NBI, FP8, OUTK>(p, acc, mw, nw, lr, kg, sx, sw, bias);
+    } else {
+        if constexpr (DUMP) dump_tile16<NBJ, NBI, FP8>(p, acc, mw, nw, lr, kg);
+        uint8_t* const to = smem + (wm * 16 * L::G + lr) * L::OUT_ROW + (wn * 16 * NBJ + 4 * kg) * 2;
+        uint8_t* const out = reinterpret_cast<uint8_t*>(p.out) + ((int64_t)m0 * p.ldo + n0) * 2;
+        v4u line[L::STEPS];
+        auto store_group = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+            for (int s = 0; s < L::STEPS; ++s) {
+                constexpr int GR = 16 * L::G;
+                const int r = s / L::PERIOD * L::PERIOD_ROWS;  // (uniform: whole segments of GR rows, or a part of one)
+                store_through(out + (int64_t)(r / GR * (16 * NBI) + r % GR + g * GR) * p.ldo * 2 + line_out[s % L::PERIOD], line[s]);
+            }
+        };
+#pragma unroll
+        for (int g = 0; g < L::GROUPS; ++g) {
+#pragma unroll
+            for (int ii = 0; ii < L::G; ++ii) {
+                const int i = g * L::G + ii;
+#pragma unroll
+                for (int j = 0; j < NBJ; ++j)
+                    *reinterpret_cast<uint2*>(to + (g * L::GROUP_ROWS + ii * 16) * L::OUT_ROW + j * 32) = outputs4<FP8, OUTK>(acc[j][i], sx[i], sw[j], bias[j]);
+                if (g > 0 && ii == 0) store_group(g - 1);  // their reads have come back meanwhile
+            }
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < L::STEPS; ++s)
+                line[s] = *reinterpret_cast<const v4u*>(smem + (g * L::GROUP_ROWS + s / L::PERIOD * L::PERIOD_ROWS) * L::OUT_ROW + line_lds[s % L::PERIOD]);
+        }
+        store_group(L::GROUPS - 1);
+    }
 }
 
 // half `half_id & 1` of the 256x256 tile quad_base - 1 + half_id / 2 of the row-group order (launches that leave tiles over after

@@ -82,6 +82,43 @@ def test_other_output_types_and_exact_fits(tile, fp8, out):
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("out", ["bf16", "fp16"])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_rows_of_outputs_that_start_anywhere(tile, fp8, out):
+    """Whole rows of a tile are stored as 16-byte pieces: column counts (and with them row starts, scales and biases) that are a multiple of
+    2, 4, 8 or nothing, a tile that is the launch and one that overlaps its neighbours, K in the short and in the pipelined form."""
+    bm, bn, ns = TILES[tile]
+    other = 5 if not fp8 else 11 if bm >= 128 else 17
+    for m, n, pairs in ((bm, bn + 1, 1), (bm + 3, bn + 2, ns + 1), (bm, 2 * bn + 36, ns + 2), (2 * bm - 1, bn, 2)):
+        if fp8 and n < 128:
+            n += 64
+        if fp8 and bm < 128:
+            m = min(m, 128)
+        xq, wq, sx, sw, b = _operands(m, n, 128 * pairs, fp8, OUT[out][1], m + n + pairs)
+        got, want = (_launch(xq, wq, sx, sw, b, fp8, out, kernel) for kernel in (32 + tile, other))
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (m, n, pairs)
+
+
+def test_fp16_sums_of_every_rounded_product():
+    """INT8 with fp16 outputs rounds the product to fp16 and adds the bias to that: every fp16 value as the product (an accumulator of
+    1, its row's and column's scales), among them subnormal ones and infinity, under biases of all sizes, against torch's two steps."""
+    bits = torch.arange(0, 0x7C01, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    bits = torch.cat([bits, bits[-1:].repeat(-len(bits) % 64)]).float()
+    m = len(bits)
+    for bias in (0.0, 1.0, -3.0e-6, 6.0e-8, -0.333, 65504.0, -1234.5):
+        n = 64
+        xq, wq = torch.zeros(m, 128, dtype=torch.int8), torch.zeros(n, 128, dtype=torch.int8)
+        xq[:, 0], wq[:, 0] = 1, 1
+        wq[1::2, 0] = -1
+        b = torch.full((n,), bias).half()
+        got = _launch(xq, wq, bits, torch.ones(n), b, False, "fp16", 32)
+        acc = xq.float() @ wq.float().T
+        want = ((acc * bits[:, None]).half().float() + b.float()).half()
+        same = (got.view(torch.int16) == want.view(torch.int16)) | (got.isnan() & want.isnan())
+        assert bool(same.all())
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("m,n,k", [(64, 16384, 256), (65, 24577, 128), (127, 8200, 1536), (128, 5120, 1024), (129, 4104, 640), (512, 5120, 384),
                                    (2900, 3080, 1024), (4096, 1536, 512), (5000, 64, 512), (5000, 127, 512), (575, 15360, 256), (700, 15360, 256)])
