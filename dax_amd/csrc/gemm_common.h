@@ -42,6 +42,7 @@ struct GemmArgs {
     int gm;  // depth (in tile rows) of the groups the tile order walks through
     // tile order of the 256x256 kernels: 0 = groups of gm tile rows, 1 = banded patches of 8 x 4 tiles (tile_order.h)
     int order;
+    int lines;     // how 16-bit outputs leave (lines_of, gemm_tile.h)
     int out_kind;  // element type of out and bias: DAXQ_BF16 / DAXQ_F16 / DAXQ_F32
     // split-K launches only: K is cut into `splits` equal ranges, one workgroup each; partial accumulators go to
     // `partials` ([tile][split][64 KiB]) and the workgroup that arrives last at `counters[tile]` adds them up

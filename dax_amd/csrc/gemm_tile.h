@@ -35,6 +35,8 @@ __device__ __forceinline__ void for_up(F&& f) {
     }
 }
 
+// GemmArgs::lines
+constexpr int kLinesNone = 0, kLinesPlain = 1, kLinesThrough = 2;
 // GemmArgs::order
 constexpr int kOrderRowGroups = 0, kOrderBanded = 1;
 
@@ -151,79 +153,109 @@ __device__ __forceinline__ void dump_tile16(const GemmArgs& p, typename Acc16<FP
         }
 }
 
-// The epilogue of a wavefront's accumulators held as NBJ x NBI blocks of 16x16 (v_mfma_i32_16x16x64_i8,
-// v_mfma_f32_16x16x128_f8f6f4): acc[j][i] is weight block j (16 output columns) and activation block i (16 output rows)
-// of the wavefront's outputs, whose first is (m0, n0).
-// In a block a lane owns output row m = l%16 and the columns n = 4*(l/16) + {0..3}.  One
-// v_permlane16_swap per word over two neighbouring blocks gives each lane 8 consecutive columns of one
-// of them: lanes 0-15 block 2jp columns 0-7, lanes 16-31 block 2jp+1 columns 0-7, lanes 32-47 block
+// In a 16x16 block a lane owns output row m = l%16 and the columns n = 4*(l/16) + {0..3}.
+// The outputs of a wavefront's accumulators held as NBJ x NBI such blocks (v_mfma_i32_16x16x64_i8, v_mfma_f32_16x16x128_f8f6f4), of
+// which (m0, n0) is the first: acc[j][i] is weight block j (16 output columns) and activation block i (16 output rows).
+// sx, sw, bias: the scales of the lane's output row in each block of rows, scales and bias of its four columns in each block of columns.
+
+// fp32 module: one rounding less and four-byte outputs, a lane's four columns of a block as one store.
+template <int NBJ, int NBI, bool FP8>
+__device__ __forceinline__ void outputs_f32(const GemmArgs& p, typename Acc16<FP8>::type (&acc)[NBJ][NBI], int m0, int n0, int l15, int g4,
+                                            const float (&sx)[NBI], const v4f (&sw)[NBJ], const v4f (&bias)[NBJ]) {
+    // a lane's place in the first block of rows; the others lie a uniform step apart, the blocks of columns at constant offsets
+    float* row = reinterpret_cast<float*>(p.out) + (int64_t)(m0 + l15) * p.ldo + n0 + 4 * g4;
+#pragma unroll
+    for (int i = 0; i < NBI; ++i) {
+#pragma unroll
+        for (int j = 0; j < NBJ; ++j) {
+            float o[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float y = (float)acc[j][i][r];  // (int8: v_cvt_f32_i32, round to nearest even)
+                y = y * sx[i];
+                y = y * sw[j][r];
+                o[r] = y + bias[j][r];
+            }
+            *reinterpret_cast<float4*>(row + j * 16) = make_float4(o[0], o[1], o[2], o[3]);
+        }
+        row += 16 * p.ldo;
+    }
+}
+
+// Outputs of 16 bits straight from the registers.  One v_permlane16_swap per word over two neighbouring blocks gives each lane 8
+// consecutive columns of one of them: lanes 0-15 block 2jp columns 0-7, lanes 16-31 block 2jp+1 columns 0-7, lanes 32-47 block
 // 2jp columns 8-15, lanes 48-63 block 2jp+1 columns 8-15.
-// (an odd NBJ leaves a block without a partner: its lanes store their own four columns).
+template <int NBJ, int NBI, bool FP8, int OUTK>
+__device__ __forceinline__ void outputs_straight(const GemmArgs& p, typename Acc16<FP8>::type (&acc)[NBJ][NBI], int m0, int n0, int l15, int g4,
+                                                 const float (&sx)[NBI], const v4f (&sw)[NBJ], const v4f (&bias)[NBJ]) {
+    static_assert(NBJ % 2 == 0, "blocks in pairs");
+    uint16_t* row = p.out + (int64_t)(m0 + l15) * p.ldo + n0 + (g4 & 1) * 16 + (g4 >> 1) * 8;
+#pragma unroll
+    for (int i = 0; i < NBI; ++i) {
+#pragma unroll
+        for (int j = 0; j < NBJ; j += 2) {
+            const uint2 lo = outputs4<FP8, OUTK>(acc[j][i], sx[i], sw[j], bias[j]), up = outputs4<FP8, OUTK>(acc[j + 1][i], sx[i], sw[j + 1], bias[j + 1]);
+            v2u s0 = __builtin_amdgcn_permlane16_swap(lo.x, up.x, false, false);
+            v2u s1 = __builtin_amdgcn_permlane16_swap(lo.y, up.y, false, false);
+            *reinterpret_cast<uint4*>(row + j * 16) = make_uint4(s0.x, s1.x, s0.y, s1.y);
+        }
+        row += 16 * p.ldo;
+    }
+}
+
+// Outputs of 16 bits as whole rows of the wavefront's, through `own`, its part of the LDS: 16 NBI rows of 32 NBJ + 16 bytes.
+template <int NBJ, int NBI, bool FP8, int OUTK, bool ALWAYS_THROUGH>
+__device__ __forceinline__ void outputs_lines(const GemmArgs& p, typename Acc16<FP8>::type (&acc)[NBJ][NBI], uint8_t* own, int m0, int n0, int lane,
+                                              const float (&sx)[NBI], const v4f (&sw)[NBJ], const v4f (&bias)[NBJ]) {
+    // groups of G blocks of rows, so that the stores of one run beside the arithmetic of the next
+    constexpr int G = 2, ROW = 32 * NBJ + 16, CHUNKS = 2 * NBJ, ROWS = 64 / CHUNKS, STEPS = 16 * G / ROWS;
+    static_assert(NBI % G == 0 && 64 % CHUNKS == 0, "whole stores");
+    uint8_t* const to = own + (lane & 15) * ROW + (lane >> 4) * 8;
+    const uint8_t* const from = own + lane / CHUNKS * ROW + lane % CHUNKS * 16;
+    uint8_t* out = reinterpret_cast<uint8_t*>(p.out) + ((int64_t)(m0 + lane / CHUNKS) * p.ldo + n0 + lane % CHUNKS * 8) * 2;
+    const int64_t step = ROWS * 2 * p.ldo;
+    v4u line[STEPS];
+    auto store_group = [&]() __attribute__((always_inline)) {
+        typedef v4u loose_v4u __attribute__((aligned(2)));
+        if (ALWAYS_THROUGH || p.lines == kLinesThrough) {
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) store_through(out + s * step, line[s]);
+        } else {
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) *reinterpret_cast<loose_v4u*>(out + s * step) = line[s];
+        }
+        out += STEPS * step;
+    };
+#pragma unroll
+    for (int g = 0; g < NBI / G; ++g) {
+#pragma unroll
+        for (int ii = 0; ii < G; ++ii) {
+            const int i = g * G + ii;
+#pragma unroll
+            for (int j = 0; j < NBJ; ++j) *reinterpret_cast<uint2*>(to + i * 16 * ROW + j * 32) = outputs4<FP8, OUTK>(acc[j][i], sx[i], sw[j], bias[j]);
+            if (g > 0 && ii == 0) store_group();  // the group before: its reads have come back meanwhile
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the LDS serves a wavefront in order)
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) line[s] = *reinterpret_cast<const v4u*>(from + (g * G * 16 + s * ROWS) * ROW);
+    }
+    store_group();
+}
+
+// The epilogue of kernels that have no registers for the scales beside their main loop: a thread has requested one of each, and they
+// pass through the LDS.
 // OUTK: element type of out and bias, DAXQ_BF16 / DAXQ_F16 / DAXQ_F32.  A template argument, i.e. a kernel
 // of its own per type: with all three forms inside one kernel behind uniform branches its code grew from 27 to 44 KB
 // and the bf16 launches at K = 1536, which change between main loop and epilogue every 24 slices, lost 2.7 %; with
 // the choice inside the loops they lost 2 to 11 % everywhere.
-// sx, sw, bias: the scales of the lane's output row in each block of rows, scales and bias of its four columns in each block of columns.
-template <bool DUMP, int NBJ, int NBI, bool FP8, int OUTK>
-__device__ __forceinline__ void tile_outputs16(const GemmArgs& p, typename Acc16<FP8>::type (&acc)[NBJ][NBI], int m0, int n0, int l15, int g4,
-                                               const float (&sx)[NBI], const v4f (&sw)[NBJ], const v4f (&bias)[NBJ]) {
-    if constexpr (DUMP) dump_tile16<NBJ, NBI, FP8>(p, acc, m0, n0, l15, g4);
-    // a lane's place in the first block of rows; the others lie a uniform step apart, the blocks of columns at constant offsets
-    constexpr int XB = OUTK == DAXQ_F32 ? 4 : 2;
-    const int64_t step = 16 * p.ldo * XB;
-    uint8_t* row = reinterpret_cast<uint8_t*>(p.out) + ((int64_t)(m0 + l15) * p.ldo + n0) * XB;
-
-    // fp32 module: one rounding less and four-byte outputs, a lane's four columns of a block as one store
-    if constexpr (OUTK == DAXQ_F32) {
-        row += 16 * g4;
-#pragma unroll
-        for (int i = 0; i < NBI; ++i) {
-#pragma unroll
-            for (int j = 0; j < NBJ; ++j) {
-                float o[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float y = (float)acc[j][i][r];  // (int8: v_cvt_f32_i32, round to nearest even)
-                    y = y * sx[i];
-                    y = y * sw[j][r];
-                    o[r] = y + bias[j][r];
-                }
-                *reinterpret_cast<float4*>(row + j * 64) = make_float4(o[0], o[1], o[2], o[3]);
-            }
-            row += step;
-        }
-    } else {
-        uint8_t* last = row + 8 * g4;  // (of a block without a partner)
-        row += (g4 & 1) * 32 + (g4 >> 1) * 16;
-#pragma unroll
-        for (int i = 0; i < NBI; ++i) {
-#pragma unroll
-            for (int jp = 0; jp < (NBJ + 1) / 2; ++jp) {
-                const int j = 2 * jp;
-                const uint2 lo = outputs4<FP8, OUTK>(acc[j][i], sx[i], sw[j], bias[j]);
-                if (j + 1 == NBJ) {
-                    *reinterpret_cast<uint2*>(last + jp * 64) = lo;
-                    continue;
-                }
-                const int pj = j + 1 < NBJ ? j + 1 : j;
-                const uint2 up = outputs4<FP8, OUTK>(acc[pj][i], sx[i], sw[pj], bias[pj]);
-                v2u s0 = __builtin_amdgcn_permlane16_swap(lo.x, up.x, false, false);
-                v2u s1 = __builtin_amdgcn_permlane16_swap(lo.y, up.y, false, false);
-                *reinterpret_cast<uint4*>(row + jp * 64) = make_uint4(s0.x, s1.x, s0.y, s1.y);
-            }
-            row += step;
-            last += step;
-        }
-    }
-}
-
-// The same for kernels that have no registers for the scales beside their main loop: a thread has requested one of each, and they
-// pass through the LDS.
-template <bool DUMP, int NBJ, int NBI, bool FP8 = false, int OUTK = DAXQ_BF16, int WM = 2, int WN = 2>
+// LINES: 16-bit outputs leave as whole rows (lines_of says when).  A template argument for the same reason: as a uniform branch in the
+// kernel it cost 1 to 2 % (75600 x 5120 x 5120 e4m3 1564 -> 1592 us, 9830 x 5120, K = 1536 84.6 -> 85.7), and some FP8 forms spilled.
+template <bool DUMP, int NBJ, int NBI, bool FP8 = false, int OUTK = DAXQ_BF16, bool LINES = false, bool ALWAYS_THROUGH = false>
 __device__ __forceinline__ void tile_epilogue16(const GemmArgs& p, typename Acc16<FP8>::type (&acc)[NBJ][NBI], uint8_t* smem, int m0, int n0, int t,
                                                 int wm, int wn, int l15, int g4, float pre_sx, float pre_sw,
                                                 float pre_bias) {
-    constexpr int WTM = 16 * NBI, WTN = 16 * NBJ, BM = WM * WTM, BN = WN * WTN, T = 64 * WM * WN;
+    constexpr int WTM = 16 * NBI, WTN = 16 * NBJ, BM = 2 * WTM, BN = 2 * WTN, T = 256;
     float* s_sx = reinterpret_cast<float*>(smem);
     float* s_sw = s_sx + BM;
     float* s_bias = s_sw + BN;
@@ -244,7 +276,16 @@ __device__ __forceinline__ void tile_epilogue16(const GemmArgs& p, typename Acc1
         bias[j] = *reinterpret_cast<const v4f*>(s_bias + nl);
     }
     __builtin_amdgcn_sched_barrier(0);
-    tile_outputs16<DUMP, NBJ, NBI, FP8, OUTK>(p, acc, m0 + wm * WTM, n0 + wn * WTN, l15, g4, sx, sw, bias);
+    const int mw = m0 + wm * WTM, nw = n0 + wn * WTN;
+    if constexpr (DUMP) dump_tile16<NBJ, NBI, FP8>(p, acc, mw, nw, l15, g4);
+    if constexpr (OUTK == DAXQ_F32) {
+        outputs_f32<NBJ, NBI, FP8>(p, acc, mw, nw, l15, g4, sx, sw, bias);
+    } else if constexpr (LINES) {
+        uint8_t* const own = smem + (BM + 2 * BN) * 4 + (t >> 6) * (WTM * (2 * WTN + 16));
+        outputs_lines<NBJ, NBI, FP8, OUTK, ALWAYS_THROUGH>(p, acc, own, mw, nw, t & 63, sx, sw, bias);
+    } else {
+        outputs_straight<NBJ, NBI, FP8, OUTK>(p, acc, mw, nw, l15, g4, sx, sw, bias);
+    }
 }
 
 // CUs of the current device (0 if the query fails), asked once per device
@@ -291,6 +332,27 @@ static inline int tail_half_tiles(const GemmArgs& a, int tail) {
     const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n, rounds = tiles / cus, left = tiles - rounds * cus;
     if (rounds < 1 || 4 * left <= cus || 2 * left > cus) return 0;
     return (tail == 2 || rounds <= kTailMaxRounds) ? (int)left : 0;
+}
+
+// How the 16-bit outputs of 256x256 tiles leave (GemmArgs::lines).  128x128 and fitted tiles run in one round, or as a launch's last
+// one, and always take whole rows through the L2.
+// Straight from the registers a store instruction writes 16 rows x 64 bytes.  Whole rows (outputs_lines, 256 bytes each) cost a trip
+// through the LDS, which other workgroups' main loops hide as well or better over many rounds; with rows through the L2 less is left to
+// write back when the launch ends, which short launches feel.  Rows that start on odd elements are split by the path to the L2.
+// GEMM and quantiser, us, straight / whole rows / and through, INT8 unless noted:
+//   rounds, K = 1536: 3200 x 5120 (1.02) 36.2 / 35.9 / 35.3   6400 x 5120 (1.95) 53.5 / 54.1 / 51.9   9830 x 5120 (3.05) 84.6 / 85.3 / 83.7
+//     13000 x 5120 (4.0) 101.0 / 102.5 / 100.0   19600 x 5120 (6.0) 155.3 / 157.2 / 155.2   26000 x 5120 (8.0) 199.3 / 203.3 / 201.4
+//     32760 x 4608 (9) 228.1 / 230.2 / 230.3
+//   K = 5120: 4096 x 5120 per-tensor e5m2 (1.25) 99.7 / 99.1 / 96.7   6400 x 5120 (1.95) 132.7 / 132.9 / 132.3   9830 x 5120 (3.05) 213.0 / 213.1 / 211.5
+//     13000 x 5120 (4.0) 262.0 / 262.6 / 264.4   75600 x 5120 e4m3 1523 / 1526 / 1530
+//   row starts, 6400 rows, K = 1536: N = 5119 73.5 / 54.6 / 54.6   5124 62.6 / 62.2 / 63.3   5136 61.2 / 62.1 / 61.8   5152 61.3 / 62.0 / 60.8
+//     20000 rows: N = 5119 219.1 / 162.3 / 167.2   5124 164.7 / 164.7 / 170.3   5152 160.1 / 163.6 / 164.7
+static inline int lines_of(const GemmArgs& a) {
+    if (a.acc || a.out_kind == DAXQ_F32) return kLinesNone;
+    const uint64_t at = (uint64_t)(uintptr_t)a.out | (uint64_t)a.ldo * 2;
+    if (at & 2) return kLinesPlain;  // (the last bit of ldo: rows on odd elements)
+    const int64_t rounds = a.k < 4096 ? 4 : 2;
+    return (at & 63) == 0 && (int64_t)a.m * a.n <= rounds * 65536 * cu_count() ? kLinesThrough : kLinesNone;
 }
 
 }  // namespace daxq

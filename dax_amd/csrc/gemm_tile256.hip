@@ -141,7 +141,7 @@ struct TileAcc<false, true> {
 // counts itself in at the tile's counter; the workgroup that arrives last adds the partial results of all ranges
 // in range order (so FP8 sums do not depend on who was last) and runs the epilogue.  No workgroup waits for
 // another.  The last one sets the counter back to zero.
-template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, bool SPLITK = false, int D = 2, int OUTK = DAXQ_BF16>
+template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, bool SPLITK = false, int D = 2, int OUTK = DAXQ_BF16, bool LINES = false>
 __device__ __forceinline__ void gemm_tile256s5_body(const GemmArgs& p, const int block) {
     static_assert(OUTK == DAXQ_BF16 || (N16 && !SPLITK && !DUMP), "fp16 / fp32 outputs exist in the 16x16 int8 form");
     using namespace t5;
@@ -482,39 +482,39 @@ __device__ __forceinline__ void gemm_tile256s5_body(const GemmArgs& p, const int
         __syncthreads();                      // every thread has read the flag before the epilogue reuses the LDS
     }
     if constexpr (N16)
-        tile_epilogue16<DUMP, NB, NB, false, OUTK>(p, acc, smem, m0, n0, t, wm, wn, lr, lane >> 4, pre_sx, pre_sw,
+        tile_epilogue16<DUMP, NB, NB, false, OUTK, LINES || BT == 128, BT == 128>(p, acc, smem, m0, n0, t, wm, wn, lr, lane >> 4, pre_sx, pre_sw,
                                                   !p.bias ? -0.0f : OUTK == DAXQ_F32 ? __uint_as_float(pre_b) : OUTK == DAXQ_F16 ? f16_bits_to_f32((uint16_t)pre_b) : bf16_bits_to_f32(pre_b));
     else
         tile256_epilogue<NB>(p, acc, smem, m0, n0, t, wm, wn, l31, hi, pre_sx, pre_sw,
                                         p.bias ? bf16_bits_to_f32(pre_b) : -0.0f);
 }
 
-template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, bool SPLITK = false, int D = 2, int OUTK = DAXQ_BF16>
+template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, bool SPLITK = false, int D = 2, int OUTK = DAXQ_BF16, bool LINES = false>
 __global__ __launch_bounds__(256) void gemm_tile256s5_kernel(const GemmArgs p) {
-    gemm_tile256s5_body<FP8, DUMP, F8, N16, BT, SPLITK, D, OUTK>(p, (int)blockIdx.x);
+    gemm_tile256s5_body<FP8, DUMP, F8, N16, BT, SPLITK, D, OUTK, LINES>(p, (int)blockIdx.x);
 }
 
 // One grid for a launch of few rounds whose left-over tiles run as halves (tail_half_tiles): workgroups 0 .. p.grid - 1
 // compute whole 256x256 tiles, the rest the 256x128 halves of the tiles from id quad_base - 1 on.  The halves start on
 // the CUs that finish their whole tiles first instead of behind the whole first kernel.
-template <bool DUMP, int OUTK>
+template <bool DUMP, int OUTK, bool LINES>
 __global__ __launch_bounds__(256) void gemm_tile256_then_halves_kernel(const GemmArgs p) {
-    if ((int)blockIdx.x < p.grid) gemm_tile256s5_body<false, DUMP, 0, true, 256, false, 2, OUTK>(p, (int)blockIdx.x);
+    if ((int)blockIdx.x < p.grid) gemm_tile256s5_body<false, DUMP, 0, true, 256, false, 2, OUTK, LINES>(p, (int)blockIdx.x);
     else gemm_half_body<false, 0, DUMP, OUTK>(p, (int)blockIdx.x - p.grid);
 }
 
 // The same for left-over tiles that run as 128x128 quadrants (tail_tiles): workgroups 0 .. p.grid - 1 compute whole
 // tiles, the rest the quadrants of the tiles from id quad_base - 1 on (D: pairs of slices the quadrants keep in flight).
-template <bool DUMP, int OUTK, int D>
+template <bool DUMP, int OUTK, int D, bool LINES>
 __global__ __launch_bounds__(256) void gemm_tile256_then_quadrants_kernel(const GemmArgs p) {
-    if ((int)blockIdx.x < p.grid) gemm_tile256s5_body<false, DUMP, 0, true, 256, false, 2, OUTK>(p, (int)blockIdx.x);
+    if ((int)blockIdx.x < p.grid) gemm_tile256s5_body<false, DUMP, 0, true, 256, false, 2, OUTK, LINES>(p, (int)blockIdx.x);
     else gemm_tile256s5_body<false, DUMP, 0, true, 128, false, D, OUTK>(p, (int)blockIdx.x - p.grid);
 }
 
-template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, bool SPLITK = false, int D = 2, int OUTK = DAXQ_BF16>
+template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, bool SPLITK = false, int D = 2, int OUTK = DAXQ_BF16, bool LINES = false>
 static int prepare_tile256s5() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256s5_kernel<FP8, DUMP, F8, N16, BT, SPLITK, D, OUTK>),
+    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256s5_kernel<FP8, DUMP, F8, N16, BT, SPLITK, D, OUTK, LINES>),
                               (2 * D + 1) * BT * t5::BKP, lds_set);
 }
 
@@ -536,6 +536,7 @@ int launch_tile128_splitk(const GemmArgs& a0, int f8, hipStream_t st) {
     GemmArgs a = a0;
     a.tiles_m = (a.m + 127) / 128;
     a.tiles_n = (a.n + 127) / 128;
+    a.lines = lines_of(a);
     if constexpr (FP8) {
         switch (f8) {
             case 1: return launch_splitk_impl<true, 1>(a, st);
@@ -551,13 +552,13 @@ int launch_tile128_splitk(const GemmArgs& a0, int f8, hipStream_t st) {
 template int launch_tile128_splitk<false>(const GemmArgs&, int, hipStream_t);
 template int launch_tile128_splitk<true>(const GemmArgs&, int, hipStream_t);
 
-template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, int D = 2, int OUTK = DAXQ_BF16>
+template <bool FP8, bool DUMP, int F8, bool N16 = false, int BT = 256, int D = 2, int OUTK = DAXQ_BF16, bool LINES = false>
 static int launch_tile256s5_impl(const GemmArgs& a, hipStream_t st) {
     using namespace t5;
     constexpr int SMEM = (2 * D + 1) * BT * BKP;  // 160 KB (256 tile), 80 KB (128 tile), 144 KB (128 tile, nine parts)
     if (a.out_kind != OUTK) return fail(DAXQ_ERR_ARG, "gemm: this kernel writes output type %d, not %d", OUTK, a.out_kind);
-    auto kern = gemm_tile256s5_kernel<FP8, DUMP, F8, N16, BT, false, D, OUTK>;
-    if (int rc = prepare_tile256s5<FP8, DUMP, F8, N16, BT, false, D, OUTK>()) return rc;
+    auto kern = gemm_tile256s5_kernel<FP8, DUMP, F8, N16, BT, false, D, OUTK, LINES>;
+    if (int rc = prepare_tile256s5<FP8, DUMP, F8, N16, BT, false, D, OUTK, LINES>()) return rc;
     const int64_t nt = grid_of_order(a);
     if (nt > 0x7fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
     launch_kernel(kern, dim3((unsigned)nt), dim3(T), SMEM, st, a);
@@ -590,24 +591,25 @@ static int launch_i8_one(const GemmArgs& a, bool small, hipStream_t st) {
         if (a.out_kind == DAXQ_F32) return launch_i8_128_out<DAXQ_F32>(a, st);
         return launch_i8_128_out<DAXQ_BF16>(a, st);
     }
-    if (a.out_kind == DAXQ_F16) return launch_tile256s5_impl<false, false, 0, true, 256, 2, DAXQ_F16>(a, st);
     if (a.out_kind == DAXQ_F32) return launch_tile256s5_impl<false, false, 0, true, 256, 2, DAXQ_F32>(a, st);
+    if (a.lines) return a.out_kind == DAXQ_F16 ? launch_tile256s5_impl<false, false, 0, true, 256, 2, DAXQ_F16, true>(a, st) : launch_tile256s5_impl<false, false, 0, true, 256, 2, DAXQ_BF16, true>(a, st);
+    if (a.out_kind == DAXQ_F16) return launch_tile256s5_impl<false, false, 0, true, 256, 2, DAXQ_F16>(a, st);
     return a.acc ? launch_tile256s5_impl<false, true, 0, true>(a, st) : launch_tile256s5_impl<false, false, 0, true>(a, st);
 }
 
 // The last, partial round of a launch of 256x256 tiles in smaller pieces with a CU each: tail_tiles (quadrants) and
 // tail_half_tiles (halves) in gemm_tile.h say which tiles, the kernels above run them in the same grid, behind the
 // whole tiles.  tail: 0 = by shape, 1 = never, 2 = whenever every piece gets a CU
-template <bool DUMP, int OUTK>
+template <bool DUMP, int OUTK, bool LINES>
 static int prepare_then_halves() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256_then_halves_kernel<DUMP, OUTK>), 5 * 256 * t5::BKP, lds_set);
+    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256_then_halves_kernel<DUMP, OUTK, LINES>), 5 * 256 * t5::BKP, lds_set);
 }
 
-template <bool DUMP, int OUTK>
+template <bool DUMP, int OUTK, bool LINES>
 static int launch_then_halves_impl(const GemmArgs& a, int64_t nt, hipStream_t st) {
-    if (int rc = prepare_then_halves<DUMP, OUTK>()) return rc;
-    launch_kernel((gemm_tile256_then_halves_kernel<DUMP, OUTK>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
+    if (int rc = prepare_then_halves<DUMP, OUTK, LINES>()) return rc;
+    launch_kernel((gemm_tile256_then_halves_kernel<DUMP, OUTK, LINES>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
     return check_launch("gemm_tile256_then_halves");
 }
 
@@ -619,30 +621,32 @@ static int launch_then_halves(const GemmArgs& a0, int whole, int halves, hipStre
     const int64_t nt = (int64_t)whole + 2 * (int64_t)halves;
     if (nt > 0x7fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
     if (a.acc && a.out_kind != DAXQ_BF16) return fail(DAXQ_ERR_ARG, "gemm: the accumulator dump exists with bf16 outputs");
-    if (a.out_kind == DAXQ_F16) return launch_then_halves_impl<false, DAXQ_F16>(a, nt, st);
-    if (a.out_kind == DAXQ_F32) return launch_then_halves_impl<false, DAXQ_F32>(a, nt, st);
-    return a.acc ? launch_then_halves_impl<true, DAXQ_BF16>(a, nt, st) : launch_then_halves_impl<false, DAXQ_BF16>(a, nt, st);
+    if (a.out_kind == DAXQ_F32) return launch_then_halves_impl<false, DAXQ_F32, false>(a, nt, st);
+    if (a.acc) return launch_then_halves_impl<true, DAXQ_BF16, false>(a, nt, st);
+    if (a.lines) return a.out_kind == DAXQ_F16 ? launch_then_halves_impl<false, DAXQ_F16, true>(a, nt, st) : launch_then_halves_impl<false, DAXQ_BF16, true>(a, nt, st);
+    return a.out_kind == DAXQ_F16 ? launch_then_halves_impl<false, DAXQ_F16, false>(a, nt, st) : launch_then_halves_impl<false, DAXQ_BF16, false>(a, nt, st);
 }
 
-template <bool DUMP, int OUTK, int D>
+template <bool DUMP, int OUTK, int D, bool LINES>
 static int prepare_then_quadrants() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D>), 5 * 256 * t5::BKP, lds_set);
+    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D, LINES>), 5 * 256 * t5::BKP, lds_set);
 }
 
-template <bool DUMP, int OUTK, int D>
+template <bool DUMP, int OUTK, int D, bool LINES>
 static int launch_then_quadrants_impl(const GemmArgs& a, int64_t nt, hipStream_t st) {
-    if (int rc = prepare_then_quadrants<DUMP, OUTK, D>()) return rc;
-    launch_kernel((gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
+    if (int rc = prepare_then_quadrants<DUMP, OUTK, D, LINES>()) return rc;
+    launch_kernel((gemm_tile256_then_quadrants_kernel<DUMP, OUTK, D, LINES>), dim3((unsigned)nt), dim3(t5::T), 5 * 256 * t5::BKP, st, a);
     return check_launch("gemm_tile256_then_quadrants");
 }
 
 template <int D>
 static int launch_then_quadrants_out(const GemmArgs& a, int64_t nt, hipStream_t st) {
     if (a.acc && a.out_kind != DAXQ_BF16) return fail(DAXQ_ERR_ARG, "gemm: the accumulator dump exists with bf16 outputs");
-    if (a.out_kind == DAXQ_F16) return launch_then_quadrants_impl<false, DAXQ_F16, D>(a, nt, st);
-    if (a.out_kind == DAXQ_F32) return launch_then_quadrants_impl<false, DAXQ_F32, D>(a, nt, st);
-    return a.acc ? launch_then_quadrants_impl<true, DAXQ_BF16, D>(a, nt, st) : launch_then_quadrants_impl<false, DAXQ_BF16, D>(a, nt, st);
+    if (a.out_kind == DAXQ_F32) return launch_then_quadrants_impl<false, DAXQ_F32, D, false>(a, nt, st);
+    if (a.acc) return launch_then_quadrants_impl<true, DAXQ_BF16, D, false>(a, nt, st);
+    if (a.lines) return a.out_kind == DAXQ_F16 ? launch_then_quadrants_impl<false, DAXQ_F16, D, true>(a, nt, st) : launch_then_quadrants_impl<false, DAXQ_BF16, D, true>(a, nt, st);
+    return a.out_kind == DAXQ_F16 ? launch_then_quadrants_impl<false, DAXQ_F16, D, false>(a, nt, st) : launch_then_quadrants_impl<false, DAXQ_BF16, D, false>(a, nt, st);
 }
 
 // `whole` 256x256 tiles of the row-group order, then the four quadrants of each of the `left` tiles behind them, in one
@@ -662,6 +666,7 @@ int launch_halves_i8(const GemmArgs& a0, hipStream_t st) {
     a.tiles_m = (a.m + 255) / 256;
     a.tiles_n = (a.n + 255) / 256;
     a.order = kOrderRowGroups;
+    a.lines = lines_of(a);
     const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
     if (tiles > 0x3fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
     return launch_then_halves(a, 0, (int)tiles, st);
@@ -673,6 +678,7 @@ int launch_tile_i8(const GemmArgs& a0, bool small, int tail, hipStream_t st) {
     a.tiles_m = (a.m + bt - 1) / bt;
     a.tiles_n = (a.n + bt - 1) / bt;
     a.grid = a.quad_base = 0;
+    a.lines = lines_of(a);
     if (small) a.order = kOrderRowGroups;
     const int left = small ? 0 : tail_tiles(a, tail);
     if (left == 0) {
@@ -690,6 +696,8 @@ int prepare_tile256_kernels() {
 #define DAXQ_PREP(...) if (!rc) rc = __VA_ARGS__()
     DAXQ_PREP(prepare_tile256s5<false, false, 0, true, 256>);
     DAXQ_PREP(prepare_tile256s5<false, true, 0, true, 256>);
+    DAXQ_PREP(prepare_tile256s5<false, false, 0, true, 256, false, 2, DAXQ_BF16, true>);
+    DAXQ_PREP(prepare_tile256s5<false, false, 0, true, 256, false, 2, DAXQ_F16, true>);
     DAXQ_PREP(prepare_tile256s5<false, false, 0, true, 128>);
     DAXQ_PREP(prepare_tile256s5<false, true, 0, true, 128>);
     DAXQ_PREP(prepare_tile256s5<false, false, 0, true, 128, false, 4>);
@@ -705,18 +713,24 @@ int prepare_tile256_kernels() {
     DAXQ_PREP(prepare_tile256s5<true, false, 1, false, 128, true>);
     DAXQ_PREP(prepare_tile256s5<true, false, 2, false, 128, true>);
     DAXQ_PREP(prepare_tile256s5<true, false, 3, false, 128, true>);
-    DAXQ_PREP(prepare_then_halves<false, DAXQ_BF16>);
-    DAXQ_PREP(prepare_then_halves<true, DAXQ_BF16>);
-    DAXQ_PREP(prepare_then_halves<false, DAXQ_F16>);
-    DAXQ_PREP(prepare_then_halves<false, DAXQ_F32>);
-    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_BF16, 2>);
-    DAXQ_PREP(prepare_then_quadrants<true, DAXQ_BF16, 2>);
-    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F16, 2>);
-    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F32, 2>);
-    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_BF16, 4>);
-    DAXQ_PREP(prepare_then_quadrants<true, DAXQ_BF16, 4>);
-    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F16, 4>);
-    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F32, 4>);
+    DAXQ_PREP(prepare_then_halves<false, DAXQ_BF16, false>);
+    DAXQ_PREP(prepare_then_halves<false, DAXQ_BF16, true>);
+    DAXQ_PREP(prepare_then_halves<true, DAXQ_BF16, false>);
+    DAXQ_PREP(prepare_then_halves<false, DAXQ_F16, false>);
+    DAXQ_PREP(prepare_then_halves<false, DAXQ_F16, true>);
+    DAXQ_PREP(prepare_then_halves<false, DAXQ_F32, false>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_BF16, 2, false>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_BF16, 2, true>);
+    DAXQ_PREP(prepare_then_quadrants<true, DAXQ_BF16, 2, false>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F16, 2, false>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F16, 2, true>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F32, 2, false>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_BF16, 4, false>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_BF16, 4, true>);
+    DAXQ_PREP(prepare_then_quadrants<true, DAXQ_BF16, 4, false>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F16, 4, false>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F16, 4, true>);
+    DAXQ_PREP(prepare_then_quadrants<false, DAXQ_F32, 4, false>);
 #undef DAXQ_PREP
     return rc;
 }

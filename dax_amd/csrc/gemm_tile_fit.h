@@ -291,10 +291,10 @@ __device__ __forceinline__ void gemm_fit_body(const GemmArgs& p, const int m0, c
             }
             if (!p.bias) bias[j][r] = -0.0f;
         }
+    if constexpr (DUMP) dump_tile16<NBJ, NBI, FP8>(p, acc, mw, nw, lr, kg);
     if constexpr (!LINES) {
-        tile_outputs16<DUMP, NBJ, NBI, FP8, OUTK>(p, acc, mw, nw, lr, kg, sx, sw, bias);
+        outputs_f32<NBJ, NBI, FP8>(p, acc, mw, nw, lr, kg, sx, sw, bias);
     } else {
-        if constexpr (DUMP) dump_tile16<NBJ, NBI, FP8>(p, acc, mw, nw, lr, kg);
         uint8_t* const to = smem + (wm * 16 * L::G + lr) * L::OUT_ROW + (wn * 16 * NBJ + 4 * kg) * 2;
         uint8_t* const out = reinterpret_cast<uint8_t*>(p.out) + ((int64_t)m0 * p.ldo + n0) * 2;
         v4u line[L::STEPS];

@@ -42,7 +42,7 @@ namespace f16 {
 constexpr int BKP = 128, T = 256, NPART = 5;
 }  // namespace f16
 
-template <bool DUMP, int F8, int BT = 256, int OUTK = DAXQ_BF16>
+template <bool DUMP, int F8, int BT = 256, int OUTK = DAXQ_BF16, bool LINES = false>
 __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int block) {
     using namespace f16;
     static_assert(BT == 256 || BT == 128, "tile edge");
@@ -351,52 +351,54 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
                            "+a"(acc[j + 1][1]), "+a"(acc[j + 1][2]), "+a"(acc[j + 1][3]));
         }
     }
-    tile_epilogue16<DUMP, NB, NB, true, OUTK>(p, acc, smem, m0, n0, t, wm, wn, lr, kg, pre_sx, pre_sw,
+    tile_epilogue16<DUMP, NB, NB, true, OUTK, LINES || BT == 128, BT == 128>(p, acc, smem, m0, n0, t, wm, wn, lr, kg, pre_sx, pre_sw,
                                              !p.bias ? -0.0f : OUTK == DAXQ_F32 ? __uint_as_float(pre_b) : OUTK == DAXQ_F16 ? f16_bits_to_f32((uint16_t)pre_b) : bf16_bits_to_f32(pre_b));
 }
 
-template <bool DUMP, int F8, int BT = 256, int OUTK = DAXQ_BF16>
+template <bool DUMP, int F8, int BT, int OUTK, bool LINES>
 __global__ __launch_bounds__(256) void gemm_tile_fp8_kernel(const GemmArgs p) {
-    gemm_tile_fp8_body<DUMP, F8, BT, OUTK>(p, (int)blockIdx.x);
+    gemm_tile_fp8_body<DUMP, F8, BT, OUTK, LINES>(p, (int)blockIdx.x);
 }
 
 // One grid for a launch of few rounds whose left-over tiles run as halves (tail_half_tiles): workgroups 0 .. p.grid - 1
 // compute whole 256x256 tiles, the rest the 256x128 halves of the tiles from id quad_base - 1 on.  The halves start on
 // the CUs that finish their whole tiles first instead of behind the whole first kernel.
-template <bool DUMP, int F8, int OUTK>
+template <bool DUMP, int F8, int OUTK, bool LINES>
 __global__ __launch_bounds__(256) void gemm_tile_fp8_then_halves_kernel(const GemmArgs p) {
-    if ((int)blockIdx.x < p.grid) gemm_tile_fp8_body<DUMP, F8, 256, OUTK>(p, (int)blockIdx.x);
+    if ((int)blockIdx.x < p.grid) gemm_tile_fp8_body<DUMP, F8, 256, OUTK, LINES>(p, (int)blockIdx.x);
     else gemm_half_body<true, F8, DUMP, OUTK>(p, (int)blockIdx.x - p.grid);
 }
 
 // The same for left-over tiles that run as 128x128 quadrants (tail_tiles): workgroups 0 .. p.grid - 1 compute whole
 // tiles, the rest the quadrants of the tiles from id quad_base - 1 on.
-template <bool DUMP, int F8, int OUTK>
+template <bool DUMP, int F8, int OUTK, bool LINES>
 __global__ __launch_bounds__(256) void gemm_tile_fp8_then_quadrants_kernel(const GemmArgs p) {
-    if ((int)blockIdx.x < p.grid) gemm_tile_fp8_body<DUMP, F8, 256, OUTK>(p, (int)blockIdx.x);
+    if ((int)blockIdx.x < p.grid) gemm_tile_fp8_body<DUMP, F8, 256, OUTK, LINES>(p, (int)blockIdx.x);
     else gemm_tile_fp8_body<DUMP, F8, 128, OUTK>(p, (int)blockIdx.x - p.grid);
 }
 
-template <bool DUMP, int F8, int BT, int OUTK>
+template <bool DUMP, int F8, int BT, int OUTK, bool LINES>
 static int prepare_fp8() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK>), f16::NPART * BT * f16::BKP, lds_set);
+    return ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK, LINES>), f16::NPART * BT * f16::BKP, lds_set);
 }
 
-template <bool DUMP, int F8, int BT, int OUTK>
+template <bool DUMP, int F8, int BT, int OUTK, bool LINES>
 static int launch_fp8_impl(const GemmArgs& a, hipStream_t st) {
-    if (int rc = prepare_fp8<DUMP, F8, BT, OUTK>()) return rc;
+    if (int rc = prepare_fp8<DUMP, F8, BT, OUTK, LINES>()) return rc;
     const int64_t nt = grid_of_order(a);
     if (nt > 0x7fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
-    launch_kernel((gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK>), dim3((unsigned)nt), dim3(f16::T), f16::NPART * BT * f16::BKP, st, a);
+    launch_kernel((gemm_tile_fp8_kernel<DUMP, F8, BT, OUTK, LINES>), dim3((unsigned)nt), dim3(f16::T), f16::NPART * BT * f16::BKP, st, a);
     return check_launch("gemm_tile_fp8");
 }
 
 template <int F8, int BT>
 static int launch_fp8_out(const GemmArgs& a, hipStream_t st) {
-    if (a.out_kind == DAXQ_F16) return a.acc ? fail(DAXQ_ERR_ARG, "gemm: the accumulator dump exists with bf16 outputs") : launch_fp8_impl<false, F8, BT, DAXQ_F16>(a, st);
-    if (a.out_kind == DAXQ_F32) return a.acc ? fail(DAXQ_ERR_ARG, "gemm: the accumulator dump exists with bf16 outputs") : launch_fp8_impl<false, F8, BT, DAXQ_F32>(a, st);
-    return a.acc ? launch_fp8_impl<true, F8, BT, DAXQ_BF16>(a, st) : launch_fp8_impl<false, F8, BT, DAXQ_BF16>(a, st);
+    if (a.acc && a.out_kind != DAXQ_BF16) return fail(DAXQ_ERR_ARG, "gemm: the accumulator dump exists with bf16 outputs");
+    if (a.out_kind == DAXQ_F32) return launch_fp8_impl<false, F8, BT, DAXQ_F32, false>(a, st);
+    if (a.acc) return launch_fp8_impl<true, F8, BT, DAXQ_BF16, false>(a, st);
+    if (BT == 256 && a.lines) return a.out_kind == DAXQ_F16 ? launch_fp8_impl<false, F8, BT, DAXQ_F16, BT == 256>(a, st) : launch_fp8_impl<false, F8, BT, DAXQ_BF16, BT == 256>(a, st);
+    return a.out_kind == DAXQ_F16 ? launch_fp8_impl<false, F8, BT, DAXQ_F16, false>(a, st) : launch_fp8_impl<false, F8, BT, DAXQ_BF16, false>(a, st);
 }
 
 template <int BT>
@@ -410,33 +412,34 @@ static int launch_fp8_one(const GemmArgs& a, int f8, hipStream_t st) {
 }
 
 // QUADS: the second part of the grid is quadrants (else halves)
-template <bool QUADS, bool DUMP, int F8, int OUTK>
+template <bool QUADS, bool DUMP, int F8, int OUTK, bool LINES>
 static const void* fp8_then_kernel() {
-    if constexpr (QUADS) return reinterpret_cast<const void*>(gemm_tile_fp8_then_quadrants_kernel<DUMP, F8, OUTK>);
-    else return reinterpret_cast<const void*>(gemm_tile_fp8_then_halves_kernel<DUMP, F8, OUTK>);
+    if constexpr (QUADS) return reinterpret_cast<const void*>(gemm_tile_fp8_then_quadrants_kernel<DUMP, F8, OUTK, LINES>);
+    else return reinterpret_cast<const void*>(gemm_tile_fp8_then_halves_kernel<DUMP, F8, OUTK, LINES>);
 }
 
-template <bool QUADS, bool DUMP, int F8, int OUTK>
+template <bool QUADS, bool DUMP, int F8, int OUTK, bool LINES>
 static int prepare_fp8_then() {
     static std::atomic<uint64_t> lds_set{0};  // per instantiation
-    return ensure_dynamic_lds(fp8_then_kernel<QUADS, DUMP, F8, OUTK>(), f16::NPART * 256 * f16::BKP, lds_set);
+    return ensure_dynamic_lds(fp8_then_kernel<QUADS, DUMP, F8, OUTK, LINES>(), f16::NPART * 256 * f16::BKP, lds_set);
 }
 
-template <bool QUADS, bool DUMP, int F8, int OUTK>
+template <bool QUADS, bool DUMP, int F8, int OUTK, bool LINES>
 static int launch_fp8_then_impl(const GemmArgs& a, int64_t nt, hipStream_t st) {
-    if (int rc = prepare_fp8_then<QUADS, DUMP, F8, OUTK>()) return rc;
+    if (int rc = prepare_fp8_then<QUADS, DUMP, F8, OUTK, LINES>()) return rc;
     constexpr int SMEM = f16::NPART * 256 * f16::BKP;
-    if constexpr (QUADS) launch_kernel((gemm_tile_fp8_then_quadrants_kernel<DUMP, F8, OUTK>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
-    else launch_kernel((gemm_tile_fp8_then_halves_kernel<DUMP, F8, OUTK>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
+    if constexpr (QUADS) launch_kernel((gemm_tile_fp8_then_quadrants_kernel<DUMP, F8, OUTK, LINES>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
+    else launch_kernel((gemm_tile_fp8_then_halves_kernel<DUMP, F8, OUTK, LINES>), dim3((unsigned)nt), dim3(f16::T), SMEM, st, a);
     return check_launch(QUADS ? "gemm_tile_fp8_then_quadrants" : "gemm_tile_fp8_then_halves");
 }
 
 template <bool QUADS, int F8>
 static int launch_fp8_then_out(const GemmArgs& a, int64_t nt, hipStream_t st) {
     if (a.acc && a.out_kind != DAXQ_BF16) return fail(DAXQ_ERR_ARG, "gemm: the accumulator dump exists with bf16 outputs");
-    if (a.out_kind == DAXQ_F16) return launch_fp8_then_impl<QUADS, false, F8, DAXQ_F16>(a, nt, st);
-    if (a.out_kind == DAXQ_F32) return launch_fp8_then_impl<QUADS, false, F8, DAXQ_F32>(a, nt, st);
-    return a.acc ? launch_fp8_then_impl<QUADS, true, F8, DAXQ_BF16>(a, nt, st) : launch_fp8_then_impl<QUADS, false, F8, DAXQ_BF16>(a, nt, st);
+    if (a.out_kind == DAXQ_F32) return launch_fp8_then_impl<QUADS, false, F8, DAXQ_F32, false>(a, nt, st);
+    if (a.acc) return launch_fp8_then_impl<QUADS, true, F8, DAXQ_BF16, false>(a, nt, st);
+    if (a.lines) return a.out_kind == DAXQ_F16 ? launch_fp8_then_impl<QUADS, false, F8, DAXQ_F16, true>(a, nt, st) : launch_fp8_then_impl<QUADS, false, F8, DAXQ_BF16, true>(a, nt, st);
+    return a.out_kind == DAXQ_F16 ? launch_fp8_then_impl<QUADS, false, F8, DAXQ_F16, false>(a, nt, st) : launch_fp8_then_impl<QUADS, false, F8, DAXQ_BF16, false>(a, nt, st);
 }
 
 // `whole` 256x256 tiles of the row-group order, then the pieces of each of the `left` tiles behind them (QUADS: four
@@ -462,6 +465,7 @@ int launch_halves_fp8(const GemmArgs& a0, int f8, hipStream_t st) {
     a.tiles_m = (a.m + 255) / 256;
     a.tiles_n = (a.n + 255) / 256;
     a.order = kOrderRowGroups;
+    a.lines = lines_of(a);
     const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
     if (tiles > 0x3fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
     return launch_fp8_then<false>(a, f8, 0, (int)tiles, st);
@@ -476,6 +480,7 @@ int launch_tile_fp8(const GemmArgs& a0, int f8, bool small, int tail, hipStream_
     a.tiles_m = (a.m + bt - 1) / bt;
     a.tiles_n = (a.n + bt - 1) / bt;
     a.grid = a.quad_base = 0;
+    a.lines = lines_of(a);
     if (small) {
         a.order = kOrderRowGroups;
         return launch_fp8_one<128>(a, f8, st);
@@ -495,23 +500,29 @@ int launch_tile_fp8(const GemmArgs& a0, int f8, bool small, int tail, hipStream_
 int prepare_tile_fp8_kernels() {
     int rc = 0;
 #define DAXQ_PREP(...) if (!rc) rc = __VA_ARGS__()
-#define DAXQ_PREP_F8(F8)                                  \
-    DAXQ_PREP(prepare_fp8<false, F8, 256, DAXQ_BF16>);    \
-    DAXQ_PREP(prepare_fp8<true, F8, 256, DAXQ_BF16>);     \
-    DAXQ_PREP(prepare_fp8<false, F8, 256, DAXQ_F16>);     \
-    DAXQ_PREP(prepare_fp8<false, F8, 256, DAXQ_F32>);     \
-    DAXQ_PREP(prepare_fp8<false, F8, 128, DAXQ_BF16>);    \
-    DAXQ_PREP(prepare_fp8<true, F8, 128, DAXQ_BF16>);     \
-    DAXQ_PREP(prepare_fp8<false, F8, 128, DAXQ_F16>);     \
-    DAXQ_PREP(prepare_fp8<false, F8, 128, DAXQ_F32>);     \
-    DAXQ_PREP(prepare_fp8_then<false, false, F8, DAXQ_BF16>); \
-    DAXQ_PREP(prepare_fp8_then<false, true, F8, DAXQ_BF16>);  \
-    DAXQ_PREP(prepare_fp8_then<false, false, F8, DAXQ_F16>);  \
-    DAXQ_PREP(prepare_fp8_then<false, false, F8, DAXQ_F32>);  \
-    DAXQ_PREP(prepare_fp8_then<true, false, F8, DAXQ_BF16>);  \
-    DAXQ_PREP(prepare_fp8_then<true, true, F8, DAXQ_BF16>);   \
-    DAXQ_PREP(prepare_fp8_then<true, false, F8, DAXQ_F16>);   \
-    DAXQ_PREP(prepare_fp8_then<true, false, F8, DAXQ_F32>)
+#define DAXQ_PREP_F8(F8)                                                 \
+    DAXQ_PREP(prepare_fp8<false, F8, 256, DAXQ_BF16, false>);            \
+    DAXQ_PREP(prepare_fp8<false, F8, 256, DAXQ_BF16, true>);             \
+    DAXQ_PREP(prepare_fp8<true, F8, 256, DAXQ_BF16, false>);             \
+    DAXQ_PREP(prepare_fp8<false, F8, 256, DAXQ_F16, false>);             \
+    DAXQ_PREP(prepare_fp8<false, F8, 256, DAXQ_F16, true>);              \
+    DAXQ_PREP(prepare_fp8<false, F8, 256, DAXQ_F32, false>);             \
+    DAXQ_PREP(prepare_fp8<false, F8, 128, DAXQ_BF16, false>);            \
+    DAXQ_PREP(prepare_fp8<true, F8, 128, DAXQ_BF16, false>);             \
+    DAXQ_PREP(prepare_fp8<false, F8, 128, DAXQ_F16, false>);             \
+    DAXQ_PREP(prepare_fp8<false, F8, 128, DAXQ_F32, false>);             \
+    DAXQ_PREP(prepare_fp8_then<false, false, F8, DAXQ_BF16, false>);     \
+    DAXQ_PREP(prepare_fp8_then<false, false, F8, DAXQ_BF16, true>);      \
+    DAXQ_PREP(prepare_fp8_then<false, true, F8, DAXQ_BF16, false>);      \
+    DAXQ_PREP(prepare_fp8_then<false, false, F8, DAXQ_F16, false>);      \
+    DAXQ_PREP(prepare_fp8_then<false, false, F8, DAXQ_F16, true>);       \
+    DAXQ_PREP(prepare_fp8_then<false, false, F8, DAXQ_F32, false>);      \
+    DAXQ_PREP(prepare_fp8_then<true, false, F8, DAXQ_BF16, false>);      \
+    DAXQ_PREP(prepare_fp8_then<true, false, F8, DAXQ_BF16, true>);       \
+    DAXQ_PREP(prepare_fp8_then<true, true, F8, DAXQ_BF16, false>);       \
+    DAXQ_PREP(prepare_fp8_then<true, false, F8, DAXQ_F16, false>);       \
+    DAXQ_PREP(prepare_fp8_then<true, false, F8, DAXQ_F16, true>);        \
+    DAXQ_PREP(prepare_fp8_then<true, false, F8, DAXQ_F32, false>)
     DAXQ_PREP_F8(0);
     DAXQ_PREP_F8(1);
     DAXQ_PREP_F8(2);

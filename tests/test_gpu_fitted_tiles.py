@@ -119,6 +119,17 @@ def test_fp16_sums_of_every_rounded_product():
         assert bool(same.all())
 
 
+@pytest.mark.parametrize("out", ["bf16", "fp16"])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("n", [4088, 4089, 4092])  # rows of outputs 8192 bytes apart, an odd number of elements, neither
+@pytest.mark.parametrize("m", [300, 4300, 5300])  # whole tiles, a last round of quadrants, of halves
+def test_ways_of_the_outputs_of_whole_tiles(m, n, fp8, out):
+    """256x256 tiles store whole rows through the L2, whole rows, or straight from the registers, by the distance of the rows."""
+    xq, wq, sx, sw, b = _operands(m, n, 384, fp8, OUT[out][1], m + n)
+    got, want = (_launch(xq, wq, sx, sw, b, fp8, out, kernel) for kernel in (8, 11 if fp8 else 5))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("m,n,k", [(64, 16384, 256), (65, 24577, 128), (127, 8200, 1536), (128, 5120, 1024), (129, 4104, 640), (512, 5120, 384),
                                    (2900, 3080, 1024), (4096, 1536, 512), (5000, 64, 512), (5000, 127, 512), (575, 15360, 256), (700, 15360, 256)])
