@@ -271,9 +271,9 @@ __global__ __launch_bounds__(256, (PRE == PRE_LN && NCH <= 12 && !WRITE_Y) ? 2 :
         for (int i = 0; i < NCH; ++i) {
             const int c = i * 64 + lane;
             if (c < nch) {
-                store_stream_8(qr + c, quant_chunk<FMT, false, DAXQ_BF16, false>(v[i], s, inv));  // own scale at the format's maximum: no clamp
+                store_through_8(qr + c, quant_chunk<FMT, false, DAXQ_BF16, false>(v[i], s, inv));  // own scale at the format's maximum: no clamp
             } else if (c < npad) {
-                store_stream_8(qr + c, make_uint2(0, 0));
+                store_through_8(qr + c, make_uint2(0, 0));
             }
         }
         if constexpr (AHEAD) {
@@ -430,9 +430,9 @@ __global__ __launch_bounds__(256, NCOL <= 3 ? 7 : NCOL <= 4 ? 6 : NCOL <= 5 ? 5 
         uint2* qr = reinterpret_cast<uint2*>(q + row * ld_q) + lane;
 #pragma unroll
         for (int i = 0; i < NCOL; ++i) {
-            if (i < FULL) store_stream_8(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv));
+            if (i < FULL) store_through_8(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv));
             else if (i * 64 + lane < npad)  // (zeros in the padding columns [k, kfill), whatever the scale is)
-                store_stream_8(qr + i * 64, i * 64 + lane < nch ? quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv) : make_uint2(0, 0));
+                store_through_8(qr + i * 64, i * 64 + lane < nch ? quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv) : make_uint2(0, 0));
         }
     };
     uint4 ra[NCOL], rb[NCOL];
@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256) void gelu_rows_exact(const uint16_t* __restric
     const float inv = 1.0f / s;
     uint2* qr = reinterpret_cast<uint2*>(q + row * ld_q) + lane;
 #pragma unroll
-    for (int i = 0; i < NCOL; ++i) store_stream_8(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(v[i], s, inv));
+    for (int i = 0; i < NCOL; ++i) store_through_8(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(v[i], s, inv));
 }
 
 template <int NCOL, int FMT>
