@@ -235,11 +235,15 @@ constexpr int64_t kKeepBytes = (int64_t)128 << 20;
 //   1024 x 5120 x 5120 e4m3 (5) 29.8 / 29.2    1230 x 2712, K = 5120 (6) 26.5 / 25.8    887 x 5120, K = 8960 e4m3 (7.6) 40.9 / 40.3
 //   2225 x 5120, K = 4608 (9.8) 51.1 / 51.3    1003 x 4608, K = 13824 (13) 60.5 / 61.0    2358 x 5120, K = 8960 (20) 92.7 / 93.0
 //   4071 x 5120, K = 13824 (54) 216.7 / 216.2  13198 x 1536, K = 5120 (64) 111.8 / 109.2   16034 x 5120, K = 5160 e4m3 (80) 320 / 312
-constexpr int64_t kThroughFrom = (int64_t)1 << 20, kThroughTo = (int64_t)8 << 20, kThroughAgain = (int64_t)32 << 20;
+// and past the caches / through, beyond kKeepBytes, up to the Infinity Cache's 256 MB:
+//   27000 x 512, K = 5120 (138) 122.0 / 113.6    30000 x 1536, K = 5120 (154) 246.7 / 236.8    20000 x 5120, K = 8960 e4m3 (179) 697 / 688
+//   37800 x 13824, K = 5120 (194) 1951 / 1953    18000 x 5120, K = 13824 (249) 985 / 975    32760 x 1536, K = 8960 (294) 438.3 / 435.6
+//   75600 x 5120 x 5120 e4m3 (387) 1540 / 1548   INT8 1565 / 1560    75600 x 5120, K = 13824 e4m3 (1045) 3965 / 3972
+constexpr int64_t kThroughFrom = (int64_t)1 << 20, kThroughTo = (int64_t)8 << 20, kThroughAgain = (int64_t)32 << 20, kThroughMost = (int64_t)256 << 20;
 static int store_of(int64_t bytes, const void* q, int64_t ld_q) {
-    if (bytes > kKeepBytes) return kStorePast;
     const bool aligned = (((uintptr_t)q | (uintptr_t)ld_q) & 7) == 0;
-    return aligned && bytes >= kThroughFrom && (bytes <= kThroughTo || bytes >= kThroughAgain) ? kStoreThrough : kStoreKeep;
+    if (aligned && ((bytes >= kThroughFrom && bytes <= kThroughTo) || (bytes >= kThroughAgain && bytes <= kThroughMost))) return kStoreThrough;
+    return bytes > kKeepBytes ? kStorePast : kStoreKeep;
 }
 
 // Rows that a workgroup of quant_rows_kernel takes where a row has more than one wavefront (the instantiations that

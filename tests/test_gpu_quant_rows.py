@@ -353,10 +353,10 @@ def test_bytes_over_the_rows_they_are_made_from(ops, dtype, fmt, m, k):
             assert torch.equal(q[:, :k], apart[:, :k]) and torch.equal(scale[0], scale[1])
 
 
-@pytest.mark.parametrize("k,m", [(1536, 681), (1536, 683), (1537, 5041), (5120, 205), (5120, 1639), (2560, 3277), (5120, 6557), (1536, 21847)])
+@pytest.mark.parametrize("k,m", [(1536, 681), (1536, 683), (1537, 5041), (5120, 205), (5120, 1639), (2560, 3277), (5120, 6557), (1536, 21847), (5120, 26215), (5120, 52429)])
 @pytest.mark.parametrize("form", ["token", "one_scale", "tensor"])
 def test_matrices_whose_bytes_are_stored_through_the_l2(form, k, m):
-    """On either side of the lines between the ways of storing the bytes (1, 8 and 32 MB), numbers of rows that leave the XCDs' ranges
+    """On either side of the lines between the ways of storing the bytes (1, 8, 32, 128 and 256 MB), numbers of rows that leave the XCDs' ranges
     uneven: the bytes and scales of the whole matrix are those of slices of a few rows, at an address that is a multiple of 8 and at one
     that is not, and nothing around them is written."""
     from dax_amd import _capi
