@@ -244,7 +244,8 @@ __device__ __forceinline__ void outputs_lines(const GemmArgs& p, typename Acc16<
 }
 
 // The epilogue of kernels that have no registers for the scales beside their main loop: a thread has requested one of each, and they
-// pass through the LDS.
+// pass through the LDS, which it begins to write at once: a barrier lies between the workgroup's last fragment read and this call (in
+// the pipelined loops the one in front of the last pair's MFMAs).
 // OUTK: element type of out and bias, DAXQ_BF16 / DAXQ_F16 / DAXQ_F32.  A template argument, i.e. a kernel
 // of its own per type: with all three forms inside one kernel behind uniform branches its code grew from 27 to 44 KB
 // and the bf16 launches at K = 1536, which change between main loop and epilogue every 24 slices, lost 2.7 %; with

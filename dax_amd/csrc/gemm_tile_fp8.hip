@@ -333,6 +333,7 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        __syncthreads();  // (the epilogue writes where other wavefronts may still read pair Q-1's fragments)
         mfma_settle();
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     }

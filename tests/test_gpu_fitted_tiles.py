@@ -130,6 +130,18 @@ def test_ways_of_the_outputs_of_whole_tiles(m, n, fp8, out):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("k", [128, 256, 384])
+@pytest.mark.parametrize("m,n,kernel", [(300, 700, 8), (300, 700, 11), (4300, 4088, 8), (5300, 4088, 8), (4300, 4088, 11)])
+def test_short_k_of_fp8_tiles(m, n, kernel, k):
+    """Up to three pairs of K slices FP8 tiles of 256x256 (alone, with a last round of quadrants, of halves) and 128x128 do not pipeline,
+    and their epilogue's scales go where the last pair's weights were read: every wavefront has to be past them.  Several launches,
+    more than a round of workgroups among them, against a fitted tile, whose epilogue keeps its scales in registers."""
+    xq, wq, sx, sw, b = _operands(m, n, k, True, torch.bfloat16, m + k)
+    want = _launch(xq, wq, sx, sw, b, True, "bf16", 32 + 10)
+    for _ in range(4):
+        assert torch.equal(_launch(xq, wq, sx, sw, b, True, "bf16", kernel).view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("m,n,k", [(64, 16384, 256), (65, 24577, 128), (127, 8200, 1536), (128, 5120, 1024), (129, 4104, 640), (512, 5120, 384),
                                    (2900, 3080, 1024), (4096, 1536, 512), (5000, 64, 512), (5000, 127, 512), (575, 15360, 256), (700, 15360, 256)])
