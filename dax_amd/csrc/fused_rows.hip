@@ -101,7 +101,7 @@ __device__ __forceinline__ float gelu_tanh_f32(float x) {
 // Requires k % 8 == 0, 16-byte aligned rows of x (and y), 8-byte aligned rows of q, kfill/8 <= NCH*64.
 // The quantise-only LayerNorm form for rows of up to 12 x 64 chunks holds two rows (the current and the requested
 // next one); what the blocks run, quantise-only rows in groups of four rows and more, takes ln_rows below instead.
-template <int NCH, int FMT, int PRE, bool WRITE_Y>
+template <int NCH, int FMT, int PRE, bool WRITE_Y, bool THROUGH>
 __global__ __launch_bounds__(256, (PRE == PRE_LN && NCH <= 12 && !WRITE_Y) ? 2 : 1) void fused_rows_wave(
     const uint16_t* __restrict__ x, int64_t m, int k, int64_t ld_x, const float* __restrict__ mul,
     const float* __restrict__ add, int64_t rows_per_group, float eps, uint16_t* __restrict__ y, int64_t ld_y,
@@ -271,9 +271,9 @@ __global__ __launch_bounds__(256, (PRE == PRE_LN && NCH <= 12 && !WRITE_Y) ? 2 :
         for (int i = 0; i < NCH; ++i) {
             const int c = i * 64 + lane;
             if (c < nch) {
-                store_through_8(qr + c, quant_chunk<FMT, false, DAXQ_BF16, false>(v[i], s, inv));  // own scale at the format's maximum: no clamp
+                store_row_8<THROUGH>(qr + c, quant_chunk<FMT, false, DAXQ_BF16, false>(v[i], s, inv));  // own scale at the format's maximum: no clamp
             } else if (c < npad) {
-                store_through_8(qr + c, make_uint2(0, 0));
+                store_row_8<THROUGH>(qr + c, make_uint2(0, 0));
             }
         }
         if constexpr (AHEAD) {
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256, (PRE == PRE_LN && NCH <= 12 && !WRITE_Y) ? 2 :
 // Bound by HBM and VALU together (3 bytes and about ten VALU instructions per element).  Measured at 9450 x 5120 (one
 // group of 9450 rows, e4m3): 41.5 us in fused_rows_wave, where lane predicates and the path for rows of another group make
 // the compiler wait for the requested row in front of every chunk; 31.9 us here (behind a GEMM, vectors and rows far away:
-// 58.7 -> 38.7 us); 75600 x 5120 213 us = 5.4 TB/s.
+// 58.7 -> 38.7 us); 75600 x 5120 214 us = 5.4 TB/s (bytes past the caches, fused_store_through).
 template <int NCOL>
 constexpr int kTailChunks = NCOL > 10 ? 2 : 1;  // chunks per lane that may lie beyond the row (NCOL > 10 exists in steps of two)
 
@@ -317,7 +317,7 @@ __device__ __forceinline__ void stage_vector(float* dst, const float* src, float
     }
 }
 
-template <int NCOL, int FMT>
+template <int NCOL, int FMT, bool THROUGH>
 __global__ __launch_bounds__(256, NCOL <= 3 ? 7 : NCOL <= 4 ? 6 : NCOL <= 5 ? 5 : NCOL <= 10 ? 4 : NCOL <= 12 ? 3 : 2) void ln_rows(const uint16_t* __restrict__ x, int64_t m, int k, int64_t ld_x,
                                                                    const float* __restrict__ mul, const float* __restrict__ add,
                                                                    int64_t rows_per_group, int64_t quads_per_group, int64_t quads,
@@ -430,9 +430,9 @@ __global__ __launch_bounds__(256, NCOL <= 3 ? 7 : NCOL <= 4 ? 6 : NCOL <= 5 ? 5 
         uint2* qr = reinterpret_cast<uint2*>(q + row * ld_q) + lane;
 #pragma unroll
         for (int i = 0; i < NCOL; ++i) {
-            if (i < FULL) store_through_8(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv));
+            if (i < FULL) store_row_8<THROUGH>(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv));
             else if (i * 64 + lane < npad)  // (zeros in the padding columns [k, kfill), whatever the scale is)
-                store_through_8(qr + i * 64, i * 64 + lane < nch ? quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv) : make_uint2(0, 0));
+                store_row_8<THROUGH>(qr + i * 64, i * 64 + lane < nch ? quant_chunk<FMT, false, DAXQ_BF16, false>(cur[i], s, inv) : make_uint2(0, 0));
         }
     };
     uint4 ra[NCOL], rb[NCOL];
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(256, NCOL <= 3 ? 7 : NCOL <= 4 ? 6 : NCOL <= 5 ? 5 
 // keeps one execution mask per chunk alive, 28 of them, which the compiler spills from scalar registers into vector lanes:
 // some 300 v_writelane / v_readlane per row on a kernel that is bound by VALU issue) and a scalar row number.  Same
 // arithmetic, same bits.  One row per wavefront, four per workgroup.
-template <int NCOL, int FMT>
+template <int NCOL, int FMT, bool THROUGH>
 __global__ __launch_bounds__(256) void gelu_rows_exact(const uint16_t* __restrict__ x, int64_t m, int64_t ld_x, uint8_t* __restrict__ q,
                                                        int64_t ld_q, float* __restrict__ scale, float qmax) {
     const int lane = threadIdx.x & 63;
@@ -480,10 +480,10 @@ __global__ __launch_bounds__(256) void gelu_rows_exact(const uint16_t* __restric
     const float inv = 1.0f / s;
     uint2* qr = reinterpret_cast<uint2*>(q + row * ld_q) + lane;
 #pragma unroll
-    for (int i = 0; i < NCOL; ++i) store_through_8(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(v[i], s, inv));
+    for (int i = 0; i < NCOL; ++i) store_row_8<THROUGH>(qr + i * 64, quant_chunk<FMT, false, DAXQ_BF16, false>(v[i], s, inv));
 }
 
-template <int NCOL, int FMT>
+template <int NCOL, int FMT, bool THROUGH>
 static int launch_ln_rows(const char* what, const uint16_t* x, int64_t m, int64_t k, int64_t ld_x, const float* mul, const float* add,
                           int64_t rows_per_group, float eps, uint8_t* q, int64_t ld_q, int64_t kfill, float* scale, float qmax, int cus,
                           hipStream_t st) {
@@ -491,35 +491,22 @@ static int launch_ln_rows(const char* what, const uint16_t* x, int64_t m, int64_
     static int per_cu = 0;  // asked once per instantiation; a race between two threads stores the same value twice
     if (per_cu <= 0) {
         int v = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, ln_rows<NCOL, FMT>, 256, lds) != hipSuccess || v <= 0)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, ln_rows<NCOL, FMT, THROUGH>, 256, lds) != hipSuccess || v <= 0)
             return fail(DAXQ_ERR_LAUNCH, "%s: occupancy query failed", what);
         per_cu = v;
     }
     const int64_t rpg = rows_per_group < m ? rows_per_group : m, qpg = (rpg + 3) / 4, quads = (m / rpg) * qpg + (m % rpg + 3) / 4;
     const int64_t want = (int64_t)cus * per_cu;
-    launch_kernel((ln_rows<NCOL, FMT>), dim3((unsigned)(quads < want ? quads : want)), dim3(256), lds, st, x, m, (int)k, ld_x, mul,
+    launch_kernel((ln_rows<NCOL, FMT, THROUGH>), dim3((unsigned)(quads < want ? quads : want)), dim3(256), lds, st, x, m, (int)k, ld_x, mul,
                        add, rpg, qpg, quads, eps, q, ld_q, (int)kfill, scale, qmax);
     return check_launch(what);
 }
 
-template <int FMT, int PRE>
-static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t k, int64_t ld_x, const float* mul,
-                             const float* add, int64_t rows_per_group, float eps, void* y, int64_t ld_y, void* q,
-                             int64_t ld_q, float* scale, float qmax, hipStream_t st) {
-    if (m < 0 || k <= 0 || ld_x < k || ld_q < k || (y && ld_y < k))
-        return fail(DAXQ_ERR_ARG, "%s: bad shape m=%lld k=%lld ld_x=%lld ld_q=%lld", what, (long long)m, (long long)k,
-                    (long long)ld_x, (long long)ld_q);
-    if (PRE == PRE_LN && (rows_per_group <= 0 || !(eps >= 0.0f))) return fail(DAXQ_ERR_ARG, "%s: rows_per_group and eps must be positive", what);
-    if (m == 0) return DAXQ_OK;
-    if (!x || !q || !scale) return fail(DAXQ_ERR_ARG, "%s: null pointer", what);
-    const int64_t kfill = fill_width(k, ld_q);
-    // the row has to fit the registers of one wavefront and move in 16-byte pieces
-    const bool ok = (k % 8 == 0) && (ld_x % 8 == 0) && (ld_q % 8 == 0) && (!y || ld_y % 8 == 0) && (((uintptr_t)x & 15) == 0) &&
-                    (((uintptr_t)y & 15) == 0) && (((uintptr_t)q & 7) == 0) && (((uintptr_t)scale & 3) == 0) &&
-                    (((uintptr_t)mul & 3) == 0) && (((uintptr_t)add & 3) == 0) && (kfill / 8 <= 28 * 64) &&
-                    (PRE != PRE_LN || k <= 8192);
-    if (!ok)
-        return fail(DAXQ_ERR_ALIGN, "%s: needs k %% 8 == 0, k <= 14336 (8192 with LayerNorm), 16-byte aligned rows of x / y and 8-byte aligned rows of q", what);
+// (a call that launch_fused_rows has checked)
+template <int FMT, int PRE, bool THROUGH>
+static int launch_fused_rows_to(const char* what, const void* x, int64_t m, int64_t k, int64_t ld_x, const float* mul,
+                                const float* add, int64_t rows_per_group, float eps, void* y, int64_t ld_y, void* q,
+                                int64_t ld_q, int64_t kfill, float* scale, float qmax, hipStream_t st) {
     const uint16_t* xp = static_cast<const uint16_t*>(x);
     uint16_t* yp = static_cast<uint16_t*>(y);
     uint8_t* qp = static_cast<uint8_t*>(q);
@@ -533,7 +520,7 @@ static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t
         if (!yp && (rows_per_group >= 4 || rows_per_group >= m)) {
             const int cols = (int)((k + 511) / 512);
 #define DAXQ_LN_ROWS(N) \
-    if (cols <= N) return launch_ln_rows<N, FMT>(what, xp, m, k, ld_x, mul, add, rows_per_group, eps, qp, ld_q, kfill, scale, qmax, cus, st);
+    if (cols <= N) return launch_ln_rows<N, FMT, THROUGH>(what, xp, m, k, ld_x, mul, add, rows_per_group, eps, qp, ld_q, kfill, scale, qmax, cus, st);
             DAXQ_LN_ROWS(1)
             DAXQ_LN_ROWS(2)
             DAXQ_LN_ROWS(3)
@@ -556,7 +543,7 @@ static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t
             switch (k / 512) {
 #define DAXQ_GELU_EXACT(N)                                                                                                        \
     case N:                                                                                                                       \
-        launch_kernel((gelu_rows_exact<N, FMT>), grid, dim3(256), 0, st, xp, m, ld_x, qp, ld_q, scale, qmax);                 \
+        launch_kernel((gelu_rows_exact<N, FMT, THROUGH>), grid, dim3(256), 0, st, xp, m, ld_x, qp, ld_q, scale, qmax);                 \
         return check_launch(what);
                 DAXQ_GELU_EXACT(12)
                 DAXQ_GELU_EXACT(16)
@@ -583,8 +570,8 @@ static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t
             const int slot = yp ? 1 : 0;                                                                                 \
             if (cached_per_cu[slot] <= 0 || cached_k[slot] != k) {                                                       \
                 int per_cu = 0;                                                                                          \
-                hipError_t oe = yp ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fused_rows_wave<N, FMT, PRE, true>, 256, lds) \
-                                   : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fused_rows_wave<N, FMT, PRE, false>, 256, lds); \
+                hipError_t oe = yp ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fused_rows_wave<N, FMT, PRE, true, THROUGH>, 256, lds) \
+                                   : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fused_rows_wave<N, FMT, PRE, false, THROUGH>, 256, lds); \
                 if (oe != hipSuccess || per_cu <= 0) return fail(DAXQ_ERR_LAUNCH, "%s: occupancy query failed", what);   \
                 cached_k[slot] = k;                                                                                      \
                 cached_per_cu[slot] = per_cu;                                                                            \
@@ -593,10 +580,10 @@ static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t
         }                                                                                                                \
         const dim3 grid((unsigned)(quads < want ? quads : want));                                                        \
         if (yp)                                                                                                          \
-            launch_kernel((fused_rows_wave<N, FMT, PRE, true>), grid, block, lds, st, xp, m, (int)k, ld_x, mul, add, \
+            launch_kernel((fused_rows_wave<N, FMT, PRE, true, THROUGH>), grid, block, lds, st, xp, m, (int)k, ld_x, mul, add, \
                                rows_per_group, eps, yp, ld_y, qp, ld_q, (int)kfill, scale, qmax);                                    \
         else                                                                                                             \
-            launch_kernel((fused_rows_wave<N, FMT, PRE, false>), grid, block, lds, st, xp, m, (int)k, ld_x, mul, add, \
+            launch_kernel((fused_rows_wave<N, FMT, PRE, false, THROUGH>), grid, block, lds, st, xp, m, (int)k, ld_x, mul, add, \
                                rows_per_group, eps, yp, ld_y, qp, ld_q, (int)kfill, scale, qmax);                                    \
         return check_launch(what);                                                                                       \
     }
@@ -606,6 +593,28 @@ static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t
     DAXQ_F_CASE(28)
 #undef DAXQ_F_CASE
     return fail(DAXQ_ERR_ARG, "%s: row too long", what);
+}
+
+template <int FMT, int PRE>
+static int launch_fused_rows(const char* what, const void* x, int64_t m, int64_t k, int64_t ld_x, const float* mul,
+                             const float* add, int64_t rows_per_group, float eps, void* y, int64_t ld_y, void* q,
+                             int64_t ld_q, float* scale, float qmax, hipStream_t st) {
+    if (m < 0 || k <= 0 || ld_x < k || ld_q < k || (y && ld_y < k))
+        return fail(DAXQ_ERR_ARG, "%s: bad shape m=%lld k=%lld ld_x=%lld ld_q=%lld", what, (long long)m, (long long)k,
+                    (long long)ld_x, (long long)ld_q);
+    if (PRE == PRE_LN && (rows_per_group <= 0 || !(eps >= 0.0f))) return fail(DAXQ_ERR_ARG, "%s: rows_per_group and eps must be positive", what);
+    if (m == 0) return DAXQ_OK;
+    if (!x || !q || !scale) return fail(DAXQ_ERR_ARG, "%s: null pointer", what);
+    const int64_t kfill = fill_width(k, ld_q);
+    // the row has to fit the registers of one wavefront and move in 16-byte pieces
+    const bool ok = (k % 8 == 0) && (ld_x % 8 == 0) && (ld_q % 8 == 0) && (!y || ld_y % 8 == 0) && (((uintptr_t)x & 15) == 0) &&
+                    (((uintptr_t)y & 15) == 0) && (((uintptr_t)q & 7) == 0) && (((uintptr_t)scale & 3) == 0) &&
+                    (((uintptr_t)mul & 3) == 0) && (((uintptr_t)add & 3) == 0) && (kfill / 8 <= 28 * 64) &&
+                    (PRE != PRE_LN || k <= 8192);
+    if (!ok)
+        return fail(DAXQ_ERR_ALIGN, "%s: needs k %% 8 == 0, k <= 14336 (8192 with LayerNorm), 16-byte aligned rows of x / y and 8-byte aligned rows of q", what);
+    auto launch = fused_store_through(m * kfill) ? launch_fused_rows_to<FMT, PRE, true> : launch_fused_rows_to<FMT, PRE, false>;
+    return launch(what, x, m, k, ld_x, mul, add, rows_per_group, eps, y, ld_y, q, ld_q, kfill, scale, qmax, st);
 }
 
 }  // namespace daxq

@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "daxq_common.h"
+#include "store_rule.h"
 
 namespace daxq {
 
@@ -207,21 +208,19 @@ __device__ __forceinline__ uint32_t chunk_absmax(uint32_t mx, const uint4& v) {
 }
 
 // Accesses of the kernels that fuse a producer and the quantiser.  The bf16 row is read once, past the caches with the non-temporal
-// hint.  The quantised row goes into the L2 and through it to memory at once (a device-coherent store): the GEMM behind finds what
-// the caches hold, and nothing is left to write back when the kernel ends.  A feed-forward (LayerNorm, up, GELU, down) on the GPU
-// alone, us, bytes past the caches (non-temporal) / kept in the L2s / through them:
-//   256 x 1536 x 8960 e4m3 46.3 / 38.9 / 38.5    512 x 5120 x 13824 INT8 104.3 / 89.0 / 88.6    1600 x 2560 x 4608 INT8 67.8 / 60.0 / 59.0
-//   2048 x 1536 x 8960 e4m3 92.3 / 83.7 / 83.5   4095 x 1536 x 8960 INT8 151.8 / 141.6 / 141.3  5000 x 512 x 1024 e4m3 31.8 / 31.0 / 29.2
-//   9450 x 5120 x 13824 e4m3 1012 / 1006 / 1004  16380 x 1536 x 8960 e4m3 493 / 486 / 481       32760 x 1536 x 8960 INT8 929 / 921 / 916
-// only the smallest lose, 256 x 512 x 1024 14.9 / 14.8 / 15.2 (the host takes 107 for such a block).
+// hint; where the quantised row goes: fused_store_through.
 typedef unsigned daxq_v4u __attribute__((ext_vector_type(4)));
 typedef unsigned daxq_v2u __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint4 load_stream_16(const uint4* p) {
     const daxq_v4u t = __builtin_nontemporal_load(reinterpret_cast<const daxq_v4u*>(p));
     return make_uint4(t.x, t.y, t.z, t.w);
 }
-__device__ __forceinline__ void store_through_8(uint2* p, uint2 v) {
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// p is a multiple of 8
+template <bool THROUGH>
+__device__ __forceinline__ void store_row_8(uint2* p, uint2 v) {
+    const daxq_v2u t = {v.x, v.y};
+    if constexpr (THROUGH) __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else __builtin_nontemporal_store(t, reinterpret_cast<daxq_v2u*>(p));
 }
 
 // A row is cut into chunks of 8 elements.  Any alignment is taken: the loads and stores are the same 16- and 8-byte
@@ -246,9 +245,7 @@ __device__ __forceinline__ void load_chunk_shared(Chunk<XT>& v, const char* p) {
     for (int h = 0; h < (XT == DAXQ_F32 ? 2 : 1); ++h) v.w[h] = reinterpret_cast<const loose*>(p)[h];
 }
 
-// Where the stored bytes go: past the caches (non-temporal), into them for the GEMM behind the quantiser, or into them and through
-// the L2 to memory at once (a device-coherent store; p is a multiple of 8 then)
-enum { kStorePast = 0, kStoreKeep = 1, kStoreThrough = 2 };
+// STORE: where the bytes go (store_of; p is a multiple of 8 with kStoreThrough)
 template <int STORE>
 __device__ __forceinline__ void store_chunk(uint8_t* p, uint2 v) {
     typedef daxq_v2u loose __attribute__((aligned(1)));

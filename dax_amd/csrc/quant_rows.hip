@@ -221,31 +221,6 @@ struct ScaleKind {
     bool weight = false;                 // rows of a weight: the leaf quantiser's bytes also under a scale that is not finite
 };
 
-// Activations of at most this many quantised bytes are stored where the GEMM finds them again, in the caches (the Infinity Cache
-// holds 256 MB), larger ones past them.  Forwards, us, past the caches -> kept: 512 x 5120 x 5120 25.5 -> 22.4, 4096 x 1536 x 1536
-// 21.9 -> 19.8, 2900 x 1000 x 3080 fp16 20.4 -> 19.7, 4725 x 5120 x 5120 static e4m3 104.8 -> 102.6, 32760 x 4608, K = 1536 238.6 -> 229.9,
-// 75600 x 5120 x 5120 e4m3 1498 -> 1505; converting a weight of 13824 x 5120 37.0 -> 38.3.  (The rows' own loads without the hint as
-// well: 512 x 5120 22.2, 4096 x 1536 19.6, but 4725 x 5120 105.2 and 32760 x 1536 234.8.)
-constexpr int64_t kKeepBytes = (int64_t)128 << 20;
-// Kept bytes that only lie in the L2s are written back when the kernel has ended, and the GEMM waits for that: it starts 1.5 us
-// behind the last acknowledged store with nothing to write back, 3.1 us with 2.6 MB (512 x 5120), 4.5 us with 6.3 MB (4096 x 1536).
-// Stores through the L2 write while the kernel runs.  Quantiser + GEMM, us, kept / through (rows of one wavefront in ranges):
-//   134 x 3472, K = 5120 (0.65 MB) 12.5 / 12.5    17 x 5120 x 5120 e4m3 (0.1) 9.05 / 9.22    64 x 5120 x 5120 (0.3) 12.1 / 12.4
-//   512 x 5120 x 5120 (2.5) 22.3 / 22.0    2900 x 3080, K = 1000 (2.8) 19.7 / 19.4    313 x 4608, K = 13824 (4.1) 31.9 / 31.3
-//   1024 x 5120 x 5120 e4m3 (5) 29.8 / 29.2    1230 x 2712, K = 5120 (6) 26.5 / 25.8    887 x 5120, K = 8960 e4m3 (7.6) 40.9 / 40.3
-//   2225 x 5120, K = 4608 (9.8) 51.1 / 51.3    1003 x 4608, K = 13824 (13) 60.5 / 61.0    2358 x 5120, K = 8960 (20) 92.7 / 93.0
-//   4071 x 5120, K = 13824 (54) 216.7 / 216.2  13198 x 1536, K = 5120 (64) 111.8 / 109.2   16034 x 5120, K = 5160 e4m3 (80) 320 / 312
-// and past the caches / through, beyond kKeepBytes, up to the Infinity Cache's 256 MB:
-//   27000 x 512, K = 5120 (138) 122.0 / 113.6    30000 x 1536, K = 5120 (154) 246.7 / 236.8    20000 x 5120, K = 8960 e4m3 (179) 697 / 688
-//   37800 x 13824, K = 5120 (194) 1951 / 1953    18000 x 5120, K = 13824 (249) 985 / 975    32760 x 1536, K = 8960 (294) 438.3 / 435.6
-//   75600 x 5120 x 5120 e4m3 (387) 1540 / 1548   INT8 1565 / 1560    75600 x 5120, K = 13824 e4m3 (1045) 3965 / 3972
-constexpr int64_t kThroughFrom = (int64_t)1 << 20, kThroughTo = (int64_t)8 << 20, kThroughAgain = (int64_t)32 << 20, kThroughMost = (int64_t)256 << 20;
-static int store_of(int64_t bytes, const void* q, int64_t ld_q) {
-    const bool aligned = (((uintptr_t)q | (uintptr_t)ld_q) & 7) == 0;
-    if (aligned && ((bytes >= kThroughFrom && bytes <= kThroughTo) || (bytes >= kThroughAgain && bytes <= kThroughMost))) return kStoreThrough;
-    return bytes > kKeepBytes ? kStorePast : kStoreKeep;
-}
-
 // Rows that a workgroup of quant_rows_kernel takes where a row has more than one wavefront (the instantiations that
 // launch_quant_rows_t goes through), else 0.
 static int quant_unit(int x_dtype, int64_t kfill) {
@@ -287,7 +262,7 @@ static int launch_quant_rows_t(const void* x, int64_t m, int64_t k, int64_t ld_x
         constexpr float kFmtMax = FMT == 0 ? 127.0f : FMT == 1 ? 448.0f : 57344.0f;
         const bool plain = kMayBePlain && ((k | kfill) & 7) == 0 && !a.leaf && qmax <= kFmtMax && (FMT == 0 || round_x);
         // (the rows of a weight, and those under a scale each from the caller, have no GEMM behind them)
-        const int to = t.weight || (SCALE_IN && !t.one_scale) ? kStorePast : store_of(m * kfill, q, ld_q);
+        const int to = t.weight || (SCALE_IN && !t.one_scale) ? kStorePast : store_of(m * kfill, (((uintptr_t)q | (uintptr_t)ld_q) & 7) == 0);
         // A launch holds fewer than 2^32 work items, i.e. 2^24 workgroups: more rows are as many launches as they need
 #define DAXQ_Q_CASE(N, W)                                                                                                  \
     if (cols <= N * W) {                                                                                                   \

@@ -76,6 +76,20 @@ def test_patch_tile_order_covers_every_tile_once():
     assert r.returncode == 0 and " 0 errors" in r.stdout, r.stdout + r.stderr
 
 
+def test_where_quantised_bytes_go():
+    """tests/host/store_rule_check, built like the check above: the row quantiser's stores and the fused producers' on either side of
+    every line, bytes of matrices far beyond the caches past them in both."""
+    import subprocess
+
+    exe = os.path.join(ROOT, "tests", "host", "store_rule_check")
+    if not os.path.exists(exe):
+        import __graft_entry__
+
+        __graft_entry__._build_host_checks()
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout == "0 errors\n", r.stdout + r.stderr
+
+
 def test_tile_order_by_shape():
     """daxq_linear_tile_order_choice (host arithmetic only): the four Wan2.1-14B launches at 75600 tokens and their
     neighbours take the banded order; a 1/8 share of the rows, short K, narrow N and small launches keep the row

@@ -193,3 +193,23 @@ def test_fused_errors_are_loud(ops):
         ops.gelu_tanh_act_quant_i8(torch.randn(4, 64).bfloat16())   # CPU tensor
     with pytest.raises(ValueError):
         ops.layernorm_act_quant_i8(dev(torch.randn(4, 64).bfloat16()), dev(torch.ones(3, 64)), None, 4, 1e-6)
+
+
+@pytest.mark.parametrize("fmt", ["i8", "e4m3"])
+@pytest.mark.parametrize("producer,k,y", [("layernorm", 5120, False), ("layernorm", 1000, True), ("gelu_tanh", 6144, False), ("gelu_tanh", 200, False), ("gelu_tanh", 200, True)])
+def test_bytes_past_the_caches(ops, fmt, producer, k, y):
+    """Producers whose bytes are more than 280 MB store them past the caches, smaller ones through the L2: a launch over the line against
+    the same rows in two launches under it, in every kernel (rows beyond the last workgroup's are ragged)."""
+    m = (280 << 20) // ops.pad_k(k) + 3
+    x = torch.randn(m, k, generator=torch.Generator("cuda").manual_seed(k), device="cuda", dtype=torch.bfloat16)
+    if producer == "layernorm":
+        g = torch.Generator("cuda").manual_seed(1)
+        mul, add = torch.randn(1, k, generator=g, device="cuda"), torch.randn(1, k, generator=g, device="cuda")
+        fn = lambda rows: getattr(ops, "layernorm_act_quant_" + fmt)(rows, mul, add, rows.shape[0], 1e-6, y)
+    else:
+        fn = lambda rows: getattr(ops, "gelu_tanh_act_quant_" + fmt)(rows, y)
+    whole, cut = fn(x), m // 2 + 1
+    for rows, part in ((slice(0, cut), fn(x[:cut])), (slice(cut, m), fn(x[cut:]))):
+        for a, b in zip(whole, part):
+            a, b = (a[rows], b) if a.shape[0] else (a, b)
+            assert torch.equal(a.view(torch.int16) if a.dtype == torch.bfloat16 else a, b.view(torch.int16) if b.dtype == torch.bfloat16 else b)
