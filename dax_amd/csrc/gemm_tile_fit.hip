@@ -38,35 +38,6 @@ __global__ __launch_bounds__(TILE::T) void gemm_fit_kernel(const GemmArgs p) {
     gemm_fit_body<TILE, FP8, F8, false, OUTK>(p, m0, n0);
 }
 
-// Depth of the tile order's groups: which part of the tile grid the CUs of an XCD hold, `depth` tile rows x an eighth of the tiles / depth
-// columns.  What that part costs goes like 3 x its rows + its columns: the activation was written a moment ago, all over the
-// chip, and arrives later than the weight.  The groups are even, and one with fewer rows than the others counts for 5 % more: with a
-// last tile row of its own its tiles fetch a weight of many columns once more.
-// Forwards, us, by depth, INT8 unless noted (* the rule's):
-//   4096 x 1536 x 1536 (16 rows of 256 x 96)  1 16.9  2 16.9*  3 17.4  4 18.4  8 20.7     2900 x 3080, K = 1000 fp16 (12 of 256 x 160)  1 18.1  2 17.9  3 17.8*  4 18.2  8 18.9
-//   2000 x 4608, K = 1536 (8 of 256 x 160)  1 20.8  2 19.9*  3 20.1  4 20.1  8 21.3     1000 x 8960, K = 1536 (4 of 256 x 160)  1 20.4  2 19.2*  4 19.9
-//   512 x 5120 x 5120 (4 of 128 x 96)  1 23.2  2 21.7*  4 21.9     1024 x 5120 x 5120 (8 of 128 x 160)  1 39.2  2 30.2  3 29.7  4 29.5*  8 30.1
-//   1500 x 5120 x 5120 (6 of 256 x 128)  1 41.1  2 39.9*  3 39.8  6 41.3     343 x 1536, K = 4608 (6 of 64 x 64)  1 13.4  2 13.2  3 12.7*  6 13.4
-//   300 x 8960 x 8960 (5 of 64 x 192)  1 62.0  2 50.6  3 49.6  5 48.7*     570 x 5120, K = 8960 (9 of 64 x 192)  2 46.8  3 36.1  5 35.5*  9 46.0
-//   444 x 6664, K = 12160 (7 of 64 x 192)  3 65.1  4 63.7  7 63.2*     600 x 4608, K = 5120 (5 of 128 x 96)  2 22.3  3 21.9*  5 22.2
-static int group_depth(int bm, int bn, int tiles_m, int tiles_n) {
-    const float t = 0.125f * (float)tiles_m * (float)tiles_n, r = 3.0f * (float)bm, c = (float)bn;
-    auto cost = [&](int depth) {
-        const float rows = (float)depth * (float)tiles_n < t ? t / (float)tiles_n : (float)depth;  // (whole groups, if they are small)
-        return r * (rows < t ? rows : t) + c * (t > rows ? t / rows : 1.0f);
-    };
-    // the least of r d + c t / d lies at sqrt(c t / r): the even groups on either side of it
-    int groups = (int)((float)tiles_m * __builtin_sqrtf(r / (c * t))), best = tiles_m;
-    if (groups < 1) groups = 1;
-    float least = 0.0f;
-    for (int g = groups; g <= groups + 1 && g <= tiles_m; ++g) {
-        const int depth = (tiles_m + g - 1) / g, last = tiles_m - (tiles_m - 1) / depth * depth;
-        const float full = cost(depth), part = 1.05f * cost(last), most = last == depth || full > part ? full : part;
-        if (g == groups || most < least) best = depth, least = most;
-    }
-    return best;
-}
-
 // args null: only raises the kernel's LDS limit on the current device
 template <class TILE, bool FP8, int F8, int OUTK>
 static int launch_fit_one(const GemmArgs* args, hipStream_t st) {

@@ -1,5 +1,6 @@
-// Banded tile order of the 256x256 GEMM kernels (gfx950: 8 XCDs of 32 CUs, workgroup ids dealt round-robin over the
-// XCDs).  Plain C++ on purpose: the host-side check in tests/host compiles this file without the HIP headers.
+// Banded tile order of the 256x256 GEMM kernels and the depth of the row groups of the fitted tiles (gfx950: 8 XCDs of 32 CUs,
+// workgroup ids dealt round-robin over the XCDs).  Plain C++ on purpose: the host-side check in tests/host compiles this
+// file without the HIP headers.
 #pragma once
 
 #include <stdint.h>
@@ -124,6 +125,38 @@ inline int64_t banded_xcd_rounds(int tiles_m, int tiles_n, int W) {
     int64_t most = 0;
     for (int x = 0; x < 8; ++x) most = load[x] > most ? load[x] : most;
     return (most + 31) / 32;
+}
+
+// Depth of the tile order's groups: which part of the tile grid the CUs of an XCD hold, `depth` tile rows x an eighth of the tiles / depth
+// columns.  What that part costs goes like 3 x its rows + its columns: the activation was written a moment ago, all over the
+// chip, and arrives later than the weight.  The groups are even, and one with fewer rows than the others counts for 5 % more: with a
+// last tile row of its own its tiles fetch a weight of many columns once more.
+// Forwards, us, by depth, INT8 unless noted (* the rule's):
+//   4096 x 1536 x 1536 (16 rows of 256 x 96)  1 16.9  2 16.9*  3 17.4  4 18.4  8 20.7     2900 x 3080, K = 1000 fp16 (12 of 256 x 160)  1 18.1  2 17.9  3 17.8*  4 18.2  8 18.9
+//   2000 x 4608, K = 1536 (8 of 256 x 160)  1 20.8  2 19.9*  3 20.1  4 20.1  8 21.3     1000 x 8960, K = 1536 (4 of 256 x 160)  1 20.4  2 19.2*  4 19.9
+//   512 x 5120 x 5120 (4 of 128 x 96)  1 23.2  2 21.7*  4 21.9     1024 x 5120 x 5120 (8 of 128 x 160)  1 39.2  2 30.2  3 29.7  4 29.5*  8 30.1
+//   1500 x 5120 x 5120 (6 of 256 x 128)  1 41.1  2 39.9*  3 39.8  6 41.3     343 x 1536, K = 4608 (6 of 64 x 64)  1 13.4  2 13.2  3 12.7*  6 13.4
+//   300 x 8960 x 8960 (5 of 64 x 192)  1 62.0  2 50.6  3 49.6  5 48.7*     570 x 5120, K = 8960 (9 of 64 x 192)  2 46.8  3 36.1  5 35.5*  9 46.0
+//   444 x 6664, K = 12160 (7 of 64 x 192)  3 65.1  4 63.7  7 63.2*     600 x 4608, K = 5120 (5 of 128 x 96)  2 22.3  3 21.9*  5 22.2
+// (bm x bn: the tile.)  What a group of `depth` tile rows costs the XCD that works in it:
+inline float group_cost(int bm, int bn, int tiles_m, int tiles_n, int depth) {
+    const float t = 0.125f * (float)tiles_m * (float)tiles_n, r = 3.0f * (float)bm, c = (float)bn;
+    const float rows = (float)depth * (float)tiles_n < t ? t / (float)tiles_n : (float)depth;  // (whole groups, if they are small)
+    return r * (rows < t ? rows : t) + c * (t > rows ? t / rows : 1.0f);
+}
+// ... and the costliest of the groups that lie `depth` tile rows apart
+inline float groups_cost(int bm, int bn, int tiles_m, int tiles_n, int depth) {
+    const int last = tiles_m - (tiles_m - 1) / depth * depth;
+    const float full = group_cost(bm, bn, tiles_m, tiles_n, depth), part = 1.05f * group_cost(bm, bn, tiles_m, tiles_n, last);
+    return last == depth || full > part ? full : part;
+}
+inline int group_depth(int bm, int bn, int tiles_m, int tiles_n) {
+    // the least of r d + c t / d lies at sqrt(c t / r): the even groups on either side of it (below a depth of 1: single rows)
+    const float t = 0.125f * (float)tiles_m * (float)tiles_n, r = 3.0f * (float)bm, c = (float)bn;
+    int groups = (int)((float)tiles_m * __builtin_sqrtf(r / (c * t)));
+    groups = groups < 1 ? 1 : groups > tiles_m ? tiles_m : groups;
+    const int depth = (tiles_m + groups - 1) / groups, other = groups < tiles_m ? (tiles_m + groups) / (groups + 1) : depth;
+    return groups_cost(bm, bn, tiles_m, tiles_n, other) < groups_cost(bm, bn, tiles_m, tiles_n, depth) ? other : depth;
 }
 
 }  // namespace daxq

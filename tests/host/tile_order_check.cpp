@@ -2,7 +2,7 @@
 // sampled grids far beyond (tile rows up to 40000, tile columns up to 4096: the range the library's choice by shape
 // admits), the launch of banded_grid() workgroups computes every tile exactly once, padding slots map to no tile, and
 // the 32 slots that one XCD runs side by side lie in one patch of at most 32 tiles, at most 8 columns wide (wider only
-// in the dense patches of the last tile rows).  Built by
+// in the dense patches of the last tile rows); and of the depth of the fitted tiles' row groups.  Built by
 // __graft_entry__.build() with the host compiler; run by tests/test_abi_and_host.py.
 #include <cstdio>
 #include <cstdlib>
@@ -76,6 +76,21 @@ int main() {
     // 8 x 4 patches: no more rounds of tiles than the tile count itself needs on the benchmark launches
     const long want[3][2] = {{296, 20}, {296, 60}, {296, 54}};
     for (auto& w : want) bad += daxq::banded_grid((int)w[0], (int)w[1], 4) != (w[0] * w[1] + 255) / 256 * 256;
+    // depth of the fitted tiles' row groups: single rows where the rule's optimum lies below one, and nowhere more than 1.3 times the cost
+    // of the best depth (the rule looks at even groups only)
+    const int tiles[11][2] = {{64, 64}, {64, 96}, {64, 128}, {64, 192}, {128, 96}, {128, 160}, {128, 224}, {192, 192}, {256, 96}, {256, 128}, {256, 160}};
+    for (auto& w : tiles)
+        for (int tiles_m = 1; tiles_m <= 320; ++tiles_m)
+            for (int tiles_n = 1; tiles_m * tiles_n <= 512; ++tiles_n, ++grids) {
+                const int depth = daxq::group_depth(w[0], w[1], tiles_m, tiles_n);
+                float best = daxq::groups_cost(w[0], w[1], tiles_m, tiles_n, 1);
+                for (int d = 2; d <= tiles_m; ++d) {
+                    const float cost = daxq::groups_cost(w[0], w[1], tiles_m, tiles_n, d);
+                    best = cost < best ? cost : best;
+                }
+                bad += depth < 1 || depth > tiles_m || daxq::groups_cost(w[0], w[1], tiles_m, tiles_n, depth) > 1.3f * best;
+            }
+    bad += daxq::group_depth(64, 64, 5, 3) != 1 || daxq::group_depth(64, 64, 9, 2) != 1 || daxq::group_depth(128, 96, 4, 54) != 2;
     std::printf("%ld tile grids checked, %ld errors\n", grids, bad);
     return bad ? 1 : 0;
 }
