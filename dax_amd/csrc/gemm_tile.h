@@ -243,6 +243,11 @@ __device__ __forceinline__ void outputs_lines(const GemmArgs& p, typename Acc16<
     store_group();
 }
 
+// LDS bytes of the epilogue below: scales and bias of the tile, then (LINES) a part per wavefront
+constexpr int epilogue16_scales(int nbj, int nbi) { return (32 * nbi + 2 * 32 * nbj) * 4; }
+constexpr int epilogue16_part(int nbj, int nbi) { return 16 * nbi * (32 * nbj + 16); }
+constexpr int epilogue16_lds(int nbj, int nbi, bool lines) { return epilogue16_scales(nbj, nbi) + (lines ? 4 * epilogue16_part(nbj, nbi) : 0); }
+
 // The epilogue of kernels that have no registers for the scales beside their main loop: a thread has requested one of each, and they
 // pass through the LDS, which it begins to write at once: a barrier lies between the workgroup's last fragment read and this call (in
 // the pipelined loops the one in front of the last pair's MFMAs).
@@ -282,7 +287,7 @@ __device__ __forceinline__ void tile_epilogue16(const GemmArgs& p, typename Acc1
     if constexpr (OUTK == DAXQ_F32) {
         outputs_f32<NBJ, NBI, FP8>(p, acc, mw, nw, l15, g4, sx, sw, bias);
     } else if constexpr (LINES) {
-        uint8_t* const own = smem + (BM + 2 * BN) * 4 + (t >> 6) * (WTM * (2 * WTN + 16));
+        uint8_t* const own = smem + epilogue16_scales(NBJ, NBI) + (t >> 6) * epilogue16_part(NBJ, NBI);
         outputs_lines<NBJ, NBI, FP8, OUTK, ALWAYS_THROUGH>(p, acc, own, mw, nw, t & 63, sx, sw, bias);
     } else {
         outputs_straight<NBJ, NBI, FP8, OUTK>(p, acc, mw, nw, l15, g4, sx, sw, bias);

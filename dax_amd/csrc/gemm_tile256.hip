@@ -155,6 +155,7 @@ __device__ __forceinline__ void gemm_tile256s5_body(const GemmArgs& p, const int
     constexpr int NB = WT / (N16 ? 16 : 32);          // MFMA blocks per operand and wavefront: 8 / 4 (16x16, 256 / 128 tile), 2 (32x32)
     constexpr int PART = BT * BKP;                    // one operand of one pair
     constexpr int PAIR_LOADS = BT / 16;               // DMA loads per thread and pair of slices
+    static_assert(!N16 || epilogue16_lds(NB, NB, LINES || BT == 128) <= NPART * PART, "the epilogue fits into the LDS of the parts");
     constexpr int NREG = NB * NB;                     // MFMAs = scheduling regions per slice
     constexpr int DMA_EVERY = NREG / (PAIR_LOADS / 2);     // regions per DMA load
     constexpr int READ_EVERY = NREG >= 48 ? 3 : NREG / (2 * NB);  // regions per fragment read (2 * NB reads)
@@ -536,7 +537,6 @@ int launch_tile128_splitk(const GemmArgs& a0, int f8, hipStream_t st) {
     GemmArgs a = a0;
     a.tiles_m = (a.m + 127) / 128;
     a.tiles_n = (a.n + 127) / 128;
-    a.lines = lines_of(a);
     if constexpr (FP8) {
         switch (f8) {
             case 1: return launch_splitk_impl<true, 1>(a, st);
@@ -666,7 +666,6 @@ int launch_halves_i8(const GemmArgs& a0, hipStream_t st) {
     a.tiles_m = (a.m + 255) / 256;
     a.tiles_n = (a.n + 255) / 256;
     a.order = kOrderRowGroups;
-    a.lines = lines_of(a);
     const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
     if (tiles > 0x3fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
     return launch_then_halves(a, 0, (int)tiles, st);
@@ -678,8 +677,8 @@ int launch_tile_i8(const GemmArgs& a0, bool small, int tail, hipStream_t st) {
     a.tiles_m = (a.m + bt - 1) / bt;
     a.tiles_n = (a.n + bt - 1) / bt;
     a.grid = a.quad_base = 0;
-    a.lines = lines_of(a);
     if (small) a.order = kOrderRowGroups;
+    else a.lines = lines_of(a);
     const int left = small ? 0 : tail_tiles(a, tail);
     if (left == 0) {
         const int halves = small ? 0 : tail_half_tiles(a, tail);

@@ -35,6 +35,8 @@ struct FitTile {
     static_assert(GROUPS * GROUP_ROWS * OUT_ROW <= SMEM, "the outputs fit into the LDS of the pairs");
     static_assert(BM % ROWS == 0 && BN % ROWS == 0, "whole load instructions");
     static_assert(NS >= 3 && SMEM <= 160 * 1024 && NS * PAIR_LOADS < 60, "LDS and load counter");
+    static constexpr int SCALE_LOADS = NBI + 2 * NBJ;  // of the epilogue's scales and bias, behind the last tile loads
+    static_assert((NS - 2) * PAIR_LOADS + SCALE_LOADS < 64, "the waits of the last pairs fit the load counter");
 };
 typedef FitTile<2, 2, 8, 4, 3> HalfTile;  // 256 x 128
 
@@ -171,7 +173,7 @@ __device__ __forceinline__ void gemm_fit_body(const GemmArgs& p, const int m0, c
 
     // the epilogue's scales and bias, requested behind the last tile loads, each lane its own outputs': always NBI + 2 NBJ loads (a missing
     // bias reads a scale instead and is replaced by -0.0: x + (-0.0) == x bit for bit), so that the counts of the waits hold
-    constexpr int SCALE_LOADS = NBI + 2 * NBJ;
+    constexpr int SCALE_LOADS = TILE::SCALE_LOADS;
     typedef v4f loose_v4f __attribute__((aligned(4)));
     typedef v2u loose_v2u __attribute__((aligned(2)));
     const int mw = m0 + wm * 16 * NBI, nw = n0 + wn * 16 * NBJ;

@@ -51,6 +51,7 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
     constexpr int WT = BT / 2;              // edge of a wavefront's outputs
     constexpr int PART = BT * BKP;          // one operand of one pair: 32 / 16 KB
     constexpr int LPO = BT / 32;            // DMA loads per thread, operand and pair
+    static_assert(epilogue16_lds(NB, NB, LINES || BT == 128) <= NPART * PART, "the epilogue fits into the LDS of the parts");
     constexpr int NREG = NB * NB;           // MFMAs = scheduling regions per pair
     constexpr int HREG = NREG / 2;          // ... per half
     constexpr int DMA_EVERY = HREG / LPO;   // regions per DMA load: 4 / 2
@@ -466,7 +467,6 @@ int launch_halves_fp8(const GemmArgs& a0, int f8, hipStream_t st) {
     a.tiles_m = (a.m + 255) / 256;
     a.tiles_n = (a.n + 255) / 256;
     a.order = kOrderRowGroups;
-    a.lines = lines_of(a);
     const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
     if (tiles > 0x3fffffff) return fail(DAXQ_ERR_ARG, "gemm: too many tiles");
     return launch_fp8_then<false>(a, f8, 0, (int)tiles, st);
@@ -481,11 +481,11 @@ int launch_tile_fp8(const GemmArgs& a0, int f8, bool small, int tail, hipStream_
     a.tiles_m = (a.m + bt - 1) / bt;
     a.tiles_n = (a.n + bt - 1) / bt;
     a.grid = a.quad_base = 0;
-    a.lines = lines_of(a);
     if (small) {
         a.order = kOrderRowGroups;
         return launch_fp8_one<128>(a, f8, st);
     }
+    a.lines = lines_of(a);
     const int left = tail_tiles(a, tail);
     if (left == 0) {
         // more than a quarter and at most half of the CUs' worth of tiles left over: their 256x128 halves with a CU each
