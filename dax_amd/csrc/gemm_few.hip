@@ -352,20 +352,20 @@ static bool few_forms(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int sche
     return k >= 8 && k % 8 == 0 && k <= kFewMaxK && n >= (f8 ? 128 : 1) && n <= (1 << 20);
 }
 
-// a call that its entry point takes
-static int few_linear(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme, int act_scale_round, const void* x, int64_t ld_x,
+// a call that the entry point `what` takes
+static int few_linear(const char* what, int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme, int act_scale_round, const void* x, int64_t ld_x,
                       const float* in_scale, const void* wq, int64_t ld_wq, const float* sw, const void* bias, void* out, int64_t ld_out,
                       int64_t m, int64_t n, int64_t k, daxq_stream_t stream) {
     const int64_t kp = (k + DAXQ_K_ALIGN - 1) / DAXQ_K_ALIGN * DAXQ_K_ALIGN;
-    if ((scheme == kFewStatic) != (in_scale != nullptr)) return fail(DAXQ_ERR_ARG, "linear_few: scheme %d takes in_scale: %d", scheme, scheme == kFewStatic);
+    if ((scheme == kFewStatic) != (in_scale != nullptr)) return fail(DAXQ_ERR_ARG, "%s: scheme %d takes in_scale: %d", what, scheme, scheme == kFewStatic);
     if (act_scale_round != DAXQ_SCALE_ROUND_X && act_scale_round != DAXQ_SCALE_ROUND_NONE)
-        return fail(DAXQ_ERR_ARG, "linear_few: unknown scale rounding %d", act_scale_round);
-    if (!x || !wq || !sw || !out) return fail(DAXQ_ERR_ARG, "linear_few: null pointer");
-    if (ld_x < k || ld_wq < kp || ld_out < n || ld_wq >= (1 << 26)) return fail(DAXQ_ERR_ARG, "linear_few: bad leading dimension");
+        return fail(DAXQ_ERR_ARG, "%s: unknown scale rounding %d", what, act_scale_round);
+    if (!x || !wq || !sw || !out) return fail(DAXQ_ERR_ARG, "%s: null pointer", what);
+    if (ld_x < k || ld_wq < kp || ld_out < n || ld_wq >= (1 << 26)) return fail(DAXQ_ERR_ARG, "%s: bad leading dimension", what);
     const uintptr_t xa = x_dtype == DAXQ_F32 ? 3 : 1;
     if (((uintptr_t)x & xa) || ((uintptr_t)out & xa) || ((uintptr_t)bias & xa) || ((uintptr_t)sw & 3) || ((uintptr_t)in_scale & 3) ||
         ((uintptr_t)wq & 15) || (ld_wq & 15))
-        return fail(DAXQ_ERR_ALIGN, "linear_few: misaligned pointer or weight rows");
+        return fail(DAXQ_ERR_ALIGN, "%s: misaligned pointer or weight rows", what);
     FewArgs a = {};
     a.g.b = static_cast<const uint8_t*>(wq);
     a.g.sw = sw;
@@ -438,7 +438,7 @@ int daxq_linear_few(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme
     if (m == 0 || n == 0) return DAXQ_OK;
     if (!daxq_linear_few_applies(x_dtype, x_fmt, w_fmt, out_dtype, scheme, act_scale_round, m, n, k))
         return fail(DAXQ_ERR_ARG, "linear_few: does not take m=%lld n=%lld k=%lld in these formats", (long long)m, (long long)n, (long long)k);
-    return few_linear(x_dtype, x_fmt, w_fmt, out_dtype, scheme, act_scale_round, x, ld_x, in_scale, wq, ld_wq, sw, bias, out, ld_out, m, n, k, stream);
+    return few_linear("linear_few", x_dtype, x_fmt, w_fmt, out_dtype, scheme, act_scale_round, x, ld_x, in_scale, wq, ld_wq, sw, bias, out, ld_out, m, n, k, stream);
 }
 
 int daxq_linear_short_rows_applies(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int scheme, int act_scale_round, int64_t m, int64_t n, int64_t k) {
@@ -455,7 +455,7 @@ int daxq_linear_short_rows(int x_dtype, int x_fmt, int w_fmt, int out_dtype, int
     if (m == 0 || n == 0) return DAXQ_OK;
     if (!daxq_linear_short_rows_applies(x_dtype, x_fmt, w_fmt, out_dtype, scheme, act_scale_round, m, n, k))
         return fail(DAXQ_ERR_ARG, "linear_short_rows: does not take m=%lld n=%lld k=%lld in these formats", (long long)m, (long long)n, (long long)k);
-    return few_linear(x_dtype, x_fmt, w_fmt, out_dtype, scheme, act_scale_round, x, ld_x, in_scale, wq, ld_wq, sw, bias, out, ld_out, m, n, k, stream);
+    return few_linear("linear_short_rows", x_dtype, x_fmt, w_fmt, out_dtype, scheme, act_scale_round, x, ld_x, in_scale, wq, ld_wq, sw, bias, out, ld_out, m, n, k, stream);
 }
 
 }  // extern "C"

@@ -160,6 +160,21 @@ def test_quantisers_refuse_a_quant_max_that_is_not_positive():
     assert lib.daxq_act_quant_tensor(None, 0, 0, 0, 8, 8, None, 8, None, None, None, 127.0, 0.0, 1, None) == 0
 
 
+def test_forwards_in_one_launch_report_errors_under_their_own_names():
+    """daxq_linear_few and daxq_linear_short_rows share their checks, which run before anything is launched."""
+    from dax_amd import _capi
+
+    lib = _capi.lib()
+    for name, m in (("linear_few", 4), ("linear_short_rows", 16)):
+        def call(scheme=0, rounding=1, in_scale=None, p=None, ld_x=512, k=512):
+            return getattr(lib, "daxq_" + name)(0, 0, 0, 0, scheme, rounding, p, ld_x, in_scale, p, 512, p, None, p, 1536, m, 1536, k, None)
+
+        for args, said in (({}, "null pointer"), ({"scheme": 2}, "in_scale"), ({"rounding": 7}, "rounding"), ({"k": 1 << 20}, "does not take"),
+                           ({"p": 4096, "ld_x": 8}, "leading dimension"), ({"p": 4098}, "misaligned")):
+            assert call(**args) < 0
+            assert _capi.last_error().startswith(name + ": ") and said in _capi.last_error(), _capi.last_error()
+
+
 def test_no_cpu_kernels_and_clear_errors():
     import dax_amd.ops as ops
 
