@@ -24,18 +24,19 @@ def _operands(m, n, k, fp8, dtype, seed):
     return xq, wq, sx, sw, torch.randn(n, generator=g).to(dtype)
 
 
-def _launch(xq, wq, sx, sw, b, fp8, out, kernel):
-    """rows behind xq / out's own and columns behind them are checked for writes"""
+def _launch(xq, wq, sx, sw, b, fp8, out, kernel, distance=None, e5m2=False):
+    """rows behind xq / out's own and columns behind them are checked for writes; distance: elements from one row of outputs to the next"""
     from dax_amd import _capi
 
     kind, dtype = OUT[out]
     m, k = xq.shape
     n = wq.shape[0]
     d = [t.to("cuda") for t in (xq, wq, sx, sw, b)]
-    o = torch.full((m + 1, n + 8), 7.0, dtype=dtype, device="cuda")
+    distance = distance or n + 8
+    o = torch.full((m + 1, distance), 7.0, dtype=dtype, device="cuda")
     f = 1 if fp8 else 0
-    rc = _capi.lib().daxq_linear_w8a8(f, f, kind, d[0].data_ptr(), k, d[2].data_ptr(), d[1].data_ptr(), k, d[3].data_ptr(), d[4].data_ptr(),
-                                      o.data_ptr(), n + 8, None, 0, m, n, k, kernel, torch.cuda.current_stream().cuda_stream)
+    rc = _capi.lib().daxq_linear_w8a8(2 if e5m2 else f, f, kind, d[0].data_ptr(), k, d[2].data_ptr(), d[1].data_ptr(), k, d[3].data_ptr(), d[4].data_ptr(),
+                                      o.data_ptr(), distance, None, 0, m, n, k, kernel, torch.cuda.current_stream().cuda_stream)
     _capi.check(rc, "linear")
     torch.cuda.synchronize()
     assert bool((o[m:] == 7.0).all()) and bool((o[:, n:] == 7.0).all())
@@ -120,14 +121,20 @@ def test_fp16_sums_of_every_rounded_product():
 
 
 @pytest.mark.parametrize("out", ["bf16", "fp16"])
-@pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("n", [4088, 4089, 4092])  # rows of outputs 8192 bytes apart, an odd number of elements, neither
+@pytest.mark.parametrize("fmt", ["int8", "e4m3", "e5m2"])
+@pytest.mark.parametrize("k", [384, 640])  # FP8 tiles pipeline from four pairs on
+@pytest.mark.parametrize("n", [4088, 4089])
 @pytest.mark.parametrize("m", [300, 4300, 5300])  # whole tiles, a last round of quadrants, of halves
-def test_ways_of_the_outputs_of_whole_tiles(m, n, fp8, out):
-    """256x256 tiles store whole rows through the L2, whole rows, or straight from the registers, by the distance of the rows."""
-    xq, wq, sx, sw, b = _operands(m, n, 384, fp8, OUT[out][1], m + n)
-    got, want = (_launch(xq, wq, sx, sw, b, fp8, out, kernel) for kernel in (8, 11 if fp8 else 5))
-    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+def test_ways_of_the_outputs_of_whole_tiles(m, n, k, fmt, out):
+    """256x256 tiles store whole rows through the L2 (rows 8256 bytes apart), whole rows (an odd number of elements), or straight from the
+    registers (8200 bytes), by the distance of the rows; the same operands all three ways, and in 128x128 tiles."""
+    fp8, e5m2 = fmt != "int8", fmt == "e5m2"
+    xq, wq, sx, sw, b = _operands(m, n, k, fp8, OUT[out][1], m + n)
+    if e5m2:
+        xq = xq.view(torch.float8_e4m3fn).float().to(torch.float8_e5m2).view(torch.uint8)
+    want = _launch(xq, wq, sx, sw, b, fp8, out, 11 if fp8 else 5, e5m2=e5m2).view(torch.int16)
+    for distance in (4100, 4101, 4128):
+        assert torch.equal(_launch(xq, wq, sx, sw, b, fp8, out, 8, distance, e5m2).view(torch.int16), want), distance
 
 
 @pytest.mark.parametrize("k", [128, 256, 384])
