@@ -309,7 +309,6 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
         // as above, so the sums are the same bits as the pipelined path would give.
         request_scales();
         for (int q = 0; q < Q; ++q) {
-            if (q) __builtin_amdgcn_s_barrier();  // every wavefront has read pair q-1 out of the two parts
 #pragma unroll
             for (int g = 0; g < LPO; ++g) issue_a(r1, g);
 #pragma unroll
@@ -324,6 +323,7 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
 #pragma unroll
             for (int i = 0; i < NB; ++i) read_into(fa0[i], false, r1, i);
             __builtin_amdgcn_s_waitcnt(lgkmcnt0_mask() & vmcnt_imm(63));
+            __builtin_amdgcn_s_barrier();  // every wavefront has read pair q out of the two parts, which the next pair or the epilogue overwrites
             __builtin_amdgcn_sched_barrier(0);
             if (q == 0) {
 #pragma unroll
@@ -334,7 +334,6 @@ __device__ __forceinline__ void gemm_tile_fp8_body(const GemmArgs& p, const int 
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();  // (the epilogue writes where other wavefronts may still read pair Q-1's fragments)
         mfma_settle();
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     }
