@@ -1,16 +1,16 @@
-// The whole forward of a W8A8 linear of at most eight rows (or up to 64 short ones) in one launch: every workgroup quantises the activation for itself, in
-// LDS, while its share of the weight arrives, and multiplies (gfx950).
+// The whole forward of a W8A8 linear of at most eight rows (or up to 64 short ones) in one launch: every workgroup quantises the activation
+// for itself, in LDS, while its share of the weight arrives, and multiplies (gfx950).
 //
 // What bounds it: the launches.  The quantiser and the GEMM of such a call take 2 and 3 to 7 us, their launches cost the host 2.8 to
 // 3.6 us each (a per-tensor scale is a third one), and the second one starts when the first has ended and drained.  The quantised rows
-// are few (m x K <= 40 KB), so that quantising them once per workgroup costs about what waiting for the weight does anyway.
+// are few (40 KB up to eight rows, 64 KB beyond), so that quantising them once per workgroup costs about what waiting for the weight does anyway.
 // Forwards back to back, us, separate launches -> this: 1 x 1536 x 1536 8.2 -> 5.5, 4 x 1536 x 1536 e5m2 under a per-tensor scale
 // 10.9 -> 5.7, 1 x 5120 x 5120 e4m3 8.2 -> 7.9 (its kernel).
 //
 // Work decomposition
 //   workgroup  8 wavefronts, two groups (CG) of 16 output columns
-//   quantiser  the wavefronts are dealt to the rows (more than eight: each takes several); all of the activation is in flight at once, maxima meet in LDS once, and the
-//              bytes go to LDS rows of K + 16 bytes (the rows a fragment read touches then lie in different banks)
+//   quantiser  the wavefronts are dealt to the rows (more than eight: each takes several); all of the activation is in flight at once,
+//              maxima meet in LDS once, and the bytes go to LDS rows of K + 16 bytes (the rows a fragment read touches then lie in different banks)
 //   GEMM       as gemm_rows.hip: wavefront w < CG x KS streams K / KS bytes of 16 weight rows through an LDS ring of its own, the
 //              first R steps of 128 bytes requested behind the activation's loads and in front of the quantiser's arithmetic.  INT8 cuts
 //              K over KS = 4 wavefronts (sums of integers); FP8 runs KS = 1, so that an output element is the sequence of MFMAs over
@@ -318,7 +318,10 @@ int prepare_few_kernels() {
 // K and the number of rows draw the line (the quantiser's arithmetic: FP8 elements take more of it than int8 ones, fp32 ones more
 // loads), up to N = 8192, where a workgroup has a CU to itself; beyond, two share one and quantise one after the other.  A tensor's scale
 // saves a third launch or the second reading of the matrix.  us per call on the GPU, separate launches / one; weights near, out of reach
-// of the caches (forwards back to back besides save the 3 us that the host takes for a launch and its buffers):
+// of the caches.  The lines are drawn for forwards back to back, which besides save the 3.6 us that the host takes for a launch and its
+// buffers (every size here 10.5 / 6.9), and for weights out of reach, a model's: what loses is FP8 of 17 to 32 rows beyond K = 512 and
+// 16 rows at K = 2048 in a graph that replays one weight, up to 0.9 us (32 x 5120, K = 512 e4m3 4.6 / 4.4; 6.0 / 5.2, K = 640 4.8 / 5.6; 6.6 / 6.2;
+// 17 rows, K = 768 4.7 / 5.1; 6.5 / 5.8).
 //   own scales        16 x 1536 x 1536 int8 5.1 / 4.7; 7.1 / 5.0    e4m3 5.4 / 5.3; 7.2 / 5.3         16 x 8192, K = 2048 int8 6.2 / 5.7; 8.0 / 7.5   e4m3 6.0 / 6.2; 8.0 / 7.4
 //                     16 x 4096, K = 2560 int8 6.3 / 5.8; 7.2 / 7.5  e4m3 6.2 / 7.0; 7.1 / 7.5         16 x 1536, K = 2048 fp32 5.4 / 5.8; 6.9 / 6.2   K = 1536 5.2 / 5.1; 6.8 / 5.3
 //                     32 x 1536, K = 512 int8 5.0 / 4.4; 6.9 / 4.6   e4m3 5.2 / 4.9; 6.7 / 4.9         32 x 5120, K = 1024 int8 5.3 / 5.4; 6.5 / 6.3   e4m3 5.3 / 6.3; 7.1 / 6.6

@@ -249,8 +249,8 @@ constexpr int epilogue16_part(int nbj, int nbi) { return 16 * nbi * (32 * nbj + 
 constexpr int epilogue16_lds(int nbj, int nbi, bool lines) { return epilogue16_scales(nbj, nbi) + (lines ? 4 * epilogue16_part(nbj, nbi) : 0); }
 
 // The epilogue of kernels that have no registers for the scales beside their main loop: a thread has requested one of each, and they
-// pass through the LDS, which it begins to write at once: a barrier lies between the workgroup's last fragment read and this call (in
-// the pipelined loops the one in front of the last pair's MFMAs).
+// pass through the LDS, which it begins to write at once: a barrier lies between the workgroup's last fragment read and this call (the one
+// in front of the last MFMAs).
 // OUTK: element type of out and bias, DAXQ_BF16 / DAXQ_F16 / DAXQ_F32.  A template argument, i.e. a kernel
 // of its own per type: with all three forms inside one kernel behind uniform branches its code grew from 27 to 44 KB
 // and the bf16 launches at K = 1536, which change between main loop and epilogue every 24 slices, lost 2.7 %; with

@@ -22,7 +22,11 @@ constexpr int64_t kKeepBytes = (int64_t)128 << 20;
 //   134 x 3472, K = 5120 (0.65 MB) 12.5 / 12.5    17 x 5120 x 5120 e4m3 (0.1) 9.05 / 9.22    64 x 5120 x 5120 (0.3) 12.1 / 12.4
 //   512 x 5120 x 5120 (2.5) 22.3 / 22.0    2900 x 3080, K = 1000 (2.8) 19.7 / 19.4    313 x 4608, K = 13824 (4.1) 31.9 / 31.3
 //   1024 x 5120 x 5120 e4m3 (5) 29.8 / 29.2    1230 x 2712, K = 5120 (6) 26.5 / 25.8    887 x 5120, K = 8960 e4m3 (7.6) 40.9 / 40.3
-//   2225 x 5120, K = 4608 (9.8) 51.1 / 51.3    1003 x 4608, K = 13824 (13) 60.5 / 61.0    2358 x 5120, K = 8960 (20) 92.7 / 93.0
+// 8 to 32 MB, medians of eleven turns that differ by 0.5 to 3 %, INT8; e4m3: shapes go either way, and the losses are the larger ones
+//   1500 x 5120, K = 13824 (21) 91.4 / 94.1; 89.0 / 92.2    1003 x 4608, K = 13824 (14) 62.0 / 63.2; 60.7 / 62.4    600 x 5120, K = 15360 (9) 58.2 / 58.7; 57.9 / 58.5
+//   3200 x 1536, K = 8960 (29) 54.0 / 54.6; 53.0 / 55.1    8000 x 5120, K = 1536 (12) 71.1 / 72.4; 70.5 / 71.6    1800 x 5120 x 5120 (9) 47.4 / 47.9; 46.6 / 46.7
+//   2225 x 5120, K = 4608 (10) 52.4 / 52.2; 51.5 / 50.9    16000 x 4608, K = 1536 (25) 117.8 / 116.6; 117.3 / 116.9    4725 x 5120 x 5120 (24) 107.6 / 107.2; 105.7 / 104.0
+// from 32 MB on
 //   4071 x 5120, K = 13824 (54) 216.7 / 216.2  13198 x 1536, K = 5120 (64) 111.8 / 109.2   16034 x 5120, K = 5160 e4m3 (80) 320 / 312
 // and past the caches / through, beyond kKeepBytes, up to the Infinity Cache's 256 MB:
 //   27000 x 512, K = 5120 (138) 122.0 / 113.6    30000 x 1536, K = 5120 (154) 246.7 / 236.8    20000 x 5120, K = 8960 e4m3 (179) 697 / 688
