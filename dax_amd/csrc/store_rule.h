@@ -22,6 +22,9 @@ constexpr int64_t kKeepBytes = (int64_t)128 << 20;
 //   134 x 3472, K = 5120 (0.65 MB) 12.5 / 12.5    17 x 5120 x 5120 e4m3 (0.1) 9.05 / 9.22    64 x 5120 x 5120 (0.3) 12.1 / 12.4
 //   512 x 5120 x 5120 (2.5) 22.3 / 22.0    2900 x 3080, K = 1000 (2.8) 19.7 / 19.4    313 x 4608, K = 13824 (4.1) 31.9 / 31.3
 //   1024 x 5120 x 5120 e4m3 (5) 29.8 / 29.2    1230 x 2712, K = 5120 (6) 26.5 / 25.8    887 x 5120, K = 8960 e4m3 (7.6) 40.9 / 40.3
+// ... in front of GEMMs against a hundred columns either way, by what the quantiser does not know (1 to 8 MB, bf16; fp32):
+//   865 x 133, K = 2909 11.8 / 11.9; 12.6 / 12.3    1500 x 133, K = 5120 20.9 / 22.0; 23.7 / 22.8    2000 x 133, K = 1001 7.5 / 7.9; 7.7 / 8.0
+//   2500 x 133, K = 2909 15.8 / 14.8; 18.2 / 16.7   600 x 133, K = 5120 13.1 / 12.9; 14.4 / 13.9     4000 x 100, K = 800 13.2 / 13.0; 14.8 / 14.4
 // 8 to 32 MB, medians of eleven turns that differ by 0.5 to 3 %, INT8; e4m3: shapes go either way, and the losses are the larger ones
 //   1500 x 5120, K = 13824 (21) 91.4 / 94.1; 89.0 / 92.2    1003 x 4608, K = 13824 (14) 62.0 / 63.2; 60.7 / 62.4    600 x 5120, K = 15360 (9) 58.2 / 58.7; 57.9 / 58.5
 //   3200 x 1536, K = 8960 (29) 54.0 / 54.6; 53.0 / 55.1    8000 x 5120, K = 1536 (12) 71.1 / 72.4; 70.5 / 71.6    1800 x 5120 x 5120 (9) 47.4 / 47.9; 46.6 / 46.7
